@@ -875,8 +875,8 @@ bool numeric(const std::vector<int>& ptr, const std::vector<int>& adj, const std
 
 // The device numeric factorization run on the host, step for step as the kernels run it
 // (one height at a time; per supernode: zeroed workspace, original entries, children's update
-// matrices in child order, left-looking Cholesky of the pivot block, its inverse, D^{-1},
-// G = F_os D^{-1}, the update matrix), with every index checked against its block. Leaves the
+// matrices in child order, D^{-1} by block sweeps of the pivot block, G = F_os D^{-1}, the update
+// matrix), with every index checked against its block. Leaves the
 // FP64 panels in f.panel.
 bool numeric_device_emulation(const std::vector<int>& ptr, const std::vector<int>& adj,
                               const std::vector<double>& val, const std::vector<double>& diag, Factor& f,
@@ -898,19 +898,23 @@ bool numeric_device_emulation(const std::vector<int>& ptr, const std::vector<int
             const int64_t po = f.poff[t], so = f.woff_s[t], to = f.woff_t[t], uo = f.woff_u[t];
             auto Pp = [&](int r, int c) -> double& { return P[po + (int64_t)c * m + r]; };
             auto Sp = [&](int r, int c) -> double& { return S[so + (int64_t)c * no + r]; };
-            auto Tp = [&](int r, int c) -> double& { return T[to + (int64_t)r * w + c]; };  // row-major
+            auto Tp = [&](int r, int c) -> double& { return T[to + (int64_t)c * w + r]; };
+            constexpr int kFb = 64;
+            const int nb = (w + kFb - 1) / kFb;
+            // the pivot block before sweep step s: in T or P, such that the last step leaves it in P
+            auto Dp = [&](int s, int r, int c) -> double& { return (nb - s) & 1 ? Tp(r, c) : Pp(r, c); };
             auto Up = [&](int r, int c) -> double& { return U[uo + (int64_t)c * no + r]; };
             const int* rows = f.offrows.data() + f.roff[t];
             // original entries, one column at a time
             for (int k = 0; k < w; ++k) {
                 const int j = c0 + k;
                 MD_FCHECK(f.col_sn[j] == t, "column owner");
-                Pp(k, k) = diag[j];
+                Dp(0, k, k) = diag[j];
                 for (int e = ptr[j]; e < ptr[j + 1]; ++e) {
                     const int i = adj[e];
                     if (i <= j) continue;
                     if (i < c0 + w) {
-                        Pp(i - c0, k) += val[e];
+                        Dp(0, i - c0, k) += val[e];
                     } else {
                         const int r = (int)(std::lower_bound(rows, rows + no, i) - rows);
                         MD_FCHECK(r < no && rows[r] == i, "off row of an original entry");
@@ -929,85 +933,63 @@ bool numeric_device_emulation(const std::vector<int>& ptr, const std::vector<int
                     const int ra = rel[a], rb = rel[b];
                     MD_FCHECK(ra >= rb && ra < m && rb >= 0, "update position");
                     if (rb < w) {
-                        if (ra < w) Pp(ra, rb) += v;
+                        if (ra < w) Dp(0, ra, rb) += v;
                         else Sp(ra - w, rb) += v;
                     } else {
                         Up(ra - w, rb - w) += v;
                     }
                 }
             }
-            // Cholesky factor and its inverse X of the pivot block, blocked by 64 columns
-            // (right-looking), in the device's workspaces; the device orders the work within a
-            // front differently (an unscaled LDL^T chain per block, the X blocks inside the
-            // right-looking loop, products split over K), so the two agree to rounding.
-            constexpr int kFb = 64;
-            const int nb = (w + kFb - 1) / kFb;
+            // the pivot block by symmetric block sweeps, 64 columns at a time, from one workspace to
+            // the other (the device inverts a block as soon as it is complete, and sweeps it by 16
+            // and 4 columns; here by single columns: the two agree to rounding)
             for (int s = 0; s < nb; ++s) {
                 const int kb = s * kFb, b = std::min(kFb, w - kb);
-                // diagonal block: unblocked Cholesky, then its inverse (row-major, upper part zero)
+                std::vector<double> Sv((size_t)b * b), W((size_t)w * b), As((size_t)w * b);
+                for (int r = 0; r < b; ++r)
+                    for (int c = 0; c <= r; ++c) Sv[(size_t)r * b + c] = Sv[(size_t)c * b + r] = Dp(s, kb + r, kb + c);
                 for (int k = 0; k < b; ++k) {
-                    const double d0 = Pp(kb + k, kb + k);
-                    if (!(d0 > 1e-14 * amax)) {
+                    const double d = Sv[(size_t)k * b + k];
+                    if (!(d > 1e-14 * amax)) {
                         err = "factorization failed: pivot block of supernode " + std::to_string(t) +
                               " is not positive definite (a mesh component without constraints?)";
                         return false;
                     }
-                    const double d = std::sqrt(d0);
-                    for (int r = k + 1; r < b; ++r) Pp(kb + r, kb + k) /= d;
-                    Pp(kb + k, kb + k) = d;
-                    for (int c = k + 1; c < b; ++c)
-                        for (int r = c; r < b; ++r) Pp(kb + r, kb + c) -= Pp(kb + r, kb + k) * Pp(kb + c, kb + k);
+                    for (int r = 0; r < b; ++r)
+                        for (int c = 0; c < b; ++c)
+                            if (r != k && c != k) Sv[(size_t)r * b + c] -= Sv[(size_t)r * b + k] * Sv[(size_t)k * b + c] / d;
+                    for (int r = 0; r < b; ++r)
+                        if (r != k) Sv[(size_t)r * b + k] = Sv[(size_t)k * b + r] = Sv[(size_t)r * b + k] / d;
+                    Sv[(size_t)k * b + k] = -1.0 / d;
                 }
-                for (int r = 0; r < b; ++r)
-                    for (int c = 0; c < b; ++c) Tp(kb + r, kb + c) = r == c ? 1.0 : 0.0;
-                for (int k = 0; k < b; ++k) {
-                    const double lkk = Pp(kb + k, kb + k);
-                    for (int c = 0; c <= k; ++c) Tp(kb + k, kb + c) = c == k ? 1.0 / lkk : Tp(kb + k, kb + c) / lkk;
-                    for (int r = k + 1; r < b; ++r)
-                        for (int c = 0; c <= k; ++c) Tp(kb + r, kb + c) -= Pp(kb + r, kb + k) * Tp(kb + k, kb + c);
-                }
-                if (s == nb - 1) break;
-                // rows below: forward substitution against the diagonal block
-                for (int r = kb + kFb; r < w; ++r)
-                    for (int j = 0; j < kFb; ++j) {
-                        double v = Pp(r, kb + j);
-                        for (int q = 0; q < j; ++q) v -= Pp(r, kb + q) * Pp(kb + j, kb + q);
-                        Pp(r, kb + j) = v / Pp(kb + j, kb + j);
-                    }
-                // trailing lower part: A(r, c) -= sum_q L(r, kb + q) L(c, kb + q)
-                for (int c = kb + kFb; c < w; ++c)
-                    for (int r = c; r < w; ++r) {
+                for (double& v : Sv) v = -v;  // A_ss^{-1}
+                for (int r = 0; r < w; ++r)
+                    for (int q = 0; q < b; ++q)
+                        As[(size_t)r * b + q] = r / kFb >= s ? Dp(s, r, kb + q) : Dp(s, kb + q, r);
+                for (int r = 0; r < w; ++r)
+                    for (int q = 0; q < b; ++q) {
                         double acc = 0.0;
-                        for (int q = 0; q < kFb; ++q) acc += Pp(r, kb + q) * Pp(c, kb + q);
-                        Pp(r, c) -= acc;
+                        for (int k = 0; k < b; ++k) acc += As[(size_t)r * b + k] * Sv[(size_t)k * b + q];
+                        W[(size_t)r * b + q] = acc;
+                    }
+                const double sign = s == nb - 1 ? -1.0 : 1.0;  // the last step leaves D^{-1}
+                for (int c = 0; c < w; ++c)
+                    for (int r = c; r < w; ++r) {
+                        const bool rs = r / kFb == s, cs = c / kFb == s;
+                        double v;
+                        if (rs && cs) v = -Sv[(size_t)(r - kb) * b + (c - kb)];
+                        else if (cs) v = W[(size_t)r * b + (c - kb)];
+                        else if (rs) v = W[(size_t)c * b + (r - kb)];
+                        else {
+                            v = Dp(s, r, c);
+                            for (int k = 0; k < b; ++k) v -= W[(size_t)r * b + k] * As[(size_t)c * b + k];
+                        }
+                        Dp(s + 1, r, c) = sign * v;
                     }
             }
-            // off-diagonal blocks of X, one block diagonal at a time:
-            // X_IJ = -X_II sum_{K=J}^{I-1} L_IK X_KJ
-            for (int d = 1; d < nb; ++d)
-                for (int I = d; I < nb; ++I) {
-                    const int J = I - d, r0 = I * kFb, c0 = J * kFb, rb = std::min(kFb, w - r0);
-                    std::vector<double> Y((size_t)kFb * kFb, 0.0);
-                    for (int K = J; K < I; ++K)
-                        for (int k = 0; k < kFb; ++k)
-                            for (int x = 0; x < rb; ++x)
-                                for (int y = 0; y < kFb; ++y)
-                                    Y[(size_t)x * kFb + y] += Pp(r0 + x, K * kFb + k) * Tp(K * kFb + k, c0 + y);
-                    for (int x = 0; x < rb; ++x)
-                        for (int y = 0; y < kFb; ++y) {
-                            double acc = 0.0;
-                            for (int k = 0; k < rb; ++k) acc += Tp(r0 + x, r0 + k) * Y[(size_t)k * kFb + y];
-                            Tp(r0 + x, c0 + y) = -acc;
-                        }
-                }
-            // D^{-1} = Linv^T Linv (symmetric)
-            for (int r = 0; r < w; ++r)
-                for (int c = 0; c <= r; ++c) {
-                    double acc = 0.0;
-                    for (int k = r; k < w; ++k) acc += Tp(k, r) * Tp(k, c);
-                    Pp(r, c) = acc;
-                    Pp(c, r) = acc;
-                }
+            // D^{-1} is symmetric: its upper triangle too
+            for (int c = 0; c < w; ++c)
+                for (int r = c + 1; r < w; ++r) Pp(c, r) = Pp(r, c);
             if (no > 0) {
                 // G = F_os D^{-1} (panel rows [w, m))
                 for (int q = 0; q < w; ++q)

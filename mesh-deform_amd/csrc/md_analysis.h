@@ -110,7 +110,7 @@ struct Factor {
     std::vector<double> panel;       // FP64 panels (host factorization)
     // device numeric factorization (multifrontal, one height at a time): per height the
     // supernodes of that height; per supernode the offsets of its workspace blocks: the
-    // off-diagonal front block (noff x w), the inverse of the pivot block's Cholesky factor
+    // off-diagonal front block (noff x w), the pivot block's second workspace of the sweeps
     // (w x w) and the update matrix for the parent (noff x noff), all column-major FP64
     std::vector<int> hptr, hlist;    // height h: hlist[hptr[h] .. hptr[h+1])
     std::vector<int64_t> woff_s, woff_t, woff_u;  // ns + 1 each

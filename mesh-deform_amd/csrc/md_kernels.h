@@ -96,8 +96,9 @@ struct MeshDev {
 struct FacDev {
     int c0, w, noff, roff;          // columns, off rows (offrows[roff ..], rel[roff ..])
     int cb, ce, m, pad;             // children child[cb .. ce), m = w + noff
-    long long poff, soff, toff, uoff;  // FP64 panel (m x w), F_os copy (noff x w), L^{-1} (w x w),
-                                       // update matrix (noff x noff); all column-major
+    long long poff, soff, toff, uoff;  // FP64 panel (m x w), F_os copy (noff x w), the pivot block's
+                                       // second workspace (w x w), update matrix (noff x noff); all
+                                       // column-major
     long long pc_off, pr_off;       // solve-precision panels of the sweeps
 };
 
@@ -156,9 +157,9 @@ void launch_pcg_init(hipStream_t s, LaunchSet L, int blocks, bool fp64);
 void launch_pcg_step(hipStream_t s, LaunchSet L, int blocks, int step, bool fp64);
 void launch_pcg_apply(hipStream_t s, LaunchSet L, int blocks, bool fp64);
 // Device numeric factorization: diagonal and its maximum, then per height (the `count`
-// supernodes from hlist[h0]) the front assembly and the pivot block's Cholesky and inverse (one
-// workgroup per supernode), D^{-1}, G and the update matrix (one workgroup per output tile, or
-// several split over K); D^{-1} and G also go to the solve-precision panels.
+// supernodes from hlist[h0]) the front assembly, the pivot blocks' inverses, G and the update
+// matrices (one workgroup per output tile, or several split over K); D^{-1} and G also go to the
+// solve-precision panels.
 void launch_fac_diag(hipStream_t s, const FacArgs &A);
 // A product stage of a height: workgroups per supernode (one per 64 x 64 output tile, lower tiles
 // for the symmetric ones; the height's most) and splits over K (1: none); a split stage needs
@@ -166,11 +167,11 @@ void launch_fac_diag(hipStream_t s, const FacArgs &A);
 struct FacSplit {
     int per, ks;
 };
-// One height: assembly (per_asm workgroups per supernode, one per asm_cols front columns), blocked
-// Cholesky and inverse of the pivot blocks (nb = column blocks of 64 in the widest one), D^{-1},
-// G and the update matrices (g.per = 0 when no supernode of the height has off rows).
+// One height: assembly (per_asm workgroups per supernode, one per asm_cols front columns), the
+// pivot blocks' inverses D^{-1} by block sweeps (nb = column blocks of 64 in the widest one), G and
+// the update matrices (g.per = 0 when no supernode of the height has off rows).
 void launch_fac_height(hipStream_t s, const FacArgs &A, int h0, int count, int nb, int asm_cols, int per_asm,
-                       const FacSplit &dinv, const FacSplit &g, const FacSplit &u);
+                       const FacSplit &g, const FacSplit &u);
 // Split of a product over K: `tiles` output tiles of 64 x 64 and `chunks` chunks of K (32 values).
 // Splits only launches of few tiles (tiles x 2 <= kSplitWorkgroups) with at least 8 chunks, into
 // shares of at least 4 chunks, at most kSplitWorkgroups workgroups in all.
@@ -181,11 +182,12 @@ inline int fac_split_k(long long tiles, int chunks) {
     return ks > 1 ? (int)ks : 1;
 }
 constexpr long long fac_split_k_doubles(long long workgroups) { return workgroups * 16 * 256; }
-// A height whose fronts all have m <= mm <= kFacSmallFront and w <= mw: every step of
-// launch_fac_height for one front in one wavefront (front in mm^2 + mm mw doubles of LDS: under
-// 64 KiB), without the FP64 panel workspace.
-constexpr int kFacSmallFront = 62;
-void launch_fac_small(hipStream_t s, const FacArgs &A, int h0, int count, int mm, int mw);
+// A height whose fronts all have m <= mm <= kFacSmallFront: every step of launch_fac_height for one
+// front in one workgroup (of one wavefront on heights of more than kSmallManyFronts fronts, else
+// of four), without the FP64 panel workspace.
+constexpr int kFacSmallFront = 64;
+constexpr int kSmallManyFronts = 1024;
+void launch_fac_small(hipStream_t s, const FacArgs &A, int h0, int count, int mm);
 // Internal-order vectors (positions, normals) to packed xyz in original order (perm: original
 // id per internal id), and packed xyz to internal order (p and/or pp; pp takes the targets tgt,
 // internal order, for the constrained ids [nf, n)).

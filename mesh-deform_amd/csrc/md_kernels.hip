@@ -11,6 +11,7 @@
 
 #include <cmath>
 #include <string>
+#include <type_traits>
 
 namespace md {
 
@@ -1427,6 +1428,22 @@ constexpr int kFacBlock = 256;
 constexpr int kAsmU = 8;      // child update entries per assembly thread in flight
 constexpr int kAsmRows = 2048;  // off rows of a front searched in LDS (longer lists: in memory)
 
+constexpr int kFb = 64;  // columns of a pivot block swept at a time
+
+// A front's pivot block during the sweeps: step s reads one of its two workspaces (P, rows m apart,
+// and T, rows w apart, column-major) and writes the other, so no workgroup overwrites what another
+// still reads; step nb - 1 writes P. Block (s, s) of the workspace that step s reads holds
+// S = A_ss^{-1} (its inverse is formed where the block is completed).
+struct PivotBuf {
+    MD_G double *p;
+    long long ld;
+};
+__device__ __forceinline__ PivotBuf pivot_buf(const FacArgs &A, const FacDev &S, int s) {
+    const int nb = (S.w + kFb - 1) / kFb;
+    if ((nb - s) & 1) return PivotBuf{A.T + S.toff, S.w};
+    return PivotBuf{A.P + S.poff, S.m};
+}
+
 // L_jj = sum of the weights of every neighbour of j, in slot order, and their maximum.
 __global__ __launch_bounds__(kBlock) void k_fac_diag(FacArgs A) {
     const int j = blockIdx.x * kBlock + threadIdx.x;
@@ -1453,7 +1470,9 @@ __global__ __launch_bounds__(kFacBlock) void k_fac_assemble(FacArgs A, int h0, i
     const int tid = threadIdx.x, w = S.w, no = S.noff, m = S.m;
     const int t0 = (int)(blockIdx.x % per) * cols, t1 = min(m, t0 + cols);
     if (t0 >= m) return;
-    MD_G double *P = A.P + S.poff, *F = A.S + S.soff, *U = A.U + S.uoff;
+    const PivotBuf D = pivot_buf(A, S, 0);  // where the sweeps start
+    MD_G double *P = D.p, *F = A.S + S.soff, *U = A.U + S.uoff;
+    const long long ldp = D.ld;
     const MD_G int *rows = A.offrows + S.roff;
     // the front's row list in LDS for the searches of the original entries (pivot columns), and
     // each child's row map in turn
@@ -1480,7 +1499,7 @@ __global__ __launch_bounds__(kFacBlock) void k_fac_assemble(FacArgs A, int h0, i
     // zero the owned columns: contiguous ranges of P and F (pivot columns) and of U
     const int kend = min(t1, w);
     if (t0 < w) {
-        for (long long e = (long long)t0 * m + tid; e < (long long)kend * m; e += kFacBlock) P[e] = 0.0;
+        for (long long e = t0 * ldp + tid; e < kend * ldp; e += kFacBlock) P[e] = 0.0;
         for (long long e = (long long)t0 * no + tid; e < (long long)kend * no; e += kFacBlock) F[e] = 0.0;
     }
     if (t1 > w)
@@ -1491,14 +1510,14 @@ __global__ __launch_bounds__(kFacBlock) void k_fac_assemble(FacArgs A, int h0, i
     // front receives at most one, right after its zero, so it is stored
     for (int k = t0 + tid / kAsmSlotLanes; k < kend; k += kFacBlock / kAsmSlotLanes) {
         const int j = S.c0 + k, sl = j / kSlice, l = j % kSlice;
-        if (tid % kAsmSlotLanes == 0) P[(long long)k * m + k] = A.diag[j];
+        if (tid % kAsmSlotLanes == 0) P[k * ldp + k] = A.diag[j];
         for (int q = A.slice_ptr[sl] + tid % kAsmSlotLanes; q < A.slice_ptr[sl + 1]; q += kAsmSlotLanes) {
             const long long g = (long long)q * kSlice + l;
             const int i = A.sell_col[g];
             if (i <= j || i >= A.nf) continue;
             const double v = -A.w64[g];
             if (i < S.c0 + w) {
-                P[(long long)k * m + (i - S.c0)] = v;
+                P[k * ldp + (i - S.c0)] = v;
             } else {
                 int lo = 0, hi = no;  // first off row >= i
                 while (lo < hi) {
@@ -1548,7 +1567,7 @@ __global__ __launch_bounds__(kFacBlock) void k_fac_assemble(FacArgs A, int h0, i
                     const int ra = rstaged ? relsh[a] : relg[a], rb = rstaged ? relsh[b] : relg[b];
                     v[u] = Uc[(long long)b * nc + a];
                     if (ra >= m || rb > ra) *A.flag = 2;
-                    else if (rb < w) dst[u] = ra < w ? P + (long long)rb * m + ra : F + (long long)rb * no + (ra - w);
+                    else if (rb < w) dst[u] = ra < w ? P + rb * ldp + ra : F + (long long)rb * no + (ra - w);
                     else dst[u] = U + (long long)(rb - w) * no + (ra - w);
                 }
             }
@@ -1563,264 +1582,282 @@ __global__ __launch_bounds__(kFacBlock) void k_fac_assemble(FacArgs A, int h0, i
     }
 }
 
-// The pivot block's Cholesky factor and its inverse X = L^{-1}, blocked by kFb columns
-// (right-looking): for each column block s, the diagonal block is factored and inverted (the
-// diagonal block of X, row-major in the T workspace; k_fac_potrf for block 0, later blocks by the
-// workgroup of k_fac_syrk that completes them), k_fac_trsm forms the rows below it (times that
-// inverse) and row block s of X, k_fac_syrk updates the trailing lower blocks and accumulates the
-// X blocks below: X_IJ = -X_II W_IJ with W_IJ = sum_{K=J}^{I-1} L_IK X_KJ, the term K = s added at
-// step s (in X's place), so W_sJ is complete when step s begins.
-constexpr int kFb = 64;
-// operands of the MFMA products are staged in LDS kMk values of k at a time, rows kMpad doubles apart
-constexpr int kMk = 32;
-constexpr int kMpad = 66;
+// Pivot blocks are inverted by symmetric block sweeps. A sweep on the columns of block s with
+// S = A_ss^{-1} maps A_ss -> -S, A_Is -> A_Is S, A_IJ -> A_IJ - A_Is S A_Js^T; it keeps the matrix
+// symmetric, and after the sweeps on every block A is -A^{-1}. Swept at 64 columns over the front's
+// pivot block (k_fac_inv0, k_fac_step), at 16 within a 64 x 64 block (invert64), at 4 within a
+// 16 x 16 block (sweep_panel). k_fac_small sweeps a whole small front by panels of 4 pivots, which
+// leaves [-D^{-1}, G^T; G, U] in place.
+// LDS rows of the 64 x 64 operands, in doubles (odd: a column of a row-major tile hits 32 banks)
+constexpr int kLdT = kFb + 1;
 
-// Diagonal block s, by four wavefronts (unrolled over the block's columns: a loop over them with
-// the same work per step measured almost twice as slow). Cholesky (unblocked, right-looking) as an
-// unscaled LDL^T: lane i of wave v holds row i of the block's columns [16 v, 16 v + 16) (a[j] =
-// A(kb + i, kb + 16 v + j), then u). The wave owning a panel of kPanel columns factors it in
-// registers: at step k it takes the pivot d_k = u_k(k) from lane k (v_readlane, two 32-bit halves
-// per double), forms 1/d_k (v_rcp_f64 and one cubic Newton step) and updates the panel's later
-// columns, a(i, c) -= (u_k(i) / d_k) u_k(c) (entries above the diagonal too, never used). It puts
-// u_k and u_k / d_k in LDS; after one barrier the waves with columns past the panel apply the
-// rank-kPanel update, the next panel's wave first and in the same basic block as that panel's
-// factorisation, so the chain starts while the rest of its update is still being issued. At the
-// end every wave scales its columns, L(:, k) = u_k / sqrt(d_k) (v_rsq_f64 and two Newton steps).
-//
-// Inverse X = L^{-1} by 16 x 16 blocks: wave v inverts diagonal block v by columns (four lanes per
-// column, lane r of column i holding X(t, i) for t = r mod 4; X(k, i) = (delta_ki - sum_{t<k}
-// L(k, t) X(t, i)) / L(k, k), the sum split over the four lanes and joined by a DPP butterfly), and
-// after one barrier wave J forms block column J downwards on the matrix cores, X_IJ = -X_II W_IJ
-// with W_IJ = sum_{K=J}^{I-1} L_IK X_KJ. X is zero above the diagonal, exactly. Rows and columns
-// past a partial block (b < 64) hold zero in L and in the slot of 1 / L(k, k), so X is zero there.
+// v_mfma_f64_16x16x4f64: A(i, k) from lane i + 16 k, B(k, j) from lane j + 16 k, D(i, j) in lane
+// j + 16 (i % 4), register i / 4. Register c of a D block is the B operand of k in [4 c, 4 c + 4), and
+// for a symmetric block also its transpose's A operand.
 typedef double dv4 __attribute__((ext_vector_type(4)));
+#define MD_MFMA64(a, b, c) __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0)
 
-__device__ __forceinline__ double readlane_f64(double v, int l) {
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, l);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), l);
+__device__ __forceinline__ double f64_of(unsigned lo, unsigned hi) {
     return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
-// v from the lane whose index is this lane's xor Q (Q = 1, 2: within a quad), by DPP.
-template <int Q>
-__device__ __forceinline__ double quad_xor(double v) {
-    constexpr int ctrl = Q == 1 ? 0xB1 : 0x4E;  // quad_perm [1,0,3,2] / [2,3,0,1]
+// x[t] = p of lane (lane % 16) + 16 t, in every lane: the four rows of 16 lanes to all rows
+// (v_permlane16_swap exchanges odd rows of one operand with even rows of the other, v_permlane32_swap
+// the halves).
+__device__ __forceinline__ void rows4(double p, double (&x)[4]) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, p);
+    const unsigned w[2] = {(unsigned)u, (unsigned)(u >> 32)};
+    unsigned r[4][2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const auto a = __builtin_amdgcn_permlane16_swap(w[h], w[h], false, false);
+        const auto b = __builtin_amdgcn_permlane32_swap(a[0], a[0], false, false);
+        const auto c = __builtin_amdgcn_permlane32_swap(a[1], a[1], false, false);
+        r[0][h] = b[0]; r[2][h] = b[1]; r[1][h] = c[0]; r[3][h] = c[1];
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) x[t] = f64_of(r[t][0], r[t][1]);
+}
+
+// v of lane N of each row of 16 lanes, to the whole row (DPP row_newbcast).
+template <int N>
+__device__ __forceinline__ double row_bcast(double v) {
     const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)u, ctrl, 0xF, 0xF, false);
-    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), ctrl, 0xF, 0xF, false);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)u, 0x150 + N, 0xF, 0xF, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), 0x150 + N, 0xF, 0xF, true);
+    return f64_of(lo, hi);
 }
 
-constexpr int kPotrfCols = kFb / 4;  // columns per wave
-constexpr int kLdsPad = kFb + 1;
-constexpr int kIb = 16;              // blocks of the inverse (one per wave)
-static_assert(kFb == 4 * kIb && kFacBlock == 4 * 64, "four wavefronts, one 16-row block of the inverse each");
+// 1 / d: v_rcp_f64 (relative error below 2^-22) and y (1 + e + e^2), e = 1 - d y.
+__device__ __forceinline__ double recip64(double d) {
+    double y = __builtin_amdgcn_rcp(d);
+    const double e = __builtin_fma(-d, y, 1.0);
+    return __builtin_fma(y, __builtin_fma(e, e, e), y);
+}
 
-// kPanel columns per barrier. FULL: a block of kFb columns (no per-column bound checks, so a
-// panel's chain is one basic block); else b columns, the rest zero. Panel buffers: cu[parity][k][i]
-// = u_k(i), cv[parity][k][i] = u_k(i) / d_k.
-constexpr int kPanel = 8;
-static_assert(kPotrfCols % kPanel == 0, "a panel lies within one wave's columns");
-template <int K, bool FULL>
-__device__ __forceinline__ void factor_panel(double (&a)[kPotrfCols], double (*cu)[kPanel][kFb], double (*cv)[kPanel][kFb],
-                                             int lane, int b, double amax, bool &bad) {
-    constexpr int j0 = K % kPotrfCols, buf = (K / kPanel) & 1;
-#pragma unroll
-    for (int kk = 0; kk < kPanel; ++kk) {
-        double v = 0.0;  // columns past the block stay zero
-        if (FULL || K + kk < b) {
-            const double d = readlane_f64(a[j0 + kk], K + kk);
-            if (!(d > 1e-14 * amax)) bad = true;
-            // 1/d: v_rcp_f64 (relative error below 2^-22) and y (1 + e + e^2), e = 1 - d y
-            double y = __builtin_amdgcn_rcp(d);
-            const double e = __builtin_fma(-d, y, 1.0);
-            y = __builtin_fma(y, __builtin_fma(e, e, e), y);
-            v = a[j0 + kk] * y;
-#pragma unroll
-            for (int c = kk + 1; c < kPanel; ++c) a[j0 + c] -= v * readlane_f64(a[j0 + kk], K + c);
-        }
-        cu[buf][kk][lane] = a[j0 + kk];
-        cv[buf][kk][lane] = v;
+// Sweep of a symmetric matrix of NB x NB blocks of 16 x 16 (all blocks stored, in the layout of D),
+// by one wavefront, on the four columns 4 C .. 4 C + 3 of block 0 (PARTIAL: on the first cnt of
+// them). Register C of block (0, J) holds a(16 J + j, 4 C + k) at lane j + 16 k: the panel is one
+// register per block, already in the layout of both operands of the rank-4 update, one MFMA per
+// block. W = P B^{-1} (B the panel's 4 x 4 pivot block) comes from B's LDL^T, whose entries every lane
+// forms for itself, and a substitution along the lane's row; the rows of the panel itself are solved
+// for minus the unit rows, which gives -B^{-1}. The columns of the panel are cleared and their B
+// operand set to minus the unit columns, so that the update leaves W there, exactly.
+// Pivots with index < real must exceed thr, else bad is set.
+template <int NB, int C, bool PARTIAL>
+__device__ __forceinline__ void sweep_panel(dv4 (&a)[NB][NB], int lane, int cnt, int real, double thr, bool &bad) {
+    const int j = lane & 15, g = lane >> 4, jj = j & 3;
+    double x[4];
+    rows4(a[0][0][C], x);
+    const double d0 = row_bcast<4 * C>(x[0]);
+    double a10 = row_bcast<4 * C + 1>(x[0]), a20 = row_bcast<4 * C + 2>(x[0]), a30 = row_bcast<4 * C + 3>(x[0]);
+    double a11 = row_bcast<4 * C + 1>(x[1]), a21 = row_bcast<4 * C + 2>(x[1]), a31 = row_bcast<4 * C + 3>(x[1]);
+    double a22 = row_bcast<4 * C + 2>(x[2]), a32 = row_bcast<4 * C + 3>(x[2]), a33 = row_bcast<4 * C + 3>(x[3]);
+    if (PARTIAL) {  // pivots past cnt: the unit matrix
+        if (cnt < 2) { a10 = 0.0; a21 = 0.0; a31 = 0.0; a11 = 1.0; }
+        if (cnt < 3) { a20 = 0.0; a21 = 0.0; a32 = 0.0; a22 = 1.0; }
+        if (cnt < 4) { a30 = 0.0; a31 = 0.0; a32 = 0.0; a33 = 1.0; }
     }
-}
-
-// Panel K is in LDS once the barrier is passed: the update of the columns past it (from column jn of
-// the next panel's wave, all columns of the waves after it), then the next panel's factorisation.
-template <int K, bool FULL>
-__device__ __forceinline__ void chol_step(double (&a)[kPotrfCols], double (*cu)[kPanel][kFb], double (*cv)[kPanel][kFb],
-                                          int wv, int lane, int b, double amax, bool &bad) {
-    if constexpr (K < kFb) {
-        if (FULL || K < b) {
-            constexpr int buf = (K / kPanel) & 1;
-            __syncthreads();
-            constexpr int nxt = K + kPanel, nown = nxt / kPotrfCols, jn = nxt % kPotrfCols;
-            if constexpr (nxt < kFb) {
-                double lik[kPanel];
+    const double r0 = recip64(d0);
+    const double l10 = a10 * r0, l20 = a20 * r0, l30 = a30 * r0;
+    const double d1 = __builtin_fma(-l10, a10, a11), r1 = recip64(d1);
+    const double b21 = __builtin_fma(-l10, a20, a21), b31 = __builtin_fma(-l10, a30, a31);
+    const double b22 = __builtin_fma(-l20, a20, a22), b32 = __builtin_fma(-l20, a30, a32), b33 = __builtin_fma(-l30, a30, a33);
+    const double l21 = b21 * r1, l31 = b31 * r1;
+    const double d2 = __builtin_fma(-l21, b21, b22), r2 = recip64(d2);
+    const double c32 = __builtin_fma(-l21, b31, b32), c33 = __builtin_fma(-l31, b31, b33);
+    const double l32 = c32 * r2;
+    const double d3 = __builtin_fma(-l32, c32, c33), r3 = recip64(d3);
+    if ((4 * C < real && !(d0 > thr)) || (4 * C + 1 < real && !(d1 > thr)) || (4 * C + 2 < real && !(d2 > thr)) ||
+        (4 * C + 3 < real && !(d3 > thr)))
+        bad = true;
+    double w[NB], p[NB];
 #pragma unroll
-                for (int kk = 0; kk < kPanel; ++kk) lik[kk] = cv[buf][kk][lane];
-                if (wv == nown) {
+    for (int J = 0; J < NB; ++J) {
+        const bool inp = J == 0 && (j >> 2) == C && (!PARTIAL || jj < cnt);
+        const double P = a[0][J][C];
+        if (J > 0) rows4(P, x);
 #pragma unroll
-                    for (int j = jn; j < kPotrfCols; ++j)
+        for (int t = 0; t < 4; ++t) {
+            if (PARTIAL && t >= cnt) x[t] = 0.0;
+            if (J == 0) x[t] = inp ? (jj == t ? -1.0 : 0.0) : x[t];
+        }
+        const double u1 = __builtin_fma(-l10, x[0], x[1]);
+        const double u2 = __builtin_fma(-l21, u1, __builtin_fma(-l20, x[0], x[2]));
+        const double u3 = __builtin_fma(-l32, u2, __builtin_fma(-l31, u1, __builtin_fma(-l30, x[0], x[3])));
+        const double w3 = u3 * r3;
+        const double w2 = __builtin_fma(-l32, w3, u2 * r2);
+        const double w1 = __builtin_fma(-l31, w3, __builtin_fma(-l21, w2, u1 * r1));
+        const double w0 = __builtin_fma(-l30, w3, __builtin_fma(-l20, w2, __builtin_fma(-l10, w1, x[0] * r0)));
+        w[J] = g == 0 ? w0 : g == 1 ? w1 : g == 2 ? w2 : w3;
+        p[J] = inp ? (g == jj ? -1.0 : 0.0) : P;
+        if (J == 0) {
 #pragma unroll
-                        for (int kk = 0; kk < kPanel; ++kk) a[j] -= lik[kk] * cu[buf][kk][kPotrfCols * nown + j];
-                    if (FULL || nxt < b) factor_panel<nxt, FULL>(a, cu, cv, lane, b, amax, bad);
-                } else if (wv > nown) {
+            for (int I = 0; I < NB; ++I)
 #pragma unroll
-                    for (int j = 0; j < kPotrfCols; ++j)
-#pragma unroll
-                        for (int kk = 0; kk < kPanel; ++kk) a[j] -= lik[kk] * cu[buf][kk][kPotrfCols * wv + j];
-                }
-            }
-            chol_step<nxt, FULL>(a, cu, cv, wv, lane, b, amax, bad);
+                for (int k = 0; k < 4; ++k) a[I][0][k] = inp ? 0.0 : a[I][0][k];
         }
     }
+#pragma unroll
+    for (int I = 0; I < NB; ++I)
+#pragma unroll
+        for (int J = 0; J < NB; ++J) a[I][J] = MD_MFMA64(-w[I], p[J], a[I][J]);
+#pragma unroll
+    for (int J = 0; J < NB; ++J) a[0][J][C] = !PARTIAL || g < cnt ? w[J] : a[0][J][C];
 }
 
-// Diagonal block o / 16 of the inverse: lane (4 ii + r) forms X(o + t, o + ii) for t = r mod 4,
-// x[q] for t = 4 q + r; the slot (k, k) of Lsh holds 1 / L(k, k).
+// LDS of invert64: the inverse of the current 16 x 16 diagonal block and the current block column,
+// two buffers each.
+constexpr int kIb = 16, kIbLd = kIb + 1;
+struct InvLds {
+    double s[2][kIb][kIbLd];
+    double a[2][4][kIb][kIbLd];
+};
+static_assert(kFb == 4 * kIb, "one block column of 16 per wavefront");
+
+// Step K of invert64: wave K sweeps its diagonal block and publishes its inverse and the block
+// column; after one barrier the other waves form T_J = S A_KJ and update their columns,
+// A_IJ -= A_IK T_J, and wave K forms A_IK S.
 template <int K>
-__device__ __forceinline__ void inv_diag(const double (*Lsh)[kLdsPad], double (&x)[kIb / 4], int r, int ii, int o) {
-    if constexpr (K < kIb) {
-        double part = 0.0;
-#pragma unroll
-        for (int q = 0; q < (K + 3) / 4; ++q) {
-            const int t = 4 * q + r;
-            part += t < K ? Lsh[o + K][o + t] * x[q] : 0.0;
-        }
-        part += quad_xor<1>(part);
-        part += quad_xor<2>(part);
-        const double xk = ((ii == K ? 1.0 : 0.0) - part) * Lsh[o + K][o + K];
-        if (r == (K & 3)) x[K / 4] = xk;
-        inv_diag<K + 1>(Lsh, x, r, ii, o);
-    }
-}
-
-// Block column J of the inverse on the matrix cores (v_mfma_f64_16x16x4f64: A(i, k) from lane
-// i + 16 k, B(k, j) from lane j + 16 k, D(i, j) in lane j + 16 (i % 4), register i / 4). Register c
-// of a D block is the B operand of k in [4 c, 4 c + 4), so the blocks X_KJ feed the next products
-// as they are. Writes the block column to T (row-major), zero above the diagonal block.
-template <int J>
-__device__ __forceinline__ void inv_blockcol(const double (*Lsh)[kLdsPad], const double (*Xd)[kIb][kIb + 1], int lane,
-                                             MD_G double *T, int w, int kb, int b) {
-    const int i = lane & 15, m = lane >> 4;
-    dv4 xb[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) xb[J][c] = Xd[J][4 * c + m][i];
-#pragma unroll
-    for (int I = J + 1; I < 4; ++I) {
-        dv4 acc = dv4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int K = J; K < I; ++K)
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(Lsh[kIb * I + i][kIb * K + 4 * c + m], xb[K][c], acc, 0, 0, 0);
-        dv4 d = dv4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int c = 0; c < 4; ++c) d = __builtin_amdgcn_mfma_f64_16x16x4f64(Xd[I][i][4 * c + m], acc[c], d, 0, 0, 0);
-        xb[I] = -d;
-    }
-    const int colx = kIb * J + i;
-    if (colx < b) {
+__device__ __forceinline__ void invert64_step(dv4 (&acc)[4], InvLds &L, int wv, int lane, int b, double thr, bool &bad) {
+    if (kIb * K >= b) return;  // past a partial block: identity, untouched
+    const int j = lane & 15, g = lane >> 4, buf = K & 1;
+    if (wv == K) {
 #pragma unroll
         for (int I = 0; I < 4; ++I)
+            if (I != K)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const int row = kIb * I + 4 * c + m;
-                if (row < b) T[(long long)(kb + row) * w + kb + colx] = I < J ? 0.0 : xb[I][c];
-            }
-    }
-}
-
-// LDS of the pivot block, two arrays: the panel buffers (later the inverse's diagonal blocks; sized
-// to also hold the staged A operand of k_fac_syrk), and L (also holds the staged B operand).
-constexpr int kPbPanels = 2 * 2 * kPanel * kFb;
-constexpr int kPbPan = kPbPanels > kMk * kMpad ? kPbPanels : kMk * kMpad;
-constexpr int kPbL = kFb * kLdsPad > kMk * kMpad ? kFb * kLdsPad : kMk * kMpad;
-static_assert(kFb / kIb * kIb * (kIb + 1) <= kPbPanels, "the diagonal blocks of the inverse fit the panel buffers");
-
-// Diagonal block s of front S by the whole workgroup: L into the panel, X = L^{-1} into T. FROM_LDS:
-// the block's lower entries are in lsh (row-major, rows kLdsPad apart), not yet in the panel.
-template <bool FROM_LDS>
-__device__ __forceinline__ void pivot_block(const FacArgs &A, const FacDev &S, int s, double *pan, double *lsh) {
-    const int w = S.w, m = S.m, kb = s * kFb;
-    if (kb >= w) return;
-    const int b = min(kFb, w - kb), wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    MD_G double *P = A.P + S.poff;
-    MD_G double *T = A.T + S.toff;
-    double (*cu)[kPanel][kFb] = reinterpret_cast<double (*)[kPanel][kFb]>(pan);
-    double (*cv)[kPanel][kFb] = cu + 2;
-    double (*Lsh)[kLdsPad] = reinterpret_cast<double (*)[kLdsPad]>(lsh);
-    double a[kPotrfCols];
+                for (int c = 0; c < 4; ++c) L.a[buf][I][4 * c + g][j] = acc[I][c];
+        dv4 d[1][1];
+        d[0][0] = acc[K];
+        const int real = b - kIb * K;
+        sweep_panel<1, 0, false>(d, lane, 4, real, thr, bad);
+        sweep_panel<1, 1, false>(d, lane, 4, real, thr, bad);
+        sweep_panel<1, 2, false>(d, lane, 4, real, thr, bad);
+        sweep_panel<1, 3, false>(d, lane, 4, real, thr, bad);
+        acc[K] = d[0][0];
 #pragma unroll
-    for (int j = 0; j < kPotrfCols; ++j) {
-        // column-major panel: A(kb + lane, kb + c) at (kb + c) m + kb + lane (lower part only)
-        const int c = kPotrfCols * wv + j;
-        if constexpr (FROM_LDS) a[j] = (lane < b && c < b && c <= lane) ? lsh[lane * kLdsPad + c] : 0.0;
-        else a[j] = (lane < b && c < b && c <= lane) ? P[(long long)(kb + c) * m + kb + lane] : 0.0;
+        for (int c = 0; c < 4; ++c) L.s[buf][4 * c + g][j] = -acc[K][c];
     }
-    if constexpr (FROM_LDS) __syncthreads();  // every entry read before lsh takes L
-    const double amax = __longlong_as_double((long long)*A.amax);
-    bool bad = false;
-    if (b == kFb) {
-        if (wv == 0) factor_panel<0, true>(a, cu, cv, lane, b, amax, bad);
-        chol_step<0, true>(a, cu, cv, wv, lane, b, amax, bad);
+    __syncthreads();
+    if (wv == K) {
+        dv4 t[4];
+#pragma unroll
+        for (int I = 0; I < 4; ++I) t[I] = dv4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int I = 0; I < 4; ++I)
+                if (I != K) t[I] = MD_MFMA64(L.a[buf][I][j][4 * c + g], -acc[K][c], t[I]);
+#pragma unroll
+        for (int I = 0; I < 4; ++I)
+            if (I != K) acc[I] = t[I];
     } else {
-        if (wv == 0) factor_panel<0, false>(a, cu, cv, lane, b, amax, bad);
-        chol_step<0, false>(a, cu, cv, wv, lane, b, amax, bad);
-    }
-    if (bad && threadIdx.x == 0) *A.flag = 1;
-    // L(:, k) = u_k / sqrt(d_k), d_k = u_k(k); lower part to the panel, all of the wave's columns to
-    // LDS (the diagonal as 1 / L(i, i))
-    double rdiag = 0.0;
+        dv4 t = dv4{0.0, 0.0, 0.0, 0.0}, t2 = t;
 #pragma unroll
-    for (int j = 0; j < kPotrfCols; ++j) {
-        const int c = kPotrfCols * wv + j;
-        const double d = readlane_f64(a[j], c);
-        double rd = 0.0;
-        if (c < b) {
-            rd = __builtin_amdgcn_rsq(d);
-            rd = rd * (1.5 - 0.5 * d * rd * rd);
-            rd = rd * (1.5 - 0.5 * d * rd * rd);
+        for (int c = 0; c < 4; c += 2) {
+            t = MD_MFMA64(L.s[buf][j][4 * c + g], acc[K][c], t);
+            t2 = MD_MFMA64(L.s[buf][j][4 * c + 4 + g], acc[K][c + 1], t2);
         }
-        if (lane == c) rdiag = rd;
-        a[j] *= rd;
-    }
+        t += t2;
 #pragma unroll
-    for (int j = 0; j < kPotrfCols; ++j) {
-        const int c = kPotrfCols * wv + j;
-        if (lane < b && c < b && c <= lane) P[(long long)(kb + c) * m + kb + lane] = a[j];
-        Lsh[lane][c] = c == lane ? rdiag : a[j];
-    }
-    __syncthreads();
-    double (*Xd)[kIb][kIb + 1] = reinterpret_cast<double (*)[kIb][kIb + 1]>(pan);
-    {
-        const int r = lane & 3, ii = lane >> 2;
-        double x[kIb / 4] = {0.0, 0.0, 0.0, 0.0};
-        inv_diag<0>(Lsh, x, r, ii, kIb * wv);
+        for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int q = 0; q < kIb / 4; ++q) Xd[wv][4 * q + r][ii] = x[q];
+            for (int I = 0; I < 4; ++I)
+                if (I != K) acc[I] = MD_MFMA64(-L.a[buf][I][j][4 * c + g], t[c], acc[I]);
+        acc[K] = t;
     }
-    __syncthreads();
-    if (wv == 0) inv_blockcol<0>(Lsh, Xd, lane, T, w, kb, b);
-    else if (wv == 1) inv_blockcol<1>(Lsh, Xd, lane, T, w, kb, b);
-    else if (wv == 2) inv_blockcol<2>(Lsh, Xd, lane, T, w, kb, b);
-    else inv_blockcol<3>(Lsh, Xd, lane, T, w, kb, b);
 }
 
-__global__ __launch_bounds__(kFacBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_fac_potrf(FacArgs A, int h0, int s) {
-    __shared__ double pan[kPbPanels];
-    __shared__ double lsh[kFb * kLdsPad];
-    pivot_block<false>(A, A.sn[A.hlist[h0 + blockIdx.x]], s, pan, lsh);
+static_assert(kFacBlock == 4 * 64, "four wavefronts");
+
+// The symmetric 64 x 64 block in m (lower part, row r at r * kLdT) replaced by minus its inverse
+// in the layout of D: wave v holds block column v in acc. b < 64: the leading b x b block (rows and
+// columns past it are taken as the identity). Ends without a barrier; work may not alias m.
+// A chain of b pivots: one 64 x 64 block takes about 9 us, 2.9 of it sixteen panel sweeps' worth of
+// dependent FP64 arithmetic per 16 columns (740 cycles per panel of 4, DPP and permlane broadcasts
+// in place of LDS), the rest the updates between (one v_mfma_f64_16x16x4 per 16 cycles and CU). The
+// unscaled LDL^T with a blocked triangular inverse that stood here took 14 us, plus X^T X.
+__device__ __forceinline__ void invert64(const double *m, InvLds &work, int b, double thr, dv4 (&acc)[4], bool &bad) {
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int I = 0; I < 4; ++I)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int r = kIb * I + 4 * c + g, q = kIb * wv + j;
+            acc[I][c] = r < b && q < b ? m[max(r, q) * kLdT + min(r, q)] : r == q ? 1.0 : 0.0;
+        }
+    invert64_step<0>(acc, work, wv, lane, b, thr, bad);
+    invert64_step<1>(acc, work, wv, lane, b, thr, bad);
+    invert64_step<2>(acc, work, wv, lane, b, thr, bad);
+    invert64_step<3>(acc, work, wv, lane, b, thr, bad);
+}
+
+// Entry (r, c), r >= c, of D^{-1}: both triangles of the panel's pivot block and of the backward
+// panel [D^{-1}; G] (row-major) in the solve precision.
+__device__ __forceinline__ void put_dinv(const FacArgs &A, const FacDev &S, int r, int c, double v) {
+    MD_G double *P = A.P + S.poff;
+    P[(long long)c * S.m + r] = v;
+    P[(long long)r * S.m + c] = v;
+    const long long o1 = S.pr_off + (long long)r * S.w + c, o2 = S.pr_off + (long long)c * S.w + r;
+    if (A.solve64) {
+        static_cast<MD_G double *>(A.pr)[o1] = v;
+        static_cast<MD_G double *>(A.pr)[o2] = v;
+    } else {
+        static_cast<MD_G float *>(A.pr)[o1] = (float)v;
+        static_cast<MD_G float *>(A.pr)[o2] = (float)v;
+    }
+}
+
+// Block s of the pivot block, complete in m (LDS): S = A_ss^{-1} into `out` (block (s, s) of the
+// workspace the next step reads), or D^{-1} itself when it is the only block.
+__device__ __forceinline__ void pivot_inverse(const FacArgs &A, const FacDev &S, int s, const double *m, InvLds &work,
+                                              PivotBuf out) {
+    const int kb = s * kFb, b = min(kFb, S.w - kb);
+    const double thr = 1e-14 * __longlong_as_double((long long)*A.amax);
+    dv4 acc[4];
+    bool bad = false;
+    invert64(m, work, b, thr, acc, bad);
+    if (bad && (threadIdx.x & 63) == 0) *A.flag = 1;
+    const int wv = threadIdx.x >> 6, j = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4, r = kIb * wv + j;
+    if (r >= b) return;
+#pragma unroll
+    for (int I = 0; I < 4; ++I)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int q = kIb * I + 4 * c + g;  // entry (r, q) = (q, r): lanes along r
+            if (q >= b) continue;
+            if (S.w <= kFb) {
+                if (r >= q) put_dinv(A, S, r, q, -acc[I][c]);
+            } else {
+                out.p[(long long)(kb + q) * out.ld + kb + r] = -acc[I][c];
+            }
+        }
+}
+
+// Block 0 of every pivot block of a height (one workgroup per front).
+__global__ __launch_bounds__(kFacBlock) void k_fac_inv0(FacArgs A, int h0) {
+    const FacDev S = A.sn[A.hlist[h0 + blockIdx.x]];
+    __shared__ double m[kFb * kLdT];
+    __shared__ InvLds work;
+    const PivotBuf B = pivot_buf(A, S, 0);
+    const int b = min(kFb, S.w);
+#pragma unroll
+    for (int i = 0; i < kFb * kFb / kFacBlock; ++i) {
+        const int e = threadIdx.x + kFacBlock * i, r = e % kFb, c = e / kFb;
+        if (r < b && c <= r) m[r * kLdT + c] = B.p[(long long)c * B.ld + r];
+    }
+    __syncthreads();
+    pivot_inverse(A, S, 0, m, work, B);
 }
 
 // ---- FP64 dense products of the factorization on the matrix cores ----------------------
 //
-// v_mfma_f64_16x16x4f64 (one wavefront): D(16x16) = A(16x4) B(4x16) + C with A(i, k) from
-// lane i + 16 k, B(k, j) from lane j + 16 k, and D(i, j) in lane j + 16 (i % 4), register
-// i / 4. A 64 x 64 output tile per workgroup of 256 threads: wave v computes rows
-// [32 (v / 2), +32) and columns [32 (v % 2), +32) as 2 x 2 such blocks, with the operands
-// staged in LDS kMk values of k at a time (As[k][i] = A(i, k), Bs[k][j] = B(k, j)).
+// A 64 x 64 output tile per workgroup of 256 threads: wave v computes rows [32 (v / 2), +32) and
+// columns [32 (v % 2), +32) as 2 x 2 blocks of v_mfma_f64_16x16x4, with the operands staged in LDS,
+// kMk values of k at a time (As[k][i] = A(i, k), Bs[k][j] = B(k, j); rows kMpad doubles apart).
+constexpr int kMk = 32;
+constexpr int kMpad = 66;
 
 struct MmaAcc {
     dv4 c[2][2];
@@ -1916,77 +1953,6 @@ __device__ __forceinline__ void acc_sum(const MD_G double *wp, int ks, MmaAcc &a
 #pragma unroll
                     for (int r = 0; r < 4; ++r) acc.c[x][y][r] += v[dz][(x * 2 + y) * 4 + r];
     }
-}
-
-// D^{-1} = X^T X into the pivot block of the panel (symmetric): lower 64 x 64 tile (I, J)
-// of D^{-1}(r, c) = sum_{k >= r} X(k, r) X(k, c), X = L^{-1} row-major in T (zero above its
-// diagonal inside the diagonal blocks), `per` workgroups per supernode.
-template <int MODE>
-__global__ __launch_bounds__(kFacBlock) __attribute__((amdgpu_waves_per_eu(MODE == 2 ? 2 : 4))) void k_fac_dinv(FacArgs A, int h0, int per, int ks) {
-    const int tile = MODE == 1 ? (int)blockIdx.x / ks : (int)blockIdx.x, z = MODE == 1 ? (int)blockIdx.x % ks : 0;
-    MmaAcc acc;
-    mma_zero(acc);
-    // MODE 2: the partials' loads go out first (a tile with no work stored none and returns below)
-    if constexpr (MODE == 2) acc_sum(A.Wk + (long long)tile * ks * kAccVals, ks, acc);
-    const FacDev S = A.sn[A.hlist[h0 + tile / per]];
-    const int w = S.w, m = S.m, nb = (w + 63) / 64, q = tile % per;
-    if (q >= nb * (nb + 1) / 2) return;
-    int I, J;
-    lower_tile(q, I, J);
-    const int r0 = 64 * I, c0 = 64 * J;
-    double *P = A.P + S.poff;
-    const double *X = A.T + S.toff;
-    __shared__ double As[kMk][kMpad];
-    __shared__ double Bs[kMk][kMpad];
-    if constexpr (MODE != 2) {
-        const int nch = (w - r0 + kMk - 1) / kMk, cb = z * nch / ks, ce = (z + 1) * nch / ks;
-        mma_pipeline(
-            ce - cb,
-            [&](int c, double (&ra)[kPer], double (&rb)[kPer]) {
-#pragma unroll
-                for (int i = 0; i < kPer; ++i) {
-                    const int e = threadIdx.x + kFacBlock * i, x = e % 64, k = r0 + (cb + c) * kMk + e / 64;
-                    const bool kin = k < w;
-                    ra[i] = kin && r0 + x < w ? X[(long long)k * w + r0 + x] : 0.0;
-                    rb[i] = kin && c0 + x < w ? X[(long long)k * w + c0 + x] : 0.0;
-                }
-            },
-            [&](const double (&ra)[kPer], const double (&rb)[kPer]) {
-#pragma unroll
-                for (int i = 0; i < kPer; ++i) {
-                    const int e = threadIdx.x + kFacBlock * i;
-                    As[e / 64][e % 64] = ra[i];
-                    Bs[e / 64][e % 64] = rb[i];
-                }
-            },
-            As, Bs, acc);
-    }
-    if constexpr (MODE == 1) {
-        acc_store(A.Wk + ((long long)tile * ks + z) * kAccVals, acc);
-        return;
-    }
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int rr = r0 + mma_row(x, r), cc = c0 + mma_col(y);
-                if (rr < w && cc < w && cc <= rr) {
-                    const double v = acc.c[x][y][r];
-                    P[(long long)cc * m + rr] = v;
-                    P[(long long)rr * m + cc] = v;
-                    // the backward panel [D^{-1}; G] (row-major) in the solve precision
-                    const long long o1 = S.pr_off + (long long)rr * w + cc, o2 = S.pr_off + (long long)cc * w + rr;
-                    if (A.solve64) {
-                        static_cast<MD_G double *>(A.pr)[o1] = v;
-                        static_cast<MD_G double *>(A.pr)[o2] = v;
-                    } else {
-                        static_cast<MD_G float *>(A.pr)[o1] = (float)v;
-                        static_cast<MD_G float *>(A.pr)[o2] = (float)v;
-                    }
-                }
-            }
 }
 
 // G = F_os D^{-1} into panel rows [w, m): 64 x 64 tile (rows of G, columns), `per`
@@ -2114,245 +2080,334 @@ __global__ __launch_bounds__(kFacBlock) __attribute__((amdgpu_waves_per_eu(MODE 
             }
 }
 
-// Step s of the right-looking loop, first launch (`per` tiles per supernode; tiles q < split
-// are row blocks, the others X blocks). Row block s + 1 + q below diagonal block s, as a product
-// with the diagonal block's inverse that k_fac_potrf left in T: L(r, kb + j) = sum_t A(r, kb + t)
-// X(kb + j, kb + t) (L_below = A_below L_ss^{-T}); A(i, t) from the panel (column-major), B(t, j)
-// = X(kb + j, kb + t) (row-major X). X block (s, J), J = q - split < s: X_sJ = -X_ss W_sJ, where
-// W_sJ = sum_{K=J}^{s-1} L_sK X_KJ, accumulated in X's place by the second launches of the
-// earlier steps. Each tile is read whole before it is written.
-__global__ __launch_bounds__(kFacBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_fac_trsm(FacArgs A, int h0, int s, int split, int per) {
-    const FacDev S = A.sn[A.hlist[h0 + blockIdx.x / per]];
-    const int w = S.w, m = S.m, kb = s * kFb, q = (int)(blockIdx.x % per);
-    MD_G double *P = A.P + S.poff;
-    MD_G double *T = A.T + S.toff;
-    __shared__ double As[kMk][kMpad];
-    __shared__ double Bs[kMk][kMpad];
-    MmaAcc acc;
-    mma_zero(acc);
-    if (q < split) {
-        const int r0 = (s + 1 + q) * kFb;
-        if (r0 >= w) return;  // also kb + kFb <= r0 < w: the diagonal block is full
-        mma_pipeline(
-            kFb / kMk,
-            [&](int c, double (&ra)[kPer], double (&rb)[kPer]) {
-#pragma unroll
-                for (int i = 0; i < kPer; ++i) {
-                    const int e = threadIdx.x + kFacBlock * i, x = e % 64, k0 = c * kMk;
-                    ra[i] = r0 + x < w ? P[(long long)(kb + k0 + e / 64) * m + r0 + x] : 0.0;
-                    // B(t, j) = X(kb + j, kb + t): consecutive threads read consecutive t of one row
-                    rb[i] = T[(long long)(kb + e / kMk) * w + kb + k0 + e % kMk];
-                }
-            },
-            [&](const double (&ra)[kPer], const double (&rb)[kPer]) {
-#pragma unroll
-                for (int i = 0; i < kPer; ++i) {
-                    const int e = threadIdx.x + kFacBlock * i;
-                    As[e / 64][e % 64] = ra[i];
-                    Bs[e % kMk][e / kMk] = rb[i];
-                }
-            },
-            As, Bs, acc);
-        __syncthreads();  // every wave has staged its last reads of the tile before any write
-#pragma unroll
-        for (int x = 0; x < 2; ++x)
-#pragma unroll
-            for (int y = 0; y < 2; ++y)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int rr = r0 + mma_row(x, r), jj = kb + mma_col(y);
-                    if (rr < w) P[(long long)jj * m + rr] = acc.c[x][y][r];
-                }
-        return;
+// Two chained products of a tile, operands whole in LDS (64 values of k, rows kLdT apart): acc(i, j) +=
+// sum_{k < kn} Ar[k][i] Bc[k][j].
+__device__ __forceinline__ void mma_span(const double *Ar, const double *Bc, int kn, MmaAcc &acc) {
+    const int wv = threadIdx.x / 64, lane = threadIdx.x & 63;
+    const int rb = 32 * (wv >> 1) + (lane & 15), cb = 32 * (wv & 1) + (lane & 15);
+    for (int k4 = 0; k4 < kn; k4 += 4) {
+        const int kk = (k4 + (lane >> 4)) * kLdT;
+        const double a0 = Ar[kk + rb], a1 = Ar[kk + rb + 16];
+        const double b0 = Bc[kk + cb], b1 = Bc[kk + cb + 16];
+        acc.c[0][0] = MD_MFMA64(a0, b0, acc.c[0][0]);
+        acc.c[0][1] = MD_MFMA64(a0, b1, acc.c[0][1]);
+        acc.c[1][0] = MD_MFMA64(a1, b0, acc.c[1][0]);
+        acc.c[1][1] = MD_MFMA64(a1, b1, acc.c[1][1]);
     }
-    const int J = q - split, c0 = J * kFb;
-    if (J >= s || kb >= w) return;  // block J < s is full
-    const int bs = min(kFb, w - kb);
-    mma_pipeline(
-        kFb / kMk,
-        [&](int c, double (&ra)[kPer], double (&rb)[kPer]) {
-#pragma unroll
-            for (int i = 0; i < kPer; ++i) {
-                const int e = threadIdx.x + kFacBlock * i, k0 = c * kMk;
-                // A(i, t) = X(kb + i, kb + t): consecutive threads read consecutive t of one row
-                const int ia = e / kMk, ta = k0 + e % kMk;
-                ra[i] = ia < bs && ta < bs ? T[(long long)(kb + ia) * w + kb + ta] : 0.0;
-                // B(t, j) = W(kb + t, c0 + j)
-                const int tb = k0 + e / 64;
-                rb[i] = tb < bs ? T[(long long)(kb + tb) * w + c0 + e % 64] : 0.0;
-            }
-        },
-        [&](const double (&ra)[kPer], const double (&rb)[kPer]) {
-#pragma unroll
-            for (int i = 0; i < kPer; ++i) {
-                const int e = threadIdx.x + kFacBlock * i;
-                As[e % kMk][e / kMk] = ra[i];
-                Bs[e / 64][e % 64] = rb[i];
-            }
-        },
-        As, Bs, acc);
-    __syncthreads();  // W_sJ is read whole before X_sJ replaces it
+}
+
+constexpr int kTileVals = kFb * kFb / kFacBlock;  // values of a 64 x 64 tile per thread
+
+// fn(value, row, column) over this thread's accumulators.
+template <class Fn>
+__device__ __forceinline__ void mma_each(const MmaAcc &acc, Fn fn) {
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll
         for (int y = 0; y < 2; ++y)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int rr = kb + mma_row(x, r), cc = c0 + mma_col(y);
-                if (rr < w) T[(long long)rr * w + cc] = -acc.c[x][y][r];
-            }
+            for (int r = 0; r < 4; ++r) fn(acc.c[x][y][r], mma_row(x, r), mma_col(y));
 }
 
-// Step s, second launch (`per` tiles per supernode; tiles q < split are trailing tiles, the
-// others W tiles). Lower trailing tile q = (I, J), s < J <= I: A(r, c) -= sum_{t<64} L(r, kb + t)
-// L(c, kb + t). W tile (I, J), I = s + 1 + (q - split) / (s + 1), J = (q - split) % (s + 1):
-// W_IJ += L_Is X_sJ (stored by the first contribution, J = s), for the X blocks of row block I.
-// Tile 0 = (s + 1, s + 1) completes diagonal block s + 1, and its workgroup then factors and
-// inverts that block (pivot_block): no other tile of the launch touches it or its block of T, so
-// the next step's chain starts while the other tiles still run.
-__global__ __launch_bounds__(kFacBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_fac_syrk(FacArgs A, int h0, int s, int split, int per) {
+// Block (X, s) of a pivot block from its lower tiles, into registers and from there to LDS as
+// Z[t][x] = A(64 X + x, 64 s + t): below the diagonal the tile itself, above it the transpose of
+// tile (s, X). Zero past the matrix.
+__device__ __forceinline__ void block_fetch(PivotBuf B, int w, int X, int s, double (&v)[kTileVals]) {
+#pragma unroll
+    for (int i = 0; i < kTileVals; ++i) {
+        const int e = threadIdx.x + kFacBlock * i, lo = e % kFb, hi = e / kFb;
+        const int row = (X >= s ? X : s) * kFb + lo, col = (X >= s ? s : X) * kFb + hi;
+        v[i] = row < w && col < w ? B.p[(long long)col * B.ld + row] : 0.0;
+    }
+}
+__device__ __forceinline__ void block_put(bool below, const double (&v)[kTileVals], double *Z) {
+#pragma unroll
+    for (int i = 0; i < kTileVals; ++i) {
+        const int e = threadIdx.x + kFacBlock * i, lo = e % kFb, hi = e / kFb;
+        Z[below ? hi * kLdT + lo : lo * kLdT + hi] = v[i];
+    }
+}
+
+// Step s of the block sweeps over the pivot blocks of a height (`per` lower tiles per front): tile
+// (I, J) of the next workspace from the current one and S = A_ss^{-1}, in one launch: with
+// W = A_Is S (64 x 64, in LDS), A_IJ - W A_Js^T; W itself in block column s; -S on the diagonal. The
+// workgroup of tile (s + 1, s + 1), scheduled first, inverts it for the next step while the other
+// tiles still run. The last step writes D^{-1} (minus the swept matrix) to the panels.
+// Bound by the chain of one tile per step: load, two products (1.7 us each at one MFMA per 16 cycles
+// and CU) and the inversion: 19.6 us a step of the 164k icosphere's top heights. One launch per 64
+// columns; the Cholesky form with a triangular inverse took two (trsm, then syrk with the next pivot
+// block: 6.6 + 24 us) and X^T X afterwards (12 to 27 us a height).
+__global__ __launch_bounds__(kFacBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_fac_step(FacArgs A, int h0, int s, int per) {
     const FacDev S = A.sn[A.hlist[h0 + blockIdx.x / per]];
-    const int w = S.w, m = S.m, kb = s * kFb, q = (int)(blockIdx.x % per);
-    MD_G double *P = A.P + S.poff;
-    MD_G double *T = A.T + S.toff;
-    __shared__ double pan[kPbPan];
-    __shared__ double lsh[kPbL];
-    double (*As)[kMpad] = reinterpret_cast<double (*)[kMpad]>(pan);
-    double (*Bs)[kMpad] = reinterpret_cast<double (*)[kMpad]>(lsh);
-    MmaAcc acc;
-    mma_zero(acc);
-    if (q < split) {
-        const int nt = (w + kFb - 1) / kFb - 1 - s;  // row blocks below diagonal block s
-        if (q >= nt * (nt + 1) / 2) return;
-        int I, J;
-        lower_tile(q, I, J);
-        const int r0 = (s + 1 + I) * kFb, c0 = (s + 1 + J) * kFb;
-        mma_pipeline(
-            kFb / kMk,
-            [&](int c, double (&ra)[kPer], double (&rb)[kPer]) {
+    const int w = S.w, nb = (w + kFb - 1) / kFb;
+    if (nb < 2 || s >= nb) return;
+    int q = (int)(blockIdx.x % per);
+    if (q >= nb * (nb + 1) / 2) return;
+    const bool last = s == nb - 1;
+    if (!last) {  // tile 0 and tile (s + 1, s + 1) trade places
+        const int d = (s + 1) * (s + 2) / 2 + s + 1;
+        q = q == 0 ? d : q == d ? 0 : q;
+    }
+    int I, J;
+    lower_tile(q, I, J);
+    const PivotBuf B = pivot_buf(A, S, s), O = pivot_buf(A, S, s + 1);
+    __shared__ double Za[kFb * kLdT], Zb[kFb * kLdT];
+    static_assert(sizeof(InvLds) <= sizeof(Za), "the inversion works in the first operand's place");
+    // entry (r, c) of tile (I, J), r and c within the tile
+    auto emit = [&](int r, int c, double v) {
+        const int rr = I * kFb + r, cc = J * kFb + c;
+        if (rr >= w || cc >= w) return;
+        if (!last) O.p[(long long)cc * O.ld + rr] = v;
+        else if (rr >= cc) put_dinv(A, S, rr, cc, -v);
+    };
+    double vs[kTileVals];
+    block_fetch(B, w, s, s, vs);  // S, both triangles
+    if (I == s && J == s) {
 #pragma unroll
-                for (int i = 0; i < kPer; ++i) {
-                    const int e = threadIdx.x + kFacBlock * i, x = e % 64;
-                    const long long col = (long long)(kb + c * kMk + e / 64) * m;
-                    ra[i] = r0 + x < w ? P[col + r0 + x] : 0.0;
-                    rb[i] = c0 + x < w ? P[col + c0 + x] : 0.0;
-                }
-            },
-            [&](const double (&ra)[kPer], const double (&rb)[kPer]) {
-#pragma unroll
-                for (int i = 0; i < kPer; ++i) {
-                    const int e = threadIdx.x + kFacBlock * i;
-                    As[e / 64][e % 64] = ra[i];
-                    Bs[e / 64][e % 64] = rb[i];
-                }
-            },
-            As, Bs, acc);
-        if (q == 0) {
-            // tile (s + 1, s + 1): its entries go to LDS for the pivot block (which writes L over
-            // their place in the panel), after every wave's last read of the staged operands
-            double v[2][2][4];
-#pragma unroll
-            for (int x = 0; x < 2; ++x)
-#pragma unroll
-                for (int y = 0; y < 2; ++y)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int rr = r0 + mma_row(x, r), cc = c0 + mma_col(y);
-                        v[x][y][r] = rr < w && cc < w && rr >= cc ? P[(long long)cc * m + rr] - acc.c[x][y][r] : 0.0;
-                    }
-            __syncthreads();
-#pragma unroll
-            for (int x = 0; x < 2; ++x)
-#pragma unroll
-                for (int y = 0; y < 2; ++y)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) lsh[mma_row(x, r) * kLdsPad + mma_col(y)] = v[x][y][r];
-            __syncthreads();
-            pivot_block<true>(A, S, s + 1, pan, lsh);
-            return;
+        for (int i = 0; i < kTileVals; ++i) {
+            const int e = threadIdx.x + kFacBlock * i;
+            emit(e % kFb, e / kFb, -vs[i]);
         }
-#pragma unroll
-        for (int x = 0; x < 2; ++x)
-#pragma unroll
-            for (int y = 0; y < 2; ++y)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int rr = r0 + mma_row(x, r), cc = c0 + mma_col(y);
-                    if (rr < w && cc < w && rr >= cc) P[(long long)cc * m + rr] -= acc.c[x][y][r];
-                }
         return;
     }
-    const int qq = q - split, r0 = (s + 1 + qq / (s + 1)) * kFb, J = qq % (s + 1), c0 = J * kFb;
-    if (r0 >= w) return;  // also block s (and every block J <= s) is full
-    mma_pipeline(
-        kFb / kMk,
-        [&](int c, double (&ra)[kPer], double (&rb)[kPer]) {
-#pragma unroll
-            for (int i = 0; i < kPer; ++i) {
-                const int e = threadIdx.x + kFacBlock * i, x = e % 64, t = c * kMk + e / 64;
-                ra[i] = r0 + x < w ? P[(long long)(kb + t) * m + r0 + x] : 0.0;  // L(r0 + x, kb + t)
-                rb[i] = T[(long long)(kb + t) * w + c0 + x];                       // X(kb + t, c0 + x)
-            }
-        },
-        [&](const double (&ra)[kPer], const double (&rb)[kPer]) {
-#pragma unroll
-            for (int i = 0; i < kPer; ++i) {
-                const int e = threadIdx.x + kFacBlock * i;
-                As[e / 64][e % 64] = ra[i];
-                Bs[e / 64][e % 64] = rb[i];
-            }
-        },
-        As, Bs, acc);
+    const int X = I == s ? J : I;  // W = A_Xs S
+    double vx[kTileVals];
+    block_fetch(B, w, X, s, vx);
+    if (I == s || J == s) {
+        block_put(true, vs, Za);
+        block_put(X > s, vx, Zb);
+        __syncthreads();
+        MmaAcc acc;
+        mma_zero(acc);
+        // lanes along the stored tile's rows: (I, s) holds W(r, k), (s, J) holds W(r, k)^T
+        if (J == s) {
+            mma_span(Za, Zb, kFb, acc);
+            mma_each(acc, [&](double v, int k, int r) { emit(r, k, v); });
+        } else {
+            mma_span(Zb, Za, kFb, acc);
+            mma_each(acc, [&](double v, int r, int k) { emit(k, r, v); });
+        }
+        return;
+    }
+    double vj[kTileVals];
+    if (I != J) block_fetch(B, w, J, s, vj);
+    // the tile's own entries, where the product's accumulators will be (row c, column r)
+    double own[2][2][4];
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll
         for (int y = 0; y < 2; ++y)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int rr = r0 + mma_row(x, r), cc = c0 + mma_col(y);
-                if (rr < w) {
-                    MD_G double *dst = T + (long long)rr * w + cc;
-                    *dst = (J == s ? 0.0 : *dst) + acc.c[x][y][r];
-                }
+                const int cc = J * kFb + mma_row(x, r), rr = I * kFb + mma_col(y);
+                own[x][y][r] = rr < w && cc < w ? B.p[(long long)cc * B.ld + rr] : 0.0;
+            }
+    block_put(true, vs, Za);
+    block_put(I > s, vx, Zb);
+    __syncthreads();
+    MmaAcc acc;
+    mma_zero(acc);
+    mma_span(Za, Zb, kFb, acc);  // (k, r): W(r, k)
+    __syncthreads();
+    mma_each(acc, [&](double v, int k, int r) { Za[k * kLdT + r] = v; });
+    if (I != J) block_put(J > s, vj, Zb);
+    __syncthreads();
+    mma_zero(acc);
+    mma_span(Zb, Za, kFb, acc);  // (c, r): sum_k A_Js(c, k) W(r, k)
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc.c[x][y][r] = own[x][y][r] - acc.c[x][y][r];
+    if (last || I != s + 1 || J != s + 1) {
+        mma_each(acc, [&](double v, int c, int r) { emit(r, c, v); });
+        return;
+    }
+    __syncthreads();  // the operands are read
+    mma_each(acc, [&](double v, int c, int r) { if (r >= c) Zb[r * kLdT + c] = v; });
+    __syncthreads();
+    pivot_inverse(A, S, s + 1, Zb, *reinterpret_cast<InvLds *>(Za), O);
+}
+
+// G = F_os D^{-1} and U -= G F_os^T for a height whose pivot blocks all have w <= 64, in one launch:
+// lower tile (I, J) of U, `per` workgroups per front, forms G's row block I itself (one product with
+// D^{-1}); the tiles of block column 0 also write it to the sweeps' panels. The two launches that
+// this replaces cost a launch and a round trip of G through memory for fronts of a few tiles.
+__global__ __launch_bounds__(kFacBlock) void k_fac_gu(FacArgs A, int h0, int per) {
+    const FacDev S = A.sn[A.hlist[h0 + blockIdx.x / per]];
+    const int w = S.w, no = S.noff, m = S.m, nb = (no + kFb - 1) / kFb, q = (int)(blockIdx.x % per);
+    if (q >= nb * (nb + 1) / 2) return;
+    int I, J;
+    lower_tile(q, I, J);
+    const int a0 = I * kFb, b0 = J * kFb, kn = (w + 3) & ~3;
+    const MD_G double *P = A.P + S.poff, *F = A.S + S.soff;
+    MD_G double *U = A.U + S.uoff;
+    __shared__ double Za[kFb * kLdT], Zb[kFb * kLdT];
+    double vd[kTileVals], vi[kTileVals], vj[kTileVals];
+#pragma unroll
+    for (int i = 0; i < kTileVals; ++i) {
+        const int e = threadIdx.x + kFacBlock * i, x = e % kFb, t = e / kFb;
+        const bool in = t < w;
+        vd[i] = in && x < w ? P[(long long)t * m + x] : 0.0;
+        vi[i] = in && a0 + x < no ? F[(long long)t * no + a0 + x] : 0.0;
+        vj[i] = I != J && in && b0 + x < no ? F[(long long)t * no + b0 + x] : 0.0;
+    }
+    double own[2][2][4];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int bb = b0 + mma_row(x, r), aa = a0 + mma_col(y);
+                own[x][y][r] = aa < no && bb <= aa ? U[(long long)bb * no + aa] : 0.0;
+            }
+    block_put(true, vd, Za);
+    block_put(true, vi, Zb);
+    __syncthreads();
+    MmaAcc acc;
+    mma_zero(acc);
+    mma_span(Za, Zb, kn, acc);  // (k, a): G(a, k)
+    __syncthreads();
+    mma_each(acc, [&](double v, int k, int a) { Za[k * kLdT + a] = v; });
+    if (I != J) block_put(true, vj, Zb);
+    __syncthreads();
+    if (J == 0) {
+        // the forward panel G (column-major) and the backward panel's G rows (row-major)
+        for (int e = threadIdx.x; e < w * kFb; e += kFacBlock) {
+            const int a = e % kFb, k = e / kFb;
+            if (a0 + a < no) {
+                const double v = Za[k * kLdT + a];
+                const long long o = S.pc_off + (long long)k * no + a0 + a;
+                if (A.solve64) static_cast<MD_G double *>(A.pc)[o] = v;
+                else static_cast<MD_G float *>(A.pc)[o] = (float)v;
+            }
+        }
+        for (int e = threadIdx.x; e < w * min(kFb, no - a0); e += kFacBlock) {
+            const int k = e % w, a = e / w;
+            const double v = Za[k * kLdT + a];
+            const long long o = S.pr_off + (long long)(w + a0 + a) * w + k;
+            if (A.solve64) static_cast<MD_G double *>(A.pr)[o] = v;
+            else static_cast<MD_G float *>(A.pr)[o] = (float)v;
+        }
+    }
+    mma_zero(acc);
+    mma_span(Zb, Za, kn, acc);  // (b, a): sum_k F(b, k) G(a, k)
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int bb = b0 + mma_row(x, r), aa = a0 + mma_col(y);
+                if (aa < no && bb <= aa) U[(long long)bb * no + aa] = own[x][y][r] - acc.c[x][y][r];
             }
 }
 
-// A whole height of small fronts (every m = w + noff <= mm <= kSmallFront) in one launch, one
-// wavefront per front, the front in LDS (2 mm^2 doubles, sized by the launch): assembly (the
-// original entries, then the children's update matrices in child order, as k_fac_assemble adds
-// them; the front's row list staged in LDS for the searches), the pivot block's Cholesky
-// (right-looking), X = L^{-1} by columns (one lane per column), D^{-1} = X^T X, G = F_os D^{-1},
-// U = U - G F_os^T into the update workspace for the parent, and the two panel layouts in the
-// solve precision. The FP64 panel workspace is not used.
-constexpr int kSmallFront = 64;
-constexpr int kSmallBlock = 64;
+// The front in LDS (lower part, row r at r * ld) of m <= 16 NB rows, swept on its w pivots by one
+// wavefront with all of it in registers, and stored: D^{-1} and G to the sweeps' panels, U for the
+// parent. After the sweeps of block 0's columns the blocks rotate (block k to k - 1), so every
+// panel has fixed registers.
+template <int NB>
+__device__ __forceinline__ void small_front(const FacArgs &A, const FacDev &S, const double *Fs, int ld, double thr) {
+    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+    const int w = S.w, no = S.noff, m = S.m;
+    dv4 a[NB][NB];
+#pragma unroll
+    for (int I = 0; I < NB; ++I)
+#pragma unroll
+        for (int J = 0; J < NB; ++J)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int r = kIb * I + 4 * c + g, q = kIb * J + j;
+                a[I][J][c] = r < m && q < m ? Fs[max(r, q) * ld + min(r, q)] : 0.0;
+            }
+    bool bad = false;
+    int rot = 0;
+    for (int k0 = 0; k0 < w; k0 += kIb) {
+        const int left = w - k0;
+        auto panel = [&](auto tag) {
+            constexpr int C = decltype(tag)::value;
+            if (left >= 4 * C + 4) sweep_panel<NB, C, false>(a, lane, 4, left, thr, bad);
+            else if (left > 4 * C) sweep_panel<NB, C, true>(a, lane, left - 4 * C, left, thr, bad);
+        };
+        panel(std::integral_constant<int, 0>{});
+        panel(std::integral_constant<int, 1>{});
+        panel(std::integral_constant<int, 2>{});
+        panel(std::integral_constant<int, 3>{});
+        if (NB > 1) {
+            dv4 t[NB][NB];
+#pragma unroll
+            for (int I = 0; I < NB; ++I)
+#pragma unroll
+                for (int J = 0; J < NB; ++J) t[I][J] = a[(I + 1) % NB][(J + 1) % NB];
+#pragma unroll
+            for (int I = 0; I < NB; ++I)
+#pragma unroll
+                for (int J = 0; J < NB; ++J) a[I][J] = t[I][J];
+            rot = rot + 1 == NB ? 0 : rot + 1;
+        }
+    }
+    if (bad && lane == 0) *A.flag = 1;
+    MD_G double *U = A.U + S.uoff;
+    auto put = [&](MD_G void *dst, long long o, double v) {
+        if (A.solve64) static_cast<MD_G double *>(dst)[o] = v;
+        else static_cast<MD_G float *>(dst)[o] = (float)v;
+    };
+#pragma unroll
+    for (int I = 0; I < NB; ++I)
+#pragma unroll
+        for (int J = 0; J < NB; ++J) {
+            const int bi = I + rot >= NB ? I + rot - NB : I + rot, bj = J + rot >= NB ? J + rot - NB : J + rot;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int r = kIb * bi + 4 * c + g, q = kIb * bj + j;  // lanes along q
+                if (r >= m || q >= m) continue;
+                const double v = a[I][J][c];
+                if (q < w) put(A.pr, S.pr_off + (long long)r * w + q, r < w ? -v : v);
+                else if (r < w) put(A.pc, S.pc_off + (long long)r * no + (q - w), v);
+                else if (q >= r) U[(long long)(r - w) * no + (q - w)] = v;
+            }
+        }
+}
+
+// A whole height of small fronts (every m = w + noff <= mm <= 16 NBMAX) in one launch, one workgroup
+// per front: assembly in LDS (the original entries, then the children's update matrices in child
+// order, as k_fac_assemble adds them; the front's row list staged in LDS for the searches) by all of
+// its BLOCK threads, then the sweeps by its first wavefront in registers (small_front). BLOCK is 64 on
+// heights of many fronts (the leaves, which have no children) and 256 on heights of few, where the
+// additions of the children are the longer part. The FP64 panel workspace is not used.
+// 45 us for the 6,616 leaves of a 164k icosphere and 15 us for a single front of 52 columns; the
+// column-by-column Cholesky in LDS that stood here took 100 and 88 us (three barriers per column).
 constexpr int kSmallSlotLanes = 4;  // lanes per pivot column for its original entries
-__global__ __launch_bounds__(kSmallBlock) void k_fac_small(FacArgs A, int h0, int mm, int mw) {
+template <int BLOCK, int NBMAX>
+__global__ __launch_bounds__(BLOCK) void k_fac_small(FacArgs A, int h0, int mm) {
     const FacDev S = A.sn[A.hlist[h0 + blockIdx.x]];
     const int tid = threadIdx.x, w = S.w, no = S.noff, m = S.m;
-    if (m > mm || w > mw || mm > kSmallFront) {  // the host sends only heights of small fronts
+    if (m > mm || mm > kIb * NBMAX) {  // the host sends only heights of small fronts
         if (tid == 0) *A.flag = 2;
         return;
     }
+    const int ld = mm | 1;
     extern __shared__ double smem[];
-    double *Fs = smem;            // the front (lower, row stride mm), then L / D^{-1}
-    double *Xs = smem + mm * mm;  // m x w (row stride mw): X (rows < w), then G (rows >= w)
-    __shared__ int rows[kSmallFront];
-    for (int e = tid; e < no; e += kSmallBlock) rows[e] = A.offrows[S.roff + e];
-    for (int e = tid; e < m * mm; e += kSmallBlock) Fs[e] = 0.0;
+    double *Fs = smem;  // the front (lower, row stride ld)
+    __shared__ int rows[kIb * NBMAX];
+    for (int e = tid; e < no; e += BLOCK) rows[e] = A.offrows[S.roff + e];
+    for (int e = tid; e < m * ld; e += BLOCK) Fs[e] = 0.0;
     __syncthreads();
     // original entries, kSmallSlotLanes lanes per pivot column (one slot each; every front entry
     // receives at most one)
-    for (int k = tid / kSmallSlotLanes; k < w; k += kSmallBlock / kSmallSlotLanes) {
+    for (int k = tid / kSmallSlotLanes; k < w; k += BLOCK / kSmallSlotLanes) {
         const int j = S.c0 + k, sl = j / kSlice, l = j % kSlice;
-        if (tid % kSmallSlotLanes == 0) Fs[k * mm + k] = A.diag[j];
+        if (tid % kSmallSlotLanes == 0) Fs[k * ld + k] = A.diag[j];
         for (int q = A.slice_ptr[sl] + tid % kSmallSlotLanes; q < A.slice_ptr[sl + 1]; q += kSmallSlotLanes) {
             const long long g = (long long)q * kSlice + l;
             const int i = A.sell_col[g];
             if (i <= j || i >= A.nf) continue;
             const double v = -A.w64[g];
             if (i < S.c0 + w) {
-                Fs[(i - S.c0) * mm + k] += v;
+                Fs[(i - S.c0) * ld + k] += v;
             } else {
                 int lo = 0, hi = no;  // first off row >= i
                 while (lo < hi) {
@@ -2360,7 +2415,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_fac_small(FacArgs A, int h0, in
                     if (rows[mid] < i) lo = mid + 1;
                     else hi = mid;
                 }
-                if (lo < no && rows[lo] == i) Fs[(w + lo) * mm + k] += v;
+                if (lo < no && rows[lo] == i) Fs[(w + lo) * ld + k] += v;
                 else *A.flag = 2;
             }
         }
@@ -2373,87 +2428,21 @@ __global__ __launch_bounds__(kSmallBlock) void k_fac_small(FacArgs A, int h0, in
         const int nc = C.noff;
         const MD_G int *rel = A.rel + C.roff;
         const MD_G double *Uc = A.U + C.uoff;
-        for (int e = tid; e < nc * nc; e += kSmallBlock) {
+        for (int e = tid; e < nc * nc; e += BLOCK) {
             const int b = e / nc, a = e - b * nc;
             if (a < b) continue;
             const int ra = rel[a], rb = rel[b];
             if (ra >= m || rb > ra) { *A.flag = 2; continue; }
-            Fs[ra * mm + rb] += Uc[(long long)b * nc + a];
+            Fs[ra * ld + rb] += Uc[(long long)b * nc + a];
         }
         __syncthreads();
     }
-    // Cholesky of the pivot block (1 / sqrt(pivot): v_rsq_f64 and two Newton steps, kept for X)
-    const double amax = __longlong_as_double((long long)*A.amax);
-    __shared__ double rdg[kSmallFront];
-    for (int k = 0; k < w; ++k) {
-        const double piv = Fs[k * mm + k];
-        if (tid == 0 && !(piv > 1e-14 * amax)) *A.flag = 1;
-        double rd = __builtin_amdgcn_rsq(piv);
-        rd = rd * (1.5 - 0.5 * piv * rd * rd);
-        rd = rd * (1.5 - 0.5 * piv * rd * rd);
-        const double d = piv * rd;
-        __syncthreads();  // every lane has read the pivot before it changes
-        if (tid == 0) {
-            Fs[k * mm + k] = d;
-            rdg[k] = rd;
-        }
-        for (int i = k + 1 + tid; i < w; i += kSmallBlock) Fs[i * mm + k] *= rd;
-        __syncthreads();
-        const int t = w - k - 1;  // trailing lower triangle, t x t
-        for (int e = tid; e < t * t; e += kSmallBlock) {
-            const int i = k + 1 + e / t, j = k + 1 + e % t;
-            if (j <= i) Fs[i * mm + j] -= Fs[i * mm + k] * Fs[j * mm + k];
-        }
-        __syncthreads();
-    }
-    // X = L^{-1}, column i by lane i: X(r, i) = (delta_ri - sum_{i<=t<r} L(r, t) X(t, i)) / L(r, r)
-    for (int i = tid; i < w; i += kSmallBlock) {
-        for (int r = 0; r < i; ++r) Xs[r * mw + i] = 0.0;
-        for (int r = i; r < w; ++r) {
-            double acc = r == i ? 1.0 : 0.0;
-            for (int t = i; t < r; ++t) acc -= Fs[r * mm + t] * Xs[t * mw + i];
-            Xs[r * mw + i] = acc * rdg[r];
-        }
-    }
-    __syncthreads();
-    // D^{-1}(r, c) = sum_{k >= max(r, c)} X(k, r) X(k, c), over the pivot block (L is done)
-    for (int e = tid; e < w * w; e += kSmallBlock) {
-        const int r = e / w, c = e % w;
-        double acc = 0.0;
-        for (int k = max(r, c); k < w; ++k) acc += Xs[k * mw + r] * Xs[k * mw + c];
-        Fs[r * mm + c] = acc;  // the upper part too: D^{-1} is symmetric
-    }
-    __syncthreads();
-    // G(r, c) = sum_k F_os(r, k) D^{-1}(k, c) into Xs rows w + r (X is no longer needed)
-    for (int e = tid; e < no * w; e += kSmallBlock) {
-        const int r = e / w, c = e % w;
-        double acc = 0.0;
-        for (int k = 0; k < w; ++k) acc += Fs[(w + r) * mm + k] * Fs[k * mm + c];
-        Xs[(w + r) * mw + c] = acc;
-    }
-    __syncthreads();
-    // U(a, b) = U_front(a, b) - sum_k G(a, k) F_os(b, k), lower part, column-major for the parent
-    MD_G double *U = A.U + S.uoff;
-    for (int e = tid; e < no * no; e += kSmallBlock) {
-        const int b = e / no, a = e - b * no;
-        if (a < b) continue;
-        double acc = Fs[(w + a) * mm + w + b];
-        for (int k = 0; k < w; ++k) acc -= Xs[(w + a) * mw + k] * Fs[(w + b) * mm + k];
-        U[(long long)b * no + a] = acc;
-    }
-    // the sweeps' panels: row-major [D^{-1}; G] (m x w) and column-major G (no x w)
-    for (int e = tid; e < m * w; e += kSmallBlock) {
-        const int r = e / w, c = e % w;
-        const double v = r < w ? Fs[r * mm + c] : Xs[r * mw + c];
-        if (A.solve64) static_cast<MD_G double *>(A.pr)[S.pr_off + e] = v;
-        else static_cast<MD_G float *>(A.pr)[S.pr_off + e] = (float)v;
-    }
-    for (int e = tid; e < no * w; e += kSmallBlock) {
-        const int c = e / no, r = e - c * no;
-        const double v = Xs[(w + r) * mw + c];
-        if (A.solve64) static_cast<MD_G double *>(A.pc)[S.pc_off + e] = v;
-        else static_cast<MD_G float *>(A.pc)[S.pc_off + e] = (float)v;
-    }
+    if (tid >= 64) return;
+    const double thr = 1e-14 * __longlong_as_double((long long)*A.amax);
+    if (NBMAX == 1 || m <= kIb) small_front<1>(A, S, Fs, ld, thr);
+    else if (NBMAX == 2 || m <= 2 * kIb) small_front<2 < NBMAX ? 2 : NBMAX>(A, S, Fs, ld, thr);
+    else if (NBMAX == 3 || m <= 3 * kIb) small_front<3 < NBMAX ? 3 : NBMAX>(A, S, Fs, ld, thr);
+    else small_front<NBMAX>(A, S, Fs, ld, thr);
 }
 
 // Plain device copy of n 16-byte elements (grid-stride): the known-size reference kernel for
@@ -2468,27 +2457,32 @@ __global__ __launch_bounds__(kBlock) void k_copy_probe(const f4 *__restrict__ sr
 void launch_fac_diag(hipStream_t s, const FacArgs &A) {
     if (A.nf > 0) hipLaunchKernelGGL(k_fac_diag, dim3((A.nf + kBlock - 1) / kBlock), dim3(kBlock), 0, s, A);
 }
-void launch_fac_small(hipStream_t s, const FacArgs &A, int h0, int count, int mm, int mw) {
-    if (count > 0)
-        hipLaunchKernelGGL(k_fac_small, dim3(count), dim3(kSmallBlock), sizeof(double) * (mm * mm + mm * mw), s, A, h0,
-                           mm, mw);
+template <int BLOCK>
+static void fac_small_of(hipStream_t s, const FacArgs &A, int h0, int count, int mm) {
+    const size_t lds = sizeof(double) * mm * (mm | 1);
+    const dim3 grid(count), block(BLOCK);
+    if (mm <= kIb) hipLaunchKernelGGL((k_fac_small<BLOCK, 1>), grid, block, lds, s, A, h0, mm);
+    else if (mm <= 2 * kIb) hipLaunchKernelGGL((k_fac_small<BLOCK, 2>), grid, block, lds, s, A, h0, mm);
+    else if (mm <= 3 * kIb) hipLaunchKernelGGL((k_fac_small<BLOCK, 3>), grid, block, lds, s, A, h0, mm);
+    else hipLaunchKernelGGL((k_fac_small<BLOCK, 4>), grid, block, lds, s, A, h0, mm);
+}
+void launch_fac_small(hipStream_t s, const FacArgs &A, int h0, int count, int mm) {
+    if (count <= 0) return;
+    if (count > kSmallManyFronts) fac_small_of<64>(s, A, h0, count, mm);
+    else fac_small_of<256>(s, A, h0, count, mm);
 }
 void launch_fac_height(hipStream_t s, const FacArgs &A, int h0, int count, int nb, int asm_cols, int per_asm,
-                       const FacSplit &dinv, const FacSplit &g, const FacSplit &u) {
+                       const FacSplit &g, const FacSplit &u) {
     if (count <= 0) return;
     hipLaunchKernelGGL(k_fac_assemble, dim3(count * per_asm), dim3(kFacBlock), 0, s, A, h0, per_asm, asm_cols);
-    hipLaunchKernelGGL(k_fac_potrf, dim3(count), dim3(kFacBlock), 0, s, A, h0, 0);
-    // per step b: the row blocks and X blocks (X_bJ, J < b) of diagonal block b, then the trailing
-    // tiles and the W tiles of the row blocks below (W_IJ, I > b, J <= b), with diagonal block b + 1
-    for (int b = 0; b < nb; ++b) {
-        // diagonal block b is factored: by k_fac_potrf (b = 0) or by tile 0 of step b - 1's k_fac_syrk
-        const int below = nb - 1 - b;
-        if (below + b > 0)
-            hipLaunchKernelGGL(k_fac_trsm, dim3(count * (below + b)), dim3(kFacBlock), 0, s, A, h0, b, below, below + b);
-        const int tiles = below * (below + 1) / 2, wtiles = below * (b + 1);
-        if (tiles + wtiles > 0)
-            hipLaunchKernelGGL(k_fac_syrk, dim3(count * (tiles + wtiles)), dim3(kFacBlock), 0, s, A, h0, b, tiles,
-                               tiles + wtiles);
+    hipLaunchKernelGGL(k_fac_inv0, dim3(count), dim3(kFacBlock), 0, s, A, h0);
+    const int tiles = nb * (nb + 1) / 2;
+    for (int b = 0; nb > 1 && b < nb; ++b)
+        hipLaunchKernelGGL(k_fac_step, dim3(count * tiles), dim3(kFacBlock), 0, s, A, h0, b, tiles);
+    if (g.per <= 0) return;
+    if (nb == 1) {
+        hipLaunchKernelGGL(k_fac_gu, dim3(count * u.per), dim3(kFacBlock), 0, s, A, h0, u.per);
+        return;
     }
     // the products, split over K where ks > 1
     auto product = [&](auto plain, auto part, auto fix, const FacSplit &p) {
@@ -2499,11 +2493,8 @@ void launch_fac_height(hipStream_t s, const FacArgs &A, int h0, int count, int n
             hipLaunchKernelGGL(plain, dim3(count * p.per), dim3(kFacBlock), 0, s, A, h0, p.per, 1);
         }
     };
-    product(k_fac_dinv<0>, k_fac_dinv<1>, k_fac_dinv<2>, dinv);
-    if (g.per > 0) {
-        product(k_fac_g<0>, k_fac_g<1>, k_fac_g<2>, g);
-        product(k_fac_u<0>, k_fac_u<1>, k_fac_u<2>, u);
-    }
+    product(k_fac_g<0>, k_fac_g<1>, k_fac_g<2>, g);
+    product(k_fac_u<0>, k_fac_u<1>, k_fac_u<2>, u);
 }
 
 void launch_copy_probe(hipStream_t s, const void *src, void *dst, long long n16) {

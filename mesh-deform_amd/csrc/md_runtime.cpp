@@ -890,28 +890,27 @@ int factor_device(md_mesh *m) {
     // products one per 64 x 64 output tile), and the products' splits over K
     struct HeightLaunch {
         int count, mw, mm, asm_cols;
-        FacSplit dinv, g, u;
+        FacSplit g, u;
     };
     const int nh = (int)f.hptr.size() - 1;
     std::vector<HeightLaunch> hl(nh);
     size_t nW = 0;
     for (int h = 0; h < nh; ++h) {
         HeightLaunch &L = hl[h];
-        L = HeightLaunch{f.hptr[h + 1] - f.hptr[h], 0, 1, 64, {1, 1}, {0, 1}, {0, 1}};
+        L = HeightLaunch{f.hptr[h + 1] - f.hptr[h], 0, 1, 64, {0, 1}, {0, 1}};
         auto lower = [](int b) { return b * (b + 1) / 2; };
         for (int i = f.hptr[h]; i < f.hptr[h + 1]; ++i) {
             const int w = f.w[f.hlist[i]], no = f.noff[f.hlist[i]];
             const int bw = (w + 63) / 64, bo = (no + 63) / 64;
             L.mw = std::max(L.mw, w);
             L.mm = std::max(L.mm, w + no);
-            L.dinv.per = std::max(L.dinv.per, lower(bw));
             L.g.per = std::max(L.g.per, bo * bw);
             L.u.per = std::max(L.u.per, lower(bo));
         }
         if (L.mm <= kFacSmallFront) continue;  // small fronts only: one fused launch
         while (L.asm_cols > 8 && (long long)L.count * ((L.mm + L.asm_cols - 1) / L.asm_cols) < 2048) L.asm_cols /= 2;
         const int chunks = (L.mw + 31) / 32;
-        for (FacSplit *p : {&L.dinv, &L.g, &L.u}) {
+        for (FacSplit *p : {&L.g, &L.u}) {
             if (p->per == 0) continue;
             p->ks = fac_split_k((long long)L.count * p->per, chunks);
             if (p->ks > 1) nW = std::max(nW, (size_t)fac_split_k_doubles((long long)L.count * p->per * p->ks));
@@ -947,11 +946,11 @@ int factor_device(md_mesh *m) {
         for (int h = 0; h < nh; ++h) {
             const HeightLaunch &L = hl[h];
             if (L.mm <= kFacSmallFront) {  // small fronts only: one fused launch
-                launch_fac_small(st, A, f.hptr[h], L.count, L.mm, L.mw);
+                launch_fac_small(st, A, f.hptr[h], L.count, L.mm);
                 continue;
             }
             launch_fac_height(st, A, f.hptr[h], L.count, (L.mw + 63) / 64, L.asm_cols,
-                              (L.mm + L.asm_cols - 1) / L.asm_cols, L.dinv, L.g, L.u);
+                              (L.mm + L.asm_cols - 1) / L.asm_cols, L.g, L.u);
         }
         e = hipGetLastError();
     }
