@@ -460,6 +460,9 @@ void symbolic(int n, const std::vector<int>& ptr, const std::vector<int>& adj, F
     {
         std::vector<int> fill(f.hptr.begin(), f.hptr.end() - 1);
         for (int t = 0; t < nn; ++t) f.hlist[fill[f.height[t]]++] = t;
+        for (int h = 0; h < f.nlevels; ++h)
+            std::stable_sort(f.hlist.begin() + f.hptr[h], f.hlist.begin() + f.hptr[h + 1],
+                             [&](int a, int b) { return f.w[a] + f.noff[a] < f.w[b] + f.noff[b]; });
     }
     f.woff_s.assign(nn + 1, 0); f.woff_t.assign(nn + 1, 0); f.woff_u.assign(nn + 1, 0);
     for (int t = 0; t < nn; ++t) {

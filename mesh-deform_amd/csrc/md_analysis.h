@@ -112,7 +112,7 @@ struct Factor {
     // supernodes of that height; per supernode the offsets of its workspace blocks: the
     // off-diagonal front block (noff x w), the pivot block's second workspace of the sweeps
     // (w x w) and the update matrix for the parent (noff x noff), all column-major FP64
-    std::vector<int> hptr, hlist;    // height h: hlist[hptr[h] .. hptr[h+1])
+    std::vector<int> hptr, hlist;    // height h: hlist[hptr[h] .. hptr[h+1]), by rows of the front
     std::vector<int64_t> woff_s, woff_t, woff_u;  // ns + 1 each
     std::vector<int> col_sn;         // supernode of each column
     // device layout

@@ -92,29 +92,35 @@ struct MeshDev {
     double pcg_tol2;            // stop (freeze) when r.z <= tol^2 * (r.z)_0, per coordinate
 };
 
-// Device numeric factorization (multifrontal, FP64): per supernode record and the buffers.
+// Device numeric factorization (multifrontal, FP64): per supernode record (stored by height, so a
+// workgroup's is one load) and the buffers.
 struct FacDev {
     int c0, w, noff, roff;          // columns, off rows (offrows[roff ..], rel[roff ..])
-    int cb, ce, m, pad;             // children child[cb .. ce), m = w + noff
-    long long poff, soff, toff, uoff;  // FP64 panel (m x w), F_os copy (noff x w), the pivot block's
-                                       // second workspace (w x w), update matrix (noff x noff); all
-                                       // column-major
+    int cb, ce, m, pad;             // children FacArgs::child[cb .. ce), m = w + noff
+    long long poff, soff, toff, uoff;  // the front's first w columns (m x w), their second workspace
+                                       // (off rows, noff x w; pivot rows, w x w), update matrix (noff x
+                                       // noff); all column-major
     long long pc_off, pr_off;       // solve-precision panels of the sweeps
 };
 
+// A child as its parent's assembly reads it: rows, their map in rel, update matrix.
+struct FacChild {
+    int noff, roff;
+    long long uoff;
+};
+
 struct FacArgs {
-    const MD_G FacDev *sn;
-    const MD_G int *hlist;          // supernodes by height
-    const MD_G int *offrows, *rel, *child;
+    const MD_G FacDev *sn;          // by height
+    const MD_G FacChild *child;
+    const MD_G int *offrows, *rel;
     const MD_G int *slice_ptr, *sell_col;
     const MD_G double *w64;         // cotan weights over the one-ring slots
     int nf;
     MD_G double *P, *S, *T, *U, *diag;
     MD_G unsigned long long *amax;  // max |L_ii| as the bits of a non-negative double
     MD_G int *flag;                 // 1: a pivot block is not positive definite; 2: structure
-    MD_G void *pc, *pr;             // the sweeps' panels (float or double), written by the D^{-1}
-    int solve64;                    //   and G kernels in the solve precision (1: double)
-    MD_G double *Wk;                // partial products of the split-K launches (fac_split_k_doubles)
+    MD_G void *pc, *pr;             // the sweeps' panels (float or double), written in the solve
+    int solve64;                    //   precision (1: double)
 };
 
 // A set of meshes processed by one launch. Block b belongs to mesh k where
@@ -157,37 +163,44 @@ void launch_pcg_init(hipStream_t s, LaunchSet L, int blocks, bool fp64);
 void launch_pcg_step(hipStream_t s, LaunchSet L, int blocks, int step, bool fp64);
 void launch_pcg_apply(hipStream_t s, LaunchSet L, int blocks, bool fp64);
 // Device numeric factorization: diagonal and its maximum, then per height (the `count`
-// supernodes from hlist[h0]) the front assembly, the pivot blocks' inverses, G and the update
-// matrices (one workgroup per output tile, or several split over K); D^{-1} and G also go to the
-// solve-precision panels.
+// supernodes from sn[h0]) the front assembly and the block sweeps, whose last step writes D^{-1} and G
+// to the solve-precision panels.
 void launch_fac_diag(hipStream_t s, const FacArgs &A);
-// A product stage of a height: workgroups per supernode (one per 64 x 64 output tile, lower tiles
-// for the symmetric ones; the height's most) and splits over K (1: none); a split stage needs
-// fac_split_k_doubles(count * per * ks) doubles at A.Wk.
-struct FacSplit {
-    int per, ks;
+// The assembly of a height of `count` fronts of at most mm rows, at most `no` of them off rows, with
+// at most `maps` = children x rows of one front: `per` workgroups per front, each `cols` columns by one
+// of rch ranges of rlen rows. 64 columns, halved down to 4 (one quad for the four wavefronts) while
+// the height has fewer than 4,096 workgroups: the top heights' few fronts take the largest children.
+// ninv LDS entries hold the inverted row maps (as many children at a time as fit, at most 32 KB),
+// nrows the front's row list.
+constexpr int kAsmInv = 8192, kAsmRows = 4096, kAsmWorkgroups = 4096;
+struct FacAssembly {
+    int per, cols, rch, rlen, ninv, nrows;
 };
-// One height: assembly (per_asm workgroups per supernode, one per asm_cols front columns), the
-// pivot blocks' inverses D^{-1} by block sweeps (nb = column blocks of 64 in the widest one), G and
-// the update matrices (g.per = 0 when no supernode of the height has off rows).
-void launch_fac_height(hipStream_t s, const FacArgs &A, int h0, int count, int nb, int asm_cols, int per_asm,
-                       const FacSplit &g, const FacSplit &u);
-// Split of a product over K: `tiles` output tiles of 64 x 64 and `chunks` chunks of K (32 values).
-// Splits only launches of few tiles (tiles x 2 <= kSplitWorkgroups) with at least 8 chunks, into
-// shares of at least 4 chunks, at most kSplitWorkgroups workgroups in all.
-constexpr int kSplitWorkgroups = 1024;
-inline int fac_split_k(long long tiles, int chunks) {
-    if (tiles <= 0 || tiles * 2 > kSplitWorkgroups || chunks < 8) return 1;
-    const long long ks = std::min<long long>(chunks / 4, kSplitWorkgroups / tiles);
-    return ks > 1 ? (int)ks : 1;
+inline FacAssembly fac_assembly(int count, int mm, int no, long long maps) {
+    FacAssembly a;
+    a.rlen = std::min(mm, kAsmInv);
+    a.rch = (mm + a.rlen - 1) / a.rlen;
+    a.cols = 64;
+    while (a.cols > 4 && (long long)count * ((mm + a.cols - 1) / a.cols) < kAsmWorkgroups) a.cols /= 2;
+    a.per = (mm + a.cols - 1) / a.cols * a.rch;
+    a.ninv = (int)std::max<long long>(a.rlen, std::min<long long>(kAsmInv, maps));
+    a.nrows = std::min(kAsmRows, no);
+    return a;
 }
-constexpr long long fac_split_k_doubles(long long workgroups) { return workgroups * 16 * 256; }
-// A height whose fronts all have m <= mm <= kFacSmallFront: every step of launch_fac_height for one
-// front in one workgroup (of one wavefront on heights of more than kSmallManyFronts fronts, else
+// One height: assembly, then the block sweeps of its fronts, nb launches (column blocks of 64 in the
+// widest pivot block) of `tiles` workgroups per front (lower 64 x 64 tiles of the largest, pivot rows
+// and off rows each rounded up).
+void launch_fac_height(hipStream_t s, const FacArgs &A, int h0, int count, int nb, const FacAssembly &as, int tiles);
+// Fronts of m <= mm <= kFacSmallFront rows: every step of launch_fac_height for one front in one
+// workgroup (of one wavefront on heights of more than kSmallManyFronts fronts, else
 // of four), without the FP64 panel workspace.
 constexpr int kFacSmallFront = 64;
 constexpr int kSmallManyFronts = 1024;
 void launch_fac_small(hipStream_t s, const FacArgs &A, int h0, int count, int mm);
+// Whether a height's `small` such fronts of `all` leave its general launches for the fused one: when
+// they are all of it, or at least 512 and the larger part (the 164k icosphere's second and third
+// heights: 116 and 114 us split, 140 and 152 together; a smaller share only adds a launch).
+inline bool fac_split_small(int small, int all) { return small == all || (small >= 512 && 2 * small >= all); }
 // Internal-order vectors (positions, normals) to packed xyz in original order (perm: original
 // id per internal id), and packed xyz to internal order (p and/or pp; pp takes the targets tgt,
 // internal order, for the constrained ids [nf, n)).

@@ -1425,23 +1425,22 @@ __global__ __launch_bounds__(kBlock) void k_scatter_entries(const TargetEntry *e
 // children's update matrices are added in child order, so the factor is deterministic.
 
 constexpr int kFacBlock = 256;
-constexpr int kAsmU = 8;      // child update entries per assembly thread in flight
-constexpr int kAsmRows = 2048;  // off rows of a front searched in LDS (longer lists: in memory)
 
 constexpr int kFb = 64;  // columns of a pivot block swept at a time
 
-// A front's pivot block during the sweeps: step s reads one of its two workspaces (P, rows m apart,
-// and T, rows w apart, column-major) and writes the other, so no workgroup overwrites what another
-// still reads; step nb - 1 writes P. Block (s, s) of the workspace that step s reads holds
-// S = A_ss^{-1} (its inverse is formed where the block is completed).
-struct PivotBuf {
-    MD_G double *p;
-    long long ld;
+
+// The first w columns of a front during the sweeps: step s reads one of two workspaces (P, all rows m
+// apart; T, pivot rows w apart, with S, off rows noff apart; column-major) and writes the other, so no
+// workgroup overwrites what another still reads. Block (s, s) of the workspace that step s reads holds
+// A_ss^{-1} (the inverse is formed where the block is completed). The front's other columns, the update
+// matrix, are updated in place.
+struct FrontBuf {
+    MD_G double *d, *f;  // pivot rows, off rows
+    long long ldd, ldf;
 };
-__device__ __forceinline__ PivotBuf pivot_buf(const FacArgs &A, const FacDev &S, int s) {
-    const int nb = (S.w + kFb - 1) / kFb;
-    if ((nb - s) & 1) return PivotBuf{A.T + S.toff, S.w};
-    return PivotBuf{A.P + S.poff, S.m};
+__device__ __forceinline__ FrontBuf front_buf(const FacArgs &A, const FacDev &S, int s) {
+    if (s & 1) return FrontBuf{A.T + S.toff, A.S + S.soff, S.w, S.noff};
+    return FrontBuf{A.P + S.poff, A.P + S.poff + S.w, S.m, S.m};
 }
 
 // L_jj = sum of the weights of every neighbour of j, in slot order, and their maximum.
@@ -1458,136 +1457,183 @@ __global__ __launch_bounds__(kBlock) void k_fac_diag(FacArgs A) {
     atomicMax(A.amax, (unsigned long long)__double_as_longlong(fabs(acc)));
 }
 
-// Front of each supernode of one height: the pivot block and G rows (panel), F_os (copy),
-// the update matrix; original entries (L_jj and -w_ij for free i > j, slot order) first,
-// then the children's update matrices in child order. `per` workgroups per supernode, each
-// owning `cols` columns of the front (pivot columns: P and F; later ones: U), so no two write
-// the same entry and every entry receives its additions in that fixed order.
-constexpr int kAsmSlotLanes = 16;  // threads per pivot column for its original entries
-constexpr int kAsmChildren = 64;   // children whose records are staged in LDS at a time
-__global__ __launch_bounds__(kFacBlock) void k_fac_assemble(FacArgs A, int h0, int per, int cols) {
-    const FacDev S = A.sn[A.hlist[h0 + blockIdx.x / per]];
-    const int tid = threadIdx.x, w = S.w, no = S.noff, m = S.m;
-    const int t0 = (int)(blockIdx.x % per) * cols, t1 = min(m, t0 + cols);
-    if (t0 >= m) return;
-    const PivotBuf D = pivot_buf(A, S, 0);  // where the sweeps start
-    MD_G double *P = D.p, *F = A.S + S.soff, *U = A.U + S.uoff;
-    const long long ldp = D.ld;
+// Front of each supernode of one height: its first w columns and the update matrix, lower part: for
+// each entry the original one (L_jj and -w_ij for free i > j), then
+// the children's update entries in child order. A gather: the children's row maps are inverted in LDS
+// (front row -> row of the child, -1 where it has none), every entry is summed by one lane in a
+// register and written once, so there is no zeroing, no read-modify-write and no barrier between
+// children. `per` workgroups per front, each `cols` columns (by rch ranges of rlen rows where one
+// child's inverse map would not fit); a wavefront takes four columns by 64 rows at a time, whose
+// children follow from one ballot, two children's entries (eight loads) in flight.
+// Bound by round trips (record, children, maps, entries): 7 us for a few fronts of 100 rows and 29 us a
+// height on average on the 164k icosphere, where scattering into the front in memory, child by child,
+// took 13 and 41.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+constexpr int kAsmAhead = 3;   // children whose entries are loaded together (four columns each)
+constexpr int kAsmBatch = 64;  // children whose maps are inverted at a time (one per lane)
+__global__ __launch_bounds__(kFacBlock) void k_fac_assemble(FacArgs A, int h0, FacAssembly as) {
+    const FacDev S = A.sn[h0 + blockIdx.x / as.per];
+    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, w = S.w, no = S.noff, m = S.m;
+    const int part = (int)(blockIdx.x % as.per), t0 = part / as.rch * as.cols, t1 = min(m, t0 + as.cols);
+    const int r0 = max(t0, part % as.rch * as.rlen), r1 = min(m, (part % as.rch + 1) * as.rlen), len = r1 - r0;
+    if (t0 >= m || len <= 0) return;
+    MD_G double *P = A.P + S.poff, *U = A.U + S.uoff;
     const MD_G int *rows = A.offrows + S.roff;
-    // the front's row list in LDS for the searches of the original entries (pivot columns), and
-    // each child's row map in turn
-    __shared__ int rsh[kAsmRows];
-    __shared__ int relsh[kAsmRows];
-    // the children's (rows, row map, update matrix) records, kAsmChildren at a time (the first
-    // batch loaded up front, beside the zeroing)
-    __shared__ int chn[kAsmChildren], chr[kAsmChildren];
-    __shared__ long long chu[kAsmChildren];
-    const int nch = S.ce - S.cb;
-    auto stage_children = [&](int c0) {
-        if (tid < min(nch - c0, kAsmChildren)) {
-            const FacDev C = A.sn[A.child[S.cb + c0 + tid]];
-            chn[tid] = C.noff;
-            chr[tid] = C.roff;
-            chu[tid] = C.uoff;
-        }
-    };
-    static_assert(kAsmChildren <= kFacBlock, "one child record per thread");
-    stage_children(0);
-    const bool staged = t0 < w && no <= kAsmRows;
+    extern __shared__ int inv[];        // row r of child c of the batch at c * len + r - r0
+    __shared__ double obuf[4][4][64];   // original entries of a wavefront's quad
+    int *rsh = inv + as.ninv;           // the front's row list, for the searches of the original entries
+    const bool staged = t0 < w && no <= as.nrows;
     if (staged)
         for (int e = tid; e < no; e += kFacBlock) rsh[e] = rows[e];
-    // zero the owned columns: contiguous ranges of P and F (pivot columns) and of U
-    const int kend = min(t1, w);
-    if (t0 < w) {
-        for (long long e = t0 * ldp + tid; e < kend * ldp; e += kFacBlock) P[e] = 0.0;
-        for (long long e = (long long)t0 * no + tid; e < (long long)kend * no; e += kFacBlock) F[e] = 0.0;
-    }
-    if (t1 > w)
-        for (long long e = (long long)(max(t0, w) - w) * no + tid; e < (long long)(t1 - w) * no; e += kFacBlock)
-            U[e] = 0.0;
-    __syncthreads();
-    // original entries, kAsmSlotLanes threads per pivot column (one slot each); each entry of the
-    // front receives at most one, right after its zero, so it is stored
-    for (int k = t0 + tid / kAsmSlotLanes; k < kend; k += kFacBlock / kAsmSlotLanes) {
-        const int j = S.c0 + k, sl = j / kSlice, l = j % kSlice;
-        if (tid % kAsmSlotLanes == 0) P[k * ldp + k] = A.diag[j];
-        for (int q = A.slice_ptr[sl] + tid % kAsmSlotLanes; q < A.slice_ptr[sl + 1]; q += kAsmSlotLanes) {
-            const long long g = (long long)q * kSlice + l;
-            const int i = A.sell_col[g];
-            if (i <= j || i >= A.nf) continue;
-            const double v = -A.w64[g];
-            if (i < S.c0 + w) {
-                P[k * ldp + (i - S.c0)] = v;
-            } else {
+    // waves over column quads first, then over their row chunks
+    const int nq = (t1 - t0 + 3) / 4, wq = min(4, nq >= 3 ? 4 : nq), wc = 4 / wq;
+    const int nch = S.ce - S.cb, cap = min(kAsmBatch, as.ninv / len);
+    int cb = 0;
+    do {
+        const int nb = min(nch - cb, cap);
+        FacChild C{0, 0, 0};
+        if (lane < nb) C = A.child[S.cb + cb + lane];
+        if (cb > 0) __syncthreads();  // the previous batch's maps are read
+        for (int e = tid; e < nb * len; e += kFacBlock) inv[e] = -1;
+        __syncthreads();
+        for (int c = wv; c < nb; c += 4) {
+            const int nc = __builtin_amdgcn_readlane(C.noff, c), roff = __builtin_amdgcn_readlane(C.roff, c);
+            for (int a = lane; a < nc; a += 64) {
+                const int r = A.rel[roff + a];
+                if (r >= r0 && r < r1) inv[c * len + r - r0] = a;
+                if (r >= m) *A.flag = 2;
+            }
+        }
+        __syncthreads();
+        for (int q = wv % wq; q < nq; q += wq) {
+            const int tq = t0 + 4 * q;
+            // rows of the quad's columns in the children (lane: child), -1: none
+            int cbm[4];
+            unsigned long long any = 0;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int t = tq + g;
+                cbm[g] = -1;
+                if (lane < nb && t < t1) {
+                    if (t >= r0 && t < r1) {
+                        cbm[g] = inv[lane * len + t - r0];
+                    } else {  // above a later row range
+                        int lo = 0, hi = C.noff;
+                        while (lo < hi) {
+                            const int mid = (lo + hi) >> 1;
+                            if (A.rel[C.roff + mid] < t) lo = mid + 1;
+                            else hi = mid;
+                        }
+                        if (lo < C.noff && A.rel[C.roff + lo] == t) cbm[g] = lo;
+                    }
+                }
+                any |= __ballot(cbm[g] >= 0);
+            }
+            // original entries of pivot columns: lane 16 g + i holds slot i of column tq + g (and of
+            // i + 16, ... below): its front row, or -1
+            const int og = lane >> 4, ot = tq + og, oi = lane & 15;
+            const bool opiv = cb == 0 && ot < min(w, t1);
+            const int oj = S.c0 + ot, osl = opiv ? oj / kSlice : 0, ol = oj % kSlice;
+            const int oq0 = opiv ? A.slice_ptr[osl] : 0, oq1 = opiv ? A.slice_ptr[osl + 1] : 0;
+            auto original = [&](int x, int &row, double &val) {
+                row = -1;
+                val = 0.0;
+                if (oq0 + x >= oq1) return;
+                const long long gs = (long long)(oq0 + x) * kSlice + ol;
+                const int i = A.sell_col[gs];
+                if (i <= oj || i >= A.nf) return;
+                val = -A.w64[gs];
+                row = i - S.c0;
+                if (row < w) return;
                 int lo = 0, hi = no;  // first off row >= i
                 while (lo < hi) {
                     const int mid = (lo + hi) >> 1;
                     if ((staged ? rsh[mid] : rows[mid]) < i) lo = mid + 1;
                     else hi = mid;
                 }
-                if (lo < no && (staged ? rsh[lo] : rows[lo]) == i) F[(long long)k * no + lo] = v;
-                else *A.flag = 2;
-            }
-        }
-    }
-    __syncthreads();
-    // children's update matrices, child by child: the child's lower entries (a >= b) of its
-    // columns b landing in [t0, t1) (rel is increasing, so they are the columns [blo, bend),
-    // counted over the workgroup), flattened over the workgroup, kAsmU entries per thread in
-    // flight (their loads, then the read-modify-writes: distinct entries of one child land on
-    // distinct front entries)
-    for (int c = 0; c < nch; ++c) {
-        if (c > 0 && c % kAsmChildren == 0) {  // the previous child's loop ended with a barrier
-            stage_children(c);
-            __syncthreads();
-        }
-        const int nc = chn[c % kAsmChildren], roff = chr[c % kAsmChildren];
-        const long long uoff = chu[c % kAsmChildren];
-        const MD_G int *relg = A.rel + roff;
-        const bool rstaged = nc <= kAsmRows;
-        int blo = 0, bend = 0;
-        for (int a0 = 0; a0 < nc; a0 += kFacBlock) {
-            const int a = a0 + tid;
-            const int r = a < nc ? relg[a] : m;
-            if (rstaged && a < nc) relsh[a] = r;
-            blo += __syncthreads_count(r < t0);
-            bend += __syncthreads_count(r < t1);
-        }
-        const MD_G double *Uc = A.U + uoff;
-        const int total = (bend - blo) * nc;
-        for (int e0 = tid; e0 < total; e0 += kFacBlock * kAsmU) {
-            double v[kAsmU];
-            MD_G double *dst[kAsmU];
+                if (lo < no && (staged ? rsh[lo] : rows[lo]) == i) row = w + lo;
+                else { row = -1; *A.flag = 2; }
+            };
+            int orow;
+            double oval;
+            original(oi, orow, oval);
+            const double odiag = opiv && oi == 0 ? A.diag[oj] : 0.0;
+            for (int ch = wv / wq; tq + 64 * ch < r1; ch += wc) {
+                double acc[4];
+                int r[4];
+                bool on[4];
+                MD_G double *dst[4];
 #pragma unroll
-            for (int u = 0; u < kAsmU; ++u) {
-                const int e = e0 + u * kFacBlock, bb = e / nc, a = e - bb * nc, b = blo + bb;
-                dst[u] = nullptr;
-                v[u] = 0.0;
-                if (e < total && a >= b) {
-                    const int ra = rstaged ? relsh[a] : relg[a], rb = rstaged ? relsh[b] : relg[b];
-                    v[u] = Uc[(long long)b * nc + a];
-                    if (ra >= m || rb > ra) *A.flag = 2;
-                    else if (rb < w) dst[u] = ra < w ? P + rb * ldp + ra : F + (long long)rb * no + (ra - w);
-                    else dst[u] = U + (long long)(rb - w) * no + (ra - w);
+                for (int g = 0; g < 4; ++g) {
+                    const int t = tq + g;
+                    r[g] = t + 64 * ch + lane;
+                    on[g] = t < t1 && r[g] >= r0 && r[g] < r1;
+                    dst[g] = t >= w ? U + (long long)(t - w) * no + (r[g] - w) : P + (long long)t * m + r[g];
+                    acc[g] = cb > 0 && on[g] ? *dst[g] : 0.0;
                 }
+                if (cb == 0 && tq < w) {
+                    // through LDS: clear the quad's 4 x 64 entries, put the original ones, take them
+                    // (one wavefront: its LDS accesses are in order)
+                    double (*ob)[64] = obuf[wv];
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) ob[g][lane] = 0.0;
+                    wave_lds_fence();
+                    const int lo = ot + 64 * ch;
+                    if (opiv && oi == 0 && ch == 0) ob[og][0] = odiag;
+                    if (orow >= lo && orow < lo + 64) ob[og][orow - lo] = oval;
+                    for (int x = oi + 16; __any(oq0 + x < oq1); x += 16) {
+                        int row;
+                        double val;
+                        original(x, row, val);
+                        if (row >= lo && row < lo + 64) ob[og][row - lo] = val;
+                    }
+                    wave_lds_fence();
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) acc[g] = ob[g][lane];
+                    wave_lds_fence();
+                }
+                for (unsigned long long todo = any; todo;) {
+                    double v[kAsmAhead][4];
+#pragma unroll
+                    for (int k = 0; k < kAsmAhead; ++k) {
+                        const bool has = todo != 0;
+                        const int c = has ? __builtin_ctzll(todo) : 0;
+                        todo &= todo - 1;
+                        const int nc = __builtin_amdgcn_readlane(C.noff, c);
+                        const unsigned long long uo =
+                            (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)C.uoff, c) |
+                            (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(C.uoff >> 32), c) << 32;
+                        const MD_G double *Uc = A.U + (long long)uo;
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            const int bcol = __builtin_amdgcn_readlane(cbm[g], c);
+                            const int a = has && bcol >= 0 && on[g] ? inv[c * len + r[g] - r0] : -1;
+                            v[k][g] = a >= 0 ? Uc[(long long)bcol * nc + a] : 0.0;
+                        }
+                    }
+#pragma unroll
+                    for (int k = 0; k < kAsmAhead; ++k)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) acc[g] += v[k][g];
+                }
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    if (on[g]) *dst[g] = acc[g];
             }
-            double old[kAsmU];
-#pragma unroll
-            for (int u = 0; u < kAsmU; ++u) old[u] = dst[u] ? *dst[u] : 0.0;
-#pragma unroll
-            for (int u = 0; u < kAsmU; ++u)
-                if (dst[u]) *dst[u] = old[u] + v[u];
         }
-        __syncthreads();
-    }
+        cb += nb;
+    } while (cb < nch);
 }
 
-// Pivot blocks are inverted by symmetric block sweeps. A sweep on the columns of block s with
-// S = A_ss^{-1} maps A_ss -> -S, A_Is -> A_Is S, A_IJ -> A_IJ - A_Is S A_Js^T; it keeps the matrix
-// symmetric, and after the sweeps on every block A is -A^{-1}. Swept at 64 columns over the front's
-// pivot block (k_fac_inv0, k_fac_step), at 16 within a 64 x 64 block (invert64), at 4 within a
-// 16 x 16 block (sweep_panel). k_fac_small sweeps a whole small front by panels of 4 pivots, which
-// leaves [-D^{-1}, G^T; G, U] in place.
+// Fronts are factored by symmetric block sweeps. A sweep on the columns of block s with S = A_ss^{-1}
+// maps A_ss -> -S, A_Is -> A_Is S, A_IJ -> A_IJ - A_Is S A_Js^T; it keeps the matrix symmetric, and
+// after the sweeps on a front's pivot blocks it holds [-D^{-1}, G^T; G, U]: the sweeps' panels and the
+// update matrix for the parent. Swept at 64 columns over the front (k_fac_inv0, k_fac_step), at 16
+// within a 64 x 64 block (invert64), at 4 within a 16 x 16 block (sweep_panel); k_fac_small sweeps a
+// whole small front by panels of 4 pivots.
 // LDS rows of the 64 x 64 operands, in doubles (odd: a column of a row-major tile hits 32 banks)
 constexpr int kLdT = kFb + 1;
 
@@ -1715,69 +1761,19 @@ struct InvLds {
 };
 static_assert(kFb == 4 * kIb, "one block column of 16 per wavefront");
 
-// Step K of invert64: wave K sweeps its diagonal block and publishes its inverse and the block
-// column; after one barrier the other waves form T_J = S A_KJ and update their columns,
-// A_IJ -= A_IK T_J, and wave K forms A_IK S.
-template <int K>
-__device__ __forceinline__ void invert64_step(dv4 (&acc)[4], InvLds &L, int wv, int lane, int b, double thr, bool &bad) {
-    if (kIb * K >= b) return;  // past a partial block: identity, untouched
-    const int j = lane & 15, g = lane >> 4, buf = K & 1;
-    if (wv == K) {
-#pragma unroll
-        for (int I = 0; I < 4; ++I)
-            if (I != K)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) L.a[buf][I][4 * c + g][j] = acc[I][c];
-        dv4 d[1][1];
-        d[0][0] = acc[K];
-        const int real = b - kIb * K;
-        sweep_panel<1, 0, false>(d, lane, 4, real, thr, bad);
-        sweep_panel<1, 1, false>(d, lane, 4, real, thr, bad);
-        sweep_panel<1, 2, false>(d, lane, 4, real, thr, bad);
-        sweep_panel<1, 3, false>(d, lane, 4, real, thr, bad);
-        acc[K] = d[0][0];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) L.s[buf][4 * c + g][j] = -acc[K][c];
-    }
-    __syncthreads();
-    if (wv == K) {
-        dv4 t[4];
-#pragma unroll
-        for (int I = 0; I < 4; ++I) t[I] = dv4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int I = 0; I < 4; ++I)
-                if (I != K) t[I] = MD_MFMA64(L.a[buf][I][j][4 * c + g], -acc[K][c], t[I]);
-#pragma unroll
-        for (int I = 0; I < 4; ++I)
-            if (I != K) acc[I] = t[I];
-    } else {
-        dv4 t = dv4{0.0, 0.0, 0.0, 0.0}, t2 = t;
-#pragma unroll
-        for (int c = 0; c < 4; c += 2) {
-            t = MD_MFMA64(L.s[buf][j][4 * c + g], acc[K][c], t);
-            t2 = MD_MFMA64(L.s[buf][j][4 * c + 4 + g], acc[K][c + 1], t2);
-        }
-        t += t2;
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int I = 0; I < 4; ++I)
-                if (I != K) acc[I] = MD_MFMA64(-L.a[buf][I][j][4 * c + g], t[c], acc[I]);
-        acc[K] = t;
-    }
-}
-
 static_assert(kFacBlock == 4 * 64, "four wavefronts");
 
 // The symmetric 64 x 64 block in m (lower part, row r at r * kLdT) replaced by minus its inverse
 // in the layout of D: wave v holds block column v in acc. b < 64: the leading b x b block (rows and
-// columns past it are taken as the identity). Ends without a barrier; work may not alias m.
-// A chain of b pivots: one 64 x 64 block takes about 9 us, 2.9 of it sixteen panel sweeps' worth of
-// dependent FP64 arithmetic per 16 columns (740 cycles per panel of 4, DPP and permlane broadcasts
-// in place of LDS), the rest the updates between (one v_mfma_f64_16x16x4 per 16 cycles and CU). The
-// unscaled LDL^T with a blocked triangular inverse that stood here took 14 us, plus X^T X.
+// columns past it are taken as the identity, and 16-blocks past it are not swept). Ends without a
+// barrier; work may not alias m. Step K: wave K sweeps its diagonal block and publishes its inverse
+// and the block column; after one barrier the other waves form T_J = S A_KJ and update their columns,
+// A_IJ -= A_IK T_J, and wave K forms A_IK S. A loop over K: the block rows rotate (row K is acc[0]), for
+// nothing, since an MFMA may write another register than it adds to; unrolled, the code of this and its
+// callers outgrew the instruction cache, and its fetch was a third of a launch.
+// A chain of b pivots: per 16 of them 2,950 cycles of dependent FP64 arithmetic in the panel sweeps
+// (DPP and permlane broadcasts in place of LDS) and 1,900 for the exchange and the updates (one
+// v_mfma_f64_16x16x4 per 16 cycles and CU).
 __device__ __forceinline__ void invert64(const double *m, InvLds &work, int b, double thr, dv4 (&acc)[4], bool &bad) {
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
 #pragma unroll
@@ -1787,32 +1783,65 @@ __device__ __forceinline__ void invert64(const double *m, InvLds &work, int b, d
             const int r = kIb * I + 4 * c + g, q = kIb * wv + j;
             acc[I][c] = r < b && q < b ? m[max(r, q) * kLdT + min(r, q)] : r == q ? 1.0 : 0.0;
         }
-    invert64_step<0>(acc, work, wv, lane, b, thr, bad);
-    invert64_step<1>(acc, work, wv, lane, b, thr, bad);
-    invert64_step<2>(acc, work, wv, lane, b, thr, bad);
-    invert64_step<3>(acc, work, wv, lane, b, thr, bad);
-}
-
-// Entry (r, c), r >= c, of D^{-1}: both triangles of the panel's pivot block and of the backward
-// panel [D^{-1}; G] (row-major) in the solve precision.
-__device__ __forceinline__ void put_dinv(const FacArgs &A, const FacDev &S, int r, int c, double v) {
-    MD_G double *P = A.P + S.poff;
-    P[(long long)c * S.m + r] = v;
-    P[(long long)r * S.m + c] = v;
-    const long long o1 = S.pr_off + (long long)r * S.w + c, o2 = S.pr_off + (long long)c * S.w + r;
-    if (A.solve64) {
-        static_cast<MD_G double *>(A.pr)[o1] = v;
-        static_cast<MD_G double *>(A.pr)[o2] = v;
-    } else {
-        static_cast<MD_G float *>(A.pr)[o1] = (float)v;
-        static_cast<MD_G float *>(A.pr)[o2] = (float)v;
+    const int nk = (b + kIb - 1) / kIb;
+#pragma unroll 1
+    for (int K = 0; K < 4; ++K) {
+        dv4 out[4];
+        if (K < nk) {
+            double (*Ss)[kIbLd] = work.s[K & 1];
+            double (*Sa)[kIb][kIbLd] = work.a[K & 1];
+            if (wv == K) {
+#pragma unroll
+                for (int I = 1; I < 4; ++I)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) Sa[I][4 * c + g][j] = acc[I][c];
+                dv4 d[1][1];
+                d[0][0] = acc[0];
+                const int real = b - kIb * K;
+                sweep_panel<1, 0, false>(d, lane, 4, real, thr, bad);
+                sweep_panel<1, 1, false>(d, lane, 4, real, thr, bad);
+                sweep_panel<1, 2, false>(d, lane, 4, real, thr, bad);
+                sweep_panel<1, 3, false>(d, lane, 4, real, thr, bad);
+                out[3] = d[0][0];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) Ss[4 * c + g][j] = -out[3][c];
+            }
+            __syncthreads();
+            if (wv == K) {
+#pragma unroll
+                for (int I = 1; I < 4; ++I) out[I - 1] = dv4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int I = 1; I < 4; ++I) out[I - 1] = MD_MFMA64(Sa[I][j][4 * c + g], -out[3][c], out[I - 1]);
+            } else {
+                dv4 t = dv4{0.0, 0.0, 0.0, 0.0}, t2 = t;
+#pragma unroll
+                for (int c = 0; c < 4; c += 2) {
+                    t = MD_MFMA64(Ss[j][4 * c + g], acc[0][c], t);
+                    t2 = MD_MFMA64(Ss[j][4 * c + 4 + g], acc[0][c + 1], t2);
+                }
+                t += t2;
+#pragma unroll
+                for (int I = 1; I < 4; ++I) out[I - 1] = acc[I];
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int I = 1; I < 4; ++I) out[I - 1] = MD_MFMA64(-Sa[I][j][4 * c + g], t[c], out[I - 1]);
+                out[3] = t;
+            }
+        } else {  // rotate only
+#pragma unroll
+            for (int I = 0; I < 4; ++I) out[I] = acc[(I + 1) & 3];
+        }
+#pragma unroll
+        for (int I = 0; I < 4; ++I) acc[I] = out[I];
     }
 }
 
-// Block s of the pivot block, complete in m (LDS): S = A_ss^{-1} into `out` (block (s, s) of the
-// workspace the next step reads), or D^{-1} itself when it is the only block.
+// Block s of a front, complete in m (LDS): S = A_ss^{-1} into block (s, s) of the workspace `out`.
 __device__ __forceinline__ void pivot_inverse(const FacArgs &A, const FacDev &S, int s, const double *m, InvLds &work,
-                                              PivotBuf out) {
+                                              const FrontBuf &out) {
     const int kb = s * kFb, b = min(kFb, S.w - kb);
     const double thr = 1e-14 * __longlong_as_double((long long)*A.amax);
     dv4 acc[4];
@@ -1821,43 +1850,37 @@ __device__ __forceinline__ void pivot_inverse(const FacArgs &A, const FacDev &S,
     if (bad && (threadIdx.x & 63) == 0) *A.flag = 1;
     const int wv = threadIdx.x >> 6, j = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4, r = kIb * wv + j;
     if (r >= b) return;
+    MD_G double *p = out.d + (long long)(kb + g) * out.ldd + kb + r;  // entry (r, q) = (q, r): lanes along r
 #pragma unroll
     for (int I = 0; I < 4; ++I)
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const int q = kIb * I + 4 * c + g;  // entry (r, q) = (q, r): lanes along r
-            if (q >= b) continue;
-            if (S.w <= kFb) {
-                if (r >= q) put_dinv(A, S, r, q, -acc[I][c]);
-            } else {
-                out.p[(long long)(kb + q) * out.ld + kb + r] = -acc[I][c];
-            }
+            const int q = kIb * I + 4 * c;
+            if (q + g < b) p[q * out.ldd] = -acc[I][c];
         }
 }
 
-// Block 0 of every pivot block of a height (one workgroup per front).
+// Block 0 of the fronts of a height (one workgroup per front).
 __global__ __launch_bounds__(kFacBlock) void k_fac_inv0(FacArgs A, int h0) {
-    const FacDev S = A.sn[A.hlist[h0 + blockIdx.x]];
+    const FacDev S = A.sn[h0 + blockIdx.x];
     __shared__ double m[kFb * kLdT];
     __shared__ InvLds work;
-    const PivotBuf B = pivot_buf(A, S, 0);
-    const int b = min(kFb, S.w);
+    const FrontBuf B = front_buf(A, S, 0);
+    const int b = min(kFb, S.w), r = threadIdx.x % kFb;
 #pragma unroll
     for (int i = 0; i < kFb * kFb / kFacBlock; ++i) {
-        const int e = threadIdx.x + kFacBlock * i, r = e % kFb, c = e / kFb;
-        if (r < b && c <= r) m[r * kLdT + c] = B.p[(long long)c * B.ld + r];
+        const int c = threadIdx.x / kFb + 4 * i;
+        if (r < b && c <= r) m[r * kLdT + c] = B.d[c * B.ldd + r];
     }
     __syncthreads();
     pivot_inverse(A, S, 0, m, work, B);
 }
 
-// ---- FP64 dense products of the factorization on the matrix cores ----------------------
+// ---- FP64 products of the sweeps on the matrix cores ---------------------------------------
 //
 // A 64 x 64 output tile per workgroup of 256 threads: wave v computes rows [32 (v / 2), +32) and
-// columns [32 (v % 2), +32) as 2 x 2 blocks of v_mfma_f64_16x16x4, with the operands staged in LDS,
-// kMk values of k at a time (As[k][i] = A(i, k), Bs[k][j] = B(k, j); rows kMpad doubles apart).
-constexpr int kMk = 32;
-constexpr int kMpad = 66;
+// columns [32 (v % 2), +32) as 2 x 2 blocks of v_mfma_f64_16x16x4, with both operands whole in LDS
+// (64 values of k, rows kLdT apart).
 
 struct MmaAcc {
     dv4 c[2][2];
@@ -1870,233 +1893,34 @@ __device__ __forceinline__ void mma_zero(MmaAcc &acc) {
         for (int y = 0; y < 2; ++y) acc.c[x][y] = dv4{0.0, 0.0, 0.0, 0.0};
 }
 
-// acc += As^T Bs over the staged kMk values of k.
-__device__ __forceinline__ void mma_chunk(const double (*As)[kMpad], const double (*Bs)[kMpad], MmaAcc &acc) {
-    const int wv = threadIdx.x / 64, lane = threadIdx.x & 63;
-    const int rb = 32 * (wv >> 1) + (lane & 15), cb = 32 * (wv & 1) + (lane & 15);
-#pragma unroll
-    for (int k4 = 0; k4 < kMk; k4 += 4) {
-        const int kk = k4 + (lane >> 4);
-        const double a0 = As[kk][rb], a1 = As[kk][rb + 16];
-        const double b0 = Bs[kk][cb], b1 = Bs[kk][cb + 16];
-        acc.c[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc.c[0][0], 0, 0, 0);
-        acc.c[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc.c[0][1], 0, 0, 0);
-        acc.c[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc.c[1][0], 0, 0, 0);
-        acc.c[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc.c[1][1], 0, 0, 0);
-    }
-}
-
 // Tile coordinates (i, j) within the 64 x 64 output of this thread's element (x, y, r).
 __device__ __forceinline__ int mma_row(int x, int r) {
     return 32 * ((threadIdx.x / 64) >> 1) + 16 * x + 4 * r + ((threadIdx.x & 63) >> 4);
 }
 __device__ __forceinline__ int mma_col(int y) { return 32 * ((threadIdx.x / 64) & 1) + 16 * y + (threadIdx.x & 15); }
 
-// acc += sum over nchunks staged chunks of kMk values of k, software-pipelined: each thread
-// holds its kPer values of both operands of the next chunk in registers, loaded (fetch(c, ra,
-// rb)) while the matrix cores work on the current one, and put into As / Bs (put(ra, rb)) once
-// every wave is done reading them. Thread t stages the entries e = t + kFacBlock i, i < kPer.
-constexpr int kPer = kMk * 64 / kFacBlock;
-template <class Fetch, class Put>
-__device__ __forceinline__ void mma_pipeline(int nchunks, Fetch fetch, Put put, double (*As)[kMpad],
-                                             double (*Bs)[kMpad], MmaAcc &acc) {
-    double ra[kPer], rb[kPer];
-    if (nchunks > 0) fetch(0, ra, rb);
-    for (int c = 0; c < nchunks; ++c) {
-        __syncthreads();
-        put(ra, rb);
-        __syncthreads();
-        if (c + 1 < nchunks) fetch(c + 1, ra, rb);
-        mma_chunk(As, Bs, acc);
-    }
-}
-
-// Lower block (I, J), I >= J, of the q-th tile of a lower-triangular tile grid.
-__device__ __forceinline__ void lower_tile(int q, int &I, int &J) {
-    int i = 0;
-    while ((i + 1) * (i + 2) / 2 <= q) ++i;
-    I = i;
-    J = q - i * (i + 1) / 2;
-}
-
-// Split-K of the long products (few tiles, long K: the top heights): each of `ks` workgroups of a
-// tile multiplies over its share of the K chunks and stores its accumulators (kAccVals doubles per
-// workgroup, coalesced; MODE 1), and a second launch (MODE 2) sums the ks partials in split order
-// (deterministic) and finishes the tile as the unsplit kernel (MODE 0) does. (A last-arriving
-// workgroup summing in the same launch measured several times slower: every workgroup's
-// device-scope fence writes back its L2.)
-constexpr int kAccVals = 16 * kFacBlock;
-static_assert(kAccVals == fac_split_k_doubles(1), "partials per workgroup as the host sizes them");
-__device__ __forceinline__ void acc_store(MD_G double *wp, const MmaAcc &acc) {
+// acc(i, j) += sum_{k < kn} Ar[k][i] Bc[k][j], 16 values of k per turn (operands past kn are zero).
+__device__ __forceinline__ void mma_span(const double *Ar, const double *Bc, int kn, MmaAcc &acc) {
+    const int wv = threadIdx.x / 64, lane = threadIdx.x & 63;
+    const double *ap = Ar + (lane >> 4) * kLdT + 32 * (wv >> 1) + (lane & 15);
+    const double *bp = Bc + (lane >> 4) * kLdT + 32 * (wv & 1) + (lane & 15);
+    for (int k = 0; k < kn; k += 16, ap += 16 * kLdT, bp += 16 * kLdT) {
+        double a[4][2], b[4][2];
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+        for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int y = 0; y < 2; ++y)
+            for (int y = 0; y < 2; ++y) {
+                a[u][y] = ap[4 * u * kLdT + 16 * y];
+                b[u][y] = bp[4 * u * kLdT + 16 * y];
+            }
 #pragma unroll
-            for (int r = 0; r < 4; ++r) wp[((x * 2 + y) * 4 + r) * kFacBlock + threadIdx.x] = acc.c[x][y][r];
-}
-// Sums in split order; the loads of four splits are issued before their additions.
-__device__ __forceinline__ void acc_sum(const MD_G double *wp, int ks, MmaAcc &acc) {
-    for (int z0 = 0; z0 < ks; z0 += 4) {
-        double v[4][16];
-#pragma unroll
-        for (int dz = 0; dz < 4; ++dz)
-#pragma unroll
-            for (int t = 0; t < 16; ++t)
-                v[dz][t] = z0 + dz < ks ? wp[(long long)(z0 + dz) * kAccVals + t * kFacBlock + threadIdx.x] : 0.0;
-#pragma unroll
-        for (int dz = 0; dz < 4; ++dz)
+        for (int u = 0; u < 4; ++u)
 #pragma unroll
             for (int x = 0; x < 2; ++x)
 #pragma unroll
-                for (int y = 0; y < 2; ++y)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) acc.c[x][y][r] += v[dz][(x * 2 + y) * 4 + r];
+                for (int y = 0; y < 2; ++y) acc.c[x][y] = MD_MFMA64(a[u][x], b[u][y], acc.c[x][y]);
     }
 }
-
-// G = F_os D^{-1} into panel rows [w, m): 64 x 64 tile (rows of G, columns), `per`
-// workgroups per supernode. A(i, k) = F_os(r0 + i, k) (column-major), B(k, j) = D^{-1}(k, q0 + j).
-template <int MODE>
-__global__ __launch_bounds__(kFacBlock) __attribute__((amdgpu_waves_per_eu(MODE == 2 ? 2 : 4))) void k_fac_g(FacArgs A, int h0, int per, int ks) {
-    const int tile = MODE == 1 ? (int)blockIdx.x / ks : (int)blockIdx.x, z = MODE == 1 ? (int)blockIdx.x % ks : 0;
-    MmaAcc acc;
-    mma_zero(acc);
-    // MODE 2: the partials' loads go out first (a tile with no work stored none and returns below)
-    if constexpr (MODE == 2) acc_sum(A.Wk + (long long)tile * ks * kAccVals, ks, acc);
-    const FacDev S = A.sn[A.hlist[h0 + tile / per]];
-    const int w = S.w, no = S.noff, m = S.m, nr = (no + 63) / 64, nq = (w + 63) / 64;
-    const int q = tile % per;
-    if (q >= nr * nq) return;
-    const int r0 = 64 * (q % nr), q0 = 64 * (q / nr);
-    double *P = A.P + S.poff;
-    const double *F = A.S + S.soff;
-    __shared__ double As[kMk][kMpad];
-    __shared__ double Bs[kMk][kMpad];
-    if constexpr (MODE != 2) {
-        const int nch = (w + kMk - 1) / kMk, cb = z * nch / ks, ce = (z + 1) * nch / ks;
-        mma_pipeline(
-            ce - cb,
-            [&](int c, double (&ra)[kPer], double (&rb)[kPer]) {
-#pragma unroll
-                for (int i = 0; i < kPer; ++i) {
-                    const int e = threadIdx.x + kFacBlock * i, x = e % 64, k = (cb + c) * kMk + e / 64;
-                    ra[i] = k < w && r0 + x < no ? F[(long long)k * no + r0 + x] : 0.0;
-                    // B(k, q0 + x): consecutive threads read consecutive k of one column
-                    const int xb = e / kMk, kg = (cb + c) * kMk + e % kMk;
-                    rb[i] = kg < w && q0 + xb < w ? P[(long long)(q0 + xb) * m + kg] : 0.0;
-                }
-            },
-            [&](const double (&ra)[kPer], const double (&rb)[kPer]) {
-#pragma unroll
-                for (int i = 0; i < kPer; ++i) {
-                    const int e = threadIdx.x + kFacBlock * i;
-                    As[e / 64][e % 64] = ra[i];
-                    Bs[e % kMk][e / kMk] = rb[i];
-                }
-            },
-            As, Bs, acc);
-    }
-    if constexpr (MODE == 1) {
-        acc_store(A.Wk + ((long long)tile * ks + z) * kAccVals, acc);
-        return;
-    }
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int rr = r0 + mma_row(x, r), qq = q0 + mma_col(y);
-                if (rr < no && qq < w) {
-                    const double v = acc.c[x][y][r];
-                    P[(long long)qq * m + w + rr] = v;
-                    // the forward panel G (column-major) and the backward panel's G rows
-                    const long long oc = S.pc_off + (long long)qq * no + rr, orr = S.pr_off + (long long)(w + rr) * w + qq;
-                    if (A.solve64) {
-                        static_cast<MD_G double *>(A.pc)[oc] = v;
-                        static_cast<MD_G double *>(A.pr)[orr] = v;
-                    } else {
-                        static_cast<MD_G float *>(A.pc)[oc] = (float)v;
-                        static_cast<MD_G float *>(A.pr)[orr] = (float)v;
-                    }
-                }
-            }
-}
-
-// U -= G F_os^T (lower part): lower 64 x 64 tile (I, J) of U(a, b), a >= b, `per` workgroups
-// per supernode. A(i, k) = G(a0 + i, k) (panel rows [w, m)), B(k, j) = F_os(b0 + j, k).
-template <int MODE>
-__global__ __launch_bounds__(kFacBlock) __attribute__((amdgpu_waves_per_eu(MODE == 2 ? 2 : 4))) void k_fac_u(FacArgs A, int h0, int per, int ks) {
-    const int tile = MODE == 1 ? (int)blockIdx.x / ks : (int)blockIdx.x, z = MODE == 1 ? (int)blockIdx.x % ks : 0;
-    MmaAcc acc;
-    mma_zero(acc);
-    // MODE 2: the partials' loads go out first (a tile with no work stored none and returns below)
-    if constexpr (MODE == 2) acc_sum(A.Wk + (long long)tile * ks * kAccVals, ks, acc);
-    const FacDev S = A.sn[A.hlist[h0 + tile / per]];
-    const int w = S.w, no = S.noff, m = S.m, nb = (no + 63) / 64, q = tile % per;
-    if (q >= nb * (nb + 1) / 2) return;
-    int I, J;
-    lower_tile(q, I, J);
-    const int a0 = 64 * I, b0 = 64 * J;
-    const double *P = A.P + S.poff, *F = A.S + S.soff;
-    double *U = A.U + S.uoff;
-    __shared__ double As[kMk][kMpad];
-    __shared__ double Bs[kMk][kMpad];
-    if constexpr (MODE != 2) {
-        const int nch = (w + kMk - 1) / kMk, cb = z * nch / ks, ce = (z + 1) * nch / ks;
-        mma_pipeline(
-            ce - cb,
-            [&](int c, double (&ra)[kPer], double (&rb)[kPer]) {
-#pragma unroll
-                for (int i = 0; i < kPer; ++i) {
-                    const int e = threadIdx.x + kFacBlock * i, x = e % 64, k = (cb + c) * kMk + e / 64;
-                    ra[i] = k < w && a0 + x < no ? P[(long long)k * m + w + a0 + x] : 0.0;
-                    rb[i] = k < w && b0 + x < no ? F[(long long)k * no + b0 + x] : 0.0;
-                }
-            },
-            [&](const double (&ra)[kPer], const double (&rb)[kPer]) {
-#pragma unroll
-                for (int i = 0; i < kPer; ++i) {
-                    const int e = threadIdx.x + kFacBlock * i;
-                    As[e / 64][e % 64] = ra[i];
-                    Bs[e / 64][e % 64] = rb[i];
-                }
-            },
-            As, Bs, acc);
-    }
-    if constexpr (MODE == 1) {
-        acc_store(A.Wk + ((long long)tile * ks + z) * kAccVals, acc);
-        return;
-    }
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int aa = a0 + mma_row(x, r), bb = b0 + mma_col(y);
-                if (aa < no && bb < no && bb <= aa) U[(long long)bb * no + aa] -= acc.c[x][y][r];
-            }
-}
-
-// Two chained products of a tile, operands whole in LDS (64 values of k, rows kLdT apart): acc(i, j) +=
-// sum_{k < kn} Ar[k][i] Bc[k][j].
-__device__ __forceinline__ void mma_span(const double *Ar, const double *Bc, int kn, MmaAcc &acc) {
-    const int wv = threadIdx.x / 64, lane = threadIdx.x & 63;
-    const int rb = 32 * (wv >> 1) + (lane & 15), cb = 32 * (wv & 1) + (lane & 15);
-    for (int k4 = 0; k4 < kn; k4 += 4) {
-        const int kk = (k4 + (lane >> 4)) * kLdT;
-        const double a0 = Ar[kk + rb], a1 = Ar[kk + rb + 16];
-        const double b0 = Bc[kk + cb], b1 = Bc[kk + cb + 16];
-        acc.c[0][0] = MD_MFMA64(a0, b0, acc.c[0][0]);
-        acc.c[0][1] = MD_MFMA64(a0, b1, acc.c[0][1]);
-        acc.c[1][0] = MD_MFMA64(a1, b0, acc.c[1][0]);
-        acc.c[1][1] = MD_MFMA64(a1, b1, acc.c[1][1]);
-    }
-}
-
-constexpr int kTileVals = kFb * kFb / kFacBlock;  // values of a 64 x 64 tile per thread
 
 // fn(value, row, column) over this thread's accumulators.
 template <class Fn>
@@ -2109,40 +1933,55 @@ __device__ __forceinline__ void mma_each(const MmaAcc &acc, Fn fn) {
             for (int r = 0; r < 4; ++r) fn(acc.c[x][y][r], mma_row(x, r), mma_col(y));
 }
 
-// Block (X, s) of a pivot block from its lower tiles, into registers and from there to LDS as
-// Z[t][x] = A(64 X + x, 64 s + t): below the diagonal the tile itself, above it the transpose of
-// tile (s, X). Zero past the matrix.
-__device__ __forceinline__ void block_fetch(PivotBuf B, int w, int X, int s, double (&v)[kTileVals]) {
-#pragma unroll
-    for (int i = 0; i < kTileVals; ++i) {
-        const int e = threadIdx.x + kFacBlock * i, lo = e % kFb, hi = e / kFb;
-        const int row = (X >= s ? X : s) * kFb + lo, col = (X >= s ? s : X) * kFb + hi;
-        v[i] = row < w && col < w ? B.p[(long long)col * B.ld + row] : 0.0;
-    }
-}
-__device__ __forceinline__ void block_put(bool below, const double (&v)[kTileVals], double *Z) {
-#pragma unroll
-    for (int i = 0; i < kTileVals; ++i) {
-        const int e = threadIdx.x + kFacBlock * i, lo = e % kFb, hi = e / kFb;
-        Z[below ? hi * kLdT + lo : lo * kLdT + hi] = v[i];
-    }
+// Lower block (I, J), I >= J, of the q-th tile of a lower-triangular tile grid.
+__device__ __forceinline__ void lower_tile(int q, int &I, int &J) {
+    int i = 0;
+    while ((i + 1) * (i + 2) / 2 <= q) ++i;
+    I = i;
+    J = q - i * (i + 1) / 2;
 }
 
-// Step s of the block sweeps over the pivot blocks of a height (`per` lower tiles per front): tile
-// (I, J) of the next workspace from the current one and S = A_ss^{-1}, in one launch: with
-// W = A_Is S (64 x 64, in LDS), A_IJ - W A_Js^T; W itself in block column s; -S on the diagonal. The
-// workgroup of tile (s + 1, s + 1), scheduled first, inverts it for the next step while the other
-// tiles still run. The last step writes D^{-1} (minus the swept matrix) to the panels.
+constexpr int kTileVals = kFb * kFb / kFacBlock;  // values of a 64 x 64 tile per thread
+static_assert(kFacBlock == 4 * kFb, "four columns of a tile per pass of the workgroup");
+
+// Block (X, s) of a front (X: pivot blocks 0 .. nb - 1, then blocks of 64 off rows) from its lower
+// tiles, into registers and from there to LDS as Z[t][x] = A(x of block X, t of block s): from block s
+// down the tile itself, above it the transpose of tile (s, X). Zero past the matrix.
+__device__ __forceinline__ void block_fetch(const FrontBuf &B, int w, int no, int nb, int X, int s, double (&v)[kTileVals]) {
+    const int lo = threadIdx.x % kFb, hi = threadIdx.x / kFb;
+    const int col = (X >= s ? s : X) * kFb + hi;
+    const bool off = X >= nb;
+    const int row = off ? (X - nb) * kFb + lo : (X >= s ? X : s) * kFb + lo;
+    const long long ld = off ? B.ldf : B.ldd;
+    const MD_G double *p = (off ? B.f : B.d) + col * ld + row;
+    const bool in = row < (off ? no : w);
+#pragma unroll
+    for (int i = 0; i < kTileVals; ++i) v[i] = in && col + 4 * i < w ? p[4 * i * ld] : 0.0;
+}
+__device__ __forceinline__ void block_put(bool below, const double (&v)[kTileVals], double *Z) {
+    const int lo = threadIdx.x % kFb, hi = threadIdx.x / kFb, z = below ? hi * kLdT + lo : lo * kLdT + hi;
+    const int step = below ? 4 * kLdT : 4;
+#pragma unroll
+    for (int i = 0; i < kTileVals; ++i) Z[z + i * step] = v[i];
+}
+
+// Step s of the block sweeps over the fronts of a height (`per` lower tiles of 64 x 64 per front, its
+// off rows and update matrix included): tile (I, J) from S = A_ss^{-1}, in one launch: with W = A_Is S
+// (64 x 64, in LDS), A_IJ - W A_Js^T; W itself in block column s; -S on the diagonal. The workgroup of
+// tile (s + 1, s + 1), scheduled first, inverts it for the next step while the other tiles still run.
+// The last step of a front writes its panels: D^{-1} (minus the swept pivot block) and G. Tiles leave
+// through LDS, so one short loop stores every kind.
 // Bound by the chain of one tile per step: load, two products (1.7 us each at one MFMA per 16 cycles
-// and CU) and the inversion: 19.6 us a step of the 164k icosphere's top heights. One launch per 64
-// columns; the Cholesky form with a triangular inverse took two (trsm, then syrk with the next pivot
-// block: 6.6 + 24 us) and X^T X afterwards (12 to 27 us a height).
+// and CU) and the inversion: 20 us a step of the 164k icosphere's top heights, whose other tiles
+// run on CUs that the chain leaves idle. So the off rows and the update matrix are swept along: as
+// products after the sweeps (G = F D^{-1}, U -= G F^T, split over K) they took another 20 to 105 us a
+// height, waiting on their own chunks.
 __global__ __launch_bounds__(kFacBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_fac_step(FacArgs A, int h0, int s, int per) {
-    const FacDev S = A.sn[A.hlist[h0 + blockIdx.x / per]];
-    const int w = S.w, nb = (w + kFb - 1) / kFb;
-    if (nb < 2 || s >= nb) return;
+    const FacDev S = A.sn[h0 + blockIdx.x / per];
+    const int w = S.w, no = S.noff, nb = (w + kFb - 1) / kFb, nbo = nb + (no + kFb - 1) / kFb;
+    if (s >= nb) return;
     int q = (int)(blockIdx.x % per);
-    if (q >= nb * (nb + 1) / 2) return;
+    if (q >= nbo * (nbo + 1) / 2) return;
     const bool last = s == nb - 1;
     if (!last) {  // tile 0 and tile (s + 1, s + 1) trade places
         const int d = (s + 1) * (s + 2) / 2 + s + 1;
@@ -2150,299 +1989,265 @@ __global__ __launch_bounds__(kFacBlock) __attribute__((amdgpu_waves_per_eu(2))) 
     }
     int I, J;
     lower_tile(q, I, J);
-    const PivotBuf B = pivot_buf(A, S, s), O = pivot_buf(A, S, s + 1);
+    const FrontBuf B = front_buf(A, S, s), O = front_buf(A, S, s + 1);
     __shared__ double Za[kFb * kLdT], Zb[kFb * kLdT];
     static_assert(sizeof(InvLds) <= sizeof(Za), "the inversion works in the first operand's place");
-    // entry (r, c) of tile (I, J), r and c within the tile
-    auto emit = [&](int r, int c, double v) {
-        const int rr = I * kFb + r, cc = J * kFb + c;
-        if (rr >= w || cc >= w) return;
-        if (!last) O.p[(long long)cc * O.ld + rr] = v;
-        else if (rr >= cc) put_dinv(A, S, rr, cc, -v);
-    };
-    double vs[kTileVals];
-    block_fetch(B, w, s, s, vs);  // S, both triangles
-    if (I == s && J == s) {
-#pragma unroll
-        for (int i = 0; i < kTileVals; ++i) {
-            const int e = threadIdx.x + kFacBlock * i;
-            emit(e % kFb, e / kFb, -vs[i]);
-        }
-        return;
-    }
     const int X = I == s ? J : I;  // W = A_Xs S
-    double vx[kTileVals];
-    block_fetch(B, w, X, s, vx);
-    if (I == s || J == s) {
-        block_put(true, vs, Za);
+    const bool inner = I != s && J != s, upd = J >= nb;
+    const int kn = (min(kFb, w - s * kFb) + 3) & ~3;
+    // where the tile's entries are: rows, columns, and those of the tile within bounds
+    const int i0 = (I < nb ? I : I - nb) * kFb, j0 = (upd ? J - nb : J) * kFb;
+    const int rn = min(kFb, (I < nb ? w : no) - i0), cn = min(kFb, (upd ? no : w) - j0);
+    MD_G double *U = A.U + S.uoff;
+    double vs[kTileVals], vx[kTileVals], vj[kTileVals];
+    block_fetch(B, w, no, nb, s, s, vs);  // S, both triangles
+    if (X != s) block_fetch(B, w, no, nb, X, s, vx);
+    if (inner && I != J) block_fetch(B, w, no, nb, J, s, vj);
+    double own[2][2][4];  // the tile's own entries, where the accumulators will be (row c, column r)
+    if (inner) {
+        const int c0 = mma_row(0, 0), r0 = mma_col(0);
+        const long long ld = upd ? no : I < nb ? B.ldd : B.ldf;
+        const MD_G double *p = (upd ? U : I < nb ? B.d : B.f) + (j0 + c0) * ld + i0 + r0;
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    own[x][y][r] = r0 + 16 * y < rn && c0 + 16 * x + 4 * r < cn ? p[(16 * x + 4 * r) * ld + 16 * y] : 0.0;
+    }
+    block_put(true, vs, Za);
+    if (X != s) {
         block_put(X > s, vx, Zb);
         __syncthreads();
         MmaAcc acc;
         mma_zero(acc);
-        // lanes along the stored tile's rows: (I, s) holds W(r, k), (s, J) holds W(r, k)^T
-        if (J == s) {
-            mma_span(Za, Zb, kFb, acc);
-            mma_each(acc, [&](double v, int k, int r) { emit(r, k, v); });
-        } else {
-            mma_span(Zb, Za, kFb, acc);
-            mma_each(acc, [&](double v, int r, int k) { emit(k, r, v); });
+        mma_span(Za, Zb, kn, acc);  // (k, r): W(r, k)
+        __syncthreads();
+        mma_each(acc, [&](double v, int k, int r) { Za[k * kLdT + r] = v; });
+        if (inner) {
+            if (I != J) block_put(J > s, vj, Zb);
+            __syncthreads();
+            mma_zero(acc);
+            mma_span(Zb, Za, kn, acc);  // (c, r): sum_k A_Js(c, k) W(r, k)
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int y = 0; y < 2; ++y)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc.c[x][y][r] = own[x][y][r] - acc.c[x][y][r];
+            __syncthreads();  // the operands are read
+            if (!last && I == s + 1 && J == s + 1) {
+                mma_each(acc, [&](double v, int c, int r) { if (r >= c) Zb[r * kLdT + c] = v; });
+                __syncthreads();
+                pivot_inverse(A, S, s + 1, Zb, *reinterpret_cast<InvLds *>(Za), O);
+                return;
+            }
+            mma_each(acc, [&](double v, int c, int r) { Za[c * kLdT + r] = v; });
         }
+    }
+    __syncthreads();
+    // Za: entry (r, c) of the tile at c * kLdT + r (S itself on the diagonal, negated below), except that
+    // in block row s it holds W_J(r', k) for entry (k, r')
+    const bool swap = I == s && J != s, dinv = last && I < nb;
+    const double sign = (X == s) != dinv ? -1.0 : 1.0;  // -S on the diagonal; D^{-1} is minus the swept block
+    auto entry = [&](int r, int c) { return sign * Za[swap ? r * kLdT + c : c * kLdT + r]; };
+    const int lo = threadIdx.x % kFb, hi = threadIdx.x / kFb;
+    if (!last || upd) {
+        const long long ld = upd ? no : I < nb ? O.ldd : O.ldf;
+        MD_G double *p = (upd ? U : I < nb ? O.d : O.f) + j0 * ld + i0;
+        if (lo < rn)
+            for (int c = hi; c < cn; c += 4) p[c * ld + lo] = entry(lo, c);
         return;
     }
-    double vj[kTileVals];
-    if (I != J) block_fetch(B, w, J, s, vj);
-    // the tile's own entries, where the product's accumulators will be (row c, column r)
-    double own[2][2][4];
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int cc = J * kFb + mma_row(x, r), rr = I * kFb + mma_col(y);
-                own[x][y][r] = rr < w && cc < w ? B.p[(long long)cc * B.ld + rr] : 0.0;
-            }
-    block_put(true, vs, Za);
-    block_put(I > s, vx, Zb);
-    __syncthreads();
-    MmaAcc acc;
-    mma_zero(acc);
-    mma_span(Za, Zb, kFb, acc);  // (k, r): W(r, k)
-    __syncthreads();
-    mma_each(acc, [&](double v, int k, int r) { Za[k * kLdT + r] = v; });
-    if (I != J) block_put(J > s, vj, Zb);
-    __syncthreads();
-    mma_zero(acc);
-    mma_span(Zb, Za, kFb, acc);  // (c, r): sum_k A_Js(c, k) W(r, k)
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc.c[x][y][r] = own[x][y][r] - acc.c[x][y][r];
-    if (last || I != s + 1 || J != s + 1) {
-        mma_each(acc, [&](double v, int c, int r) { emit(r, c, v); });
-        return;
+    auto put = [&](MD_G void *dst, long long o, double v) {
+        if (A.solve64) static_cast<MD_G double *>(dst)[o] = v;
+        else static_cast<MD_G float *>(dst)[o] = (float)v;
+    };
+    // row-major panel [D^{-1}; G], lanes along its columns; the pivot rows' tiles also mirrored (the
+    // diagonal tile from its lower part), G also to the column-major panel
+    const long long pr = S.pr_off + (long long)((dinv ? 0 : w) + i0) * w + j0;
+    if (lo < cn)
+        for (int r = hi; r < rn; r += 4) put(A.pr, pr + (long long)r * w + lo, I == J ? entry(max(r, lo), min(r, lo)) : entry(r, lo));
+    if (I == J || lo >= rn) return;
+    for (int c = hi; c < cn; c += 4) {
+        if (dinv) put(A.pr, S.pr_off + (long long)(j0 + c) * w + i0 + lo, entry(lo, c));
+        else put(A.pc, S.pc_off + (long long)(j0 + c) * no + i0 + lo, entry(lo, c));
     }
-    __syncthreads();  // the operands are read
-    mma_each(acc, [&](double v, int c, int r) { if (r >= c) Zb[r * kLdT + c] = v; });
-    __syncthreads();
-    pivot_inverse(A, S, s + 1, Zb, *reinterpret_cast<InvLds *>(Za), O);
 }
 
-// G = F_os D^{-1} and U -= G F_os^T for a height whose pivot blocks all have w <= 64, in one launch:
-// lower tile (I, J) of U, `per` workgroups per front, forms G's row block I itself (one product with
-// D^{-1}); the tiles of block column 0 also write it to the sweeps' panels. The two launches that
-// this replaces cost a launch and a round trip of G through memory for fronts of a few tiles.
-__global__ __launch_bounds__(kFacBlock) void k_fac_gu(FacArgs A, int h0, int per) {
-    const FacDev S = A.sn[A.hlist[h0 + blockIdx.x / per]];
-    const int w = S.w, no = S.noff, m = S.m, nb = (no + kFb - 1) / kFb, q = (int)(blockIdx.x % per);
-    if (q >= nb * (nb + 1) / 2) return;
-    int I, J;
-    lower_tile(q, I, J);
-    const int a0 = I * kFb, b0 = J * kFb, kn = (w + 3) & ~3;
-    const MD_G double *P = A.P + S.poff, *F = A.S + S.soff;
-    MD_G double *U = A.U + S.uoff;
-    __shared__ double Za[kFb * kLdT], Zb[kFb * kLdT];
-    double vd[kTileVals], vi[kTileVals], vj[kTileVals];
-#pragma unroll
-    for (int i = 0; i < kTileVals; ++i) {
-        const int e = threadIdx.x + kFacBlock * i, x = e % kFb, t = e / kFb;
-        const bool in = t < w;
-        vd[i] = in && x < w ? P[(long long)t * m + x] : 0.0;
-        vi[i] = in && a0 + x < no ? F[(long long)t * no + a0 + x] : 0.0;
-        vj[i] = I != J && in && b0 + x < no ? F[(long long)t * no + b0 + x] : 0.0;
-    }
-    double own[2][2][4];
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int bb = b0 + mma_row(x, r), aa = a0 + mma_col(y);
-                own[x][y][r] = aa < no && bb <= aa ? U[(long long)bb * no + aa] : 0.0;
-            }
-    block_put(true, vd, Za);
-    block_put(true, vi, Zb);
-    __syncthreads();
-    MmaAcc acc;
-    mma_zero(acc);
-    mma_span(Za, Zb, kn, acc);  // (k, a): G(a, k)
-    __syncthreads();
-    mma_each(acc, [&](double v, int k, int a) { Za[k * kLdT + a] = v; });
-    if (I != J) block_put(true, vj, Zb);
-    __syncthreads();
-    if (J == 0) {
-        // the forward panel G (column-major) and the backward panel's G rows (row-major)
-        for (int e = threadIdx.x; e < w * kFb; e += kFacBlock) {
-            const int a = e % kFb, k = e / kFb;
-            if (a0 + a < no) {
-                const double v = Za[k * kLdT + a];
-                const long long o = S.pc_off + (long long)k * no + a0 + a;
-                if (A.solve64) static_cast<MD_G double *>(A.pc)[o] = v;
-                else static_cast<MD_G float *>(A.pc)[o] = (float)v;
-            }
-        }
-        for (int e = threadIdx.x; e < w * min(kFb, no - a0); e += kFacBlock) {
-            const int k = e % w, a = e / w;
-            const double v = Za[k * kLdT + a];
-            const long long o = S.pr_off + (long long)(w + a0 + a) * w + k;
-            if (A.solve64) static_cast<MD_G double *>(A.pr)[o] = v;
-            else static_cast<MD_G float *>(A.pr)[o] = (float)v;
-        }
-    }
-    mma_zero(acc);
-    mma_span(Zb, Za, kn, acc);  // (b, a): sum_k F(b, k) G(a, k)
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int bb = b0 + mma_row(x, r), aa = a0 + mma_col(y);
-                if (aa < no && bb <= aa) U[(long long)bb * no + aa] = own[x][y][r] - acc.c[x][y][r];
-            }
-}
-
-// The front in LDS (lower part, row r at r * ld) of m <= 16 NB rows, swept on its w pivots by one
-// wavefront with all of it in registers, and stored: D^{-1} and G to the sweeps' panels, U for the
-// parent. After the sweeps of block 0's columns the blocks rotate (block k to k - 1), so every
-// panel has fixed registers.
-template <int NB>
-__device__ __forceinline__ void small_front(const FacArgs &A, const FacDev &S, const double *Fs, int ld, double thr) {
+// The front in LDS (symmetric, row r at r * LD, zero past its m rows) of m <= 16 NB rows, swept on its w
+// pivots by one wavefront with all of it in registers, and put back: [-D^{-1}, G^T; G, U]. After the
+// sweeps of block 0's columns the blocks rotate (block k to k - 1), so every panel has fixed
+// registers.
+template <int NB, int LD>
+__device__ __forceinline__ bool small_front(double *Fs, int w, double thr) {
     const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
-    const int w = S.w, no = S.noff, m = S.m;
     dv4 a[NB][NB];
 #pragma unroll
     for (int I = 0; I < NB; ++I)
 #pragma unroll
         for (int J = 0; J < NB; ++J)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const int r = kIb * I + 4 * c + g, q = kIb * J + j;
-                a[I][J][c] = r < m && q < m ? Fs[max(r, q) * ld + min(r, q)] : 0.0;
-            }
+            for (int c = 0; c < 4; ++c) a[I][J][c] = Fs[(kIb * I + 4 * c + g) * LD + kIb * J + j];
     bool bad = false;
     int rot = 0;
+#pragma unroll 1
     for (int k0 = 0; k0 < w; k0 += kIb) {
         const int left = w - k0;
-        auto panel = [&](auto tag) {
-            constexpr int C = decltype(tag)::value;
-            if (left >= 4 * C + 4) sweep_panel<NB, C, false>(a, lane, 4, left, thr, bad);
-            else if (left > 4 * C) sweep_panel<NB, C, true>(a, lane, left - 4 * C, left, thr, bad);
-        };
-        panel(std::integral_constant<int, 0>{});
-        panel(std::integral_constant<int, 1>{});
-        panel(std::integral_constant<int, 2>{});
-        panel(std::integral_constant<int, 3>{});
-        if (NB > 1) {
-            dv4 t[NB][NB];
+        sweep_panel<NB, 0, true>(a, lane, min(4, left), left, thr, bad);
+        if (left > 4) sweep_panel<NB, 1, true>(a, lane, min(4, left - 4), left, thr, bad);
+        if (left > 8) sweep_panel<NB, 2, true>(a, lane, min(4, left - 8), left, thr, bad);
+        if (left > 12) sweep_panel<NB, 3, true>(a, lane, min(4, left - 12), left, thr, bad);
+        dv4 t[NB][NB];
 #pragma unroll
-            for (int I = 0; I < NB; ++I)
+        for (int I = 0; I < NB; ++I)
 #pragma unroll
-                for (int J = 0; J < NB; ++J) t[I][J] = a[(I + 1) % NB][(J + 1) % NB];
+            for (int J = 0; J < NB; ++J) t[I][J] = a[(I + 1) % NB][(J + 1) % NB];
 #pragma unroll
-            for (int I = 0; I < NB; ++I)
+        for (int I = 0; I < NB; ++I)
 #pragma unroll
-                for (int J = 0; J < NB; ++J) a[I][J] = t[I][J];
-            rot = rot + 1 == NB ? 0 : rot + 1;
-        }
+            for (int J = 0; J < NB; ++J) a[I][J] = t[I][J];
+        rot = rot + 1 == NB ? 0 : rot + 1;
     }
-    if (bad && lane == 0) *A.flag = 1;
-    MD_G double *U = A.U + S.uoff;
-    auto put = [&](MD_G void *dst, long long o, double v) {
-        if (A.solve64) static_cast<MD_G double *>(dst)[o] = v;
-        else static_cast<MD_G float *>(dst)[o] = (float)v;
-    };
 #pragma unroll
     for (int I = 0; I < NB; ++I)
 #pragma unroll
         for (int J = 0; J < NB; ++J) {
             const int bi = I + rot >= NB ? I + rot - NB : I + rot, bj = J + rot >= NB ? J + rot - NB : J + rot;
+            double *dst = Fs + (kIb * bi + g) * LD + kIb * bj + j;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const int r = kIb * bi + 4 * c + g, q = kIb * bj + j;  // lanes along q
-                if (r >= m || q >= m) continue;
-                const double v = a[I][J][c];
-                if (q < w) put(A.pr, S.pr_off + (long long)r * w + q, r < w ? -v : v);
-                else if (r < w) put(A.pc, S.pc_off + (long long)r * no + (q - w), v);
-                else if (q >= r) U[(long long)(r - w) * no + (q - w)] = v;
-            }
+            for (int c = 0; c < 4; ++c) dst[4 * c * LD] = a[I][J][c];
         }
+    return bad;
 }
 
-// A whole height of small fronts (every m = w + noff <= mm <= 16 NBMAX) in one launch, one workgroup
-// per front: assembly in LDS (the original entries, then the children's update matrices in child
-// order, as k_fac_assemble adds them; the front's row list staged in LDS for the searches) by all of
-// its BLOCK threads, then the sweeps by its first wavefront in registers (small_front). BLOCK is 64 on
-// heights of many fronts (the leaves, which have no children) and 256 on heights of few, where the
-// additions of the children are the longer part. The FP64 panel workspace is not used.
-// 45 us for the 6,616 leaves of a 164k icosphere and 15 us for a single front of 52 columns; the
+// Small fronts (m = w + noff <= 16 NB), one workgroup per front: assembly in LDS (the original
+// entries, then the children's update matrices in child order, as k_fac_assemble adds them; the
+// front's row list staged in LDS for the searches) by all of its BLOCK threads, the sweeps by its
+// first wavefront in registers (small_front), and all of it out again: D^{-1} and G to the sweeps'
+// panels, U for the parent. BLOCK is 64 for many fronts (the leaves, which have no children) and 256
+// for few, where the additions of the children are the longer part. The FP64 panel workspace is not
+// used. 51 us for the 6,616 leaves of the 164k icosphere and 14 us for a single front of 52 columns; the
 // column-by-column Cholesky in LDS that stood here took 100 and 88 us (three barriers per column).
 constexpr int kSmallSlotLanes = 4;  // lanes per pivot column for its original entries
-template <int BLOCK, int NBMAX>
-__global__ __launch_bounds__(BLOCK) void k_fac_small(FacArgs A, int h0, int mm) {
-    const FacDev S = A.sn[A.hlist[h0 + blockIdx.x]];
+constexpr int kSmallAhead = 16;     // columns of a child's update matrix in flight
+template <int BLOCK, int NB>
+__global__ __launch_bounds__(BLOCK) void k_fac_small(FacArgs A, int h0) {
+    const FacDev S = A.sn[h0 + blockIdx.x];
     const int tid = threadIdx.x, w = S.w, no = S.noff, m = S.m;
-    if (m > mm || mm > kIb * NBMAX) {  // the host sends only heights of small fronts
+    if (m > kIb * NB) {  // the host sends only small fronts
         if (tid == 0) *A.flag = 2;
         return;
     }
-    const int ld = mm | 1;
-    extern __shared__ double smem[];
-    double *Fs = smem;  // the front (lower, row stride ld)
-    __shared__ int rows[kIb * NBMAX];
+    constexpr int LD = kIb * NB + 1;
+    __shared__ double Fs[kIb * NB * LD];
+    __shared__ int rows[kIb * NB];
     for (int e = tid; e < no; e += BLOCK) rows[e] = A.offrows[S.roff + e];
-    for (int e = tid; e < m * ld; e += BLOCK) Fs[e] = 0.0;
+    const bool narrow = NB > 2 && m <= 2 * kIb;  // swept as two blocks
+    for (int e = tid; e < (narrow ? 2 * kIb : NB * kIb) * LD; e += BLOCK) Fs[e] = 0.0;
     __syncthreads();
     // original entries, kSmallSlotLanes lanes per pivot column (one slot each; every front entry
     // receives at most one)
     for (int k = tid / kSmallSlotLanes; k < w; k += BLOCK / kSmallSlotLanes) {
         const int j = S.c0 + k, sl = j / kSlice, l = j % kSlice;
-        if (tid % kSmallSlotLanes == 0) Fs[k * ld + k] = A.diag[j];
+        if (tid % kSmallSlotLanes == 0) Fs[k * LD + k] = A.diag[j];
         for (int q = A.slice_ptr[sl] + tid % kSmallSlotLanes; q < A.slice_ptr[sl + 1]; q += kSmallSlotLanes) {
             const long long g = (long long)q * kSlice + l;
             const int i = A.sell_col[g];
             if (i <= j || i >= A.nf) continue;
-            const double v = -A.w64[g];
-            if (i < S.c0 + w) {
-                Fs[(i - S.c0) * ld + k] += v;
-            } else {
+            int r = i - S.c0;
+            if (r >= w) {
                 int lo = 0, hi = no;  // first off row >= i
                 while (lo < hi) {
                     const int mid = (lo + hi) >> 1;
                     if (rows[mid] < i) lo = mid + 1;
                     else hi = mid;
                 }
-                if (lo < no && rows[lo] == i) Fs[(w + lo) * ld + k] += v;
-                else *A.flag = 2;
+                if (lo >= no || rows[lo] != i) {
+                    *A.flag = 2;
+                    continue;
+                }
+                r = w + lo;
             }
+            Fs[r * LD + k] = -A.w64[g];
         }
     }
     __syncthreads();
     // children's update matrices in child order (distinct entries of one child land on distinct
-    // front entries)
-    for (int ci = S.cb; ci < S.ce; ++ci) {
-        const FacDev C = A.sn[A.child[ci]];
-        const int nc = C.noff;
-        const MD_G int *rel = A.rel + C.roff;
-        const MD_G double *Uc = A.U + C.uoff;
-        for (int e = tid; e < nc * nc; e += BLOCK) {
-            const int b = e / nc, a = e - b * nc;
-            if (a < b) continue;
-            const int ra = rel[a], rb = rel[b];
-            if (ra >= m || rb > ra) { *A.flag = 2; continue; }
-            Fs[ra * ld + rb] += Uc[(long long)b * nc + a];
+    // front entries): a child has at most 64 rows, so its map is one register (the next child's in
+    // flight), and kSmallAhead of its columns are loaded at a time
+    const int wv = tid >> 6, lane = tid & 63;
+    for (int cb = S.cb; cb < S.ce; cb += 64) {
+        const int nb = min(S.ce - cb, 64);
+        FacChild C{0, 0, 0};
+        if (lane < nb) C = A.child[cb + lane];
+        auto map_of = [&](int c) {
+            const int nc = __builtin_amdgcn_readlane(C.noff, c), roff = __builtin_amdgcn_readlane(C.roff, c);
+            return lane < nc ? A.rel[roff + lane] : -1;
+        };
+        int next = map_of(0);
+        for (int c = 0; c < nb; ++c) {
+            const int ra = next, nc = __builtin_amdgcn_readlane(C.noff, c);
+            const unsigned long long uo = (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)C.uoff, c) |
+                                          (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(C.uoff >> 32), c) << 32;
+            const MD_G double *Uc = A.U + (long long)uo;
+            if (c + 1 < nb) next = map_of(c + 1);
+            if (nc > 64 || __any(ra >= m)) {  // the same in every wavefront
+                *A.flag = 2;
+                break;
+            }
+            for (int b0 = wv; b0 < nc; b0 += kSmallAhead * (BLOCK / 64)) {
+                double v[kSmallAhead];
+#pragma unroll
+                for (int u = 0; u < kSmallAhead; ++u) {
+                    const int col = b0 + u * (BLOCK / 64);
+                    v[u] = col < nc && lane >= col && lane < nc ? Uc[(long long)col * nc + lane] : 0.0;
+                }
+#pragma unroll
+                for (int u = 0; u < kSmallAhead; ++u) {
+                    const int col = b0 + u * (BLOCK / 64);
+                    if (col >= nc) break;
+                    const int rb = __builtin_amdgcn_readlane(ra, col);
+                    if (lane >= col && lane < nc) Fs[ra * LD + rb] += v[u];
+                }
+            }
+            __syncthreads();
         }
-        __syncthreads();
     }
-    if (tid >= 64) return;
-    const double thr = 1e-14 * __longlong_as_double((long long)*A.amax);
-    if (NBMAX == 1 || m <= kIb) small_front<1>(A, S, Fs, ld, thr);
-    else if (NBMAX == 2 || m <= 2 * kIb) small_front<2 < NBMAX ? 2 : NBMAX>(A, S, Fs, ld, thr);
-    else if (NBMAX == 3 || m <= 3 * kIb) small_front<3 < NBMAX ? 3 : NBMAX>(A, S, Fs, ld, thr);
-    else small_front<NBMAX>(A, S, Fs, ld, thr);
+    // the upper triangle from the lower one
+    for (int e = tid; e < m * m; e += BLOCK) {
+        const int r = e / m, c = e - r * m;
+        if (c > r) Fs[r * LD + c] = Fs[c * LD + r];
+    }
+    __syncthreads();
+    if (tid < 64) {
+        const double thr = 1e-14 * __longlong_as_double((long long)*A.amax);
+        bool bad;
+        if (narrow) bad = small_front<2 < NB ? 2 : NB, LD>(Fs, w, thr);
+        else bad = small_front<NB, LD>(Fs, w, thr);
+        if (bad && tid == 0) *A.flag = 1;
+    }
+    __syncthreads();
+    MD_G double *U = A.U + S.uoff;
+    auto put = [&](MD_G void *dst, long long o, double v) {
+        if (A.solve64) static_cast<MD_G double *>(dst)[o] = v;
+        else static_cast<MD_G float *>(dst)[o] = (float)v;
+    };
+    // the sweeps' panels: row-major [D^{-1}; G] (m x w) and column-major G (no x w); U, lower part
+    for (int e = tid; e < m * w; e += BLOCK) {
+        const int r = e / w, c = e - r * w;
+        const double v = Fs[r * LD + c];
+        put(A.pr, S.pr_off + e, r < w ? -v : v);
+    }
+    for (int e = tid; e < no * w; e += BLOCK) {
+        const int c = e / no, r = e - c * no;
+        put(A.pc, S.pc_off + e, Fs[c * LD + w + r]);
+    }
+    for (int e = tid; e < no * no; e += BLOCK) {
+        const int b = e / no, a = e - b * no;
+        if (a >= b) U[e] = Fs[(w + b) * LD + w + a];
+    }
 }
 
 // Plain device copy of n 16-byte elements (grid-stride): the known-size reference kernel for
@@ -2459,42 +2264,23 @@ void launch_fac_diag(hipStream_t s, const FacArgs &A) {
 }
 template <int BLOCK>
 static void fac_small_of(hipStream_t s, const FacArgs &A, int h0, int count, int mm) {
-    const size_t lds = sizeof(double) * mm * (mm | 1);
     const dim3 grid(count), block(BLOCK);
-    if (mm <= kIb) hipLaunchKernelGGL((k_fac_small<BLOCK, 1>), grid, block, lds, s, A, h0, mm);
-    else if (mm <= 2 * kIb) hipLaunchKernelGGL((k_fac_small<BLOCK, 2>), grid, block, lds, s, A, h0, mm);
-    else if (mm <= 3 * kIb) hipLaunchKernelGGL((k_fac_small<BLOCK, 3>), grid, block, lds, s, A, h0, mm);
-    else hipLaunchKernelGGL((k_fac_small<BLOCK, 4>), grid, block, lds, s, A, h0, mm);
+    if (mm <= kIb) hipLaunchKernelGGL((k_fac_small<BLOCK, 1>), grid, block, 0, s, A, h0);
+    else if (mm <= 2 * kIb) hipLaunchKernelGGL((k_fac_small<BLOCK, 2>), grid, block, 0, s, A, h0);
+    else if (mm <= 3 * kIb) hipLaunchKernelGGL((k_fac_small<BLOCK, 3>), grid, block, 0, s, A, h0);
+    else hipLaunchKernelGGL((k_fac_small<BLOCK, 4>), grid, block, 0, s, A, h0);
 }
 void launch_fac_small(hipStream_t s, const FacArgs &A, int h0, int count, int mm) {
     if (count <= 0) return;
     if (count > kSmallManyFronts) fac_small_of<64>(s, A, h0, count, mm);
     else fac_small_of<256>(s, A, h0, count, mm);
 }
-void launch_fac_height(hipStream_t s, const FacArgs &A, int h0, int count, int nb, int asm_cols, int per_asm,
-                       const FacSplit &g, const FacSplit &u) {
+void launch_fac_height(hipStream_t s, const FacArgs &A, int h0, int count, int nb, const FacAssembly &as, int tiles) {
     if (count <= 0) return;
-    hipLaunchKernelGGL(k_fac_assemble, dim3(count * per_asm), dim3(kFacBlock), 0, s, A, h0, per_asm, asm_cols);
+    hipLaunchKernelGGL(k_fac_assemble, dim3(count * as.per), dim3(kFacBlock), sizeof(int) * (as.ninv + as.nrows), s, A, h0, as);
     hipLaunchKernelGGL(k_fac_inv0, dim3(count), dim3(kFacBlock), 0, s, A, h0);
-    const int tiles = nb * (nb + 1) / 2;
-    for (int b = 0; nb > 1 && b < nb; ++b)
+    for (int b = 0; b < nb; ++b)
         hipLaunchKernelGGL(k_fac_step, dim3(count * tiles), dim3(kFacBlock), 0, s, A, h0, b, tiles);
-    if (g.per <= 0) return;
-    if (nb == 1) {
-        hipLaunchKernelGGL(k_fac_gu, dim3(count * u.per), dim3(kFacBlock), 0, s, A, h0, u.per);
-        return;
-    }
-    // the products, split over K where ks > 1
-    auto product = [&](auto plain, auto part, auto fix, const FacSplit &p) {
-        if (p.ks > 1) {
-            hipLaunchKernelGGL(part, dim3(count * p.per * p.ks), dim3(kFacBlock), 0, s, A, h0, p.per, p.ks);
-            hipLaunchKernelGGL(fix, dim3(count * p.per), dim3(kFacBlock), 0, s, A, h0, p.per, p.ks);
-        } else {
-            hipLaunchKernelGGL(plain, dim3(count * p.per), dim3(kFacBlock), 0, s, A, h0, p.per, 1);
-        }
-    };
-    product(k_fac_g<0>, k_fac_g<1>, k_fac_g<2>, g);
-    product(k_fac_u<0>, k_fac_u<1>, k_fac_u<2>, u);
 }
 
 void launch_copy_probe(hipStream_t s, const void *src, void *dst, long long n16) {

@@ -501,7 +501,7 @@ int analyze_device(md_mesh *m) {
     size_t o_pc = A.reserve(psz * std::max<int64_t>(1, last(f.pc_off)));
     size_t o_pr = A.reserve(psz * std::max<int64_t>(1, last(f.pr_off)));
     size_t o_fac = A.reserve(sizeof(FacDev) * std::max(1, ns));
-    size_t o_hl = A.reserve(sizeof(int) * std::max(1, ns));
+    size_t o_fch = A.reserve(sizeof(FacChild) * std::max<size_t>(1, f.child.size()));
     size_t o_or = A.reserve(sizeof(int) * std::max<size_t>(1, f.offrows.size()));
     size_t o_rel = A.reserve(sizeof(int) * std::max<size_t>(1, f.rel.size()));
     int eblocks = std::max(1, cdiv(t.nslices, kSlicesPerBlock));
@@ -544,7 +544,7 @@ int analyze_device(md_mesh *m) {
     d.child_ptr = (const int *)A.at(o_cp); d.child = (const int *)A.at(o_ch);
     d.pc = A.at(o_pc); d.pr = A.at(o_pr);
     m->d_fac = (const FacDev *)A.at(o_fac);
-    m->d_hlist = (const int *)A.at(o_hl);
+    m->d_fchild = (const FacChild *)A.at(o_fch);
     m->d_offrows = (const int *)A.at(o_or);
     m->d_rel = (const int *)A.at(o_rel);
     d.energy_part = (double *)A.at(o_en);
@@ -570,18 +570,24 @@ int analyze_device(md_mesh *m) {
     chk(up(d.slot_fe, t.slot_fe.data(), sizeof(int) * t.slot_fe.size()));
     chk(up(m->d_orig, t.original_of.data(), sizeof(int) * n));
     std::vector<FacDev> fh(ns);
-    for (int k = 0; k < ns; ++k) {
-        FacDev &x = fh[k];
+    for (int i = 0; i < ns; ++i) {
+        FacDev &x = fh[i];
+        const int k = f.hlist[i];
         x.c0 = f.c0[k]; x.w = f.w[k]; x.noff = f.noff[k]; x.roff = f.roff[k];
         x.cb = f.child_ptr[k]; x.ce = f.child_ptr[k + 1]; x.m = f.w[k] + f.noff[k]; x.pad = 0;
         x.poff = f.poff[k]; x.soff = f.woff_s[k]; x.toff = f.woff_t[k]; x.uoff = f.woff_u[k];
         x.pc_off = f.pc_off[k]; x.pr_off = f.pr_off[k];
     }
+    std::vector<FacChild> fch(f.child.size());
+    for (size_t k = 0; k < fch.size(); ++k) {
+        const int c = f.child[k];
+        fch[k] = FacChild{f.noff[c], f.roff[c], f.woff_u[c]};
+    }
     if (ns > 0) {
         chk(up(d.child_ptr, f.child_ptr.data(), sizeof(int) * (ns + 1)));
         chk(up(d.child, f.child.data(), sizeof(int) * f.child.size()));
         chk(up(m->d_fac, fh.data(), sizeof(FacDev) * ns));
-        chk(up(m->d_hlist, f.hlist.data(), sizeof(int) * ns));
+        chk(up(m->d_fchild, fch.data(), sizeof(FacChild) * fch.size()));
         chk(up(m->d_offrows, f.offrows.data(), sizeof(int) * f.offrows.size()));
         chk(up(m->d_rel, f.rel.data(), sizeof(int) * f.rel.size()));
     }
@@ -884,41 +890,36 @@ int factor_device(md_mesh *m) {
     const Factor &f = m->fac;
     const int ns = f.ns, nf = m->topo.nf;
     hipStream_t st = m->ctx->stream;
-    // per height: workgroups per supernode of the multi-workgroup stages, for the height's largest
-    // front (assembly one per asm_cols front columns: 64, halved down to 8 while the height has
-    // fewer than 2048 assembly workgroups, since the top fronts take the largest children; the
-    // products one per 64 x 64 output tile), and the products' splits over K
+    // what each height's launches are sized by
     struct HeightLaunch {
-        int count, mw, mm, asm_cols;
-        FacSplit g, u;
+        int small, sm;  // fronts of at most kFacSmallFront rows (first in the height) in one fused
+                        // launch, and the rows of the largest; the others:
+        int count, mw, mm, mo, tiles;
+        long long maps;  // children x rows of a front
     };
     const int nh = (int)f.hptr.size() - 1;
     std::vector<HeightLaunch> hl(nh);
-    size_t nW = 0;
     for (int h = 0; h < nh; ++h) {
         HeightLaunch &L = hl[h];
-        L = HeightLaunch{f.hptr[h + 1] - f.hptr[h], 0, 1, 64, {0, 1}, {0, 1}};
-        auto lower = [](int b) { return b * (b + 1) / 2; };
-        for (int i = f.hptr[h]; i < f.hptr[h + 1]; ++i) {
-            const int w = f.w[f.hlist[i]], no = f.noff[f.hlist[i]];
-            const int bw = (w + 63) / 64, bo = (no + 63) / 64;
+        L = HeightLaunch{0, 0, 0, 0, 1, 0, 0, 0};
+        auto rows = [&](int i) { return f.w[f.hlist[i]] + f.noff[f.hlist[i]]; };
+        const int n = f.hptr[h + 1] - f.hptr[h];
+        while (L.small < n && rows(f.hptr[h] + L.small) <= kFacSmallFront) ++L.small;
+        if (!fac_split_small(L.small, n)) L.small = 0;
+        if (L.small > 0) L.sm = rows(f.hptr[h] + L.small - 1);
+        L.count = n - L.small;
+        for (int i = f.hptr[h] + L.small; i < f.hptr[h + 1]; ++i) {
+            const int t = f.hlist[i], w = f.w[t], no = f.noff[t], b = (w + 63) / 64 + (no + 63) / 64;
             L.mw = std::max(L.mw, w);
             L.mm = std::max(L.mm, w + no);
-            L.g.per = std::max(L.g.per, bo * bw);
-            L.u.per = std::max(L.u.per, lower(bo));
-        }
-        if (L.mm <= kFacSmallFront) continue;  // small fronts only: one fused launch
-        while (L.asm_cols > 8 && (long long)L.count * ((L.mm + L.asm_cols - 1) / L.asm_cols) < 2048) L.asm_cols /= 2;
-        const int chunks = (L.mw + 31) / 32;
-        for (FacSplit *p : {&L.g, &L.u}) {
-            if (p->per == 0) continue;
-            p->ks = fac_split_k((long long)L.count * p->per, chunks);
-            if (p->ks > 1) nW = std::max(nW, (size_t)fac_split_k_doubles((long long)L.count * p->per * p->ks));
+            L.mo = std::max(L.mo, no);
+            L.tiles = std::max(L.tiles, b * (b + 1) / 2);
+            L.maps = std::max(L.maps, (long long)(f.child_ptr[t + 1] - f.child_ptr[t]) * (w + no));
         }
     }
     const size_t nP = (size_t)f.poff[ns], nS = (size_t)f.woff_s[ns], nT = (size_t)f.woff_t[ns],
                  nU = (size_t)f.woff_u[ns];
-    const size_t bytes = sizeof(double) * (nP + nS + nT + nU + nW + (size_t)nf) + 2 * sizeof(unsigned long long);
+    const size_t bytes = sizeof(double) * (nP + nS + nT + nU + (size_t)nf) + 2 * sizeof(unsigned long long);
     const bool keep = m->cfg.rest_mode == MD_REST_REFERENCE;  // refactors on every deform call
     if (m->fac_ws && m->fac_ws_bytes != bytes) m->release_fac_ws();
     if (!m->fac_ws) {
@@ -931,10 +932,10 @@ int factor_device(md_mesh *m) {
     }
     void *ws = m->fac_ws;
     FacArgs A{};
-    A.sn = m->d_fac; A.hlist = m->d_hlist; A.offrows = m->d_offrows; A.rel = m->d_rel; A.child = m->dev.child;
+    A.sn = m->d_fac; A.child = m->d_fchild; A.offrows = m->d_offrows; A.rel = m->d_rel;
     A.slice_ptr = m->dev.slice_ptr; A.sell_col = m->dev.sell_col; A.w64 = m->dev.w64; A.nf = nf;
     double *base = static_cast<double *>(ws);
-    A.P = base; A.S = A.P + nP; A.T = A.S + nS; A.U = A.T + nT; A.Wk = A.U + nU; A.diag = A.Wk + nW;
+    A.P = base; A.S = A.P + nP; A.T = A.S + nS; A.U = A.T + nT; A.diag = A.U + nU;
     A.amax = reinterpret_cast<unsigned long long *>(A.diag + nf);
     A.flag = reinterpret_cast<int *>(A.amax + 1);
     A.pc = const_cast<void *>(m->dev.pc);
@@ -945,12 +946,9 @@ int factor_device(md_mesh *m) {
         launch_fac_diag(st, A);
         for (int h = 0; h < nh; ++h) {
             const HeightLaunch &L = hl[h];
-            if (L.mm <= kFacSmallFront) {  // small fronts only: one fused launch
-                launch_fac_small(st, A, f.hptr[h], L.count, L.mm);
-                continue;
-            }
-            launch_fac_height(st, A, f.hptr[h], L.count, (L.mw + 63) / 64, L.asm_cols,
-                              (L.mm + L.asm_cols - 1) / L.asm_cols, L.g, L.u);
+            if (L.small > 0) launch_fac_small(st, A, f.hptr[h], L.small, L.sm);
+            launch_fac_height(st, A, f.hptr[h] + L.small, L.count, (L.mw + 63) / 64,
+                              fac_assembly(L.count, L.mm, L.mo, L.maps), L.tiles);
         }
         e = hipGetLastError();
     }
@@ -1201,7 +1199,7 @@ void rebind(md_mesh *m, const char *oa, size_t asz, char *na, const char *ol, si
     fix(d.pc); fix(d.pr); fix(d.ftile); fix(d.btile); fix(d.sub); fix(d.sub_h); fix(d.snode); fix(d.scp);
     fix(d.sfc); fix(d.sbo); fix(d.srow); fix(d.sfi); fix(d.lrows); fix(d.energy_part); fix(d.w32);
     fix(d.diag); fix(d.cg_x); fix(d.cg_p); fix(d.cg_v); fix(d.cg_part);
-    fix(m->d_fac); fix(m->d_hlist); fix(m->d_offrows); fix(m->d_rel); fix(m->d_tgt_xyz);
+    fix(m->d_fac); fix(m->d_fchild); fix(m->d_offrows); fix(m->d_rel); fix(m->d_tgt_xyz);
     fix(m->d_orig); fix(m->d_xyz);
 }
 

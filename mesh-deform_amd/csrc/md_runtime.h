@@ -173,7 +173,8 @@ struct md_mesh {
     uint64_t gen = 0;              // bumped whenever device pointers in dev change
     // device numeric factorization: static structure (main arena)
     const md::FacDev *d_fac = nullptr;
-    const int *d_hlist = nullptr, *d_offrows = nullptr, *d_rel = nullptr;
+    const md::FacChild *d_fchild = nullptr;
+    const int *d_offrows = nullptr, *d_rel = nullptr;
     double factor_ms = 0.0;        // last numeric factorization (host or device), wall ms
     double deform_ms[6] = {0, 0, 0, 0, 0, 0};  // phases of the last md_mesh_deform (md_mesh_stats)
     double setup_phase_ms[3] = {0, 0, 0};      // phases of the last setup: analysis, uploads +
