@@ -66,7 +66,7 @@ typedef struct {
                           single iteration for the rest; PCG: single only), captured at the
                           first md_mesh_iterate / md_batch_iterate after a (re)layout; default 1 */
     int subtree_budget;/* MD_SOLVER_LDLT: LDS vector entries (at most 1024) of one bottom
-                          subtree of the factor swept by a single wavefront (fronts + columns of
+                          subtree of the factor swept by one workgroup (fronts + columns of
                           its supernodes); 0 sweeps every supernode by level launches;
                           default 512 */
     double amalg_ratio;/* MD_SOLVER_LDLT: relaxed supernode amalgamation, the share of explicit
@@ -99,7 +99,7 @@ typedef struct {
      * array element the phase must read or write counted once */
     int64_t bytes_local, bytes_residual, bytes_forward, bytes_backward;
     int subtree_budget;      /* sweep layout in use (md_config.subtree_budget or the autotuned one) */
-    int subtrees;            /* bottom subtrees swept by one wavefront each */
+    int subtrees;            /* bottom subtrees swept by one workgroup each */
     int64_t factor_nnz_exact;/* strictly-lower nonzeros of the exact factor (no explicit zeros) */
     double factor_ms;        /* wall time of the last numeric factorization (device or host) */
     /* wall milliseconds of the last md_mesh_deform call by phase: [0] host analysis (a new

@@ -605,38 +605,40 @@ void device_layout(Factor& f, int sub_budget) {
     }
     // bottom subtrees (the subtree of root r is the id range [r - size + 1, r]): per-supernode
     // records by height, contribution entries, backward off-row sources
-    f.nsub = 0; f.sub_lds_fwd = 0; f.sub_lds_bwd = 0; f.sub_nodes = 0;
+    f.nsub = 0; f.sub_lds_fwd = 0; f.sub_lds_bwd = 0; f.sub_nodes = 0; f.sub_heights = 0; f.sub_off = 0;
     f.sub.clear(); f.sub_h.clear(); f.snode.clear(); f.scp.clear(); f.sfc.clear(); f.sbo.clear();
     f.srow.clear();
     f.sfi.assign(n, -1);
-    std::vector<int> fb(nn, 0), fbb(nn, 0);
+    std::vector<int> fb(nn, 0);
     for (int r = 0; r < nn; ++r) {
         if (sub_root[r] != r) continue;
         const int first = r - size[r] + 1, nh = f.height[r] + 1;
         const int col0 = f.c0[first], col1 = f.c0[r] + f.w[r];
         std::vector<std::vector<int>> at(nh);
         for (int t = first; t <= r; ++t) at[f.height[t]].push_back(t);
-        // forward: every front; backward: the columns, then the fronts of one height
-        int fronts = 0, height_fronts = 0;
-        for (int t = first; t <= r; ++t) { fb[t] = fronts; fronts += f.w[t] + f.noff[t]; }
+        // fronts one after another in record order (by height)
+        int fronts = 0, off = 0;
+        for (int h = 0; h < nh; ++h)
+            for (int t : at[h]) {
+                fb[t] = fronts;
+                fronts += f.w[t] + f.noff[t];
+                off += f.noff[t];
+            }
         const int ncols = col1 - col0;
-        f.srow.push_back(col0);
-        f.srow.push_back(ncols);
+        const int row[8] = {col0, ncols, (int)(f.scp.size() / 2), fronts, (int)(f.sbo.size() / 2), off, 0, 0};
+        f.srow.insert(f.srow.end(), row, row + 8);
         for (int t = first; t <= r; ++t)
             for (int q = 0; q < f.w[t]; ++q) f.sfi[f.c0[t] + q] = fb[t] + q;
-        for (int h = 0; h < nh; ++h) {
-            int off = ncols;
-            for (int t : at[h]) { fbb[t] = off; off += f.w[t] + f.noff[t]; }
-            height_fronts = std::max(height_fronts, off - ncols);
-        }
         const int rec0 = (int)(f.snode.size() / 16);
         f.sub.push_back(rec0);
         f.sub.push_back(rec0 + size[r]);
         f.sub.push_back((int)f.sub_h.size());
         f.sub.push_back(nh);
         f.sub_lds_fwd = std::max(f.sub_lds_fwd, fronts);
-        f.sub_lds_bwd = std::max(f.sub_lds_bwd, ncols + height_fronts);
+        f.sub_lds_bwd = std::max(f.sub_lds_bwd, 2 * ncols + off);
+        f.sub_off = std::max(f.sub_off, off);
         f.sub_nodes = std::max(f.sub_nodes, size[r]);
+        f.sub_heights = std::max(f.sub_heights, nh);
         ++f.nsub;
         std::vector<std::vector<int>> lists;
         for (int h = 0; h <= nh; ++h) {
@@ -647,7 +649,7 @@ void device_layout(Factor& f, int sub_budget) {
                 const int w = f.w[t], no = f.noff[t], m = w + no;
                 int rec[16] = {f.c0[t], w, no, fb[t], (int)f.pc_off[t], (int)f.pr_off[t], (int)(f.scp.size() / 2),
                                (int)(f.sbo.size() / 2), t == r ? f.roff[t] : -1, (int)f.xoff[t],
-                               f.c0[t] - col0, pa, pb, pq, fbb[t], 0};
+                               f.c0[t] - col0, pa, pb, pq, 0, 0};
                 f.snode.insert(f.snode.end(), rec, rec + 16);
                 pa += m; pb += no; pq += w;
                 // children's update entries landing on each position, in child order
@@ -1130,7 +1132,7 @@ bool solve_tiles_host(const Factor& f, const double* b, double* x, std::string& 
         for (int j = f.sub[4 * (size_t)i]; j < f.sub[4 * (size_t)i + 1]; ++j) {
             const int* R = rec(j);
             if (fwd) e = std::max(e, R[3] + R[1] + R[2]);
-            else e = std::max(e, std::max(R[10] + R[1], R[14] + R[1] + R[2]));
+            else e += 2 * R[1] + R[2];
         }
         return e;
     };
@@ -1142,11 +1144,14 @@ bool solve_tiles_host(const Factor& f, const double* b, double* x, std::string& 
         lds.assign(3 * (size_t)entries, 0.0);
         stamp.assign(entries, 0);
         int phase = 1;
-        // the one-mesh form first writes the residual of the subtree's rows into their front
-        // positions (sfi); the gathers below read it from there
-        MD_CHECK(2 * (size_t)i + 1 < f.srow.size(), "subtree row range");
-        const int col0 = f.srow[2 * (size_t)i], ncols = f.srow[2 * (size_t)i + 1];
+        // every position starts at zero, then the residual of the subtree's rows goes to theirs (sfi)
+        MD_CHECK(8 * (size_t)i + 7 < f.srow.size() && nh <= f.sub_heights, "subtree row range");
+        const int col0 = f.srow[8 * (size_t)i], ncols = f.srow[8 * (size_t)i + 1];
+        const int cp0 = f.srow[8 * (size_t)i + 2];
+        MD_CHECK(f.srow[8 * (size_t)i + 3] == entries, "subtree positions");
         MD_CHECK(col0 >= 0 && ncols > 0 && (size_t)col0 + ncols <= f.sfi.size(), "subtree rows");
+        for (int e = 0; e < entries; ++e) MD_CHECK(lds_claim(e, entries, phase), "subtree position clear");
+        ++phase;
         for (int t = 0; t < ncols; ++t) {
             const int e = f.sfi[(size_t)col0 + t];
             MD_CHECK(lds_claim(e, entries, phase), "subtree residual write");
@@ -1156,16 +1161,14 @@ bool solve_tiles_host(const Factor& f, const double* b, double* x, std::string& 
             int ra, rb;
             MD_CHECK(sub_heights(i, h, ra, rb), "subtree height range");
             ++phase;
-            const int npos = rec(rb - 1)[11] + items(rb - 1, 11);
-            for (int t = 0; t < npos; ++t) {
-                const int j = find(ra, rb, 11, t);
-                const int* R = rec(j);
-                const int p = t - R[11], w = R[1];
-                MD_CHECK(p >= 0 && p < w + R[2], "subtree position map");
-                MD_CHECK(R[6] >= 0 && 2 * ((size_t)R[6] + p) + 1 < f.scp.size(), "subtree contribution entry");
+            // positions of the height, one range; children's entries added (none at height 0)
+            const int p0 = rec(ra)[6] - cp0, p1 = rec(rb - 1)[6] - cp0 + items(rb - 1, 11);
+            MD_CHECK(p0 >= 0 && p0 < p1 && p1 <= entries, "subtree position range");
+            for (int t = p0; t < p1; ++t) {
+                MD_CHECK(2 * ((size_t)cp0 + t) + 1 < f.scp.size(), "subtree contribution entry");
                 // child entries: the first two inline, the rest from a -1-terminated list
                 std::vector<int> src;
-                const int e0 = f.scp[2 * (R[6] + p)], e1 = f.scp[2 * (R[6] + p) + 1];
+                const int e0 = f.scp[2 * ((size_t)cp0 + t)], e1 = f.scp[2 * ((size_t)cp0 + t) + 1];
                 if (e0 >= 0) src.push_back(e0);
                 if (e1 >= 0) {
                     src.push_back(e1);
@@ -1177,24 +1180,21 @@ bool solve_tiles_host(const Factor& f, const double* b, double* x, std::string& 
                         src.push_back(f.sfc[c]);
                     }
                 }
+                if (h == 0) {
+                    MD_CHECK(src.empty(), "children of a leaf");
+                    continue;
+                }
                 double v[3] = {0, 0, 0};
                 for (int c = 0; c < 3; ++c) {
-                    if (p < w) {
-                        MD_CHECK(R[0] + p < n && f.sfi[R[0] + p] == R[3] + p, "subtree residual slot");
-                        MD_CHECK(lds_read(R[3] + p, entries, phase, c, v[c]), "subtree residual read");
-                        MD_CHECK(v[c] == b[(size_t)c * n + R[0] + p], "subtree residual value");
-                    }
+                    MD_CHECK(lds_read(t, entries, phase, c, v[c]), "subtree position read");
                     for (int e : src) {
                         double u;
                         MD_CHECK(lds_read(e, entries, phase, c, u), "subtree child update read");
                         v[c] += u;
                     }
                 }
-                MD_CHECK(lds_claim(R[3] + p, entries, phase), "subtree front write");
-                for (int c = 0; c < 3; ++c) {
-                    lds[3 * (size_t)(R[3] + p) + c] = v[c];
-                    if (p < w) z[3 * (size_t)(R[0] + p) + c] = v[c];
-                }
+                MD_CHECK(lds_claim(t, entries, phase), "subtree front write");
+                for (int c = 0; c < 3; ++c) lds[3 * (size_t)t + c] = v[c];
             }
             ++phase;
             const int nrow = rec(rb - 1)[12] + items(rb - 1, 12);
@@ -1227,6 +1227,10 @@ bool solve_tiles_host(const Factor& f, const double* b, double* x, std::string& 
                 }
             }
         }
+        ++phase;
+        for (int t = 0; t < ncols; ++t)
+            for (int c = 0; c < 3; ++c)
+                MD_CHECK(lds_read(f.sfi[(size_t)col0 + t], entries, phase, c, z[3 * (size_t)(col0 + t) + c]), "subtree z");
     }
     // children's contributions to position pos of level supernode s: the sum of its uk slots
     // (unused ones zero), in slot order as the kernels sum them
@@ -1329,42 +1333,45 @@ bool solve_tiles_host(const Factor& f, const double* b, double* x, std::string& 
         MD_CHECK(entries > 0 && entries <= f.sub_lds_bwd, "subtree extent (backward)");
         lds.assign(3 * (size_t)entries, 0.0);
         stamp.assign(entries, 0);
-        // the column region starts with z of the subtree's rows; each row's x replaces it
+        // z of the subtree's rows, then their x, then the off rows of its fronts; the off rows outside
+        // the subtree are gathered at the start
         int phase = 1;
-        const int col0 = f.srow[2 * (size_t)i], ncols = f.srow[2 * (size_t)i + 1];
+        const int col0 = f.srow[8 * (size_t)i], ncols = f.srow[8 * (size_t)i + 1];
+        const int ob0 = f.srow[8 * (size_t)i + 4], nob = f.srow[8 * (size_t)i + 5];
+        MD_CHECK(2 * ncols + nob == entries && nob <= f.sub_off, "subtree off rows");
         for (int t = 0; t < ncols; ++t) {
             MD_CHECK(lds_claim(t, entries, phase), "subtree z write");
             for (int c = 0; c < 3; ++c) lds[3 * (size_t)t + c] = z[3 * (size_t)(col0 + t) + c];
+        }
+        for (int e = 0; e < nob; ++e) {
+            MD_CHECK(2 * ((size_t)ob0 + e) + 1 < f.sbo.size(), "subtree off-row source");
+            const int src = f.sbo[2 * ((size_t)ob0 + e)], info = f.sbo[2 * ((size_t)ob0 + e) + 1];
+            if (info < 0) {
+                MD_CHECK(src >= 0 && src < ncols, "subtree off-row column");
+                continue;
+            }
+            MD_CHECK((info >> 16) >= 1, "subtree outer partial count");
+            MD_CHECK(lds_claim(2 * ncols + e, entries, phase), "subtree off-row write");
+            for (int c = 0; c < 3; ++c) {
+                double v;
+                MD_CHECK(sum_part(xp, src, info >> 16, info & 0xffff, 0, c, v), "subtree outer solution");
+                lds[3 * (size_t)(2 * ncols + e) + c] = -v;
+            }
         }
         for (int h = nh - 1; h >= 0; --h) {
             int ra, rb;
             MD_CHECK(sub_heights(i, h, ra, rb), "subtree height range");
             ++phase;
-            const int npos = rec(rb - 1)[11] + items(rb - 1, 11);
-            for (int t = 0; t < npos; ++t) {
-                const int j = find(ra, rb, 11, t);
-                const int* R = rec(j);
-                const int p = t - R[11], w = R[1];
+            const int e0 = rec(ra)[7] - ob0, e1 = rec(rb - 1)[7] - ob0 + items(rb - 1, 12);
+            MD_CHECK(e0 >= 0 && e0 <= e1 && e1 <= nob, "subtree off-row range");
+            for (int e = e0; e < e1; ++e) {
+                if (f.sbo[2 * ((size_t)ob0 + e) + 1] >= 0) continue;
+                MD_CHECK(h < nh - 1, "an off row of the root inside the subtree");
                 double v[3];
-                if (p < w) {
-                    MD_CHECK(R[10] + p < ncols && col0 + R[10] + p == R[0] + p, "subtree column slot");
-                    for (int c = 0; c < 3; ++c) MD_CHECK(lds_read(R[10] + p, entries, phase, c, v[c]), "subtree z read");
-                } else {
-                    const size_t e = (size_t)R[7] + p - w;
-                    MD_CHECK(R[7] >= 0 && 2 * e + 1 < f.sbo.size(), "subtree off-row source");
-                    const int src = f.sbo[2 * e], info = f.sbo[2 * e + 1];
-                    for (int c = 0; c < 3; ++c) {
-                        if (info < 0) {
-                            MD_CHECK(lds_read(src, entries, phase, c, v[c]), "subtree solution read");
-                        } else {
-                            MD_CHECK((info >> 16) >= 1, "subtree outer partial count");
-                            MD_CHECK(sum_part(xp, src, info >> 16, info & 0xffff, 0, c, v[c]), "subtree outer solution");
-                        }
-                        v[c] = -v[c];
-                    }
-                }
-                MD_CHECK(lds_claim(R[14] + p, entries, phase), "subtree rhs write");
-                for (int c = 0; c < 3; ++c) lds[3 * (size_t)(R[14] + p) + c] = v[c];
+                for (int c = 0; c < 3; ++c)
+                    MD_CHECK(lds_read(ncols + f.sbo[2 * ((size_t)ob0 + e)], entries, phase, c, v[c]), "subtree solution read");
+                MD_CHECK(lds_claim(2 * ncols + e, entries, phase), "subtree off-row write");
+                for (int c = 0; c < 3; ++c) lds[3 * (size_t)(2 * ncols + e) + c] = -v[c];
             }
             ++phase;
             const int ncol = rec(rb - 1)[13] + items(rb - 1, 13);
@@ -1374,18 +1381,19 @@ bool solve_tiles_host(const Factor& f, const double* b, double* x, std::string& 
                 const int q = t - R[13], w = R[1], mm = w + R[2];
                 MD_CHECK(q >= 0 && q < w && mm <= kSubMaxRows && R[5] >= 0 &&
                          (int64_t)R[5] + q + (int64_t)(mm - 1) * w < (int64_t)pr.size(), "subtree P range");
-                double acc[3] = {0, 0, 0};
+                double part[4][3] = {};  // four lanes per column, rows by p mod 4
                 for (int p = 0; p < mm; ++p)
                     for (int c = 0; c < 3; ++c) {
                         double v;
-                        MD_CHECK(lds_read(R[14] + p, entries, phase, c, v), "subtree rhs read");
-                        acc[c] += pr[R[5] + q + (size_t)p * w] * v;
+                        MD_CHECK(lds_read(p < w ? R[10] + p : 2 * ncols + R[7] - ob0 + p - w, entries, phase, c, v), "subtree rhs read");
+                        part[p & 3][c] += pr[R[5] + q + (size_t)p * w] * v;
                     }
-                MD_CHECK(lds_claim(R[10] + q, entries, phase), "subtree solution write");
+                MD_CHECK(lds_claim(ncols + R[10] + q, entries, phase), "subtree solution write");
                 MD_CHECK(R[9] >= 0 && R[9] + q < nx, "subtree solution output");
                 for (int c = 0; c < 3; ++c) {
-                    lds[3 * (size_t)(R[10] + q) + c] = acc[c];
-                    xp[3 * (size_t)(R[9] + q) + c] = acc[c];
+                    const double acc = (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
+                    lds[3 * (size_t)(ncols + R[10] + q) + c] = acc;
+                    xp[3 * (size_t)(R[9] + q) + c] = acc;
                 }
             }
         }

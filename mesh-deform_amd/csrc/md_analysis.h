@@ -25,13 +25,13 @@ constexpr int kPairBudget = 128;
 constexpr int kTile = 64;
 // Vertices per one-ring slice (one wavefront).
 constexpr int kSlice = 64;
-// Default LDS budget (vector entries) of one bottom subtree swept by a single wavefront.
+// Default LDS budget (vector entries) of one bottom subtree, swept by one workgroup.
 constexpr int kSubBudgetDefault = 512;
 // Default relaxed-amalgamation limit: a child merges into its parent while the explicit zeros
 // stay below this share of the merged panel (half of it for merges wider than 48 columns).
 constexpr double kAmalgRatioDefault = 0.3;
-// Largest budget: 1024 FP64 vector entries (32 bytes each) are 32 KiB of LDS; with at most
-// kSubMaxNodes 64-byte supernode records a subtree stays within 36 KiB.
+// Largest budget: 1024 FP64 vector entries (32 bytes each) are 32 KiB of LDS; with its index lists and
+// at most kSubMaxNodes 64-byte supernode records a subtree stays within 46 KiB.
 constexpr int kSubBudgetMax = 1024;
 constexpr int kSubMaxNodes = 64;
 // Largest supernode a bottom subtree may hold: columns, and rows of the front.
@@ -76,21 +76,21 @@ struct Topology {
 //     kr_s = ceil(m/64) partials that every reader (descendants, the final update) sums.
 //
 // Bottom subtrees: a subtree whose supernodes are all small (w <= 64, m <= 128) and whose
-// fronts and columns fit an LDS budget is swept by one wavefront, height by height, with
+// fronts and columns fit an LDS budget is swept by one workgroup, height by height, with
 // every front in LDS (no level launches, no global round trips inside the subtree). Its
 // supernodes keep one partial of x_s (kr = 1); only the subtree root stores u_s (kc = 1,
 // the others kc = 0). Each supernode of a subtree has a 16-int record (SubNode layout:
 // c0, w, noff, forward front base, G offset, [Dinv; G] offset, contribution base, off-row
 // source base, u output or -1, x output, LDS column base of x, position / off-row / column
-// prefix within its height, backward front base, 0). Records of a subtree are contiguous
-// and ordered by height; the wavefront copies them to LDS and maps lane items to supernodes
-// by binary search over the prefixes. LDS holds, forward, the fronts of all the subtree's
-// supernodes; backward, the solution columns of the subtree and the fronts of one height.
+// prefix within its height, 0, 0). Records of a subtree are contiguous and ordered by height; the
+// workgroup copies them to LDS and maps its items to supernodes by binary search over the
+// prefixes. LDS holds, forward, the fronts of the subtree's supernodes one after another in record
+// order; backward, z and x of the subtree's columns and the off rows of its fronts in record order.
 // Per item only this remains in HBM:
 //   forward positions: the LDS indices of the first two children's update entries landing
 //     there (-1: none); a second index <= -2 points (-2 - i) at sfc[i ..], a -1-terminated
 //     list of the rest;
-//   backward off-row positions: (LDS index of x, -1) when the row lies in the subtree, else
+//   backward off-row positions: (column of the subtree, -1) when the row lies in the subtree, else
 //     (first partial of x, count << 16 | stride) of the row's owner.
 // Level schedule: supernodes outside subtrees get level = 1 + the largest level of their
 // children outside subtrees (0 if none); subtree sweeps run before the forward levels and
@@ -137,15 +137,16 @@ struct Factor {
     // bottom subtrees
     int nsub = 0;                    // subtrees
     int sub_lds_fwd = 0, sub_lds_bwd = 0;  // LDS vector entries of the largest, per sweep
-    int sub_nodes = 0;               // supernodes of the largest subtree
+    int sub_nodes = 0, sub_heights = 0, sub_off = 0;  // supernodes, heights, backward off rows (largest)
     std::vector<int> sub;            // 4 per subtree: (first record, end record, height table offset, heights)
     std::vector<int> sub_h;          // per (subtree, height) + a terminal per subtree: first record
     std::vector<int> snode;          // 16 per subtree supernode (SubNode), by subtree then height
     std::vector<int> scp;            // 2 per forward position: first two child entries (see above)
     std::vector<int> sfc;            // -1-terminated overflow lists of child entries
     std::vector<int> sbo;            // 2 per off-row position of a subtree supernode (backward source)
-    std::vector<int> srow;           // 2 per subtree: first row, rows
-    std::vector<int> sfi;            // per row (n): forward front slot of a subtree row, else -1
+    std::vector<int> srow;           // 8 per subtree: first row, rows, first forward position (scp),
+                                     //   positions, first backward off row (sbo), off rows, 0, 0
+    std::vector<int> sfi;            // per row (n): forward position of a subtree row, else -1
     int64_t nnz_exact = 0;           // strictly-lower nonzeros of the exact factor (no amalgamation zeros)
     int64_t factor_nnz() const { return poff.empty() ? 0 : poff.back(); }
 };

@@ -67,7 +67,7 @@ struct MeshDev {
     const MD_G int4 *xloc;      // per off row entry: rowinfo of that row
     const MD_G void *pc, *pr;   // panels (float or double), forward and backward layouts
     const MD_G TileDev *ftile, *btile; // level tiles, level by level (bases in the launch tables)
-    // bottom subtrees, one wavefront each (layouts in md_analysis.h, Factor)
+    // bottom subtrees, one workgroup each (layouts in md_analysis.h, Factor)
     const MD_G int4 *sub;       // (first record, end record, height table offset, heights)
     const MD_G int *sub_h;      // first record of each (subtree, height), + a terminal per subtree
     const MD_G int4 *snode;     // supernode records, four int4 each (SubNode)
@@ -75,8 +75,9 @@ struct MeshDev {
     const MD_G int *sfc;        // -1-terminated overflow lists of child update entries
     const MD_G int2 *sbo;       // backward off-row sources
     int nsub;                   // bottom subtrees (their rows' x is added to p' by k_sub_bwd)
-    const MD_G int2 *srow;      // per subtree: first row, rows (their residual is formed in LDS)
-    const MD_G int *sfi;        // per free row of a subtree: its forward front slot in LDS
+    const MD_G int4 *srow;      // two per subtree: (first row, rows, first forward position,
+                                //   positions), (first backward off row, off rows, 0, 0)
+    const MD_G int *sfi;        // per free row of a subtree: its forward position in LDS
     int nlrows;                 // rows of level-swept supernodes, increasing
     const MD_G int *lrows;      //   (their residual: extra blocks of k_sub_fwd; x summed from the
                                 //   partials and added to p': extra blocks of k_sub_bwd)
@@ -141,12 +142,25 @@ void launch_local(hipStream_t s, LaunchSet L, int blocks, bool fp64);
 void launch_residual(hipStream_t s, LaunchSet L, int blocks, bool fp64);
 void launch_fwd(hipStream_t s, LaunchSet L, int blocks, int level, bool fp64);
 void launch_bwd(hipStream_t s, LaunchSet L, int blocks, int level, bool fp64);
-// Bottom-subtree sweeps: one 64-lane block per subtree; LDS for `nodes` supernode records
-// and `lds_entries` vector entries.
+// Bottom-subtree sweeps, one workgroup per subtree: LDS for the largest subtree's supernode records,
+// heights, forward positions, backward vector entries and backward off rows. block: kSubBlock threads
+// where the launch's subtrees are at most kSubFew (at most four workgroups per CU, so their chain
+// counts), else fewer: 64 forward with the residual (its registers allow three wavefronts per
+// SIMD), 128 forward without it and backward. Measured, 64 / 128 / 256 threads: 91 subtrees (FP32) 17.2 /
+// 12.5 / 11.1 us forward with the residual, 18.8 / 12.4 / 10.2 backward; 612 (FP32) 18.7 / 14.2 / 15.1 and
+// 20.8 / 14.8 / 12.2; 2,825 (FP64) 40 / 42 / 63 and 38 / 31 / 34; a batch's 7,413 (FP32, without the
+// residual) 38 / 34 / 47 and 57 / 59 / 80.
 // fused: the launch also forms the residual (one-mesh plans; blocks past the subtrees take
 // the level rows), else k_residual ran before it.
-void launch_sub_fwd(hipStream_t s, LaunchSet L, int blocks, int nodes, int lds_entries, bool fused, bool fp64);
-void launch_sub_bwd(hipStream_t s, LaunchSet L, int blocks, int nodes, int lds_entries, bool fp64);
+struct SubLds {
+    int block, nodes, heights, fwd, bwd, off;
+};
+constexpr int kSubBlock = 256, kSubFew = 1024;
+// Level rows per workgroup past the subtrees (its threads).
+inline int sub_rows_fwd(const SubLds &D) { return D.block == kSubBlock ? kSubBlock : 64; }  // fused
+inline int sub_rows_bwd(const SubLds &D) { return D.block == kSubBlock ? kSubBlock : 128; }
+void launch_sub_fwd(hipStream_t s, LaunchSet L, int blocks, const SubLds &D, bool fused, bool fp64);
+void launch_sub_bwd(hipStream_t s, LaunchSet L, int blocks, const SubLds &D, bool fp64);
 void launch_energy(hipStream_t s, LaunchSet L, int blocks, bool fp64);
 void launch_identity_quat(hipStream_t s, LaunchSet L, int blocks, bool fp64);
 // A target of a served request: the device address of its vertex's p' entry and the position.

@@ -813,23 +813,13 @@ __global__ __launch_bounds__(kTile) void k_bwd(LaunchSet L, int level) {
     else bwd_tile<64, T>(M, S, q0, p0, qn, pn);
 }
 
-// acc += sum_{i < n} P[i * stride] * v[i] (n <= 64; n <= 0 adds nothing but still reads P[0]
-// and v[0]) with the unrolled width chosen per wavefront (the widest active lane's class,
-// 16 / 32 / 64), so lanes of different widths do not diverge.
-template <typename T, typename V>
-__device__ __forceinline__ void wave_dot(const T *P, long long stride, const V *v, int n, T &ax, T &ay, T &az) {
-    if (__any(n > 32)) tile_dot<64>(P, stride, v, n, ax, ay, az);
-    else if (__any(n > 16)) tile_dot<32>(P, stride, v, n, ax, ay, az);
-    else tile_dot<16>(P, stride, v, n, ax, ay, az);
-}
-
 // Record of one supernode of a bottom subtree (16 ints, as the host lays it out).
 struct SubNode {
     int c0, w, noff, fb;     // columns, off rows, forward front base in LDS
     int pc, pr, cp, ob;      // G offset, [Dinv; G] offset, contribution entries, off-row sources
     int uo, xo, xs, pa;      // root: first update-slot entry (udst) or -1; x output, LDS column base
                              //   of x, position prefix
-    int pb, pq, fbb, pad;    // off-row prefix, column prefix, backward front base in LDS
+    int pb, pq, pad0, pad1;  // off-row prefix, column prefix (within the height)
 };
 
 // Last record j in [a, b) whose prefix (field F) is <= t.
@@ -844,124 +834,195 @@ __device__ __forceinline__ int sub_find(const SubNode *N, int a, int b, int t) {
     return lo;
 }
 
-// Copies the records [sd.x, sd.y) of a subtree to LDS.
-__device__ __forceinline__ void sub_records(const MD_G MeshDev &M, const int4 &sd, SubNode *N) {
-    int4 *dst = reinterpret_cast<int4 *>(N);
-    for (int i = threadIdx.x; i < 4 * (sd.y - sd.x); i += kTile) dst[i] = M.snode[4 * sd.x + i];
-    __syncthreads();
+// v from the lane whose index is this lane's xor Q (Q = 1, 2: within a quad), by DPP.
+template <int Q>
+__device__ __forceinline__ double quad_xor(double v) {
+    constexpr int ctrl = Q == 1 ? 0xB1 : 0x4E;  // quad_perm [1,0,3,2] / [2,3,0,1]
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)u, ctrl, 0xF, 0xF, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), ctrl, 0xF, 0xF, true);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
-// Bottom subtree, forward sweep, one wavefront per subtree (sd = first record, end record,
-// height table offset, heights). Heights bottom-up, each in two phases with every front in
-// LDS:
-//   positions: front[p] = (p < w ? r[c0 + p] : 0) + children's update entries; z = front[p < w],
-//   off rows:  front[w + i] -= G_s[i, 0..w) front[0 .. w)  (u_s in place; the root also stores
-//              u_s for its parent outside the subtree).
+// One subtree as the host lays it out: records [sub.x, sub.y), height table offset sub.z, sub.w
+// heights; rows [row.x, +row.y); forward positions [row.z, +row.w), backward off rows [ext.x, +ext.y).
+struct SubTree {
+    int4 sub, row;
+    int2 ext;
+};
+__device__ __forceinline__ SubTree sub_tree(const MD_G MeshDev &M, int k) {
+    const int4 e = M.srow[2 * k + 1];
+    return SubTree{M.sub[k], M.srow[2 * k], make_int2(e.x, e.y)};
+}
+
+// Panel entries of a sweep item kept in registers, loaded while the positions before it are formed
+// (their addresses depend on the layout alone).
+constexpr int kSubAhead = 16;
+
+// Bottom subtree, forward sweep, one workgroup per subtree, heights bottom-up with every front in LDS
+// (position t of the subtree at F[t], its records' fronts one after another):
+//   F = residual on the rows, else 0; per height
+//   positions: F[t] += the children's update entries (none at height 0),
+//   off rows:  F[w + i] -= G_s[i, 0..w) F[0 .. w)  (u_s in place; the root also stores u_s for its
+//              parent outside the subtree);
+// z = F on the rows at the end. Index lists are in LDS from the start and the next height's panel
+// entries are loaded ahead, so a height costs no round trip of its own.
 // With Fused (one-mesh launches), the residual is formed here: subtree rows straight into
 // their front positions, level rows by blocks past the subtrees (no k_residual launch; more
 // registers, so batches keep the separate residual).
-template <typename T, bool Fused>
-__global__ __launch_bounds__(kTile) void k_sub_fwd(LaunchSet L, int node_cap) {
+// Bound by its chain of heights where the subtrees are few (a 10k icosphere's 91 in FP32: 11 us with the
+// residual, 18 with one wavefront per subtree and dependent loads in every height), by occupancy
+// where they are many.
+template <typename T, bool Fused, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_sub_fwd(LaunchSet L, SubLds D) {
     using V = typename V4T<T>::type;
     extern __shared__ __align__(32) unsigned char sub_smem[];
-    SubNode *N = reinterpret_cast<SubNode *>(sub_smem);
-    V *F = reinterpret_cast<V *>(sub_smem + sizeof(SubNode) * node_cap);
+    V *F = reinterpret_cast<V *>(sub_smem);
+    SubNode *N = reinterpret_cast<SubNode *>(F + D.fwd);
+    int2 *cp = reinterpret_cast<int2 *>(N + D.nodes);
+    int *H = reinterpret_cast<int *>(cp + D.fwd);
     const int k = find_mesh(L, blockIdx.x);
     const MD_G MeshDev &M = L.meshes[k];
-    const int lane = threadIdx.x;
+    const int tid = threadIdx.x;
     const int bk = blockIdx.x - L.prefix[k];
     if (Fused && bk >= M.nsub) {
-        // blocks past the subtrees: the residual of 64 rows of level supernodes
-        const int j = (bk - M.nsub) * kTile + lane;
+        // blocks past the subtrees: the residual of BLOCK rows of level supernodes
+        const int j = (bk - M.nsub) * BLOCK + tid;
         if (j < M.nlrows) {
             const int i = M.lrows[j];
             reinterpret_cast<V *>(M.r)[i] = residual_of<T, 8>(M, i);
         }
         return;
     }
-    const int4 sd = M.sub[bk];
+    const SubTree S = sub_tree(M, bk);
     const V *R = reinterpret_cast<const V *>(M.r);
     V *Z = reinterpret_cast<V *>(M.z);
     V *U = reinterpret_cast<V *>(M.upart);
     const T *G = tptr<T>(M.pc);
-    if (Fused) {
-        // the residual of the subtree's rows, straight into their front positions (it is
-        // read by nothing else)
-        const int2 rr = M.srow[bk];
-        for (int t = lane; t < rr.y; t += kTile) F[M.sfi[rr.x + t]] = residual_of<T, 8>(M, rr.x + t);
+    {
+        int4 *dst = reinterpret_cast<int4 *>(N);
+        for (int i = tid; i < 4 * (S.sub.y - S.sub.x); i += BLOCK) dst[i] = M.snode[4 * S.sub.x + i];
+        for (int i = tid; i <= S.sub.w; i += BLOCK) H[i] = M.sub_h[S.sub.z + i] - S.sub.x;
+        V zero;
+        zero.x = 0; zero.y = 0; zero.z = 0; zero.w = 0;
+        for (int i = tid; i < S.row.w; i += BLOCK) {
+            cp[i] = M.scp[S.row.z + i];
+            F[i] = zero;
+        }
     }
-    sub_records(M, sd, N);  // ends with a barrier
-    for (int h = 0; h < sd.w; ++h) {
-        const int a = M.sub_h[sd.z + h] - sd.x, b = M.sub_h[sd.z + h + 1] - sd.x;
-        const int npos = N[b - 1].pa + N[b - 1].w + N[b - 1].noff;
-        for (int t = lane; t < npos; t += kTile) {
-            const SubNode &S = N[sub_find<&SubNode::pa>(N, a, b, t)];
-            const int p = t - S.pa;
-            V v;
-            v.x = 0; v.y = 0; v.z = 0; v.w = 0;
-            if (p < S.w) v = Fused ? F[S.fb + p] : R[S.c0 + p];  // the residual
-            // children's update entries: two inline, the rest from a -1-terminated list
-            const int2 e = M.scp[S.cp + p];
-            if (e.x >= 0) {
-                const V u = F[e.x];
-                v.x += u.x; v.y += u.y; v.z += u.z;
-            }
-            if (e.y >= 0) {
-                const V u = F[e.y];
-                v.x += u.x; v.y += u.y; v.z += u.z;
-            } else if (e.y <= -2) {
-                for (int c = -2 - e.y;; ++c) {
-                    const int q = M.sfc[c];
-                    if (q < 0) break;
-                    const V u = F[q];
+    __syncthreads();
+    for (int t = tid; t < S.row.y; t += BLOCK)
+        F[M.sfi[S.row.x + t]] = Fused ? residual_of<T, 8>(M, S.row.x + t) : R[S.row.x + t];
+    // off row t of height h: its record and the first kSubAhead entries of its row of G_s
+    T g[kSubAhead];
+    int item = 0;
+    auto load = [&](int a, int b, int t) {
+        item = sub_find<&SubNode::pb>(N, a, b, t);
+        const SubNode &s = N[item];
+        panel_load<kSubAhead, T>(G + s.pc + (t - s.pb), s.noff, s.w, g);
+    };
+    auto rows_of = [&](int h) { return N[H[h + 1] - 1].pb + N[H[h + 1] - 1].noff; };
+    if (tid < rows_of(0)) load(H[0], H[1], tid);
+    __syncthreads();
+    for (int h = 0; h < S.sub.w; ++h) {
+        const int a = H[h], b = H[h + 1];
+        if (h > 0) {
+            const int p0 = N[a].cp - S.row.z, p1 = N[b - 1].cp - S.row.z + N[b - 1].w + N[b - 1].noff;
+            for (int t = p0 + tid; t < p1; t += BLOCK) {
+                // children's update entries: two inline, the rest from a -1-terminated list
+                const int2 e = cp[t];
+                V v = F[t];
+                if (e.x >= 0) {
+                    const V u = F[e.x];
                     v.x += u.x; v.y += u.y; v.z += u.z;
                 }
+                if (e.y >= 0) {
+                    const V u = F[e.y];
+                    v.x += u.x; v.y += u.y; v.z += u.z;
+                } else if (e.y <= -2) {
+                    for (int c = -2 - e.y;; ++c) {
+                        const int q = M.sfc[c];
+                        if (q < 0) break;
+                        const V u = F[q];
+                        v.x += u.x; v.y += u.y; v.z += u.z;
+                    }
+                }
+                F[t] = v;
             }
-            v.w = 0;
-            F[S.fb + p] = v;
-            if (p < S.w) Z[S.c0 + p] = v;
+            __syncthreads();
         }
-        __syncthreads();
-        const int nrow = N[b - 1].pb + N[b - 1].noff;
-        for (int t0 = 0; t0 < nrow; t0 += kTile) {
-            const int t = t0 + lane;
-            const bool on = t < nrow;
-            const SubNode &S = N[sub_find<&SubNode::pb>(N, a, b, on ? t : nrow - 1)];
-            const int i = (on ? t : nrow - 1) - S.pb;
+        const int nrow = rows_of(h);
+        for (int t = tid; t < nrow; t += BLOCK) {
+            if (t != tid) load(a, b, t);
+            const SubNode &s = N[item];
+            const int i = t - s.pb;
+            const V *v = F + s.fb;
             T ax = 0, ay = 0, az = 0;
             // column-major G_s: entry (row i, column q) at q * noff + i
-            wave_dot<T, V>(G + S.pc + i, S.noff, F + S.fb, on ? S.w : 0, ax, ay, az);
-            if (on) {
-                V o = F[S.fb + S.w + i];
-                o.x -= ax; o.y -= ay; o.z -= az;
-                F[S.fb + S.w + i] = o;
-                if (S.uo >= 0) U[M.udst[S.uo + i]] = o;  // the root: into the parent's slot
+            for (int q0 = 0; q0 < s.w; q0 += kSubAhead) {
+                if (q0 > 0) panel_load<kSubAhead, T>(G + s.pc + i + (long long)q0 * s.noff, s.noff, s.w - q0, g);
+#pragma unroll
+                for (int u0 = 0; u0 < kSubAhead; u0 += 4) {
+                    if (q0 + u0 < s.w) {
+#pragma unroll
+                        for (int u = u0; u < u0 + 4; ++u) {
+                            const V x = v[min(q0 + u, s.w - 1)];
+                            const T e = q0 + u < s.w ? g[u] : T(0);
+                            ax += e * x.x; ay += e * x.y; az += e * x.z;
+                        }
+                    }
+                }
             }
+            V o = F[s.fb + s.w + i];
+            o.x -= ax; o.y -= ay; o.z -= az;
+            F[s.fb + s.w + i] = o;
+            if (s.uo >= 0) U[M.udst[s.uo + i]] = o;  // the root: into the parent's slot
         }
+        if (h + 1 < S.sub.w && tid < rows_of(h + 1)) load(b, H[h + 2], tid);
         __syncthreads();
     }
+    for (int t = tid; t < S.row.y; t += BLOCK) Z[S.row.x + t] = F[M.sfi[S.row.x + t]];
 }
 
-// Bottom subtree, backward sweep, one wavefront per subtree. Heights top-down, with the
-// subtree's solution columns and the fronts of one height in LDS:
-//   positions: t[p] = z[c0 + p] (p < w), else -x of the off row, from LDS when the row lies
-//              in the subtree, else the sum of its owner's partials,
-//   columns:   x_s[q] = sum_p [Dinv_s; G_s][p, q] t[p], to LDS and to the single partial.
+// Bottom subtree, backward sweep, one workgroup per subtree, heights top-down with the subtree's z and
+// solution columns and the fronts' off rows in LDS (z at F[t], x at F[ncols + t], off row e at
+// F[2 ncols + e]). Off rows outside the subtree are gathered once at the start (-x, the sum of their
+// owner's partials); per height
+//   off rows: -x of those inside, from LDS,
+//   columns:  x_s[q] = sum_p [Dinv_s; G_s][p, q] t[p], t = [z_s; off rows], four lanes per column
+//             (rows p = lane mod 4, joined by DPP: a front of up to 64 rows is one load of kSubAhead
+//             entries per lane, made a height ahead).
+// A 10k icosphere's 91 subtrees in FP32: 9.5 us; one wavefront per subtree, one lane per column and
+// a round trip for the sources and one for the panel in every height took 19. The 164k icosphere's
+// 2,825 in FP64: 31 us (50), a batch's 7,413 in FP32: 59 us (73).
 template <typename T>
-__global__ __launch_bounds__(kTile) void k_sub_bwd(LaunchSet L, int node_cap) {
+__device__ __forceinline__ T quad_sum(T v) {
+    if constexpr (sizeof(T) == 8) {
+        v += quad_xor<1>(v);
+        v += quad_xor<2>(v);
+    } else {
+        v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));
+        v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, true));
+    }
+    return v;
+}
+template <typename T, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_sub_bwd(LaunchSet L, SubLds D) {
     using V = typename V4T<T>::type;
     extern __shared__ __align__(32) unsigned char sub_smem[];
-    SubNode *N = reinterpret_cast<SubNode *>(sub_smem);
-    V *F = reinterpret_cast<V *>(sub_smem + sizeof(SubNode) * node_cap);
+    V *F = reinterpret_cast<V *>(sub_smem);
+    SubNode *N = reinterpret_cast<SubNode *>(F + D.bwd);
+    int *src = reinterpret_cast<int *>(N + D.nodes);  // x column of an off row inside the subtree, else -1
+    int *H = src + D.off;
     const int k = find_mesh(L, blockIdx.x);
     const MD_G MeshDev &M = L.meshes[k];
-    const int lane = threadIdx.x;
+    const int tid = threadIdx.x;
     const V *X = reinterpret_cast<const V *>(M.xpart);
     const int bk = blockIdx.x - L.prefix[k];
     if (bk >= M.nsub) {
-        // blocks past the subtrees: p' += x for 64 rows of level supernodes (x summed from
+        // blocks past the subtrees: p' += x for BLOCK rows of level supernodes (x summed from
         // the partials of the level sweeps)
-        const int j = (bk - M.nsub) * kTile + lane;
+        const int j = (bk - M.nsub) * BLOCK + tid;
         if (j < M.nlrows) {
             const int i = M.lrows[j];
             const int4 ri = M.rowinfo[i];
@@ -972,64 +1033,99 @@ __global__ __launch_bounds__(kTile) void k_sub_bwd(LaunchSet L, int node_cap) {
         }
         return;
     }
-    const int4 sd = M.sub[bk];
+    const SubTree S = sub_tree(M, bk);
     const T *P = tptr<T>(M.pr);
-    // the column region F[0 .. ncols) starts with z of the subtree's rows (read at the row's
-    // height, then replaced by its x)
-    const int2 rr = M.srow[bk];
+    const int nc = S.row.y;
+    V *x = F + nc, *off = F + 2 * nc;
     {
+        int4 *dst = reinterpret_cast<int4 *>(N);
+        for (int i = tid; i < 4 * (S.sub.y - S.sub.x); i += BLOCK) dst[i] = M.snode[4 * S.sub.x + i];
+        for (int i = tid; i <= S.sub.w; i += BLOCK) H[i] = M.sub_h[S.sub.z + i] - S.sub.x;
         const V *Zs = reinterpret_cast<const V *>(M.z);
-        for (int t = lane; t < rr.y; t += kTile) F[t] = Zs[rr.x + t];
-    }
-    sub_records(M, sd, N);  // ends with a barrier
-    for (int h = sd.w - 1; h >= 0; --h) {
-        const int a = M.sub_h[sd.z + h] - sd.x, b = M.sub_h[sd.z + h + 1] - sd.x;
-        const int npos = N[b - 1].pa + N[b - 1].w + N[b - 1].noff;
-        for (int t = lane; t < npos; t += kTile) {
-            const SubNode &S = N[sub_find<&SubNode::pa>(N, a, b, t)];
-            const int p = t - S.pa;
-            V v;
-            if (p < S.w) {
-                v = F[S.xs + p];
-            } else {
-                const int2 d = M.sbo[S.ob + p - S.w];
-                // x of the row: from LDS, or the owner's partials loaded 8 at a time
-                const V g = d.y < 0 ? F[d.x] : sum_partials<V>(X + d.x, d.y >> 16, d.y & 0xffff, 0);
-                v.x = -g.x; v.y = -g.y; v.z = -g.z;
+        for (int t = tid; t < nc; t += BLOCK) F[t] = Zs[S.row.x + t];
+        for (int e = tid; e < S.ext.y; e += BLOCK) {
+            const int2 d = M.sbo[S.ext.x + e];
+            src[e] = d.y < 0 ? d.x : -1;
+            if (d.y >= 0) {
+                const V u = sum_partials<V>(X + d.x, d.y >> 16, d.y & 0xffff, 0);
+                V o;
+                o.x = -u.x; o.y = -u.y; o.z = -u.z; o.w = 0;
+                off[e] = o;
             }
-            v.w = 0;
-            F[S.fbb + p] = v;
         }
-        __syncthreads();
-        const int ncol = N[b - 1].pq + N[b - 1].w;
-        for (int t0 = 0; t0 < ncol; t0 += kTile) {
-            const int t = t0 + lane;
-            const bool on = t < ncol;
-            const SubNode &S = N[sub_find<&SubNode::pq>(N, a, b, on ? t : ncol - 1)];
-            const int q = (on ? t : ncol - 1) - S.pq, m = S.w + S.noff;
+    }
+    __syncthreads();
+    // column t of height h: its record and the first entries of the lane's rows
+    const int part = tid & 3;
+    T g[kSubAhead];
+    int item = 0;
+    auto rows4 = [&](const SubNode &s, int q, int p0) {  // rows p0 + part, + 4, ...
+        const int m = s.w + s.noff;
+        const T *p = P + s.pr + q;
+#pragma unroll
+        for (int u = 0; u < kSubAhead; ++u) g[u] = p[(long long)min(p0 + part + 4 * u, m - 1) * s.w];
+    };
+    auto load = [&](int a, int b, int t) {
+        item = sub_find<&SubNode::pq>(N, a, b, t);
+        rows4(N[item], t - N[item].pq, 0);
+    };
+    auto cols_of = [&](int h) { return N[H[h + 1] - 1].pq + N[H[h + 1] - 1].w; };
+    const int t0 = tid >> 2;
+    if (t0 < cols_of(S.sub.w - 1)) load(H[S.sub.w - 1], H[S.sub.w], t0);
+    for (int h = S.sub.w - 1; h >= 0; --h) {
+        const int a = H[h], b = H[h + 1];
+        if (h < S.sub.w - 1) {
+            const int e0 = N[a].ob - S.ext.x, e1 = N[b - 1].ob - S.ext.x + N[b - 1].noff;
+            for (int e = e0 + tid; e < e1; e += BLOCK) {
+                const int c = src[e];
+                if (c >= 0) {
+                    const V u = x[c];
+                    V o;
+                    o.x = -u.x; o.y = -u.y; o.z = -u.z; o.w = 0;
+                    off[e] = o;
+                }
+            }
+            __syncthreads();
+        }
+        const int ncol = cols_of(h);
+        for (int t = t0; t < ncol; t += BLOCK / 4) {
+            if (t != t0) load(a, b, t);
+            const SubNode &s = N[item];
+            const int q = t - s.pq, m = s.w + s.noff;
+            const V *zs = F + s.xs, *os = off + (s.ob - S.ext.x) - s.w;
             T ax = 0, ay = 0, az = 0;
             // row-major [Dinv_s; G_s]: entry (row p, column q) at p * w + q
-            wave_dot<T, V>(P + S.pr + q, S.w, F + S.fbb, on ? min(m, kTile) : 0, ax, ay, az);
-            if (__any(on && m > kTile)) {
-                // rows 64 .. m-1; lanes with m <= 64 keep their own base and add nothing
-                const bool two = on && m > kTile;
-                wave_dot<T, V>(P + S.pr + q + (two ? (long long)kTile * S.w : 0), S.w, F + S.fbb + (two ? kTile : 0),
-                               two ? m - kTile : 0, ax, ay, az);
+            for (int p0 = 0; p0 < m; p0 += 4 * kSubAhead) {
+                if (p0 > 0) rows4(s, q, p0);
+#pragma unroll
+                for (int u0 = 0; u0 < kSubAhead; u0 += 4) {
+                    if (p0 + 4 * u0 < m) {
+#pragma unroll
+                        for (int u = u0; u < u0 + 4; ++u) {
+                            const int p = p0 + part + 4 * u, pc = min(p, m - 1);
+                            const V v = *(pc < s.w ? zs + pc : os + pc);
+                            const T e = p < m ? g[u] : T(0);
+                            ax += e * v.x; ay += e * v.y; az += e * v.z;
+                        }
+                    }
+                }
             }
-            if (on) {
+            ax = quad_sum(ax); ay = quad_sum(ay); az = quad_sum(az);
+            if (part == 0) {
                 V o;
                 o.x = ax; o.y = ay; o.z = az; o.w = 0;
-                F[S.xs + q] = o;
+                x[s.xs + q] = o;
             }
         }
+        if (h > 0 && t0 < cols_of(h - 1)) load(H[h - 1], a, t0);
         __syncthreads();
     }
     // x of the subtree's rows is final and read by nothing outside the subtree: p' += x
-    for (int t = lane; t < rr.y; t += kTile) {
-        const V o = F[t];
-        d4 pv = M.pp[rr.x + t];
+    for (int t = tid; t < nc; t += BLOCK) {
+        const V o = x[t];
+        d4 pv = M.pp[S.row.x + t];
         pv.x += (double)o.x; pv.y += (double)o.y; pv.z += (double)o.z;
-        M.pp[rr.x + t] = pv;
+        M.pp[S.row.x + t] = pv;
     }
 }
 
@@ -2367,23 +2463,32 @@ void launch_bwd(hipStream_t s, LaunchSet L, int blocks, int level, bool fp64) {
         else hipLaunchKernelGGL((k_bwd<float, false>), dim3(blocks), dim3(kTile), 0, s, L, level);
     }
 }
-void launch_sub_fwd(hipStream_t s, LaunchSet L, int blocks, int nodes, int lds_entries, bool fused, bool fp64) {
-    if (blocks <= 0) return;
-    const size_t rec = sizeof(SubNode) * (size_t)nodes;
-    const size_t lds = rec + (fp64 ? sizeof(d4) : sizeof(f4)) * lds_entries;
-    if (fused) {
-        if (fp64) hipLaunchKernelGGL((k_sub_fwd<double, true>), dim3(blocks), dim3(kTile), lds, s, L, nodes);
-        else hipLaunchKernelGGL((k_sub_fwd<float, true>), dim3(blocks), dim3(kTile), lds, s, L, nodes);
-    } else {
-        if (fp64) hipLaunchKernelGGL((k_sub_fwd<double, false>), dim3(blocks), dim3(kTile), lds, s, L, nodes);
-        else hipLaunchKernelGGL((k_sub_fwd<float, false>), dim3(blocks), dim3(kTile), lds, s, L, nodes);
-    }
+static size_t sub_lds(const SubLds &D, int entries, int index_bytes, bool fp64) {
+    return (fp64 ? sizeof(d4) : sizeof(f4)) * (size_t)entries + sizeof(SubNode) * (size_t)D.nodes + (size_t)index_bytes +
+           sizeof(int) * (size_t)(D.heights + 1);
 }
-void launch_sub_bwd(hipStream_t s, LaunchSet L, int blocks, int nodes, int lds_entries, bool fp64) {
+template <typename T, bool Fused>
+static void sub_fwd_of(hipStream_t s, LaunchSet L, int blocks, const SubLds &D, size_t lds) {
+    constexpr int kMany = Fused ? 64 : 128;
+    if (D.block == kSubBlock) hipLaunchKernelGGL((k_sub_fwd<T, Fused, kSubBlock>), dim3(blocks), dim3(kSubBlock), lds, s, L, D);
+    else hipLaunchKernelGGL((k_sub_fwd<T, Fused, kMany>), dim3(blocks), dim3(kMany), lds, s, L, D);
+}
+void launch_sub_fwd(hipStream_t s, LaunchSet L, int blocks, const SubLds &D, bool fused, bool fp64) {
     if (blocks <= 0) return;
-    const size_t rec = sizeof(SubNode) * (size_t)nodes;
-    if (fp64) hipLaunchKernelGGL(k_sub_bwd<double>, dim3(blocks), dim3(kTile), rec + sizeof(d4) * lds_entries, s, L, nodes);
-    else hipLaunchKernelGGL(k_sub_bwd<float>, dim3(blocks), dim3(kTile), rec + sizeof(f4) * lds_entries, s, L, nodes);
+    const size_t lds = sub_lds(D, D.fwd, (int)sizeof(int2) * D.fwd, fp64);
+    if (fp64) fused ? sub_fwd_of<double, true>(s, L, blocks, D, lds) : sub_fwd_of<double, false>(s, L, blocks, D, lds);
+    else fused ? sub_fwd_of<float, true>(s, L, blocks, D, lds) : sub_fwd_of<float, false>(s, L, blocks, D, lds);
+}
+template <typename T>
+static void sub_bwd_of(hipStream_t s, LaunchSet L, int blocks, const SubLds &D, size_t lds) {
+    if (D.block == kSubBlock) hipLaunchKernelGGL((k_sub_bwd<T, kSubBlock>), dim3(blocks), dim3(kSubBlock), lds, s, L, D);
+    else hipLaunchKernelGGL((k_sub_bwd<T, 128>), dim3(blocks), dim3(128), lds, s, L, D);
+}
+void launch_sub_bwd(hipStream_t s, LaunchSet L, int blocks, const SubLds &D, bool fp64) {
+    if (blocks <= 0) return;
+    const size_t lds = sub_lds(D, D.bwd, (int)sizeof(int) * D.off, fp64);
+    if (fp64) sub_bwd_of<double>(s, L, blocks, D, lds);
+    else sub_bwd_of<float>(s, L, blocks, D, lds);
 }
 void launch_energy(hipStream_t s, LaunchSet L, int blocks, bool fp64) {
     if (blocks <= 0) return;

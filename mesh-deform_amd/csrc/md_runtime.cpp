@@ -72,7 +72,7 @@ hipError_t build_plan(Plan &plan, const std::vector<const MeshDev *> &meshes,
     plan.nlevels = 0;
     for (const Factor *f : factors) plan.nlevels = std::max(plan.nlevels, f->nlevels);
     int nl = plan.nlevels;
-    int ntables = 7 + 2 * nl;
+    int ntables = 8 + 2 * nl;
     plan.h_prefix.assign((size_t)ntables * (na + 1), 0);
     plan.h_tbase.assign((size_t)ntables * (na + 1), 0);
     plan.off_fwd.assign(nl, 0);
@@ -94,22 +94,25 @@ hipError_t build_plan(Plan &plan, const std::vector<const MeshDev *> &meshes,
     table(3, plan.off_ident, plan.blk_ident, [&](int k) { return cdiv(meshes[k]->n, kBlock); });
     table(4, plan.off_apply, plan.blk_apply, [&](int k) { return cdiv(meshes[k]->nf, kBlock); });
     table(5, plan.off_sub, plan.blk_sub, [&](int k) { return factors[k]->nsub; });
-    table(6, plan.off_subb, plan.blk_subb,
-          [&](int k) { return factors[k]->nsub + cdiv(meshes[k]->nlrows, kTile); });
-    plan.sub_lds_fwd = 0;
-    plan.sub_lds_bwd = 0;
-    plan.sub_nodes = 0;
+    plan.sub = SubLds{};
     for (const Factor *f : factors) {
-        plan.sub_lds_fwd = std::max(plan.sub_lds_fwd, f->sub_lds_fwd);
-        plan.sub_lds_bwd = std::max(plan.sub_lds_bwd, f->sub_lds_bwd);
-        plan.sub_nodes = std::max(plan.sub_nodes, f->sub_nodes);
+        plan.sub.fwd = std::max(plan.sub.fwd, f->sub_lds_fwd);
+        plan.sub.bwd = std::max(plan.sub.bwd, f->sub_lds_bwd);
+        plan.sub.off = std::max(plan.sub.off, f->sub_off);
+        plan.sub.nodes = std::max(plan.sub.nodes, f->sub_nodes);
+        plan.sub.heights = std::max(plan.sub.heights, f->sub_heights);
     }
+    plan.sub.block = plan.blk_sub <= kSubFew ? kSubBlock : 0;
+    table(6, plan.off_subb, plan.blk_subb,
+          [&](int k) { return factors[k]->nsub + cdiv(meshes[k]->nlrows, sub_rows_bwd(plan.sub)); });
+    table(7, plan.off_subf, plan.blk_subf,
+          [&](int k) { return factors[k]->nsub + cdiv(meshes[k]->nlrows, sub_rows_fwd(plan.sub)); });
     for (int l = 0; l < nl; ++l) {
-        table(7 + 2 * l, plan.off_fwd[l], plan.blk_fwd[l], [&](int k) {
+        table(8 + 2 * l, plan.off_fwd[l], plan.blk_fwd[l], [&](int k) {
             const Factor *f = factors[k];
             return l < f->nlevels ? f->ft_ptr[l + 1] - f->ft_ptr[l] : 0;
         });
-        table(8 + 2 * l, plan.off_bwd[l], plan.blk_bwd[l], [&](int k) {
+        table(9 + 2 * l, plan.off_bwd[l], plan.blk_bwd[l], [&](int k) {
             const Factor *f = factors[k];
             return l < f->nlevels ? f->bt_ptr[l + 1] - f->bt_ptr[l] : 0;
         });
@@ -170,7 +173,9 @@ hipError_t build_plan(Plan &plan, const std::vector<const MeshDev *> &meshes,
 
 // One-mesh plans with at most this many bottom subtrees form the residual inside the subtree
 // forward launch: its registers allow 3 waves per SIMD, and 3 x 1024 SIMDs of a 256-CU device
-// then hold every subtree at once (more subtrees would queue behind the longer waves).
+// then hold every subtree at once, one wave each (more would queue behind the longer waves). Two
+// launches against one: 642 vertices 14 / 10 us, 164k icosphere at budget 128 21 / 17.5 us, at 512 in
+// FP64 41 / 40 us.
 constexpr int kFusedResidualMaxSubtrees = 3072;
 
 void enqueue_iteration(const Plan &plan, hipStream_t stream, hipEvent_t *ev) {
@@ -198,18 +203,16 @@ void enqueue_iteration(const Plan &plan, hipStream_t stream, hipEvent_t *ev) {
         if (!fused) launch_residual(stream, plan.set(plan.off_resid), plan.blk_resid, plan.fp64);
         if (ev && r == 0) hipEventRecord(ev[2], stream);
         if (fused)
-            launch_sub_fwd(stream, plan.set(plan.off_subb), plan.blk_subb, plan.sub_nodes, plan.sub_lds_fwd, true,
-                           plan.fp64);
+            launch_sub_fwd(stream, plan.set(plan.off_subf), plan.blk_subf, plan.sub, true, plan.fp64);
         else
-            launch_sub_fwd(stream, plan.set(plan.off_sub), plan.blk_sub, plan.sub_nodes, plan.sub_lds_fwd, false,
-                           plan.fp64);
+            launch_sub_fwd(stream, plan.set(plan.off_sub), plan.blk_sub, plan.sub, false, plan.fp64);
         for (int l = 0; l < plan.nlevels; ++l)
             launch_fwd(stream, plan.level_set(plan.off_fwd[l], true), plan.blk_fwd[l], l, plan.fp64);
         if (ev && r == 0) hipEventRecord(ev[3], stream);
         for (int l = plan.nlevels - 1; l >= 0; --l)
             launch_bwd(stream, plan.level_set(plan.off_bwd[l], false), plan.blk_bwd[l], l, plan.fp64);
         // subtrees, then p' += x (subtree rows inside their blocks, level rows in extra blocks)
-        launch_sub_bwd(stream, plan.set(plan.off_subb), plan.blk_subb, plan.sub_nodes, plan.sub_lds_bwd, plan.fp64);
+        launch_sub_bwd(stream, plan.set(plan.off_subb), plan.blk_subb, plan.sub, plan.fp64);
         if (ev && r == 0) hipEventRecord(ev[4], stream);
     }
 }
@@ -633,7 +636,7 @@ int upload_layout(md_mesh *m) {
         if (f.level[k] >= 0)
             for (int q = 0; q < f.w[k]; ++q) lrows.push_back(f.c0[k] + q);
     size_t o_lr = A.reserve(sizeof(int) * std::max<size_t>(1, lrows.size()));
-    size_t o_srow = A.reserve(sizeof(int) * std::max<size_t>(2, f.srow.size()));
+    size_t o_srow = A.reserve(sizeof(int) * std::max<size_t>(8, f.srow.size()));
     size_t o_sfi = A.reserve(sizeof(int) * std::max<size_t>(1, f.sfi.size()));
     if (A.allocate() != hipSuccess) {
         set_error("device allocation of " + std::to_string(A.size()) + " bytes (sweep layout) failed");
@@ -651,7 +654,7 @@ int upload_layout(md_mesh *m) {
     d.nsub = f.nsub;
     d.nlrows = (int)lrows.size();
     d.lrows = (const int *)A.at(o_lr);
-    d.srow = (const int2 *)A.at(o_srow);
+    d.srow = (const int4 *)A.at(o_srow);
     d.sfi = (const int *)A.at(o_sfi);
     hipStream_t st = m->ctx->stream;
     auto up = [&](const void *dst, const void *src, size_t bytes) -> hipError_t {

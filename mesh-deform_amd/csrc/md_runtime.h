@@ -51,10 +51,10 @@ struct Plan {
     int nlevels = 0;
     int blk_face = 0, blk_slice = 0, blk_resid = 0, blk_ident = 0, blk_apply = 0, blk_sub = 0;
     int blk_subb = 0, off_subb = 0;    // k_sub_bwd: subtrees, then the p' update of level rows
+    int blk_subf = 0, off_subf = 0;    // k_sub_fwd with the residual: subtrees, then the level rows
     std::vector<int> blk_fwd, blk_bwd;
     int off_face = 0, off_slice = 0, off_resid = 0, off_ident = 0, off_apply = 0, off_sub = 0;
-    int sub_lds_fwd = 0, sub_lds_bwd = 0;  // LDS vector entries of the largest bottom subtree
-    int sub_nodes = 0;                 // supernode records of the largest bottom subtree
+    SubLds sub{};                      // bottom subtrees: workgroup size, LDS of the largest
     std::vector<int> off_fwd, off_bwd;
     MeshDev *d_meshes = nullptr;       // views into d_tables: the mesh records,
     int *d_prefix = nullptr;           //   the prefix tables,
