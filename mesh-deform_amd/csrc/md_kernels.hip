@@ -1129,7 +1129,6 @@ __global__ __launch_bounds__(BLOCK) void k_sub_bwd(LaunchSet L, SubLds D) {
     }
 }
 
-// p'_i += x_i for every free vertex, x_i the sum of its supernode's partials.
 // ---- Jacobi-preconditioned CG on the correction system (alternative to the sweeps) -------
 //
 // Solves A d = r for the three coordinates at once (three independent CG recurrences, one
@@ -1142,58 +1141,78 @@ template <typename T> __device__ __forceinline__ const T *wts(const MD_G MeshDev
 template <> __device__ __forceinline__ const float *wts<float>(const MD_G MeshDev &M) { return M.w32; }
 template <> __device__ __forceinline__ const double *wts<double>(const MD_G MeshDev &M) { return M.w64; }
 
-// Two block sums at once (six values in one tree): a into pa[blk], b into pb[blk].
-template <typename T, typename V>
-__device__ __forceinline__ void block_partial2(const T (&a)[3], const T (&b)[3], MD_G V *pa, MD_G V *pb, int blk,
-                                               T (*red)[kBlock]) {
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        red[q][threadIdx.x] = a[q];
-        red[3 + q][threadIdx.x] = b[q];
+// Lane moves inside a row of 16 lanes (DPP control CTRL).
+template <int CTRL> __device__ __forceinline__ float dpp_move(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+template <int CTRL> __device__ __forceinline__ double dpp_move(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)u, CTRL, 0xF, 0xF, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), CTRL, 0xF, 0xF, true);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+// v + the value of the other row of each pair (Half: of the other half of the wavefront).
+template <bool Half> __device__ __forceinline__ void rows_swap(unsigned u, unsigned (&o)[2]) {
+    if constexpr (Half) {
+        const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        o[0] = a[0]; o[1] = a[1];
+    } else {
+        const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        o[0] = a[0]; o[1] = a[1];
     }
+}
+template <bool Half> __device__ __forceinline__ float rows_sum(float v) {
+    unsigned a[2];
+    rows_swap<Half>(__builtin_bit_cast(unsigned, v), a);
+    return __builtin_bit_cast(float, a[0]) + __builtin_bit_cast(float, a[1]);
+}
+template <bool Half> __device__ __forceinline__ double rows_sum(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    unsigned lo[2], hi[2];
+    rows_swap<Half>((unsigned)u, lo);
+    rows_swap<Half>((unsigned)(u >> 32), hi);
+    return __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]) +
+           __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
+}
+// Sum over the wavefront, in every lane (quads, half rows, rows, row pairs, halves).
+template <typename T> __device__ __forceinline__ T wave_sum(T v) {
+    v += dpp_move<0xB1>(v);
+    v += dpp_move<0x4E>(v);
+    v += dpp_move<0x141>(v);
+    v += dpp_move<0x140>(v);
+    v = rows_sum<false>(v);
+    return rows_sum<true>(v);
+}
+
+// Six block sums, in every thread: a wavefront's by lane moves, the wavefronts' through LDS
+// (two LDS trees of eight barriers each took 4 of a CG step's 11 us). red is written once
+// per kernel.
+template <typename T> __device__ __forceinline__ void block_sum6(T (&v)[6], T (*red)[6]) {
+    constexpr int kWaves = kBlock / 64;
+#pragma unroll
+    for (int q = 0; q < 6; ++q) v[q] = wave_sum(v[q]);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int q = 0; q < 6; ++q) red[threadIdx.x >> 6][q] = v[q];
     __syncthreads();
-    for (int o = kBlock / 2; o > 0; o >>= 1) {
-        if (threadIdx.x < o) {
 #pragma unroll
-            for (int q = 0; q < 6; ++q) red[q][threadIdx.x] += red[q][threadIdx.x + o];
-        }
-        __syncthreads();
+    for (int q = 0; q < 6; ++q) {
+        v[q] = red[0][q];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) v[q] += red[w][q];
     }
+}
+// A block's sums of (r, u) and (w, u) into pa[blk] and pb[blk].
+template <typename T, typename V>
+__device__ __forceinline__ void block_partial2(T (&v)[6], MD_G V *pa, MD_G V *pb, int blk, T (*red)[6]) {
+    block_sum6(v, red);
     if (threadIdx.x == 0) {
         V va, vb;
-        va.x = red[0][0]; va.y = red[1][0]; va.z = red[2][0]; va.w = 0;
-        vb.x = red[3][0]; vb.y = red[4][0]; vb.z = red[5][0]; vb.w = 0;
+        va.x = v[0]; va.y = v[1]; va.z = v[2]; va.w = 0;
+        vb.x = v[3]; vb.y = v[4]; vb.z = v[5]; vb.w = 0;
         pa[blk] = va;
         pb[blk] = vb;
     }
-}
-
-// Two partial arrays summed at once (fixed order); the results broadcast through LDS.
-template <typename T, typename V>
-__device__ __forceinline__ void reduce_partials2(const MD_G V *pa, const MD_G V *pb, int nb, T (&oa)[3], T (&ob)[3],
-                                                 T (*red)[kBlock]) {
-    T a[6] = {0, 0, 0, 0, 0, 0};
-    for (int k = threadIdx.x; k < nb; k += kBlock) {
-        const V x = pa[k], y = pb[k];
-        a[0] += x.x; a[1] += x.y; a[2] += x.z;
-        a[3] += y.x; a[4] += y.y; a[5] += y.z;
-    }
-#pragma unroll
-    for (int q = 0; q < 6; ++q) red[q][threadIdx.x] = a[q];
-    __syncthreads();
-    for (int o = kBlock / 2; o > 0; o >>= 1) {
-        if (threadIdx.x < o) {
-#pragma unroll
-            for (int q = 0; q < 6; ++q) red[q][threadIdx.x] += red[q][threadIdx.x + o];
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        oa[q] = red[q][0];
-        ob[q] = red[3 + q][0];
-    }
-    __syncthreads();
 }
 
 // L_ii = sum of every neighbour weight (arap.h:332), once per factorisation.
@@ -1221,23 +1240,15 @@ __global__ __launch_bounds__(kBlock) void k_pcg_diag(LaunchSet L) {
 // its r, w and s of the previous step, which live in the other buffer of each pair (parity i),
 // so no lane reads what another writes. Per coordinate, a solve whose gamma fell below
 // tol^2 gamma_0 keeps alpha = 0 (its x and r stay).
-template <typename T, typename V> struct CgVecs {
-    MD_G V *r[2], *w[2], *s[2], *x, *p;
+template <typename V> struct CgVecs {
+    MD_G V *r[2], *w[2], *s[2], *x, *p;  // [0]: the parity a step reads, [1]: the one it writes
 };
-template <typename T, typename V>
-__device__ __forceinline__ CgVecs<T, V> cg_vecs(const MD_G MeshDev &M) {
-    CgVecs<T, V> c;
-    MD_G V *v = reinterpret_cast<MD_G V *>(M.cg_v);
-    const long long nf = M.nf;
-    c.r[0] = reinterpret_cast<MD_G V *>(M.r);
-    c.r[1] = v;
-    c.w[0] = v + nf;
-    c.w[1] = v + 2 * nf;
-    c.s[0] = v + 3 * nf;
-    c.s[1] = v + 4 * nf;
-    c.x = reinterpret_cast<MD_G V *>(M.cg_x);
-    c.p = reinterpret_cast<MD_G V *>(M.cg_p);
-    return c;
+template <typename V>
+__device__ __forceinline__ CgVecs<V> cg_vecs(const MD_G MeshDev &M, int parity) {
+    MD_G V *r = reinterpret_cast<MD_G V *>(M.r), *v = reinterpret_cast<MD_G V *>(M.cg_v);
+    const long long nf = M.nf, o = parity ? nf : 0;
+    return {{parity ? v : r, parity ? r : v}, {v + nf + o, v + 2 * nf - o}, {v + 3 * nf + o, v + 4 * nf - o},
+            reinterpret_cast<MD_G V *>(M.cg_x), reinterpret_cast<MD_G V *>(M.cg_p)};
 }
 
 // x = p = s_0 = 0, u = M^-1 r, w_0 = A u, partials of (r, u) and (w, u) (parity 0). One lane
@@ -1245,15 +1256,15 @@ __device__ __forceinline__ CgVecs<T, V> cg_vecs(const MD_G MeshDev &M) {
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_pcg_init(LaunchSet L) {
     using V = typename V4T<T>::type;
-    __shared__ T red[6][kBlock];
+    __shared__ T red[kBlock / 64][6];
     const int k = find_mesh(L, blockIdx.x);
     const MD_G MeshDev &M = L.meshes[k];
     const int blk = blockIdx.x - L.prefix[k];
     const int slice = blk * kSlicesPerBlock + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int iv = slice * kSlice + lane;
-    const CgVecs<T, V> c = cg_vecs<T, V>(M);
+    const CgVecs<V> c = cg_vecs<V>(M, 0);
     const MD_G T *D = reinterpret_cast<const MD_G T *>(M.diag);
-    T gam[3] = {0, 0, 0}, del[3] = {0, 0, 0};
+    T dots[6] = {0, 0, 0, 0, 0, 0};  // (r, u), (w, u)
     if (slice < M.nslices_free && iv < M.nf) {
         const T *W = wts<T>(M);
         const int s0 = M.slice_ptr[slice], wd = M.slice_ptr[slice + 1] - s0;
@@ -1278,34 +1289,79 @@ __global__ __launch_bounds__(kBlock) void k_pcg_init(LaunchSet L) {
         c.s[0][iv] = z;
         c.x[iv] = z;
         c.p[iv] = z;
-        gam[0] = r.x * ux; gam[1] = r.y * uy; gam[2] = r.z * uz;
-        del[0] = yx * ux; del[1] = yy * uy; del[2] = yz * uz;
+        dots[0] = r.x * ux; dots[1] = r.y * uy; dots[2] = r.z * uz;
+        dots[3] = yx * ux; dots[4] = yy * uy; dots[5] = yz * uz;
     }
     MD_G V *part = reinterpret_cast<MD_G V *>(M.cg_part);
     const int nb = M.nblk_free;
-    block_partial2<T, V>(gam, del, part, part + nb, blk, red);
+    block_partial2<T, V>(dots, part, part + nb, blk, red);
 }
 
 // Step i (parity c = i & 1): reads r, w, s and the partials of parity c, writes those of 1 - c.
+// Bound by the chain of one launch (10k icosphere: 34 workgroups): everything a lane reads,
+// kPcgAhead slots of its one-ring included, is on its way before the partials are summed.
+// A step of the 10k icosphere in FP32 takes 7.8 us (11.4 with LDS trees and the loads behind them), of
+// the 164k one 16.4 (21.3) in FP32 and 27 (32) in FP64; with 8 slots ahead in FP64 the registers leave one
+// wavefront per SIMD and that took 33.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_pcg_step(LaunchSet L, int step) {
     using V = typename V4T<T>::type;
-    __shared__ T red[6][kBlock];
+    constexpr int kPcgAhead = sizeof(T) == 4 ? 8 : 4;
+    __shared__ T red[2][kBlock / 64][6];
     const int k = find_mesh(L, blockIdx.x);
     const MD_G MeshDev &M = L.meshes[k];
     const int blk = blockIdx.x - L.prefix[k];
-    const int slice = blk * kSlicesPerBlock + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int slice = __builtin_amdgcn_readfirstlane(blk * kSlicesPerBlock + (int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int iv = slice * kSlice + lane;
     const int c = step & 1, n = 1 - c;
-    const CgVecs<T, V> v = cg_vecs<T, V>(M);
+    const CgVecs<V> v = cg_vecs<V>(M, c);
     const MD_G T *D = reinterpret_cast<const MD_G T *>(M.diag);
     MD_G V *part = reinterpret_cast<MD_G V *>(M.cg_part);
     const int nb = M.nblk_free;
-    T ga[3], de[3];
-    reduce_partials2<T, V>(part + 2 * c * nb, part + (2 * c + 1) * nb, nb, ga, de, red);
     MD_G V *scal = part + 4 * nb;  // (gamma, alpha) of each parity, then the first gamma
-    T al[3], be[3];
     const V gp = scal[2 * c], ap = scal[2 * c + 1], gz = scal[4];
+    T sum[6] = {0, 0, 0, 0, 0, 0};
+    for (int b = threadIdx.x; b < nb; b += kBlock) {
+        const V x = part[2 * c * nb + b], y = part[(2 * c + 1) * nb + b];
+        sum[0] += x.x; sum[1] += x.y; sum[2] += x.z;
+        sum[3] += y.x; sum[4] += y.y; sum[5] += y.z;
+    }
+    const bool live = slice < M.nslices_free && iv < M.nf;
+    const T *W = wts<T>(M);
+    const bool inside = slice < M.nslices_free;
+    const int s0 = inside ? M.slice_ptr[slice] : 0, wd = inside ? M.slice_ptr[slice + 1] - s0 : 0;
+    V r = {}, w = {}, so = {}, p = {}, x = {}, nr[kPcgAhead], nw[kPcgAhead], ns[kPcgAhead];
+    T di = T(1), wq[kPcgAhead], nd[kPcgAhead];
+#pragma unroll
+    for (int q = 0; q < kPcgAhead; ++q) {
+        nr[q] = nw[q] = ns[q] = V{};
+        wq[q] = T(0);
+        nd[q] = T(1);
+    }
+    if (live) {
+        r = v.r[0][iv]; w = v.w[0][iv]; so = v.s[0][iv];
+        p = v.p[iv]; x = v.x[iv];
+        di = D[iv];
+        if (wd > 0) {
+            int nj[kPcgAhead];
+#pragma unroll
+            for (int q = 0; q < kPcgAhead; ++q) {
+                const long long g = (long long)(s0 + min(q, wd - 1)) * kSlice + lane;
+                nj[q] = M.sell_col[g];
+                wq[q] = W[g];
+            }
+#pragma unroll
+            for (int q = 0; q < kPcgAhead; ++q) {
+                // padding, constrained neighbours and slots past the slice's count as zero
+                if (q >= wd || nj[q] >= M.nf || nj[q] == iv) { nj[q] = iv; wq[q] = T(0); }
+                nr[q] = v.r[0][nj[q]]; nw[q] = v.w[0][nj[q]]; ns[q] = v.s[0][nj[q]];
+                nd[q] = D[nj[q]];
+            }
+        }
+    }
+    block_sum6(sum, red[0]);
+    const T ga[3] = {sum[0], sum[1], sum[2]}, de[3] = {sum[3], sum[4], sum[5]};
+    T al[3], be[3];
     const T gprev[3] = {gp.x, gp.y, gp.z}, aprev[3] = {ap.x, ap.y, ap.z};
     const T g0[3] = {step == 0 ? ga[0] : gz.x, step == 0 ? ga[1] : gz.y, step == 0 ? ga[2] : gz.z};
     for (int q = 0; q < 3; ++q) {
@@ -1330,13 +1386,9 @@ __global__ __launch_bounds__(kBlock) void k_pcg_step(LaunchSet L, int step) {
         scal[2 * n + 1] = a;
         if (step == 0) scal[4] = g;  // the first gamma, for the stopping test
     }
-    T gam[3] = {0, 0, 0}, del[3] = {0, 0, 0};
-    if (slice < M.nslices_free && iv < M.nf) {
-        const T *W = wts<T>(M);
-        const int s0 = M.slice_ptr[slice], wd = M.slice_ptr[slice + 1] - s0;
-        const T di = D[iv], rdi = T(1) / di;
-        const V r = v.r[c][iv], w = v.w[c][iv], so = v.s[c][iv];
-        V p = v.p[iv], x = v.x[iv];
+    T dots[6] = {0, 0, 0, 0, 0, 0};
+    if (live) {
+        const T rdi = T(1) / di;
         // p = u + beta p, s = w + beta s, x += alpha p, r -= alpha s
         p.x = r.x * rdi + be[0] * p.x; p.y = r.y * rdi + be[1] * p.y; p.z = r.z * rdi + be[2] * p.z;
         V sn;
@@ -1346,29 +1398,31 @@ __global__ __launch_bounds__(kBlock) void k_pcg_step(LaunchSet L, int step) {
         rn.x = r.x - al[0] * sn.x; rn.y = r.y - al[1] * sn.y; rn.z = r.z - al[2] * sn.z; rn.w = 0;
         v.p[iv] = p;
         v.x[iv] = x;
-        v.s[n][iv] = sn;
-        v.r[n][iv] = rn;
+        v.s[1][iv] = sn;
+        v.r[1][iv] = rn;
         // w = A u with u = M^-1 r of the new r; a neighbour's new u from its previous r, w, s
         const T ux = rn.x * rdi, uy = rn.y * rdi, uz = rn.z * rdi;
         T yx = di * ux, yy = di * uy, yz = di * uz;
-        for (int q = 0; q < wd; ++q) {
+        auto slot = [&](T wj, const V &rj, const V &uj, const V &sj) {
+            yx -= wj * (rj.x - al[0] * (uj.x + be[0] * sj.x));
+            yy -= wj * (rj.y - al[1] * (uj.y + be[1] * sj.y));
+            yz -= wj * (rj.z - al[2] * (uj.z + be[2] * sj.z));
+        };
+#pragma unroll
+        for (int q = 0; q < kPcgAhead; ++q)
+            if (q < wd) slot(wq[q] / nd[q], nr[q], nw[q], ns[q]);
+        for (int q = kPcgAhead; q < wd; ++q) {
             const long long g = (long long)(s0 + q) * kSlice + lane;
             const int j = M.sell_col[g];
-            if (j != iv && j < M.nf) {
-                const V rj = v.r[c][j], wj = v.w[c][j], sj = v.s[c][j];
-                const T wq = W[g] / D[j];
-                yx -= wq * (rj.x - al[0] * (wj.x + be[0] * sj.x));
-                yy -= wq * (rj.y - al[1] * (wj.y + be[1] * sj.y));
-                yz -= wq * (rj.z - al[2] * (wj.z + be[2] * sj.z));
-            }
+            if (j != iv && j < M.nf) slot(W[g] / D[j], v.r[0][j], v.w[0][j], v.s[0][j]);
         }
         V wn;
         wn.x = yx; wn.y = yy; wn.z = yz; wn.w = 0;
-        v.w[n][iv] = wn;
-        gam[0] = rn.x * ux; gam[1] = rn.y * uy; gam[2] = rn.z * uz;
-        del[0] = yx * ux; del[1] = yy * uy; del[2] = yz * uz;
+        v.w[1][iv] = wn;
+        dots[0] = rn.x * ux; dots[1] = rn.y * uy; dots[2] = rn.z * uz;
+        dots[3] = yx * ux; dots[4] = yy * uy; dots[5] = yz * uz;
     }
-    block_partial2<T, V>(gam, del, part + 2 * n * nb, part + (2 * n + 1) * nb, blk, red);
+    block_partial2<T, V>(dots, part + 2 * n * nb, part + (2 * n + 1) * nb, blk, red[1]);
 }
 
 // p' += d for the free vertices.
