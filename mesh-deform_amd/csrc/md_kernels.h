@@ -122,6 +122,7 @@ struct FacArgs {
     MD_G int *flag;                 // 1: a pivot block is not positive definite; 2: structure
     MD_G void *pc, *pr;             // the sweeps' panels (float or double), written in the solve
     int solve64;                    //   precision (1: double)
+    unsigned long long *stamp;      // clock at the start (may be null)
 };
 
 // A set of meshes processed by one launch. Block b belongs to mesh k where
@@ -162,7 +163,6 @@ inline int sub_rows_bwd(const SubLds &D) { return D.block == kSubBlock ? kSubBlo
 void launch_sub_fwd(hipStream_t s, LaunchSet L, int blocks, const SubLds &D, bool fused, bool fp64);
 void launch_sub_bwd(hipStream_t s, LaunchSet L, int blocks, const SubLds &D, bool fp64);
 void launch_energy(hipStream_t s, LaunchSet L, int blocks, bool fp64);
-void launch_identity_quat(hipStream_t s, LaunchSet L, int blocks, bool fp64);
 // A target of a served request: the device address of its vertex's p' entry and the position.
 struct alignas(16) TargetEntry {
     unsigned long long addr;
@@ -170,7 +170,8 @@ struct alignas(16) TargetEntry {
 };
 // *entry.addr = (x, y, z) for k entries (targets of several meshes in one launch).
 void launch_scatter_entries(hipStream_t s, const TargetEntry *e, int k);
-void launch_normals(hipStream_t s, LaunchSet Lf, int blocks_face, LaunchSet Ls, int blocks_slice, double *fn, d4 *out);
+void launch_normals(hipStream_t s, LaunchSet Lf, int blocks_face, LaunchSet Ls, int blocks_slice, double *fn, d4 *out,
+                    double *packed = nullptr, const int *orig = nullptr);
 void launch_pcg_diag(hipStream_t s, LaunchSet L, int blocks, bool fp64);
 // Jacobi-PCG in the Chronopoulos-Gear form: one launch per CG iteration (step i).
 void launch_pcg_init(hipStream_t s, LaunchSet L, int blocks, bool fp64);
@@ -215,12 +216,23 @@ void launch_fac_small(hipStream_t s, const FacArgs &A, int h0, int count, int mm
 // they are all of it, or at least 512 and the larger part (the 164k icosphere's second and third
 // heights: 116 and 114 us split, 140 and 152 together; a smaller share only adds a launch).
 inline bool fac_split_small(int small, int all) { return small == all || (small >= 512 && 2 * small >= all); }
-// Internal-order vectors (positions, normals) to packed xyz in original order (perm: original
-// id per internal id), and packed xyz to internal order (p and/or pp; pp takes the targets tgt,
-// internal order, for the constrained ids [nf, n)).
-void launch_pack_xyz(hipStream_t s, const d4 *v, const int *perm, int n, double *dst);
-void launch_unpack_xyz(hipStream_t s, const double *xyz, const int *perm, int n, int nf, const double *tgt, d4 *p,
-                       d4 *pp);
+// Internal-order vectors (positions, normals) to packed xyz in original order (internal: internal
+// id per original id); stamp: clock at the start (may be null).
+void launch_pack_xyz(hipStream_t s, const d4 *v, const int *internal, int n, double *dst, unsigned long long *stamp);
+// Packed xyz to internal order (p and/or pp; pp takes the targets tgt, internal order, for the
+// constrained ids [nf, n), and comes with identity rotations in quat).
+struct UnpackArgs {
+    const double *xyz;
+    const int *internal;
+    int n, nf;
+    const double *tgt;
+    d4 *p, *pp;
+    void *quat;
+    unsigned long long *clear, *stamp;
+};
+void launch_unpack_xyz(hipStream_t s, const UnpackArgs &a, bool fp64);
+// Clock and *flag to pinned host memory.
+void launch_publish(hipStream_t s, unsigned long long *stamp, const int *flag, int *out);
 
 // Per-GPU device workspace of the non-allocating entry points (a static device array of
 // kScratchBytes): its address on the current device, from hipGetSymbolAddress. Call once per

@@ -403,18 +403,6 @@ __global__ __launch_bounds__(kBlock) void k_local(LaunchSet L) {
     reinterpret_cast<V *>(M.quat)[iv] = out;
 }
 
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_identity_quat(LaunchSet L) {
-    using V = typename V4T<T>::type;
-    int k = find_mesh(L, blockIdx.x);
-    const MD_G MeshDev &M = L.meshes[k];
-    int iv = (blockIdx.x - L.prefix[k]) * kBlock + threadIdx.x;
-    if (iv >= M.n) return;
-    V out;
-    out.x = 0; out.y = 0; out.z = 0; out.w = 1;
-    reinterpret_cast<V *>(M.quat)[iv] = out;
-}
-
 // ---- right-hand side and residual (arap.h:393-414) --------------------------------------
 
 // One lane per free vertex i:
@@ -1458,8 +1446,10 @@ __global__ __launch_bounds__(kBlock) void k_face_normals(LaunchSet L, double *fn
 
 // Per vertex: every incident face appears on exactly two of its one-ring slots (the two face
 // edges at the vertex), so half the sum over the slots' face lists is the sum of incident
-// face normals; normalised (zero stays zero). Output in internal order.
-__global__ __launch_bounds__(kBlock) void k_vertex_normals(LaunchSet L, const double *fn, d4 *out) {
+// face normals; normalised (zero stays zero). Output in internal order, or packed in original order
+// (orig: original id of each internal id).
+__global__ __launch_bounds__(kBlock) void k_vertex_normals(LaunchSet L, const double *fn, d4 *out, double *packed,
+                                                           const int *orig) {
     int k = find_mesh(L, blockIdx.x);
     const MD_G MeshDev &M = L.meshes[k];
     int slice = (blockIdx.x - L.prefix[k]) * kSlicesPerBlock + (threadIdx.x >> 6);
@@ -1478,19 +1468,27 @@ __global__ __launch_bounds__(kBlock) void k_vertex_normals(LaunchSet L, const do
     }
     double nrm = sqrt(x * x + y * y + z * z);
     double inv = nrm > 0.0 ? 1.0 / nrm : 0.0;
+    if (packed) {
+        double *o = packed + 3 * (size_t)orig[iv];
+        o[0] = x * inv; o[1] = y * inv; o[2] = z * inv;
+        return;
+    }
     d4 o;
     o.x = x * inv; o.y = y * inv; o.z = z * inv; o.w = 0.0;
     out[iv] = o;
 }
 
 // Internal-order vectors (positions or normals) to the caller's packed xyz in original vertex
-// order: dst[3 perm[iv] + c] = v[iv].c (perm = original id of each internal id, a bijection).
-__global__ __launch_bounds__(kBlock) void k_pack_xyz(const d4 *nrm, const int *perm, int n, double *dst) {
-    int iv = blockIdx.x * kBlock + threadIdx.x;
-    if (iv >= n) return;
-    d4 v = nrm[iv];
-    double *o = dst + 3 * (size_t)perm[iv];
-    o[0] = v.x; o[1] = v.y; o[2] = v.z;
+// order: dst[3 v + c] = x[internal[v]].c. One thread per original vertex: dst may be pinned host memory,
+// whose writes then leave in order.
+__global__ __launch_bounds__(kBlock) void k_pack_xyz(const d4 *x, const int *internal, int n, double *dst,
+                                                     unsigned long long *stamp) {
+    const int v = blockIdx.x * kBlock + threadIdx.x;
+    if (v == 0 && stamp) *stamp = wall_clock64();
+    if (v >= n) return;
+    const d4 p = x[internal[v]];
+    double *o = dst + 3 * (size_t)v;
+    o[0] = p.x; o[1] = p.y; o[2] = p.z;
 }
 
 // Device workspace of the entry points that allocate nothing (md_mesh_normals_noalloc): one
@@ -1542,23 +1540,37 @@ __global__ __launch_bounds__(kBlock) void k_energy(LaunchSet L) {
 }
 
 // p'[iv[k]] = xyz[k] for k targets (internal ids), used to move handles without a re-setup.
-// The caller's packed xyz (original order) into internal order: p[iv] = xyz[perm[iv]] (p may
-// be null), and pp[iv] the same for free vertices, the constrained ones (iv >= nf) taking their
-// targets tgt[iv - nf] (internal order) instead (pp may be null).
-__global__ __launch_bounds__(kBlock) void k_unpack_xyz(const double *xyz, const int *perm, int n, int nf,
-                                                       const double *tgt, d4 *p, d4 *pp) {
-    const int iv = blockIdx.x * kBlock + threadIdx.x;
-    if (iv >= n) return;
-    const double *s = xyz + 3 * (size_t)perm[iv];
-    const d4 v{s[0], s[1], s[2], 0.0};
-    if (p) p[iv] = v;
-    if (pp) {
-        if (iv < nf) pp[iv] = v;
-        else {
-            const double *t = tgt + 3 * (size_t)(iv - nf);
-            pp[iv] = d4{t[0], t[1], t[2], 0.0};
+// The caller's packed xyz (original order, read in order: it may be pinned host memory) into
+// internal order: p[iv] (may be null), and pp[iv] (may be null) the same for free vertices, the constrained
+// ones (iv >= nf) taking their targets tgt[iv - nf] instead; with pp, identity rotations (arap.h:246-249).
+// Thread 0 clears `clear` (two words) and writes the clock to `stamp` (each may be null).
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_unpack_xyz(UnpackArgs a) {
+    using V = typename V4T<T>::type;
+    const int v = blockIdx.x * kBlock + threadIdx.x;
+    if (v == 0 && a.clear) a.clear[0] = a.clear[1] = 0;
+    if (v == 0 && a.stamp) *a.stamp = wall_clock64();
+    if (v >= a.n) return;
+    const int iv = a.internal[v];
+    const double *s = a.xyz + 3 * (size_t)v;
+    d4 x{s[0], s[1], s[2], 0.0};
+    if (a.p) a.p[iv] = x;
+    if (a.pp) {
+        if (iv >= a.nf) {
+            const double *t = a.tgt + 3 * (size_t)(iv - a.nf);
+            x = d4{t[0], t[1], t[2], 0.0};
         }
+        a.pp[iv] = x;
+        V q;
+        q.x = 0; q.y = 0; q.z = 0; q.w = 1;
+        reinterpret_cast<V *>(a.quat)[iv] = q;
     }
+}
+
+// The clock and the factorization's flag (if any) to the host, between two phases' launches.
+__global__ void k_publish(unsigned long long *stamp, const int *flag, int *out) {
+    *stamp = wall_clock64();
+    if (flag) *out = *flag;
 }
 
 // Targets of several meshes: entry t writes its position into the p' entry at its address.
@@ -1596,6 +1608,7 @@ __device__ __forceinline__ FrontBuf front_buf(const FacArgs &A, const FacDev &S,
 // L_jj = sum of the weights of every neighbour of j, in slot order, and their maximum.
 __global__ __launch_bounds__(kBlock) void k_fac_diag(FacArgs A) {
     const int j = blockIdx.x * kBlock + threadIdx.x;
+    if (j == 0 && A.stamp) *A.stamp = wall_clock64();
     if (j >= A.nf) return;
     const int sl = j / kSlice, l = j % kSlice;
     double acc = 0.0;
@@ -2452,9 +2465,11 @@ void launch_pcg_step(hipStream_t s, LaunchSet L, int blocks, int step, bool fp64
 }
 void launch_pcg_apply(hipStream_t s, LaunchSet L, int blocks, bool fp64) { MD_LAUNCH_T(k_pcg_apply, blocks, s, L); }
 
-void launch_normals(hipStream_t s, LaunchSet Lf, int blocks_face, LaunchSet Ls, int blocks_slice, double *fn, d4 *out) {
+void launch_normals(hipStream_t s, LaunchSet Lf, int blocks_face, LaunchSet Ls, int blocks_slice, double *fn, d4 *out,
+                    double *packed, const int *orig) {
     if (blocks_face > 0) hipLaunchKernelGGL(k_face_normals, dim3(blocks_face), dim3(kBlock), 0, s, Lf, fn);
-    if (blocks_slice > 0) hipLaunchKernelGGL(k_vertex_normals, dim3(blocks_slice), dim3(kBlock), 0, s, Ls, (const double *)fn, out);
+    if (blocks_slice > 0)
+        hipLaunchKernelGGL(k_vertex_normals, dim3(blocks_slice), dim3(kBlock), 0, s, Ls, (const double *)fn, out, packed, orig);
 }
 
 hipError_t scratch_address(void **ptr) {
@@ -2462,14 +2477,16 @@ hipError_t scratch_address(void **ptr) {
     return hipGetSymbolAddress(ptr, HIP_SYMBOL(scratch));
 }
 
-void launch_pack_xyz(hipStream_t s, const d4 *v, const int *perm, int n, double *dst) {
-    if (n > 0) hipLaunchKernelGGL(k_pack_xyz, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, v, perm, n, dst);
+void launch_pack_xyz(hipStream_t s, const d4 *v, const int *internal, int n, double *dst, unsigned long long *stamp) {
+    if (n > 0) hipLaunchKernelGGL(k_pack_xyz, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, v, internal, n, dst, stamp);
 }
-void launch_unpack_xyz(hipStream_t s, const double *xyz, const int *perm, int n, int nf, const double *tgt, d4 *p,
-                       d4 *pp) {
-    if (n > 0)
-        hipLaunchKernelGGL(k_unpack_xyz, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, xyz, perm, n, nf, tgt, p,
-                           pp);
+void launch_unpack_xyz(hipStream_t s, const UnpackArgs &a, bool fp64) {
+    if (a.n <= 0) return;
+    if (fp64) hipLaunchKernelGGL(k_unpack_xyz<double>, dim3((a.n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, a);
+    else hipLaunchKernelGGL(k_unpack_xyz<float>, dim3((a.n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, a);
+}
+void launch_publish(hipStream_t s, unsigned long long *stamp, const int *flag, int *out) {
+    hipLaunchKernelGGL(k_publish, dim3(1), dim3(1), 0, s, stamp, flag, out);
 }
 
 void launch_scatter_entries(hipStream_t s, const TargetEntry *e, int k) {
@@ -2486,11 +2503,6 @@ void launch_local(hipStream_t s, LaunchSet L, int blocks, bool fp64) {
     if (blocks <= 0) return;
     if (fp64) hipLaunchKernelGGL(k_local<double>, dim3(blocks), dim3(kBlock), 0, s, L);
     else hipLaunchKernelGGL(k_local<float>, dim3(blocks), dim3(kBlock), 0, s, L);
-}
-void launch_identity_quat(hipStream_t s, LaunchSet L, int blocks, bool fp64) {
-    if (blocks <= 0) return;
-    if (fp64) hipLaunchKernelGGL(k_identity_quat<double>, dim3(blocks), dim3(kBlock), 0, s, L);
-    else hipLaunchKernelGGL(k_identity_quat<float>, dim3(blocks), dim3(kBlock), 0, s, L);
 }
 void launch_residual(hipStream_t s, LaunchSet L, int blocks, bool fp64) {
     if (blocks <= 0) return;

@@ -28,7 +28,34 @@ void ctx_release(md_ctx *c) {
     hipSetDevice(c->device);
     hipStreamSynchronize(c->stream);
     hipStreamDestroy(c->stream);
+    for (char *p : c->slots) hipHostFree(p);
     delete c;
+}
+
+CallSlot::CallSlot(md_ctx *c) : ctx_(c) {
+    {
+        std::lock_guard<std::mutex> g(c->slot_mu);
+        if (!c->slots.empty()) {
+            base_ = c->slots.back();
+            c->slots.pop_back();
+        }
+    }
+    void *h = nullptr;
+    if (!base_ && hipHostMalloc(&h, kHeadBytes + kStageBytes, hipHostMallocDefault) == hipSuccess)
+        base_ = static_cast<char *>(h);
+    if (base_) *head() = Head{};
+}
+CallSlot::~CallSlot() {
+    if (!base_) return;
+    if (queued) hipStreamSynchronize(ctx_->stream);
+    {
+        std::lock_guard<std::mutex> g(ctx_->slot_mu);
+        if (ctx_->slots.size() < kSlotsKept) {
+            ctx_->slots.push_back(base_);
+            return;
+        }
+    }
+    hipHostFree(base_);
 }
 
 #define MD_HIP(call)                                                                    \
@@ -55,8 +82,7 @@ Plan::~Plan() {
 
 void Plan::drop_graph() {
     if (graph) hipGraphExecDestroy(graph);
-    if (graph_multi) hipGraphExecDestroy(graph_multi);
-    graph = graph_multi = nullptr;
+    graph = nullptr;
 }
 
 static int cdiv(int a, int b) { return (a + b - 1) / b; }
@@ -72,7 +98,7 @@ hipError_t build_plan(Plan &plan, const std::vector<const MeshDev *> &meshes,
     plan.nlevels = 0;
     for (const Factor *f : factors) plan.nlevels = std::max(plan.nlevels, f->nlevels);
     int nl = plan.nlevels;
-    int ntables = 8 + 2 * nl;
+    int ntables = 7 + 2 * nl;
     plan.h_prefix.assign((size_t)ntables * (na + 1), 0);
     plan.h_tbase.assign((size_t)ntables * (na + 1), 0);
     plan.off_fwd.assign(nl, 0);
@@ -91,7 +117,6 @@ hipError_t build_plan(Plan &plan, const std::vector<const MeshDev *> &meshes,
           [&](int k) { return cdiv(meshes[k]->nslices, kSlicesPerBlock); });
     table(2, plan.off_resid, plan.blk_resid,
           [&](int k) { return cdiv(meshes[k]->nslices_free, kSlicesPerBlock); });
-    table(3, plan.off_ident, plan.blk_ident, [&](int k) { return cdiv(meshes[k]->n, kBlock); });
     table(4, plan.off_apply, plan.blk_apply, [&](int k) { return cdiv(meshes[k]->nf, kBlock); });
     table(5, plan.off_sub, plan.blk_sub, [&](int k) { return factors[k]->nsub; });
     plan.sub = SubLds{};
@@ -105,14 +130,14 @@ hipError_t build_plan(Plan &plan, const std::vector<const MeshDev *> &meshes,
     plan.sub.block = plan.blk_sub <= kSubFew ? kSubBlock : 0;
     table(6, plan.off_subb, plan.blk_subb,
           [&](int k) { return factors[k]->nsub + cdiv(meshes[k]->nlrows, sub_rows_bwd(plan.sub)); });
-    table(7, plan.off_subf, plan.blk_subf,
+    table(3, plan.off_subf, plan.blk_subf,
           [&](int k) { return factors[k]->nsub + cdiv(meshes[k]->nlrows, sub_rows_fwd(plan.sub)); });
     for (int l = 0; l < nl; ++l) {
-        table(8 + 2 * l, plan.off_fwd[l], plan.blk_fwd[l], [&](int k) {
+        table(7 + 2 * l, plan.off_fwd[l], plan.blk_fwd[l], [&](int k) {
             const Factor *f = factors[k];
             return l < f->nlevels ? f->ft_ptr[l + 1] - f->ft_ptr[l] : 0;
         });
-        table(9 + 2 * l, plan.off_bwd[l], plan.blk_bwd[l], [&](int k) {
+        table(8 + 2 * l, plan.off_bwd[l], plan.blk_bwd[l], [&](int k) {
             const Factor *f = factors[k];
             return l < f->nlevels ? f->bt_ptr[l + 1] - f->bt_ptr[l] : 0;
         });
@@ -217,8 +242,10 @@ void enqueue_iteration(const Plan &plan, hipStream_t stream, hipEvent_t *ev) {
     }
 }
 
-// Graph replays of one iteration each leave a few microseconds between launches (about 6 us on
-// a 0.16 ms iteration); a graph of kGraphIterations iterations takes the bulk of a longer run.
+// A graph of kGraphIterations iterations takes the bulk of a longer run. The rest is launched
+// directly: a launch costs the host under a microsecond here and the device 4.5 at least, while each
+// graph leaves about 8 us before the next one and its capture and instantiation take half a
+// millisecond (five iterations of a 642-vertex sphere: 190 us launched, 230 as one-iteration graphs).
 constexpr int kGraphIterations = 8;
 
 static hipError_t capture_iterations(Plan &plan, hipStream_t stream, int count, hipGraphExec_t *out) {
@@ -233,22 +260,20 @@ static hipError_t capture_iterations(Plan &plan, hipStream_t stream, int count, 
     return e;
 }
 
+hipError_t prepare_iterations(Plan &plan, hipStream_t stream, int iters, bool use_graph) {
+    // a PCG iteration is already hundreds of launches: one-iteration graphs
+    const int count = plan.pcg ? 1 : kGraphIterations;
+    if (!use_graph || iters < count || plan.graph) return hipSuccess;
+    return capture_iterations(plan, stream, count, &plan.graph);
+}
+
 hipError_t run_iterations(Plan &plan, hipStream_t stream, int iters, bool use_graph) {
     if (iters <= 0) return hipSuccess;
-    if (!use_graph) {
-        for (int i = 0; i < iters; ++i) enqueue_iteration(plan, stream, nullptr);
-        return hipGetLastError();
-    }
-    // a PCG iteration is already hundreds of launches: one-iteration graphs only
-    const bool multi = !plan.pcg;
-    if (!plan.graph || (multi && !plan.graph_multi)) {  // both at the first replay: a warm-up call captures them
-        plan.drop_graph();
-        MD_HIP_E(capture_iterations(plan, stream, 1, &plan.graph));
-        if (multi) MD_HIP_E(capture_iterations(plan, stream, kGraphIterations, &plan.graph_multi));
-    }
-    if (multi)
-        for (; iters >= kGraphIterations; iters -= kGraphIterations) MD_HIP_E(hipGraphLaunch(plan.graph_multi, stream));
-    for (; iters > 0; --iters) MD_HIP_E(hipGraphLaunch(plan.graph, stream));
+    MD_HIP_E(prepare_iterations(plan, stream, iters, use_graph));
+    const int count = plan.pcg ? 1 : kGraphIterations;
+    if (use_graph)
+        for (; iters >= count; iters -= count) MD_HIP_E(hipGraphLaunch(plan.graph, stream));
+    for (; iters > 0; --iters) enqueue_iteration(plan, stream, nullptr);
     return hipGetLastError();
 }
 
@@ -314,6 +339,8 @@ extern "C" int md_ctx_create(int device, md_ctx **out) {
         set_error(std::string("md_ctx_create: address of the device workspace: ") + hipGetErrorString(e));
         return MD_ERR_HIP;
     }
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && khz > 0) ctx->clock_khz = khz;
     *out = ctx.release();
     return MD_OK;
 }
@@ -520,6 +547,7 @@ int analyze_device(md_mesh *m) {
     size_t o_cpt = A.reserve(vsz * (pcg ? 4 * (size_t)nblk + 5 : 1));
     size_t o_tx = A.reserve(sizeof(double) * 3 * std::max(1, n - nf));
     size_t o_orig = A.reserve(sizeof(int) * std::max(1, n));
+    size_t o_int = A.reserve(sizeof(int) * std::max(1, n));
     size_t o_xyz = A.reserve(sizeof(double) * 3 * std::max(1, n));
     if (A.allocate() != hipSuccess) {
         set_error("device allocation of " + std::to_string(A.size()) + " bytes failed");
@@ -558,6 +586,7 @@ int analyze_device(md_mesh *m) {
     d.pcg_tol2 = m->cfg.pcg_tol * m->cfg.pcg_tol;
     m->d_tgt_xyz = (double *)A.at(o_tx);
     m->d_orig = (const int *)A.at(o_orig);
+    m->d_internal = (const int *)A.at(o_int);
     m->d_xyz = (double *)A.at(o_xyz);
     hipStream_t st = m->ctx->stream;
     auto up = [&](const void *dst, const void *src, size_t bytes) -> hipError_t {
@@ -572,6 +601,7 @@ int analyze_device(md_mesh *m) {
     chk(up(d.slot_fe_ptr, t.slot_fe_ptr.data(), sizeof(int) * (slots + 1)));
     chk(up(d.slot_fe, t.slot_fe.data(), sizeof(int) * t.slot_fe.size()));
     chk(up(m->d_orig, t.original_of.data(), sizeof(int) * n));
+    chk(up(m->d_internal, t.internal_of.data(), sizeof(int) * n));
     std::vector<FacDev> fh(ns);
     for (int i = 0; i < ns; ++i) {
         FacDev &x = fh[i];
@@ -718,9 +748,6 @@ hipError_t copy_on_stream(md_mesh *m, void *dst, const void *src, size_t bytes, 
     return e == hipSuccess ? hipStreamSynchronize(m->ctx->stream) : e;
 }
 
-// Uploads the caller's positions (original order, 3 per vertex) and spreads them to internal
-// order on the device: into p (rest, may be null) and pp (current positions with the targets
-// of the constrained vertices pasted, may be null). Stream-ordered, no synchronisation.
 // Pinned staging of the packed positions on their way back: downloads of at least kPinMinBytes,
 // from a mesh's second one on, in at most kPinChunks chunks of at least kPinChunkMin bytes, each
 // chunk copied to the caller's buffer as soon as its DMA has arrived. For 3.9 MB (the 164k
@@ -752,38 +779,74 @@ static size_t pin_chunk(size_t bytes) {
     return (c + 7) & ~size_t(7);
 }
 
-hipError_t upload_positions(md_mesh *m, const double *xyz, d4 *p, d4 *pp) {
+// Uploads the caller's positions (original order, 3 per vertex) and spreads them to internal
+// order on the device: into p (rest, may be null) and pp (current positions with the targets
+// of the constrained vertices pasted, and identity rotations; may be null). Stream-ordered, no
+// synchronisation: xyz and the block must stay until the stream has passed. clear: two words of
+// device memory to clear (may be null).
+hipError_t upload_positions(md_mesh *m, const double *xyz, d4 *p, d4 *pp, CallSlot &slot,
+                            unsigned long long *clear = nullptr) {
     hipStream_t st = m->ctx->stream;
     const int n = m->n, nf = m->topo.nf;
     if (n == 0) return hipSuccess;
-    hipError_t e = hipMemcpyAsync(m->d_xyz, xyz, sizeof(double) * 3 * (size_t)n, hipMemcpyHostToDevice, st);
-    if (e == hipSuccess && pp && n > nf) {
+    if (slot.queued) MD_HIP_E(slot.wait());  // an earlier upload of the call may still read the block
+    const size_t bytes = sizeof(double) * 3 * (size_t)n, tb = pp ? sizeof(double) * 3 * (size_t)(n - nf) : 0;
+    const bool staged = bytes + tb <= CallSlot::kStageBytes;
+    UnpackArgs a{m->d_xyz, m->d_internal, n, nf, m->d_tgt_xyz, p, pp, m->dev.quat, clear, &slot.head()->stamp[0]};
+    double *tgt = staged ? slot.data() + 3 * (size_t)n : slot.data();
+    if (tb > CallSlot::kStageBytes) {
         m->tgt_stage.resize(3 * (size_t)(n - nf));
-        for (int iv = nf; iv < n; ++iv)
-            std::memcpy(&m->tgt_stage[3 * (size_t)(iv - nf)], &m->con[3 * (size_t)m->topo.original_of[iv]],
-                        3 * sizeof(double));
-        e = hipMemcpyAsync(m->d_tgt_xyz, m->tgt_stage.data(), sizeof(double) * m->tgt_stage.size(),
-                           hipMemcpyHostToDevice, st);
+        tgt = m->tgt_stage.data();
     }
-    if (e != hipSuccess) return e;
-    launch_unpack_xyz(st, m->d_xyz, m->d_orig, n, nf, m->d_tgt_xyz, p, pp);
+    slot.queued = true;
+    if (staged) {
+        std::memcpy(slot.data(), xyz, bytes);
+        a.xyz = slot.data();
+    } else {
+        MD_HIP_E(hipMemcpyAsync(m->d_xyz, xyz, bytes, hipMemcpyHostToDevice, st));
+    }
+    if (tb) {
+        for (int iv = nf; iv < n; ++iv)
+            std::memcpy(tgt + 3 * (size_t)(iv - nf), &m->con[3 * (size_t)m->topo.original_of[iv]], 3 * sizeof(double));
+        if (staged) a.tgt = tgt;
+        else MD_HIP_E(hipMemcpyAsync(m->d_tgt_xyz, tgt, tb, hipMemcpyHostToDevice, st));
+    }
+    launch_unpack_xyz(st, a, m->fp64());
     return hipGetLastError();
 }
 
-// Current positions to the caller's packed xyz (original order), packed on the device.
-hipError_t download_positions(md_mesh *m, double *xyz) {
+// Packed vectors of every vertex (original order) to the caller: `fill` queues the kernel that
+// writes them to the device-visible address it is given, `arrived` (after everything queued before
+// has finished) may refuse the result by a status other than MD_OK, and out is then left as it was.
+template <class Fill, class Arrived>
+int download_packed(md_mesh *m, double *out, CallSlot &slot, const char *what, Fill fill, Arrived arrived) {
     hipStream_t st = m->ctx->stream;
-    if (m->n == 0) return hipSuccess;
-    launch_pack_xyz(st, m->dev.pp, m->d_orig, m->n, m->d_xyz);
-    hipError_t e = hipGetLastError();
     const size_t bytes = sizeof(double) * 3 * (size_t)m->n;
+    auto fail = [&](hipError_t e) {
+        if (slot.queued) slot.wait();
+        set_error(std::string(what) + " failed: " + hipGetErrorString(e));
+        return (int)MD_ERR_HIP;
+    };
+    hipError_t e = hipSuccess;
+    slot.queued = true;
+    if (bytes <= CallSlot::kStageBytes) {
+        if (m->n > 0) fill(slot.data());
+        e = hipGetLastError();
+        if (e == hipSuccess) e = slot.wait();
+        if (e != hipSuccess) return fail(e);
+        if (int rc = arrived()) return rc;
+        std::memcpy(out, slot.data(), bytes);
+        return MD_OK;
+    }
+    fill(m->d_xyz);
+    e = hipGetLastError();
     if (e == hipSuccess && pin_ready(m, bytes, ++m->downloads)) {
         // every chunk's DMA queued (each followed by its event), then each chunk copied out as
         // soon as it has arrived
         const size_t ch = pin_chunk(bytes);
-        char *pin = reinterpret_cast<char *>(m->xyz_pin), *out = reinterpret_cast<char *>(xyz);
+        char *pin = reinterpret_cast<char *>(m->xyz_pin), *dst = reinterpret_cast<char *>(out);
         const char *src = reinterpret_cast<const char *>(m->d_xyz);
-        int c = 0;
+        int c = 0, rc = MD_OK;
         for (size_t off = 0; off < bytes && e == hipSuccess; off += ch, ++c) {
             e = hipMemcpyAsync(pin + off, src + off, std::min(ch, bytes - off), hipMemcpyDeviceToHost, st);
             if (e == hipSuccess) e = hipEventRecord(m->pin_ev[c], st);
@@ -791,13 +854,32 @@ hipError_t download_positions(md_mesh *m, double *xyz) {
         c = 0;
         for (size_t off = 0; off < bytes && e == hipSuccess; off += ch, ++c) {
             e = hipEventSynchronize(m->pin_ev[c]);
-            if (e == hipSuccess) std::memcpy(out + off, pin + off, std::min(ch, bytes - off));
+            if (e == hipSuccess && c == 0 && (rc = arrived())) return rc;
+            if (e == hipSuccess) std::memcpy(dst + off, pin + off, std::min(ch, bytes - off));
         }
-        return e;
+        if (e != hipSuccess) return fail(e);
+        slot.queued = false;  // the last event was the stream's last work
+        return MD_OK;
     }
-    if (e == hipSuccess) e = hipMemcpyAsync(xyz, m->d_xyz, bytes, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = slot.wait();
+    if (e != hipSuccess) return fail(e);
+    if (int rc = arrived()) return rc;
+    e = hipMemcpyAsync(out, m->d_xyz, bytes, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
-    return e;
+    return e == hipSuccess ? MD_OK : fail(e);
+}
+
+// Current positions to the caller's packed xyz (original order), packed on the device.
+template <class Arrived> int download_positions(md_mesh *m, double *xyz, CallSlot &slot, Arrived arrived) {
+    return download_packed(m, xyz, slot, "position download", [&](double *dst) {
+        launch_pack_xyz(m->ctx->stream, m->dev.pp, m->d_internal, m->n, dst, &slot.head()->stamp[3]);
+    }, arrived);
+}
+
+int no_slot(const char *who) {
+    set_error(std::string(who) + ": pinned host block of " +
+              std::to_string(CallSlot::kHeadBytes + CallSlot::kStageBytes) + " bytes: allocation failed");
+    return MD_ERR_NOMEM;
 }
 
 hipError_t compute_cotan(md_mesh *m) {
@@ -808,15 +890,13 @@ hipError_t compute_cotan(md_mesh *m) {
     return hipGetLastError();
 }
 
-// FP64 numeric factorization on the host from the device cotan weights; uploads panels.
-// With the PCG solver only the Jacobi diagonal is formed (on the device).
-int factor_pcg(md_mesh *m) {
+// With the PCG solver only the Jacobi diagonal is formed (queued on the device).
+int factor_pcg(md_mesh *m, CallSlot &slot) {
     const Plan &P = m->plan;
+    launch_publish(m->ctx->stream, &slot.head()->stamp[1], nullptr, nullptr);
     launch_pcg_diag(m->ctx->stream, P.set(P.off_resid), P.blk_resid, m->fp64());
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(m->ctx->stream);
     if (e != hipSuccess) { set_error(std::string("PCG diagonal: ") + hipGetErrorString(e)); return MD_ERR_HIP; }
-    m->factored = true;
     return MD_OK;
 }
 
@@ -884,12 +964,23 @@ bool factor_host(md_mesh *m, std::string &err) {
     return true;
 }
 
+// Bytes of the FP64 workspace of the device factorization, and its two words that start at
+// zero (the largest |L_ii|, the flag) when the workspace is there.
+size_t fac_ws_size(const md_mesh *m) {
+    const Factor &f = m->fac;
+    const size_t entries = (size_t)f.poff[f.ns] + (size_t)f.woff_s[f.ns] + (size_t)f.woff_t[f.ns] + (size_t)f.woff_u[f.ns];
+    return sizeof(double) * (entries + (size_t)m->topo.nf) + 2 * sizeof(unsigned long long);
+}
+unsigned long long *fac_ws_words(const md_mesh *m) {
+    if (!m->fac_ws || m->fac_ws_bytes != fac_ws_size(m)) return nullptr;
+    return reinterpret_cast<unsigned long long *>(static_cast<char *>(m->fac_ws) + m->fac_ws_bytes) - 2;
+}
+
 // FP64 numeric factorization on the device from the device cotan weights, straight into
 // the sweeps' panels: diagonal, then per height of the supernodal tree the front assembly and
-// the dense partial factorization, then the conversion to the solve precision. The FP64
-// workspace lives for the call only.
-int factor_device(md_mesh *m) {
-    auto t0 = Clock::now();
+// the dense partial factorization, then the conversion to the solve precision. Only queued:
+// factor_finish looks at the flag once the stream has passed. cleared: the two words are zero already.
+int factor_device(md_mesh *m, CallSlot &slot, bool cleared) {
     const Factor &f = m->fac;
     const int ns = f.ns, nf = m->topo.nf;
     hipStream_t st = m->ctx->stream;
@@ -922,8 +1013,7 @@ int factor_device(md_mesh *m) {
     }
     const size_t nP = (size_t)f.poff[ns], nS = (size_t)f.woff_s[ns], nT = (size_t)f.woff_t[ns],
                  nU = (size_t)f.woff_u[ns];
-    const size_t bytes = sizeof(double) * (nP + nS + nT + nU + (size_t)nf) + 2 * sizeof(unsigned long long);
-    const bool keep = m->cfg.rest_mode == MD_REST_REFERENCE;  // refactors on every deform call
+    const size_t bytes = fac_ws_size(m);
     if (m->fac_ws && m->fac_ws_bytes != bytes) m->release_fac_ws();
     if (!m->fac_ws) {
         if (hipMalloc(&m->fac_ws, bytes) != hipSuccess) {
@@ -939,12 +1029,14 @@ int factor_device(md_mesh *m) {
     A.slice_ptr = m->dev.slice_ptr; A.sell_col = m->dev.sell_col; A.w64 = m->dev.w64; A.nf = nf;
     double *base = static_cast<double *>(ws);
     A.P = base; A.S = A.P + nP; A.T = A.S + nS; A.U = A.T + nT; A.diag = A.U + nU;
-    A.amax = reinterpret_cast<unsigned long long *>(A.diag + nf);
+    A.amax = fac_ws_words(m);
     A.flag = reinterpret_cast<int *>(A.amax + 1);
     A.pc = const_cast<void *>(m->dev.pc);
     A.pr = const_cast<void *>(m->dev.pr);
     A.solve64 = m->fp64() ? 1 : 0;
-    hipError_t e = hipMemsetAsync(A.amax, 0, 2 * sizeof(unsigned long long), st);
+    A.stamp = &slot.head()->stamp[1];
+    slot.queued = true;
+    hipError_t e = cleared ? hipSuccess : hipMemsetAsync(A.amax, 0, 2 * sizeof(unsigned long long), st);
     if (e == hipSuccess) {
         launch_fac_diag(st, A);
         for (int h = 0; h < nh; ++h) {
@@ -953,29 +1045,32 @@ int factor_device(md_mesh *m) {
             launch_fac_height(st, A, f.hptr[h] + L.small, L.count, (L.mw + 63) / 64,
                               fac_assembly(L.count, L.mm, L.mo, L.maps), L.tiles);
         }
+        launch_publish(st, &slot.head()->stamp[2], A.flag, &slot.head()->flag);
         e = hipGetLastError();
     }
-    int flag = 0;
-    if (e == hipSuccess) e = hipMemcpyAsync(&flag, A.flag, sizeof(int), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (!keep || e != hipSuccess) m->release_fac_ws();
     if (e != hipSuccess) {
+        slot.wait();
+        m->release_fac_ws();
         set_error(std::string("device factorization: ") + hipGetErrorString(e));
         return MD_ERR_HIP;
     }
-    m->factor_ms = std::chrono::duration<double, std::milli>(Clock::now() - t0).count();
-    if (flag == 1) {
-        m->factored = false;
+    return MD_OK;
+}
+
+// Result of a queued device factorization, after the stream has passed it. The workspace stays
+// with meshes that refactor on every deform call.
+int factor_finish(md_mesh *m, const CallSlot &slot) {
+    if (m->cfg.rest_mode != MD_REST_REFERENCE) m->release_fac_ws();
+    m->factor_ms = slot.ms(1, 2);
+    if (slot.head()->flag == 1) {
         set_error("factorization failed: a pivot block is not positive definite (a mesh component "
                   "without constraints?)");
         return MD_ERR_FACTOR;
     }
-    if (flag != 0) {
-        m->factored = false;
+    if (slot.head()->flag != 0) {
         set_error("device factorization: inconsistent symbolic structure");
         return MD_ERR_INVALID;
     }
-    m->factored = true;
     return MD_OK;
 }
 
@@ -996,59 +1091,78 @@ int factor_upload(md_mesh *m) {
 }
 
 // The dirty branch of deform (arap.h:102-120), in phases so that the host work of many
-// meshes can run in parallel (md_meshes_prepare) while device work stays on one stream.
+// meshes can run in parallel (md_meshes_prepare) while device work stays on one stream. The device
+// phases only queue; prep_finish closes them once the stream has passed.
 struct Prep {
     const double *xyz = nullptr;
     bool full = false, need_analysis = false, need_factor = false, early = false;
+    bool cleared = false;        // the factorization's two words
+    Clock::time_point uploaded;  // when the upload was queued
 };
 
-// Decisions and the rest pose (arap.h:102-108,162-168).
+// Decisions and the rest pose (arap.h:102-108,162-168). Only an analysis reads the rest pose of
+// a full setup; otherwise the caller copies it while the device works (prep_keep_rest).
 void prep_begin(md_mesh *m, const double *xyz, Prep &p) {
     p.xyz = xyz;
     p.full = m->cfg.rest_mode == MD_REST_REFERENCE || !m->initialized;
-    if (p.full) m->rest.assign(xyz, xyz + 3 * (size_t)m->n);
     p.need_analysis = !m->analyzed || m->con_set_changed;
+    if (p.full && p.need_analysis) m->rest.assign(xyz, xyz + 3 * (size_t)m->n);
     if (p.need_analysis) m->factored = false;
+}
+void prep_keep_rest(md_mesh *m, const Prep &p) {
+    if (p.full && !p.need_analysis) m->rest.assign(p.xyz, p.xyz + 3 * (size_t)m->n);
 }
 
 // Device work before the factorization: arena, weights, initial guess, identity rotations.
-int prep_device_a(md_mesh *m, Prep &p) {
+int prep_device_a(md_mesh *m, Prep &p, CallSlot &slot) {
     if (p.need_analysis) {
         int rc = analyze_device(m);
         if (rc) return rc;
     }
+    const bool device = m->cfg.solver == MD_SOLVER_LDLT && m->cfg.factor_device;
+    const bool factor = m->ncon > 0 && m->topo.nf > 0 && (p.full || p.need_analysis || !m->factored);
+    unsigned long long *words = factor && device ? fac_ws_words(m) : nullptr;
+    p.cleared = words && m->n > 0;
     hipError_t e = hipSuccess;
     // rest pose (when it changes) and the initial guess: the current mesh with the targets
     // pasted (arap.h:162-168, 277-281); in reference rest mode both come from the same upload
-    if (p.full) e = upload_positions(m, p.xyz, m->dev.p, m->dev.pp);
+    if (p.full) e = upload_positions(m, p.xyz, m->dev.p, m->dev.pp, slot, words);
     else {
-        if (p.need_analysis) e = upload_positions(m, m->rest.data(), m->dev.p, nullptr);
-        if (e == hipSuccess) e = upload_positions(m, p.xyz, nullptr, m->dev.pp);
+        if (p.need_analysis) e = upload_positions(m, m->rest.data(), m->dev.p, nullptr, slot);
+        if (e == hipSuccess) e = upload_positions(m, p.xyz, nullptr, m->dev.pp, slot, words);
     }
-    if (e != hipSuccess) { set_error(std::string("position upload failed: ") + hipGetErrorString(e)); return MD_ERR_HIP; }
-    if (p.full || p.need_analysis) {
+    p.uploaded = Clock::now();
+    if (e == hipSuccess && (p.full || p.need_analysis)) {
         e = compute_cotan(m);
         if (e != hipSuccess) { set_error(std::string("cotan weights: ") + hipGetErrorString(e)); return MD_ERR_HIP; }
     }
-    // identity rotations (arap.h:246-249)
-    launch_identity_quat(m->ctx->stream, m->plan.set(m->plan.off_ident), m->plan.blk_ident, m->fp64());
     m->initialized = true;
     m->iterated = false;
-    // the caller's buffers have been read once this returns (the copies above may be
-    // asynchronous), and the cotan weights are complete for the host factorization
-    e = hipStreamSynchronize(m->ctx->stream);
+    p.early = m->ncon == 0;  // arap.h:113-114
+    p.need_factor = factor;
+    if (e == hipSuccess && p.early) e = slot.wait();
     if (e != hipSuccess) { set_error(std::string("position upload failed: ") + hipGetErrorString(e)); return MD_ERR_HIP; }
-    if (m->ncon == 0) { p.early = true; return MD_OK; }  // arap.h:113-114
-    p.need_factor = m->topo.nf > 0 && (p.full || p.need_analysis || !m->factored);
-    if (p.need_factor && m->cfg.solver == MD_SOLVER_LDLT && !m->cfg.factor_device) return weights_download(m);
+    if (p.need_factor && m->cfg.solver == MD_SOLVER_LDLT && !device) return weights_download(m);
     return MD_OK;
 }
 
-// Device work after the factorization.
-int prep_device_b(md_mesh *m, Prep &p) {
+// Device work of the factorization.
+int prep_device_b(md_mesh *m, Prep &p, CallSlot &slot) {
+    if (!p.need_factor) return MD_OK;
+    const bool pcg = m->cfg.solver == MD_SOLVER_PCG;
+    if (!pcg && m->cfg.factor_device) return factor_device(m, slot, p.cleared);
+    if (int rc = pcg ? factor_pcg(m, slot) : factor_upload(m)) return rc;
+    slot.queued = true;
+    launch_publish(m->ctx->stream, &slot.head()->stamp[2], nullptr, nullptr);
+    return MD_OK;
+}
+
+// After the stream has passed the queued work.
+int prep_finish(md_mesh *m, const Prep &p, const CallSlot &slot) {
     if (p.need_factor) {
-        int rc = m->cfg.solver == MD_SOLVER_PCG ? factor_pcg(m) : m->cfg.factor_device ? factor_device(m)
-                                                                                       : factor_upload(m);
+        const bool device = m->cfg.solver == MD_SOLVER_LDLT && m->cfg.factor_device;
+        const int rc = device ? factor_finish(m, slot) : MD_OK;
+        m->factored = rc == MD_OK;
         if (rc) return rc;
     }
     m->dirty = false;
@@ -1056,10 +1170,9 @@ int prep_device_b(md_mesh *m, Prep &p) {
     return MD_OK;
 }
 
-// Returns MD_OK with *early = true when no vertex is constrained (arap.h:113-114).
-int setup(md_mesh *m, const double *xyz, bool *early) {
+// Queues the whole setup. p.early: no vertex is constrained (arap.h:113-114), nothing is queued.
+int setup_queue(md_mesh *m, const double *xyz, Prep &p, CallSlot &slot) {
     auto ms_since = [](Clock::time_point t) { return std::chrono::duration<double, std::milli>(Clock::now() - t).count(); };
-    Prep p;
     auto t0 = Clock::now();
     prep_begin(m, xyz, p);
     m->setup_phase_ms[0] = m->setup_phase_ms[1] = m->setup_phase_ms[2] = 0.0;
@@ -1069,18 +1182,41 @@ int setup(md_mesh *m, const double *xyz, bool *early) {
     }
     m->setup_phase_ms[0] = ms_since(t0);
     t0 = Clock::now();
-    int rc = prep_device_a(m, p);
+    int rc = prep_device_a(m, p, slot);
     m->setup_phase_ms[1] = ms_since(t0);
+    if (rc || p.early) {
+        prep_keep_rest(m, p);
+        return rc;
+    }
+    if (p.need_factor && m->cfg.solver == MD_SOLVER_LDLT && !m->cfg.factor_device) {
+        t0 = Clock::now();
+        std::string err;
+        if (!factor_host(m, err)) {
+            prep_keep_rest(m, p);
+            set_error(err);
+            return MD_ERR_FACTOR;
+        }
+        m->setup_phase_ms[2] = ms_since(t0);
+    } else {
+        m->setup_phase_ms[1] = std::chrono::duration<double, std::milli>(p.uploaded - t0).count();
+    }
+    rc = prep_device_b(m, p, slot);
+    if (rc) prep_keep_rest(m, p);
+    return rc;
+}
+
+// The whole setup, waited for.
+int setup(md_mesh *m, const double *xyz, bool *early) {
+    CallSlot slot(m->ctx);
+    if (!slot.ok()) return no_slot("setup");
+    Prep p;
+    int rc = setup_queue(m, xyz, p, slot);
     *early = p.early;
     if (rc || p.early) return rc;
-    t0 = Clock::now();
-    if (p.need_factor && m->cfg.solver == MD_SOLVER_LDLT && !m->cfg.factor_device) {
-        std::string err;
-        if (!factor_host(m, err)) { set_error(err); return MD_ERR_FACTOR; }
-    }
-    rc = prep_device_b(m, p);
-    m->setup_phase_ms[2] = ms_since(t0);
-    return rc;
+    prep_keep_rest(m, p);
+    hipError_t e = slot.wait();
+    if (e != hipSuccess) { set_error(std::string("setup: ") + hipGetErrorString(e)); return MD_ERR_HIP; }
+    return prep_finish(m, p, slot);
 }
 
 // Runs fn(k) for k in [0, count) on up to nthreads threads.
@@ -1099,10 +1235,16 @@ template <class Fn> void parallel_for(int count, int nthreads, Fn fn) {
     for (auto &x : th) x.join();
 }
 
-int iterate(md_mesh *m, int iterations) {
+int iterate_queue(md_mesh *m, int iterations) {
     if (iterations <= 0) return MD_OK;
     hipError_t e = run_iterations(m->plan, m->ctx->stream, iterations, m->cfg.use_graph != 0);
-    if (e == hipSuccess) e = hipStreamSynchronize(m->ctx->stream);
+    if (e != hipSuccess) { set_error(std::string("iteration failed: ") + hipGetErrorString(e)); return MD_ERR_HIP; }
+    return MD_OK;
+}
+int iterate(md_mesh *m, int iterations) {
+    if (iterations <= 0) return MD_OK;
+    if (int rc = iterate_queue(m, iterations)) return rc;
+    hipError_t e = hipStreamSynchronize(m->ctx->stream);
     if (e != hipSuccess) { set_error(std::string("iteration failed: ") + hipGetErrorString(e)); return MD_ERR_HIP; }
     m->iterated = true;
     return MD_OK;
@@ -1151,7 +1293,8 @@ hipError_t restore_state(const std::vector<md_mesh *> &meshes, hipStream_t st, c
 
 hipError_t time_plan(Plan &plan, hipStream_t st, int iters, bool use_graph, double &ms) {
     hipEvent_t a = nullptr, b = nullptr;
-    hipError_t e = hipEventCreate(&a);
+    hipError_t e = prepare_iterations(plan, st, iters, use_graph);
+    if (e == hipSuccess) e = hipEventCreate(&a);
     if (e == hipSuccess) e = hipEventCreate(&b);
     if (e == hipSuccess) e = hipEventRecord(a, st);
     if (e == hipSuccess) e = run_iterations(plan, st, iters, use_graph);
@@ -1203,7 +1346,7 @@ void rebind(md_mesh *m, const char *oa, size_t asz, char *na, const char *ol, si
     fix(d.sfc); fix(d.sbo); fix(d.srow); fix(d.sfi); fix(d.lrows); fix(d.energy_part); fix(d.w32);
     fix(d.diag); fix(d.cg_x); fix(d.cg_p); fix(d.cg_v); fix(d.cg_part);
     fix(m->d_fac); fix(m->d_fchild); fix(m->d_offrows); fix(m->d_rel); fix(m->d_tgt_xyz);
-    fix(m->d_orig); fix(m->d_xyz);
+    fix(m->d_orig); fix(m->d_internal); fix(m->d_xyz);
 }
 
 // True when an 8-byte word of the mesh's device record still addresses an old arena (a
@@ -1356,7 +1499,7 @@ extern "C" int md_mesh_autotune(md_mesh *m, const int *budgets, int count, int i
         rc = relayout(m, budgets[i]);
         if (rc) return rc;
         double t = 0.0;
-        MD_HIP(run_iterations(m->plan, st, 1, g));  // first replay captures the graphs
+        MD_HIP(run_iterations(m->plan, st, 1, g));  // untimed first run
         MD_HIP(restore_state(ms, st, snap));
         MD_HIP(time_plan(m->plan, st, iterations, g, t));
         MD_HIP(restore_state(ms, st, snap));
@@ -1463,9 +1606,13 @@ extern "C" int md_meshes_prepare(md_ctx *ctx, int count, md_mesh *const *meshes,
             todo[k]->setup_ms_host = std::chrono::duration<double, std::milli>(Clock::now() - t0).count();
         }
     });
+    CallSlot slot(ctx);  // one mesh at a time
+    if (!slot.ok()) return no_slot("md_meshes_prepare");
     for (int k = 0; k < nt; ++k) {
-        int rc = prep_device_a(todo[k], preps[k]);
+        int rc = prep_device_a(todo[k], preps[k], slot);
+        prep_keep_rest(todo[k], preps[k]);
         if (rc) return rc;
+        MD_HIP(slot.wait());
         if (preps[k].early) {
             set_error("md_meshes_prepare: mesh without constrained vertices");
             return MD_ERR_STATE;
@@ -1480,8 +1627,10 @@ extern "C" int md_meshes_prepare(md_ctx *ctx, int count, md_mesh *const *meshes,
     for (int k = 0; k < nt; ++k)
         if (bad[k]) { set_error(errs[k]); return MD_ERR_FACTOR; }
     for (int k = 0; k < nt; ++k) {
-        int rc = prep_device_b(todo[k], preps[k]);
+        int rc = prep_device_b(todo[k], preps[k], slot);
         if (rc) return rc;
+        MD_HIP(slot.wait());
+        if ((rc = prep_finish(todo[k], preps[k], slot))) return rc;
     }
     return MD_OK;
 }
@@ -1494,23 +1643,51 @@ extern "C" int md_mesh_deform(md_mesh *m, int iterations, double *xyz, int *ok) 
     auto ms_since = [](Clock::time_point t) { return std::chrono::duration<double, std::milli>(Clock::now() - t).count(); };
     const auto t_call = Clock::now();
     for (double &x : m->deform_ms) x = 0.0;
-    if (m->dirty) {
-        bool early = false;
-        int rc = setup(m, xyz, &early);
+    // everything is queued and waited for once: the setup, the iterations (arap.h:122-129) and the
+    // packed positions; a factorization that failed leaves xyz untouched and the state that of the setup
+    CallSlot slot(m->ctx);
+    if (!slot.ok()) return no_slot("md_mesh_deform");
+    const bool dirty = m->dirty;
+    Prep p;
+    if (dirty) {
+        int rc = setup_queue(m, xyz, p, slot);
         for (int k = 0; k < 3; ++k) m->deform_ms[k] = m->setup_phase_ms[k];
         if (rc == MD_ERR_FACTOR) return rc;   // deform() == false (arap.h:116-117)
         if (rc) return rc;
-        if (early) { if (ok) *ok = 1; m->deform_ms[5] = ms_since(t_call); return MD_OK; }
+        if (p.early) { if (ok) *ok = 1; m->deform_ms[5] = ms_since(t_call); return MD_OK; }
     }
-    auto t0 = Clock::now();
-    int rc = iterate(m, iterations);  // arap.h:122-129
+    slot.queued = true;
+    int rc = iterate_queue(m, iterations);
+    if (dirty) prep_keep_rest(m, p);
     if (rc) return rc;
-    m->deform_ms[3] = ms_since(t0);
-    t0 = Clock::now();
-    hipError_t e = download_positions(m, xyz);  // write-back, arap.h:133-135
-    if (e != hipSuccess) { set_error("position download failed"); return MD_ERR_HIP; }
-    m->deform_ms[4] = ms_since(t0);
-    m->deform_ms[5] = ms_since(t_call);
+    double arrived_ms = 0.0;
+    rc = download_positions(m, xyz, slot, [&]() -> int {  // write-back, arap.h:133-135
+        arrived_ms = ms_since(t_call);
+        const int r = dirty ? prep_finish(m, p, slot) : MD_OK;
+        if (r == MD_OK) m->iterated = m->iterated || iterations > 0;
+        return r;
+    });
+    if (rc) {
+        if (dirty && m->dirty && (rc == MD_ERR_FACTOR || rc == MD_ERR_INVALID)) {
+            hipError_t e = upload_positions(m, xyz, nullptr, m->dev.pp, slot);
+            if (e == hipSuccess) e = slot.wait();
+            if (e != hipSuccess) { set_error("position upload failed"); return MD_ERR_HIP; }
+        }
+        return rc;
+    }
+    // phases: the host's clock outside the device's work, the kernels' clocks within
+    double *t = m->deform_ms;
+    t[5] = ms_since(t_call);
+    if (dirty) {
+        const bool device = p.need_factor && (m->cfg.solver == MD_SOLVER_PCG || m->cfg.factor_device);
+        if (device) t[1] += slot.ms(0, 1);
+        if (device) t[2] = slot.ms(1, 2);
+        t[3] = slot.ms(p.need_factor ? 2 : 0, 3);
+        t[4] = std::max(0.0, t[5] - t[0] - t[1] - t[2] - t[3]);
+    } else {
+        t[3] = arrived_ms;
+        t[4] = t[5] - arrived_ms;
+    }
     if (ok) *ok = 1;
     return MD_OK;
 }
@@ -1528,8 +1705,9 @@ extern "C" int md_mesh_download(md_mesh *m, double *xyz) {
     if (!m->analyzed) { set_error("md_mesh_download: no device state yet"); return MD_ERR_STATE; }
     hipSetDevice(m->ctx->device);
     if (int rc = ensure_resident(m, "md_mesh_download")) return rc;
-    if (download_positions(m, xyz) != hipSuccess) { set_error("position download failed"); return MD_ERR_HIP; }
-    return MD_OK;
+    CallSlot slot(m->ctx);
+    if (!slot.ok()) return no_slot("md_mesh_download");
+    return download_positions(m, xyz, slot, [] { return (int)MD_OK; });
 }
 
 extern "C" int md_mesh_cotan_nnz(md_mesh *m, int64_t *nnz) {
@@ -1612,34 +1790,23 @@ extern "C" int md_mesh_normals(md_mesh *m, double *nrm) {
     if (!m->analyzed) { set_error("md_mesh_normals: call deform first"); return MD_ERR_STATE; }
     hipSetDevice(m->ctx->device);
     if (int rc = ensure_resident(m, "md_mesh_normals")) return rc;
-    hipStream_t st = m->ctx->stream;
-    double *fn = nullptr;
-    d4 *out = nullptr;
-    MD_HIP(hipMalloc((void **)&fn, sizeof(double) * 3 * std::max(1, m->F)));
-    hipError_t e = hipMalloc((void **)&out, sizeof(d4) * std::max(1, m->n));
-    if (e == hipSuccess) {
-        const Plan &P = m->plan;
-        launch_normals(st, P.set(P.off_face), P.blk_face, P.set(P.off_slice), P.blk_slice, fn, out);
-        e = hipGetLastError();
-    }
-    std::vector<d4> h(m->n);
-    if (e == hipSuccess) e = hipMemcpyAsync(h.data(), out, sizeof(d4) * m->n, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    hipStreamSynchronize(st);
-    if (fn) hipFree(fn);
-    if (out) hipFree(out);
-    if (e != hipSuccess) { set_error(std::string("md_mesh_normals: ") + hipGetErrorString(e)); return MD_ERR_HIP; }
-    for (int iv = 0; iv < m->n; ++iv) {
-        double *o = nrm + 3 * (size_t)m->topo.original_of[iv];
-        o[0] = h[iv].x; o[1] = h[iv].y; o[2] = h[iv].z;
-    }
-    return MD_OK;
+    // face normals in the cotan step's per-face scratch (three doubles a face, rewritten whenever
+    // weights are computed), vertex normals packed into the positions' device buffer: nothing is allocated
+    CallSlot slot(m->ctx);
+    if (!slot.ok()) return no_slot("md_mesh_normals");
+    const Plan &P = m->plan;
+    return download_packed(m, nrm, slot, "md_mesh_normals", [&](double *dst) {
+        launch_normals(m->ctx->stream, P.set(P.off_face), P.blk_face, P.set(P.off_slice), P.blk_slice, m->dev.fe_val,
+                       nullptr, m->d_xyz, m->d_orig);
+        if (dst != m->d_xyz)
+            hipMemcpyAsync(dst, m->d_xyz, sizeof(double) * 3 * (size_t)m->n, hipMemcpyDeviceToHost, m->ctx->stream);
+    }, [] { return (int)MD_OK; });
 }
 
 namespace {
 constexpr size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 // Workspace of md_mesh_normals_noalloc: face normals, vertex normals (internal order), the
-// internal-to-original permutation and the packed result.
+// original-to-internal permutation and the packed result.
 size_t normals_scratch_bytes(size_t n, size_t F) {
     return align256(sizeof(double) * 3 * F) + align256(sizeof(d4) * n) + align256(sizeof(int) * n) +
            align256(sizeof(double) * 3 * n);
@@ -1677,9 +1844,9 @@ extern "C" int md_mesh_normals_noalloc(md_mesh *m, double *nrm) {
     launch_normals(st, P.set(P.off_face), P.blk_face, P.set(P.off_slice), P.blk_slice, fn, vn);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && n)
-        e = hipMemcpyAsync(perm, m->topo.original_of.data(), sizeof(int) * n, hipMemcpyHostToDevice, st);
+        e = hipMemcpyAsync(perm, m->topo.internal_of.data(), sizeof(int) * n, hipMemcpyHostToDevice, st);
     if (e == hipSuccess) {
-        launch_pack_xyz(st, vn, perm, m->n, dst);
+        launch_pack_xyz(st, vn, perm, m->n, dst, nullptr);
         e = hipGetLastError();
     }
     if (e == hipSuccess && n) e = hipMemcpyAsync(nrm, dst, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, st);
@@ -1791,6 +1958,7 @@ extern "C" int md_mesh_time_iterations(md_mesh *m, int warmup, int iterations, d
     hipStream_t st = m->ctx->stream;
     bool g = m->cfg.use_graph != 0;
     MD_HIP(run_iterations(m->plan, st, warmup, g));
+    MD_HIP(prepare_iterations(m->plan, st, iterations, g));
     MD_HIP(hipStreamSynchronize(st));
     hipEvent_t a, b;
     MD_HIP(hipEventCreate(&a));

@@ -4,6 +4,7 @@
 
 #include <array>
 #include <atomic>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -49,11 +50,11 @@ private:
 struct Plan {
     int nactive = 0;
     int nlevels = 0;
-    int blk_face = 0, blk_slice = 0, blk_resid = 0, blk_ident = 0, blk_apply = 0, blk_sub = 0;
+    int blk_face = 0, blk_slice = 0, blk_resid = 0, blk_apply = 0, blk_sub = 0;
     int blk_subb = 0, off_subb = 0;    // k_sub_bwd: subtrees, then the p' update of level rows
     int blk_subf = 0, off_subf = 0;    // k_sub_fwd with the residual: subtrees, then the level rows
     std::vector<int> blk_fwd, blk_bwd;
-    int off_face = 0, off_slice = 0, off_resid = 0, off_ident = 0, off_apply = 0, off_sub = 0;
+    int off_face = 0, off_slice = 0, off_resid = 0, off_apply = 0, off_sub = 0;
     SubLds sub{};                      // bottom subtrees: workgroup size, LDS of the largest
     std::vector<int> off_fwd, off_bwd;
     MeshDev *d_meshes = nullptr;       // views into d_tables: the mesh records,
@@ -72,8 +73,7 @@ struct Plan {
     int refine_steps = 1;
     bool pcg = false;
     int pcg_iters = 0;
-    hipGraphExec_t graph = nullptr;        // one iteration
-    hipGraphExec_t graph_multi = nullptr;  // kGraphIterations iterations
+    hipGraphExec_t graph = nullptr;        // kGraphIterations iterations (PCG: one)
     ~Plan();
     void drop_graph();
     LaunchSet set(int off) const {
@@ -99,7 +99,9 @@ hipError_t build_plan(Plan &plan, const std::vector<const MeshDev *> &meshes,
                       hipStream_t stream, bool sync = true, bool block_maps = false);
 // Enqueues one ARAP iteration (local step + refine_steps x (residual, sweeps)).
 void enqueue_iteration(const Plan &plan, hipStream_t stream, hipEvent_t *phase_events);
-// Runs `iters` iterations, from a captured graph when use_graph is set.
+// Runs `iters` iterations, the bulk of them from a captured graph when use_graph is set;
+// prepare_iterations captures what that many need, without running it.
+hipError_t prepare_iterations(Plan &plan, hipStream_t stream, int iters, bool use_graph);
 hipError_t run_iterations(Plan &plan, hipStream_t stream, int iters, bool use_graph);
 
 // Sweep layout of a prepared LDLT mesh with another bottom-subtree budget (device_layout +
@@ -147,11 +149,49 @@ struct md_ctx {
     // the caller's handle plus one reference per mesh, batch and server created from it:
     // the stream is destroyed with the last holder, whatever the order of destruction
     std::atomic<int> refs{1};
+    double clock_khz = 1e5;   // rate of the kernels' wall_clock64
+    std::mutex slot_mu;       // pinned blocks of calls (md::CallSlot) waiting for the next one,
+    std::vector<char *> slots;  //   at most kSlotsKept
 };
 
 namespace md {
 void ctx_retain(md_ctx *c);
 void ctx_release(md_ctx *c);
+
+// Pinned host block that one call holds from its first launch to its end (so calls of several
+// threads never share one): the factorization's flag and the kernels' clocks, then kStageBytes through
+// which small positions travel. Measured for 246 KB (10k vertices): a pageable copy up 103 us and
+// down 110, through the block (host copy, a kernel reading or writing it, both with the wait) 18 and
+// 21; for 983 KB 46 and 50 against 45 and 51, so the line lies at about one MB.
+class CallSlot {
+public:
+    struct Head {
+        int flag;                     // of the device factorization
+        unsigned long long stamp[4];  // clocks: unpack, factorization, its end, pack
+    };
+    static constexpr size_t kStageBytes = size_t(5) << 18, kHeadBytes = 256;
+    static constexpr size_t kSlotsKept = 4;
+    explicit CallSlot(md_ctx *c);
+    ~CallSlot();  // waits for the stream if work of the call may still use the block
+    CallSlot(const CallSlot &) = delete;
+    CallSlot &operator=(const CallSlot &) = delete;
+    bool ok() const { return base_ != nullptr; }
+    Head *head() const { return reinterpret_cast<Head *>(base_); }
+    double *data() const { return reinterpret_cast<double *>(base_ + kHeadBytes); }
+    double ms(int from, int to) const {
+        return head()->stamp[to] > head()->stamp[from]
+                   ? (double)(head()->stamp[to] - head()->stamp[from]) / ctx_->clock_khz : 0.0;
+    }
+    hipError_t wait() {
+        queued = false;
+        return hipStreamSynchronize(ctx_->stream);
+    }
+    bool queued = false;
+
+private:
+    md_ctx *ctx_;
+    char *base_ = nullptr;
+};
 }  // namespace md
 
 struct md_mesh {
@@ -193,9 +233,10 @@ struct md_mesh {
     std::vector<char> pc_host, pr_host;  // device panel layouts staged on the host
     double *d_tgt_xyz = nullptr;   // targets of the constrained ids, internal order (3 (n - nf))
     const int *d_orig = nullptr;   // original id of each internal id (topo.original_of)
+    const int *d_internal = nullptr;  // internal id of each original id (topo.internal_of)
     double *d_xyz = nullptr;       // packed xyz in original order (3n): positions in and out
-    std::vector<double> tgt_stage; // targets of the constrained ids in internal order (host
-                                   //   source of an upload; kept until the stream has passed it)
+    std::vector<double> tgt_stage; // targets of the constrained ids in internal order (host source of
+                                   //   an upload too large for the call's pinned block)
     // FP64 workspace of the device factorization, kept between calls by meshes that refactor
     // on every deform call (reference rest mode); others free it after each factorization
     void *fac_ws = nullptr;

@@ -109,6 +109,7 @@ extern "C" int md_batch_time_iterations(md_batch *b, int warmup, int iterations,
     hipSetDevice(b->ctx->device);
     hipStream_t st = b->ctx->stream;
     hipError_t e = run_iterations(b->plan, st, warmup, b->use_graph);
+    if (e == hipSuccess) e = prepare_iterations(b->plan, st, iterations, b->use_graph);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     hipEvent_t a = nullptr, c = nullptr;
     if (e == hipSuccess) e = hipEventCreate(&a);
@@ -163,7 +164,7 @@ extern "C" int md_batch_autotune(md_batch *b, const int *budgets, int count, int
     for (int i = 0; i < count; ++i) {
         if (int rc = use(budgets[i])) return rc;
         double t = 0.0;
-        e = run_iterations(b->plan, st, 1, b->use_graph);  // first replay captures the graph
+        e = run_iterations(b->plan, st, 1, b->use_graph);  // untimed first run
         if (e == hipSuccess) e = restore_state(b->meshes, st, snap);
         if (e == hipSuccess) e = time_plan(b->plan, st, iterations, b->use_graph, t);
         if (e == hipSuccess) e = restore_state(b->meshes, st, snap);
