@@ -172,7 +172,7 @@ std::vector<int> order_graph(int m, const int* rowptr, const int* col, const dou
 
 std::vector<int> order_free_vertices(int n, int F, const int* tri, const double* xyz,
                                      const std::vector<char>& is_con, std::vector<int>* pair_group,
-                                     double amalg_ratio) {
+                                     double amalg_ratio, int top_columns) {
     std::vector<int> rank_of, vert_of, ptr, adj;
     free_graph(n, F, tri, is_con, rank_of, vert_of, ptr, adj);
     int m = (int)vert_of.size();
@@ -180,7 +180,7 @@ std::vector<int> order_free_vertices(int n, int F, const int* tri, const double*
     for (int k = 0; k < m; ++k)
         for (int a = 0; a < 3; ++a) fx[3 * k + a] = xyz[3 * (size_t)vert_of[k] + a];
     std::vector<int> perm = nd_postorder(m, ptr, adj, fx);
-    if (pair_group) perm = pair_levels(perm, ptr, adj, kPairBudget, amalg_ratio, *pair_group);
+    if (pair_group) perm = pair_levels(perm, ptr, adj, kPairBudget, amalg_ratio, top_columns, *pair_group);
     for (int k = 0; k < m; ++k) perm[k] = vert_of[perm[k]];
     return perm;
 }
@@ -689,7 +689,7 @@ void device_layout(Factor& f, int sub_budget) {
 // ---- level pairs ------------------------------------------------------------------------
 
 std::vector<int> pair_levels(const std::vector<int>& order, const std::vector<int>& ptr, const std::vector<int>& adj,
-                             int sub_budget, double amalg_ratio, std::vector<int>& group) {
+                             int sub_budget, double amalg_ratio, int top_columns, std::vector<int>& group) {
     const int m = (int)order.size();
     group.assign(m, -1);
     if (m == 0) return order;
@@ -706,55 +706,59 @@ std::vector<int> pair_levels(const std::vector<int>& order, const std::vector<in
     Factor f;
     symbolic(m, p2, a2, f, sub_budget, amalg_ratio);
     const int ns = f.ns, top = f.nlevels - 1;
-    if (top < 2) return order;
-    // members: level supernodes whose level is an odd distance below the top level and whose
-    // parent sits one level up; they join their parent's group
+    if (top < 0) return order;
+    // the top levels [cut, top] of at most top_columns columns together, or all of a small system. Below
+    // the cut level 0 goes into the subtrees of the default budget and the others pair, so an even cut
+    // leaves as many levels as the next one, for a wider top
+    const bool whole = m <= kWholeColumns;
+    int cut = top;
+    {
+        std::vector<int64_t> width(top + 1, 0);
+        for (int t = 0; t < ns; ++t)
+            if (f.level[t] >= 0) width[f.level[t]] += f.w[t];
+        int64_t sum = width[top];
+        while (cut > 0 && sum + width[cut - 1] <= top_columns) sum += width[--cut];
+        if (cut < top && cut % 2 == 0) ++cut;
+    }
+    if (!whole && cut == top && top < 2) return order;
+    // heads: roots of merged tops; below them, level supernodes whose level is an even distance below
+    // the cut and whose parent sits one level up join their parent's group
     std::vector<int> head(ns, -1);
     for (int t = ns - 1; t >= 0; --t) {
-        if (f.level[t] < 0) continue;
-        const int p = f.parent[t];
-        const bool member = p >= 0 && (top - f.level[t]) % 2 == 0 && f.level[p] == f.level[t] + 1 && head[p] == p;
-        head[t] = member ? p : t;
+        const int p = f.parent[t], l = f.level[t];
+        head[t] = t;
+        if (p < 0) continue;
+        if (whole || l >= cut) head[t] = head[p];
+        else if (l >= 0 && (cut - l) % 2 == 0 && f.level[p] == l + 1 && head[p] == p) head[t] = p;
     }
-    // children lists in id order
-    std::vector<std::vector<int>> kids(ns);
+    // per head, in id order (children before parents): its members, and the heads right below them
+    std::vector<std::vector<int>> members(ns), below(ns);
     std::vector<int> roots;
     for (int t = 0; t < ns; ++t) {
-        if (f.parent[t] >= 0) kids[f.parent[t]].push_back(t);
+        if (head[t] != t) members[head[t]].push_back(t);
+        else if (f.parent[t] >= 0) below[head[f.parent[t]]].push_back(t);
         else roots.push_back(t);
     }
-    // new order of positions: a head's members' subtrees first, then the members' columns,
-    // then the head's; every column still follows its descendants (same fill)
-    std::vector<int> pos;
+    // new order of positions: the subtrees below a group first, then the members' columns, then the
+    // head's; every column still follows its descendants
+    std::vector<int> pos, gpos;
     pos.reserve(m);
-    std::vector<int> gpos;
     gpos.reserve(m);
     auto cols = [&](int t, int g) {
         for (int j = f.c0[t]; j < f.c0[t] + f.w[t]; ++j) { pos.push_back(j); gpos.push_back(g); }
     };
-    struct Frame { int t, stage; };
+    struct Frame { int t; size_t next; };
     std::vector<Frame> st;
     for (int r : roots) {
         st.push_back({r, 0});
         while (!st.empty()) {
             const int t = st.back().t;
-            const int stage = st.back().stage;
-            const std::vector<int>& ch = kids[t];
-            if (stage < (int)ch.size()) {
-                st.back().stage = stage + 1;
-                const int c = ch[stage];
-                if (head[c] == t && c != t) {  // a member: its children's subtrees now
-                    for (int q = (int)kids[c].size() - 1; q >= 0; --q) st.push_back({kids[c][q], 0});
-                } else {
-                    st.push_back({c, 0});
-                }
+            if (st.back().next < below[t].size()) {
+                st.push_back({below[t][st.back().next++], 0});
                 continue;
             }
-            const bool is_head = head[t] == t;
-            bool grouped = false;
-            for (int c : ch)
-                if (head[c] == t && c != t) { cols(c, t); grouped = true; }
-            cols(t, is_head && grouped ? t : -1);
+            for (int c : members[t]) cols(c, t);
+            cols(t, members[t].empty() ? -1 : t);
             st.pop_back();
         }
     }

@@ -33,7 +33,7 @@ extern "C" int md_host_factor_solve(int n, const int *rowptr, const int *col, co
                 if (col[e] != i) adj0.push_back(col[e]);
             ptr0[i + 1] = (int)adj0.size();
         }
-        perm = pair_levels(perm, ptr0, adj0, kPairBudget, kAmalgRatioDefault, group);
+        perm = pair_levels(perm, ptr0, adj0, kPairBudget, kAmalgRatioDefault, kTopColumns, group);
     }
     std::vector<int> iperm(n);
     for (int k = 0; k < n; ++k) iperm[perm[k]] = k;

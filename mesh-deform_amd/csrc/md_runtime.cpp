@@ -470,7 +470,8 @@ void analyze_host(md_mesh *m) {
     const bool pairs = m->cfg.level_pairs != 0 && m->cfg.solver == MD_SOLVER_LDLT;
     std::vector<int> group;
     std::vector<int> perm = order_free_vertices(n, m->F, m->tri.data(), m->rest.data(), m->is_con,
-                                                pairs ? &group : nullptr, m->cfg.amalg_ratio);
+                                                pairs ? &group : nullptr, m->cfg.amalg_ratio,
+                                                m->cfg.rest_mode == MD_REST_REFERENCE ? kTopColumns : kTopColumnsKept);
     m->topo = Topology();
     build_topology(n, m->F, m->tri.data(), perm, m->is_con, m->topo);
     const Topology &t = m->topo;
