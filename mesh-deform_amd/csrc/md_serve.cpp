@@ -209,7 +209,7 @@ struct ServedMesh {
     size_t bytes = 0;             // device footprint while resident (both arenas)
     bool busy = false;            // a request admitted and not completed
     uint64_t last_use = 0;        // admission stamp (least recently used eviction)
-    std::vector<d4 *> pinned_free;  // reusable pinned result buffers
+    std::vector<double *> pinned_free;  // reusable pinned result buffers
     std::vector<uint32_t> stamp;    // per vertex: the last submission that moved it (dedup)
     uint32_t stamp_gen = 0;
 };
@@ -224,7 +224,7 @@ struct Request {
     bool done = false;
     int status = MD_OK;
     std::string error;
-    d4 *pinned = nullptr;         // positions in internal order, copied at completion
+    double *pinned = nullptr;         // packed positions (original order), written at completion
     uint64_t finish_seq = 0;      // launch after which the copy of its positions is complete
 };
 }  // namespace
@@ -262,20 +262,20 @@ struct md_server {
     size_t tgt_cap_host[2] = {0, 0};
     TargetEntry *tgt_dev = nullptr;
     size_t tgt_cap_dev = 0;
-    std::vector<d4 *> pinned_all;                     // guarded by mu
+    std::vector<double *> pinned_all;                     // guarded by mu
 
-    d4 *take_pinned(ServedMesh *sm) {  // caller holds mu
+    double *take_pinned(ServedMesh *sm) {  // caller holds mu
         auto &fl = sm->pinned_free;
         if (!fl.empty()) {
-            d4 *p = fl.back();
+            double *p = fl.back();
             fl.pop_back();
             return p;
         }
         void *p = nullptr;
-        if (hipHostMalloc(&p, sizeof(d4) * (size_t)std::max(1, sm->m->n), hipHostMallocDefault) != hipSuccess)
+        if (hipHostMalloc(&p, 3 * sizeof(double) * (size_t)std::max(1, sm->m->n), hipHostMallocDefault) != hipSuccess)
             return nullptr;
-        pinned_all.push_back((d4 *)p);
-        return (d4 *)p;
+        pinned_all.push_back((double *)p);
+        return (double *)p;
     }
 };
 
@@ -552,7 +552,9 @@ void server_loop(md_server *S) {
                 if (r->status == MD_OK && !(r->pinned = S->take_pinned(r->sm)))
                     fail(*r, MD_ERR_NOMEM, "pinned result buffer");
         }
-        // the positions go to the pinned buffers on the copy stream, after this boundary's
+        // the positions are packed in original order straight into the pinned buffers (a burst to 24
+        // meshes of 5k to 60k vertices: 3.6 ms; with the scatter into the caller's order on the host 4.4) on the
+        // copy stream, after this boundary's
         // launch (or, when nothing was launched, after everything queued so far), so the copies
         // overlap the next launches; a mesh is not iterated again before its result is delivered
         if (launched) hipEventRecord(S->ev[S->seq % 2], st);
@@ -566,8 +568,8 @@ void server_loop(md_server *S) {
                     waited = true;
                 }
                 md_mesh *m = r->sm->m;
-                hipError_t x = hipMemcpyAsync(r->pinned, m->dev.pp, sizeof(d4) * m->n, hipMemcpyDeviceToHost,
-                                              S->copy_stream);
+                launch_pack_xyz(S->copy_stream, m->dev.pp, m->d_internal, m->n, r->pinned, nullptr);
+                hipError_t x = hipGetLastError();
                 if (x != hipSuccess) fail(*r, MD_ERR_HIP, hipGetErrorString(x));
             }
             r->finish_seq = launched ? S->seq : 0;
@@ -652,12 +654,12 @@ extern "C" int md_server_add_mesh(md_server *S, md_mesh *m, int *mesh_id) {
     // they would stall the worker); more are made only while earlier results wait for their
     // md_server_wait / md_server_poll
     void *buf = nullptr;
-    if (hipHostMalloc(&buf, sizeof(d4) * (size_t)std::max(1, m->n), hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc(&buf, 3 * sizeof(double) * (size_t)std::max(1, m->n), hipHostMallocDefault) != hipSuccess) {
         set_error("md_server_add_mesh: pinned result buffer: allocation failed");
         return MD_ERR_NOMEM;
     }
     std::lock_guard<std::mutex> lk(S->mu);
-    S->pinned_all.push_back(static_cast<d4 *>(buf));
+    S->pinned_all.push_back(static_cast<double *>(buf));
     if (!S->meshes.empty()) {
         md_mesh *m0 = S->meshes[0]->m;
         if (m0->cfg.precision != m->cfg.precision || m0->cfg.refine_steps != m->cfg.refine_steps ||
@@ -680,7 +682,7 @@ extern "C" int md_server_add_mesh(md_server *S, md_mesh *m, int *mesh_id) {
     sm->m = m;
     sm->id = (int)S->meshes.size();
     sm->bytes = bytes;
-    sm->pinned_free.push_back(static_cast<d4 *>(buf));
+    sm->pinned_free.push_back(static_cast<double *>(buf));
     S->meshes.push_back(std::move(sm));
     ++m->servers;
     *mesh_id = (int)S->meshes.size() - 1;
@@ -733,8 +735,7 @@ extern "C" int md_server_submit(md_server *S, int mesh_id, int k, const int *idx
 }
 
 // Called with S->mu held: takes the finished request out of the ticket map (null when another
-// caller took it first). The permutation of its positions into the original vertex order runs
-// afterwards without the lock.
+// caller took it first). Its positions are copied out afterwards without the lock.
 static std::shared_ptr<Request> take_finished(md_server *S, uint64_t ticket) {
     auto it = S->tickets.find(ticket);
     if (it == S->tickets.end()) return nullptr;
@@ -748,13 +749,7 @@ static int deliver(md_server *S, std::shared_ptr<Request> r, double *xyz, double
     int rc = r->status;
     if (rc != MD_OK) set_error("request failed: " + r->error);
     else if (xyz && r->pinned) {
-        md_mesh *m = r->sm->m;
-        for (int iv = 0; iv < m->n; ++iv) {
-            int v = m->topo.original_of[iv];
-            xyz[3 * (size_t)v] = r->pinned[iv].x;
-            xyz[3 * (size_t)v + 1] = r->pinned[iv].y;
-            xyz[3 * (size_t)v + 2] = r->pinned[iv].z;
-        }
+        std::memcpy(xyz, r->pinned, sizeof(double) * 3 * (size_t)r->sm->m->n);
     }
     if (r->pinned) {
         std::lock_guard<std::mutex> lk(S->mu);
@@ -819,7 +814,7 @@ extern "C" int md_server_destroy(md_server *S) {
     hipSetDevice(ctx->device);
     hipStreamSynchronize(S->stream);
     hipStreamSynchronize(S->copy_stream);
-    for (d4 *p : S->pinned_all) hipHostFree(p);
+    for (double *p : S->pinned_all) hipHostFree(p);
     for (TargetEntry *p : S->tgt_host)
         if (p) hipHostFree(p);
     if (S->tgt_dev) hipFree(S->tgt_dev);
