@@ -10,6 +10,39 @@ namespace md {
 
 namespace {
 
+// Neighbour lists (ascending, without repeats) of the m kept vertices of faces `tri`: rank[v] is a
+// vertex's number or -1. Counting twice sorts: the lists of the first pass, transposed in order of
+// their owners, come out ascending (the pattern is symmetric), without comparing anything.
+void face_graph(int F, const int* tri, const std::vector<int>& rank, int m, std::vector<int>& ptr, std::vector<int>& adj) {
+    std::vector<int> p(m + 1, 0), fill, list;
+    auto edges = [&](auto fn) {
+        for (int f = 0; f < F; ++f) {
+            const int v[3] = {rank[tri[3 * f]], rank[tri[3 * f + 1]], rank[tri[3 * f + 2]]};
+            for (int k = 0; k < 3; ++k) {
+                const int a = v[k], b = v[k == 2 ? 0 : k + 1];
+                if (a >= 0 && b >= 0 && a != b) fn(a, b);
+            }
+        }
+    };
+    edges([&](int a, int b) { ++p[a + 1]; ++p[b + 1]; });
+    for (int i = 0; i < m; ++i) p[i + 1] += p[i];
+    list.resize(p[m]);
+    fill.assign(p.begin(), p.end() - 1);
+    edges([&](int a, int b) { list[fill[a]++] = b; list[fill[b]++] = a; });
+    std::vector<int> sorted(p[m]);
+    fill.assign(p.begin(), p.end() - 1);
+    for (int i = 0; i < m; ++i)
+        for (int e = p[i]; e < p[i + 1]; ++e) sorted[fill[list[e]]++] = i;
+    ptr.assign(m + 1, 0);
+    adj.clear();
+    adj.reserve(p[m] / 2 + 1);
+    for (int i = 0; i < m; ++i) {
+        for (int e = p[i]; e < p[i + 1]; ++e)
+            if (e == p[i] || sorted[e] != sorted[e - 1]) adj.push_back(sorted[e]);
+        ptr[i + 1] = (int)adj.size();
+    }
+}
+
 // Free-free adjacency in "free rank" numbering (rank among free vertices, ascending id).
 void free_graph(int n, int F, const int* tri, const std::vector<char>& is_con,
                 std::vector<int>& rank_of, std::vector<int>& vert_of, std::vector<int>& ptr,
@@ -18,20 +51,7 @@ void free_graph(int n, int F, const int* tri, const std::vector<char>& is_con,
     vert_of.clear();
     for (int v = 0; v < n; ++v)
         if (!is_con[v]) { rank_of[v] = (int)vert_of.size(); vert_of.push_back(v); }
-    int m = (int)vert_of.size();
-    std::vector<std::pair<int, int>> e;
-    e.reserve((size_t)F * 6);
-    for (int f = 0; f < F; ++f)
-        for (int k = 0; k < 3; ++k) {
-            int a = rank_of[tri[3 * f + k]], b = rank_of[tri[3 * f + (k + 1) % 3]];
-            if (a >= 0 && b >= 0 && a != b) { e.emplace_back(a, b); e.emplace_back(b, a); }
-        }
-    std::sort(e.begin(), e.end());
-    e.erase(std::unique(e.begin(), e.end()), e.end());
-    ptr.assign(m + 1, 0);
-    adj.resize(e.size());
-    for (size_t k = 0; k < e.size(); ++k) { ptr[e[k].first + 1]++; adj[k] = e[k].second; }
-    for (int i = 0; i < m; ++i) ptr[i + 1] += ptr[i];
+    face_graph(F, tri, rank_of, (int)vert_of.size(), ptr, adj);
 }
 
 // ---- geometric nested dissection ------------------------------------------------------
@@ -42,6 +62,8 @@ struct ND {
     const std::vector<double>& xyz;  // 3 per free rank
     std::vector<int> stamp, side;
     int stamp_ctr = 0;
+    struct Keyed { double key; int id; };
+    std::vector<Keyed> keyed;
     std::vector<int> out;
     static constexpr int kLeaf = 8;
 
@@ -64,10 +86,12 @@ struct ND {
         for (int a = 1; a < 3; ++a)
             if (hi[a] - lo[a] > hi[axis] - lo[axis]) axis = a;
         int half = cnt / 2;
-        std::nth_element(v.begin(), v.begin() + half, v.end(), [&](int i, int j) {
-            double a = xyz[3 * i + axis], b = xyz[3 * j + axis];
-            return a < b || (a == b && i < j);
+        keyed.resize(cnt);  // keys beside their vertices: the selection reads them in order
+        for (int k = 0; k < cnt; ++k) keyed[k] = {xyz[3 * v[k] + axis], v[k]};
+        std::nth_element(keyed.begin(), keyed.begin() + half, keyed.end(), [](const Keyed& i, const Keyed& j) {
+            return i.key < j.key || (i.key == j.key && i.id < j.id);
         });
+        for (int k = 0; k < cnt; ++k) v[k] = keyed[k].id;
         int st = ++stamp_ctr;
         for (int k = 0; k < cnt; ++k) { stamp[v[k]] = st; side[v[k]] = k < half ? 0 : 1; }
         // boundary of each side; the smaller one is the separator
@@ -196,36 +220,10 @@ void build_topology(int n, int F, const int* tri, const std::vector<int>& perm,
     for (int v : perm) { t.internal_of[v] = next; t.original_of[next] = v; ++next; }
     for (int v = 0; v < n; ++v)
         if (is_con[v]) { t.internal_of[v] = next; t.original_of[next] = v; ++next; }
-    // undirected edge list with the face edges that touch it (3f + k), in face order
-    std::vector<int64_t> key;
-    key.reserve((size_t)F * 3);
-    std::vector<int> fe_order;
-    for (int f = 0; f < F; ++f)
-        for (int k = 0; k < 3; ++k) {
-            int a = tri[3 * f + k], b = tri[3 * f + (k + 1) % 3];
-            if (a == b) { key.push_back(-1); continue; }
-            int lo = std::min(a, b), hi = std::max(a, b);
-            key.push_back((int64_t)lo * n + hi);
-        }
-    // CSR adjacency in original ids (ascending neighbour ids), with per-directed-edge face lists
-    std::vector<int> deg(n, 0);
-    std::vector<int64_t> ukeys;
-    ukeys.reserve(key.size());
-    for (int64_t k : key)
-        if (k >= 0) ukeys.push_back(k);
-    std::sort(ukeys.begin(), ukeys.end());
-    ukeys.erase(std::unique(ukeys.begin(), ukeys.end()), ukeys.end());
-    for (int64_t k : ukeys) { deg[k / n]++; deg[k % n]++; }
-    std::vector<int> rp(n + 1, 0);
-    for (int v = 0; v < n; ++v) rp[v + 1] = rp[v] + deg[v];
-    std::vector<int> ci(rp[n]);
-    std::vector<int> fill(rp.begin(), rp.end() - 1);
-    for (int64_t k : ukeys) {
-        int a = (int)(k / n), b = (int)(k % n);
-        ci[fill[a]++] = b;
-        ci[fill[b]++] = a;
-    }
-    for (int v = 0; v < n; ++v) std::sort(ci.begin() + rp[v], ci.begin() + rp[v + 1]);
+    // CSR adjacency in original ids (ascending neighbour ids)
+    std::vector<int> rp, ci, ident(n);
+    std::iota(ident.begin(), ident.end(), 0);
+    face_graph(F, tri, ident, n, rp, ci);
     // slices over internal ids
     t.nslices = (n + kSlice - 1) / kSlice;
     t.slice_ptr.assign(t.nslices + 1, 0);
@@ -263,31 +261,36 @@ void build_topology(int n, int F, const int* tri, const std::vector<int>& perm,
     }
     // face edges feeding each slot, in ascending face order (deterministic summation that
     // matches setFromTriplets' insertion order, arap.h:224-238)
-    std::vector<int> cnt(slots + 1, 0);
     auto csr_find = [&](int a, int b) {
-        auto it = std::lower_bound(ci.begin() + rp[a], ci.begin() + rp[a + 1], b);
-        return (int)(it - ci.begin());
+        int e = rp[a];
+        if (rp[a + 1] - e > 32) return (int)(std::lower_bound(ci.begin() + e, ci.begin() + rp[a + 1], b) - ci.begin());
+        while (ci[e] < b) ++e;
+        return e;
     };
-    std::vector<std::pair<int64_t, int>> pairs;
-    pairs.reserve((size_t)F * 6);
+    std::vector<int64_t> at;  // slots of the two directions of every face edge
+    at.reserve((size_t)F * 6);
+    t.slot_fe_ptr.assign(slots + 1, 0);
     for (int f = 0; f < F; ++f)
         for (int k = 0; k < 3; ++k) {
             int a = tri[3 * f + k], b = tri[3 * f + (k + 1) % 3];
             if (a == b) continue;
-            pairs.emplace_back(slot_of_csr[csr_find(a, b)], 3 * f + k);
-            pairs.emplace_back(slot_of_csr[csr_find(b, a)], 3 * f + k);
+            at.push_back(slot_of_csr[csr_find(a, b)]);
+            at.push_back(slot_of_csr[csr_find(b, a)]);
+            ++t.slot_fe_ptr[at[at.size() - 2] + 1];
+            ++t.slot_fe_ptr[at.back() + 1];
         }
-    std::stable_sort(pairs.begin(), pairs.end(),
-                     [](const std::pair<int64_t, int>& x, const std::pair<int64_t, int>& y) {
-                         return x.first < y.first;
-                     });
-    t.slot_fe_ptr.assign(slots + 1, 0);
-    t.slot_fe.resize(pairs.size());
-    for (size_t k = 0; k < pairs.size(); ++k) {
-        t.slot_fe_ptr[pairs[k].first + 1]++;
-        t.slot_fe[k] = pairs[k].second;
-    }
     for (int64_t s = 0; s < slots; ++s) t.slot_fe_ptr[s + 1] += t.slot_fe_ptr[s];
+    t.slot_fe.resize(at.size());
+    {
+        std::vector<int> next_of(t.slot_fe_ptr.begin(), t.slot_fe_ptr.end() - 1);
+        size_t q = 0;
+        for (int f = 0; f < F; ++f)
+            for (int k = 0; k < 3; ++k) {
+                if (tri[3 * f + k] == tri[3 * f + (k + 1) % 3]) continue;
+                t.slot_fe[next_of[at[q++]]++] = 3 * f + k;
+                t.slot_fe[next_of[at[q++]]++] = 3 * f + k;
+            }
+    }
     t.tri_internal.resize(3 * (size_t)F);
     for (size_t k = 0; k < 3 * (size_t)F; ++k) t.tri_internal[k] = t.internal_of[tri[k]];
 }
@@ -297,8 +300,10 @@ void build_topology(int n, int F, const int* tri, const std::vector<int>& perm,
 // Supernodes of at most this many columns always merge with their parent.
 constexpr int kAmalgSmall = 16;
 
-void symbolic(int n, const std::vector<int>& ptr, const std::vector<int>& adj, Factor& f, int sub_budget,
-              double amalg_ratio, const std::vector<int>* group) {
+namespace {
+// Supernodes (columns, off rows, children, heights) of the factor of this order.
+void supernodes(int n, const std::vector<int>& ptr, const std::vector<int>& adj, Factor& f,
+                double amalg_ratio, const std::vector<int>* group) {
     f = Factor();
     f.n = n;
     std::vector<int> ident(n);
@@ -339,10 +344,10 @@ void symbolic(int n, const std::vector<int>& ptr, const std::vector<int>& adj, F
     std::vector<std::vector<int>> rows(ns);
     std::vector<int> spar(ns, -1);
     std::vector<std::vector<int>> kids(ns);
-    std::vector<int> marker(n, -1);
+    std::vector<int> marker(n, -1), r;
     for (int s = 0; s < ns; ++s) {
         int lo = first[s], hi = first[s + 1];
-        std::vector<int>& r = rows[s];
+        r.clear();
         for (int j = lo; j < hi; ++j)
             for (int e = ptr[j]; e < ptr[j + 1]; ++e) {
                 int i = adj[e];
@@ -351,10 +356,10 @@ void symbolic(int n, const std::vector<int>& ptr, const std::vector<int>& adj, F
         for (int c : kids[s])
             for (int i : rows[c])
                 if (i >= hi && marker[i] != s) { marker[i] = s; r.push_back(i); }
-        std::sort(r.begin(), r.end());
         if (!r.empty()) {
-            spar[s] = sn_of[r[0]];
+            spar[s] = sn_of[*std::min_element(r.begin(), r.end())];
             kids[spar[s]].push_back(s);
+            rows[s] = r;
         }
     }
     // relaxed amalgamation: merge the last child into its parent when the panel grows little
@@ -414,7 +419,11 @@ void symbolic(int n, const std::vector<int>& ptr, const std::vector<int>& adj, F
     for (int t = 0; t < nn; ++t) f.roff[t + 1] += f.roff[t];
     f.offrows.resize(f.roff[nn]);
     for (int s = 0; s < ns; ++s)
-        if (alive[s]) std::copy(rows[s].begin(), rows[s].end(), f.offrows.begin() + f.roff[newid[s]]);
+        if (alive[s]) {
+            int* r = f.offrows.data() + f.roff[newid[s]];
+            std::copy(rows[s].begin(), rows[s].end(), r);
+            std::sort(r, r + rows[s].size());
+        }
     // children, heights
     f.child_ptr.assign(nn + 1, 0);
     for (int t = 0; t < nn; ++t)
@@ -433,6 +442,13 @@ void symbolic(int n, const std::vector<int>& ptr, const std::vector<int>& adj, F
             f.height[t] = std::max(f.height[t], f.height[f.child[k]] + 1);
         f.nlevels = std::max(f.nlevels, f.height[t] + 1);
     }
+}
+}  // namespace
+
+void symbolic(int n, const std::vector<int>& ptr, const std::vector<int>& adj, Factor& f, int sub_budget,
+              double amalg_ratio, const std::vector<int>* group) {
+    supernodes(n, ptr, adj, f, amalg_ratio, group);
+    const int nn = f.ns;
     // rel: position of each off row of t in its parent's row list [0, m_p)
     f.rel.assign(f.offrows.size(), -1);
     for (int t = 0; t < nn; ++t) {
@@ -477,11 +493,14 @@ void symbolic(int n, const std::vector<int>& ptr, const std::vector<int>& adj, F
     device_layout(f, sub_budget);
 }
 
-void device_layout(Factor& f, int sub_budget) {
-    const int n = f.n, nn = f.ns;
+namespace {
+// Bottom subtrees: maximal subtrees of small supernodes within the LDS budget (the root of each
+// supernode's, -1: none, and the sizes of the trees), and the levels of the others.
+void sweep_levels(Factor& f, int sub_budget, std::vector<int>& sub_root, std::vector<int>& size) {
+    const int nn = f.ns;
     auto cdiv = [](int a, int b) { return (a + b - 1) / b; };
-    // bottom subtrees: maximal subtrees of small supernodes within the LDS budget
-    std::vector<int> sub_root(nn, -1), size(nn, 1);
+    sub_root.assign(nn, -1);
+    size.assign(nn, 1);
     std::vector<int64_t> lds(nn, 0);
     std::vector<char> ok(nn, 0);
     // subtree records hold int offsets, and a partial count (< 2^15) with a stride (< 2^16)
@@ -521,6 +540,14 @@ void device_layout(Factor& f, int sub_budget) {
         f.level[t] = l;
         f.nlevels = std::max(f.nlevels, l + 1);
     }
+}
+}  // namespace
+
+void device_layout(Factor& f, int sub_budget) {
+    const int n = f.n, nn = f.ns;
+    auto cdiv = [](int a, int b) { return (a + b - 1) / b; };
+    std::vector<int> sub_root, size;
+    sweep_levels(f, sub_budget, sub_root, size);
     // device layout: tiles, partial vectors, bucket pointers, row locators
     f.pc_off.assign(nn + 1, 0); f.pr_off.assign(nn + 1, 0);
     f.xoff.assign(nn + 1, 0);
@@ -609,7 +636,7 @@ void device_layout(Factor& f, int sub_budget) {
     f.sub.clear(); f.sub_h.clear(); f.snode.clear(); f.scp.clear(); f.sfc.clear(); f.sbo.clear();
     f.srow.clear();
     f.sfi.assign(n, -1);
-    std::vector<int> fb(nn, 0);
+    std::vector<int> fb(nn, 0), lptr, lent, lfill;  // (a front position's child entries)
     for (int r = 0; r < nn; ++r) {
         if (sub_root[r] != r) continue;
         const int first = r - size[r] + 1, nh = f.height[r] + 1;
@@ -640,7 +667,6 @@ void device_layout(Factor& f, int sub_budget) {
         f.sub_nodes = std::max(f.sub_nodes, size[r]);
         f.sub_heights = std::max(f.sub_heights, nh);
         ++f.nsub;
-        std::vector<std::vector<int>> lists;
         for (int h = 0; h <= nh; ++h) {
             f.sub_h.push_back((int)(f.snode.size() / 16));
             if (h == nh) break;
@@ -653,20 +679,25 @@ void device_layout(Factor& f, int sub_budget) {
                 f.snode.insert(f.snode.end(), rec, rec + 16);
                 pa += m; pb += no; pq += w;
                 // children's update entries landing on each position, in child order
-                lists.assign(m, {});
+                lptr.assign(m + 1, 0);
+                for (int k = f.child_ptr[t]; k < f.child_ptr[t + 1]; ++k)
+                    for (int e = f.roff[f.child[k]]; e < f.roff[f.child[k] + 1]; ++e) ++lptr[f.rel[e] + 1];
+                for (int p = 0; p < m; ++p) lptr[p + 1] += lptr[p];
+                lent.resize(lptr[m]);
+                lfill.assign(lptr.begin(), lptr.end() - 1);
                 for (int k = f.child_ptr[t]; k < f.child_ptr[t + 1]; ++k) {
                     int c = f.child[k];
-                    for (int e = 0; e < f.noff[c]; ++e)
-                        lists[f.rel[f.roff[c] + e]].push_back(fb[c] + f.w[c] + e);
+                    for (int e = 0; e < f.noff[c]; ++e) lent[lfill[f.rel[f.roff[c] + e]]++] = fb[c] + f.w[c] + e;
                 }
                 for (int p = 0; p < m; ++p) {
-                    const std::vector<int>& L = lists[p];
-                    f.scp.push_back(L.size() > 0 ? L[0] : -1);
-                    if (L.size() <= 2) {
-                        f.scp.push_back(L.size() > 1 ? L[1] : -1);
+                    const int* L = lent.data() + lptr[p];
+                    const int ln = lptr[p + 1] - lptr[p];
+                    f.scp.push_back(ln > 0 ? L[0] : -1);
+                    if (ln <= 2) {
+                        f.scp.push_back(ln > 1 ? L[1] : -1);
                     } else {
                         f.scp.push_back(-2 - (int)f.sfc.size());
-                        f.sfc.insert(f.sfc.end(), L.begin() + 1, L.end());
+                        f.sfc.insert(f.sfc.end(), L + 1, L + ln);
                         f.sfc.push_back(-1);
                     }
                 }
@@ -704,7 +735,11 @@ std::vector<int> pair_levels(const std::vector<int>& order, const std::vector<in
         p2[k + 1] = (int)a2.size();
     }
     Factor f;
-    symbolic(m, p2, a2, f, sub_budget, amalg_ratio);
+    supernodes(m, p2, a2, f, amalg_ratio, nullptr);
+    {
+        std::vector<int> sub_root, size;
+        sweep_levels(f, sub_budget, sub_root, size);
+    }
     const int ns = f.ns, top = f.nlevels - 1;
     if (top < 0) return order;
     // the top levels [cut, top] of at most top_columns columns together, or all of a small system. Below

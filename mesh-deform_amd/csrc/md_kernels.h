@@ -60,7 +60,6 @@ struct MeshDev {
     MD_G void *quat;            // rotations as quaternions (x, y, z, w=scalar): f4 or d4
     MD_G void *r, *z;           // residual and forward result (V4 of the solve type), nf each
     MD_G void *upart, *xpart;   // update slots of the level fronts / partial solutions (V4)
-    const MD_G int *child_ptr, *child;
     const MD_G long long *udst; // per off-row entry of a level supernode or subtree root: its
                                 //   update slot in the parent's front (partial cb: + cb * dstride)
     const MD_G int4 *rowinfo;   // per row: (first partial, stride, count, 0)
