@@ -109,6 +109,9 @@ struct FacChild {
     long long uoff;
 };
 
+// Words of the factorization that start at zero: partial maxima of |L_ii| (256 bytes apart: atomics on
+// one line follow one another), then the flag.
+constexpr int kFacMaxima = 8, kFacMaxStride = 32, kFacWords = kFacMaxima * kFacMaxStride + 1;
 struct FacArgs {
     const MD_G FacDev *sn;          // by height
     const MD_G FacChild *child;
@@ -117,11 +120,11 @@ struct FacArgs {
     const MD_G double *w64;         // cotan weights over the one-ring slots
     int nf;
     MD_G double *P, *S, *T, *U, *diag;
-    MD_G unsigned long long *amax;  // max |L_ii| as the bits of a non-negative double
+    MD_G unsigned long long *amax;  // max |L_ii| as the bits of a non-negative double, in kFacMaxima parts
     MD_G int *flag;                 // 1: a pivot block is not positive definite; 2: structure
     MD_G void *pc, *pr;             // the sweeps' panels (float or double), written in the solve
     int solve64;                    //   precision (1: double)
-    unsigned long long *stamp;      // clock at the start (may be null)
+    unsigned long long *stamp;      // clock at the first height (may be null)
 };
 
 // A set of meshes processed by one launch. Block b belongs to mesh k where
@@ -137,7 +140,8 @@ struct LaunchSet {
 
 // Launchers (grid = total blocks of the launch, from the host-side prefix table).
 void launch_cotan_face(hipStream_t s, LaunchSet L, int blocks);
-void launch_cotan_slot(hipStream_t s, LaunchSet L, int blocks);
+// One mesh, a block per slice; diag, amax: L_ii of the free vertices and their maxima (may be null).
+void launch_cotan_slot(hipStream_t s, LaunchSet L, int blocks, double *diag, unsigned long long *amax);
 void launch_local(hipStream_t s, LaunchSet L, int blocks, bool fp64);
 void launch_residual(hipStream_t s, LaunchSet L, int blocks, bool fp64);
 void launch_fwd(hipStream_t s, LaunchSet L, int blocks, int level, bool fp64);
@@ -179,7 +183,6 @@ void launch_pcg_apply(hipStream_t s, LaunchSet L, int blocks, bool fp64);
 // Device numeric factorization: diagonal and its maximum, then per height (the `count`
 // supernodes from sn[h0]) the front assembly and the block sweeps, whose last step writes D^{-1} and G
 // to the solve-precision panels.
-void launch_fac_diag(hipStream_t s, const FacArgs &A);
 // The assembly of a height of `count` fronts of at most mm rows, at most `no` of them off rows, with
 // at most `maps` = children x rows of one front: `per` workgroups per front, each `cols` columns by one
 // of rch ranges of rlen rows. 64 columns, halved down to 4 (one quad for the four wavefronts) while

@@ -94,31 +94,82 @@ __global__ __launch_bounds__(kBlock) void k_cotan_face(LaunchSet L) {
     M.fe_val[3 * f + 2] = ref_max(1e-10, cot2) * 0.5;
 }
 
-// One lane per vertex, one wavefront per 64-vertex slice: each slot sums its face-edge
-// contributions in face order (setFromTriplets' duplicate sum, arap.h:224,238) and stores
-// w_ij and the weighted rest edge a_ij = w_ij (p_i - p_j) in FP64 and FP32.
-__global__ __launch_bounds__(kBlock) void k_cotan_slot(LaunchSet L) {
-    int k = find_mesh(L, blockIdx.x);
+// One workgroup per 64-vertex slice, its slots dealt to the wavefronts column by column, four in
+// flight each: a slot sums its face-edge contributions in face order (setFromTriplets' duplicate
+// sum, arap.h:224,238) and stores w_ij and the weighted rest edge a_ij = w_ij (p_i - p_j) in FP64 and
+// FP32. With diag, the weights also pass through LDS to the first wavefront, which sums each free
+// vertex' in slot order (L_ii, arap.h:332) and the largest into amax (bits of a non-negative double; one
+// address for all slices takes 12 ns per atomic, 25 us on the 164k icosphere).
+// Bound by round trips per slot (face list, values, neighbour), so a lane taking a vertex' slots one after
+// another took 59 us on a UV sphere of 3,202 with poles of 80 neighbours, and 37 on the 164k
+// icosphere; the diagonal was a launch of its own (6 and 32 us, one atomic per vertex).
+// Now 29 and 34 us, 7 on a sphere of 642 (10 and 6 for the diagonal).
+constexpr int kCotSlots = 8;  // slot columns per round of a workgroup
+__global__ __launch_bounds__(kBlock) void k_cotan_slot(LaunchSet L, double *diag, unsigned long long *amax) {
+    __shared__ double wsh[kCotSlots][kSlice];
+    const int k = find_mesh(L, blockIdx.x);
     const MD_G MeshDev &M = L.meshes[k];
-    int slice = (blockIdx.x - L.prefix[k]) * kSlicesPerBlock + (threadIdx.x >> 6);
-    int lane = threadIdx.x & 63;
-    if (slice >= M.nslices) return;
-    int iv = slice * kSlice + lane;
-    int s0 = M.slice_ptr[slice], wd = M.slice_ptr[slice + 1] - s0;
-    d4 pi = M.p[iv < M.n ? iv : 0];
-    for (int q = 0; q < wd; ++q) {
-        long long g = (long long)(s0 + q) * kSlice + lane;
-        double w = 0.0;
-        for (int e = M.slot_fe_ptr[g]; e < M.slot_fe_ptr[g + 1]; ++e) w += M.fe_val[M.slot_fe[e]];
-        int j = M.sell_col[g];
-        d4 pj = M.p[j];
-        double ax = w * (pi.x - pj.x), ay = w * (pi.y - pj.y), az = w * (pi.z - pj.z);
-        if (iv >= M.n) { w = 0.0; ax = ay = az = 0.0; }
-        M.w64[g] = w;
-        M.w32[g] = (float)w;
-        M.a64[g] = ax; M.a64[M.slots + g] = ay; M.a64[2 * M.slots + g] = az;
-        M.a32[g] = (float)ax; M.a32[M.slots + g] = (float)ay; M.a32[2 * M.slots + g] = (float)az;
+    const int slice = blockIdx.x - L.prefix[k], lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int iv = slice * kSlice + lane;
+    const int s0 = M.slice_ptr[slice], wd = M.slice_ptr[slice + 1] - s0;
+    const d4 pi = M.p[iv < M.n ? iv : 0];
+    double acc = 0.0;
+    for (int q0 = 0; q0 < wd; q0 += kCotSlots) {
+        constexpr int kWaves = kBlock / 64, kU = kCotSlots / kWaves;
+        int j[kU], e0[kU], e1[kU], f0[kU], f1[kU];
+        d4 pj[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const int q = q0 + u * kWaves + wave;
+            j[u] = e0[u] = e1[u] = 0;
+            if (q < wd) {
+                const long long g = (long long)(s0 + q) * kSlice + lane;
+                j[u] = M.sell_col[g];
+                e0[u] = M.slot_fe_ptr[g];
+                e1[u] = M.slot_fe_ptr[g + 1];
+            }
+        }
+        // the first two face edges of every slot (all of an ordinary one's) at once
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            f0[u] = e1[u] > e0[u] ? M.slot_fe[e0[u]] : -1;
+            f1[u] = e1[u] > e0[u] + 1 ? M.slot_fe[e0[u] + 1] : -1;
+            if (q0 + u * kWaves + wave < wd) pj[u] = M.p[j[u]];
+        }
+        double w[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const double a = f0[u] >= 0 ? M.fe_val[f0[u]] : 0.0, b = f1[u] >= 0 ? M.fe_val[f1[u]] : 0.0;
+            w[u] = (0.0 + a) + b;
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const int q = q0 + u * kWaves + wave;
+            if (q >= wd) break;
+            for (int e = e0[u] + 2; e < e1[u]; ++e) w[u] += M.fe_val[M.slot_fe[e]];
+            double ax = w[u] * (pi.x - pj[u].x), ay = w[u] * (pi.y - pj[u].y), az = w[u] * (pi.z - pj[u].z);
+            if (iv >= M.n) { w[u] = 0.0; ax = ay = az = 0.0; }
+            wsh[q - q0][lane] = j[u] == iv ? 0.0 : w[u];
+            const long long g = (long long)(s0 + q) * kSlice + lane;
+            M.w64[g] = w[u];
+            M.w32[g] = (float)w[u];
+            M.a64[g] = ax; M.a64[M.slots + g] = ay; M.a64[2 * M.slots + g] = az;
+            M.a32[g] = (float)ax; M.a32[M.slots + g] = (float)ay; M.a32[2 * M.slots + g] = (float)az;
+        }
+        if (!diag) continue;
+        __syncthreads();
+        if (wave == 0)
+            for (int q = 0; q < min(kCotSlots, wd - q0); ++q) acc += wsh[q][lane];
+        __syncthreads();
     }
+    if (!diag || wave != 0) return;
+    const bool free_row = iv < M.nf;
+    if (free_row) diag[iv] = acc;
+    unsigned long long top = free_row ? (unsigned long long)__double_as_longlong(fabs(acc)) : 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) top = max(top, (unsigned long long)__shfl_xor(top, o));
+    if (lane == 0) atomicMax(amax + slice % kFacMaxima * kFacMaxStride, top);
 }
 
 // ---- local step (arap.h:354-384) ----------------------------------------------------------
@@ -1543,12 +1594,13 @@ __global__ __launch_bounds__(kBlock) void k_energy(LaunchSet L) {
 // The caller's packed xyz (original order, read in order: it may be pinned host memory) into
 // internal order: p[iv] (may be null), and pp[iv] (may be null) the same for free vertices, the constrained
 // ones (iv >= nf) taking their targets tgt[iv - nf] instead; with pp, identity rotations (arap.h:246-249).
-// Thread 0 clears `clear` (two words) and writes the clock to `stamp` (each may be null).
+// The first block clears `clear` (kFacWords) and thread 0 writes the clock to `stamp` (each may be null).
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_unpack_xyz(UnpackArgs a) {
     using V = typename V4T<T>::type;
     const int v = blockIdx.x * kBlock + threadIdx.x;
-    if (v == 0 && a.clear) a.clear[0] = a.clear[1] = 0;
+    if (a.clear && blockIdx.x == 0)
+        for (int i = v; i < kFacWords; i += kBlock) a.clear[i] = 0;
     if (v == 0 && a.stamp) *a.stamp = wall_clock64();
     if (v >= a.n) return;
     const int iv = a.internal[v];
@@ -1588,6 +1640,14 @@ __global__ __launch_bounds__(kBlock) void k_scatter_entries(const TargetEntry *e
 
 constexpr int kFacBlock = 256;
 
+// Least pivot: 1e-14 of the largest diagonal entry.
+__device__ __forceinline__ double pivot_floor(const FacArgs &A) {
+    unsigned long long m = 0;
+#pragma unroll
+    for (int i = 0; i < kFacMaxima; ++i) m = max(m, A.amax[i * kFacMaxStride]);
+    return 1e-14 * __longlong_as_double((long long)m);
+}
+
 constexpr int kFb = 64;  // columns of a pivot block swept at a time
 
 
@@ -1603,21 +1663,6 @@ struct FrontBuf {
 __device__ __forceinline__ FrontBuf front_buf(const FacArgs &A, const FacDev &S, int s) {
     if (s & 1) return FrontBuf{A.T + S.toff, A.S + S.soff, S.w, S.noff};
     return FrontBuf{A.P + S.poff, A.P + S.poff + S.w, S.m, S.m};
-}
-
-// L_jj = sum of the weights of every neighbour of j, in slot order, and their maximum.
-__global__ __launch_bounds__(kBlock) void k_fac_diag(FacArgs A) {
-    const int j = blockIdx.x * kBlock + threadIdx.x;
-    if (j == 0 && A.stamp) *A.stamp = wall_clock64();
-    if (j >= A.nf) return;
-    const int sl = j / kSlice, l = j % kSlice;
-    double acc = 0.0;
-    for (int q = A.slice_ptr[sl]; q < A.slice_ptr[sl + 1]; ++q) {
-        const long long g = (long long)q * kSlice + l;
-        if (A.sell_col[g] != j) acc += A.w64[g];
-    }
-    A.diag[j] = acc;
-    atomicMax(A.amax, (unsigned long long)__double_as_longlong(fabs(acc)));
 }
 
 // Front of each supernode of one height: its first w columns and the update matrix, lower part: for
@@ -1640,6 +1685,7 @@ constexpr int kAsmBatch = 64;  // children whose maps are inverted at a time (on
 __global__ __launch_bounds__(kFacBlock) void k_fac_assemble(FacArgs A, int h0, FacAssembly as) {
     const FacDev S = A.sn[h0 + blockIdx.x / as.per];
     const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, w = S.w, no = S.noff, m = S.m;
+    if (A.stamp && h0 == 0 && blockIdx.x == 0 && tid == 0) *A.stamp = wall_clock64();
     const int part = (int)(blockIdx.x % as.per), t0 = part / as.rch * as.cols, t1 = min(m, t0 + as.cols);
     const int r0 = max(t0, part % as.rch * as.rlen), r1 = min(m, (part % as.rch + 1) * as.rlen), len = r1 - r0;
     if (t0 >= m || len <= 0) return;
@@ -2006,7 +2052,7 @@ __device__ __forceinline__ void invert64(const double *m, InvLds &work, int b, d
 __device__ __forceinline__ void pivot_inverse(const FacArgs &A, const FacDev &S, int s, const double *m, InvLds &work,
                                               const FrontBuf &out) {
     const int kb = s * kFb, b = min(kFb, S.w - kb);
-    const double thr = 1e-14 * __longlong_as_double((long long)*A.amax);
+    const double thr = pivot_floor(A);
     dv4 acc[4];
     bool bad = false;
     invert64(m, work, b, thr, acc, bad);
@@ -2299,6 +2345,7 @@ template <int BLOCK, int NB>
 __global__ __launch_bounds__(BLOCK) void k_fac_small(FacArgs A, int h0) {
     const FacDev S = A.sn[h0 + blockIdx.x];
     const int tid = threadIdx.x, w = S.w, no = S.noff, m = S.m;
+    if (A.stamp && h0 == 0 && blockIdx.x == 0 && tid == 0) *A.stamp = wall_clock64();
     if (m > kIb * NB) {  // the host sends only small fronts
         if (tid == 0) *A.flag = 2;
         return;
@@ -2385,7 +2432,7 @@ __global__ __launch_bounds__(BLOCK) void k_fac_small(FacArgs A, int h0) {
     }
     __syncthreads();
     if (tid < 64) {
-        const double thr = 1e-14 * __longlong_as_double((long long)*A.amax);
+        const double thr = pivot_floor(A);
         bool bad;
         if (narrow) bad = small_front<2 < NB ? 2 : NB, LD>(Fs, w, thr);
         else bad = small_front<NB, LD>(Fs, w, thr);
@@ -2422,9 +2469,6 @@ __global__ __launch_bounds__(kBlock) void k_copy_probe(const f4 *__restrict__ sr
 
 }  // namespace
 
-void launch_fac_diag(hipStream_t s, const FacArgs &A) {
-    if (A.nf > 0) hipLaunchKernelGGL(k_fac_diag, dim3((A.nf + kBlock - 1) / kBlock), dim3(kBlock), 0, s, A);
-}
 template <int BLOCK>
 static void fac_small_of(hipStream_t s, const FacArgs &A, int h0, int count, int mm) {
     const dim3 grid(count), block(BLOCK);
@@ -2496,8 +2540,8 @@ void launch_scatter_entries(hipStream_t s, const TargetEntry *e, int k) {
 void launch_cotan_face(hipStream_t s, LaunchSet L, int blocks) {
     if (blocks > 0) hipLaunchKernelGGL(k_cotan_face, dim3(blocks), dim3(kBlock), 0, s, L);
 }
-void launch_cotan_slot(hipStream_t s, LaunchSet L, int blocks) {
-    if (blocks > 0) hipLaunchKernelGGL(k_cotan_slot, dim3(blocks), dim3(kBlock), 0, s, L);
+void launch_cotan_slot(hipStream_t s, LaunchSet L, int blocks, double *diag, unsigned long long *amax) {
+    if (blocks > 0) hipLaunchKernelGGL(k_cotan_slot, dim3(blocks), dim3(kBlock), 0, s, L, diag, amax);
 }
 void launch_local(hipStream_t s, LaunchSet L, int blocks, bool fp64) {
     if (blocks <= 0) return;

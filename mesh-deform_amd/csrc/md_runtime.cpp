@@ -803,7 +803,7 @@ static size_t pin_chunk(size_t bytes) {
 // Uploads the caller's positions (original order, 3 per vertex) and spreads them to internal
 // order on the device: into p (rest, may be null) and pp (current positions with the targets
 // of the constrained vertices pasted, and identity rotations; may be null). Stream-ordered, no
-// synchronisation: xyz and the block must stay until the stream has passed. clear: two words of
+// synchronisation: xyz and the block must stay until the stream has passed. clear: kFacWords of
 // device memory to clear (may be null).
 hipError_t upload_positions(md_mesh *m, const double *xyz, d4 *p, d4 *pp, CallSlot &slot,
                             unsigned long long *clear = nullptr) {
@@ -903,11 +903,13 @@ int no_slot(const char *who) {
     return MD_ERR_NOMEM;
 }
 
-hipError_t compute_cotan(md_mesh *m) {
+// Cotan weights; with words (fac_ws_words), also the diagonal and its maximum for the factorization.
+hipError_t compute_cotan(md_mesh *m, unsigned long long *words) {
     const Plan &P = m->plan;
     hipStream_t st = m->ctx->stream;
     launch_cotan_face(st, P.set(P.off_face), P.blk_face);
-    launch_cotan_slot(st, P.set(P.off_slice), P.blk_slice);
+    launch_cotan_slot(st, P.set(P.off_slice), m->topo.nslices,
+                      words ? reinterpret_cast<double *>(words) - m->topo.nf : nullptr, words);
     return hipGetLastError();
 }
 
@@ -985,23 +987,38 @@ bool factor_host(md_mesh *m, std::string &err) {
     return true;
 }
 
-// Bytes of the FP64 workspace of the device factorization, and its two words that start at
-// zero (the largest |L_ii|, the flag) when the workspace is there.
+// Bytes of the FP64 workspace of the device factorization, and its kFacWords that start at
+// zero (maxima of |L_ii|, the flag) when the workspace is there.
 size_t fac_ws_size(const md_mesh *m) {
     const Factor &f = m->fac;
     const size_t entries = (size_t)f.poff[f.ns] + (size_t)f.woff_s[f.ns] + (size_t)f.woff_t[f.ns] + (size_t)f.woff_u[f.ns];
-    return sizeof(double) * (entries + (size_t)m->topo.nf) + 2 * sizeof(unsigned long long);
+    return sizeof(double) * (entries + (size_t)m->topo.nf) + kFacWords * sizeof(unsigned long long);
 }
 unsigned long long *fac_ws_words(const md_mesh *m) {
     if (!m->fac_ws || m->fac_ws_bytes != fac_ws_size(m)) return nullptr;
-    return reinterpret_cast<unsigned long long *>(static_cast<char *>(m->fac_ws) + m->fac_ws_bytes) - 2;
+    return reinterpret_cast<unsigned long long *>(static_cast<char *>(m->fac_ws) + m->fac_ws_bytes) - kFacWords;
+}
+
+// The workspace of the coming device factorization, allocated unless kept from the last one.
+int fac_ws_ready(md_mesh *m) {
+    const size_t bytes = fac_ws_size(m);
+    if (m->fac_ws && m->fac_ws_bytes != bytes) m->release_fac_ws();
+    if (m->fac_ws) return MD_OK;
+    if (hipMalloc(&m->fac_ws, bytes) != hipSuccess) {
+        m->fac_ws = nullptr;
+        set_error("device factorization workspace of " + std::to_string(bytes) + " bytes: allocation failed");
+        return MD_ERR_NOMEM;
+    }
+    m->fac_ws_bytes = bytes;
+    return MD_OK;
 }
 
 // FP64 numeric factorization on the device from the device cotan weights, straight into
-// the sweeps' panels: diagonal, then per height of the supernodal tree the front assembly and
+// the sweeps' panels: per height of the supernodal tree the front assembly and
 // the dense partial factorization, then the conversion to the solve precision. Only queued:
-// factor_finish looks at the flag once the stream has passed. cleared: the two words are zero already.
-int factor_device(md_mesh *m, CallSlot &slot, bool cleared) {
+// factor_finish looks at the flag once the stream has passed. The workspace is there (fac_ws_ready) and
+// holds the diagonal and its maximum (compute_cotan).
+int factor_device(md_mesh *m, CallSlot &slot) {
     const Factor &f = m->fac;
     const int ns = f.ns, nf = m->topo.nf;
     hipStream_t st = m->ctx->stream;
@@ -1034,16 +1051,6 @@ int factor_device(md_mesh *m, CallSlot &slot, bool cleared) {
     }
     const size_t nP = (size_t)f.poff[ns], nS = (size_t)f.woff_s[ns], nT = (size_t)f.woff_t[ns],
                  nU = (size_t)f.woff_u[ns];
-    const size_t bytes = fac_ws_size(m);
-    if (m->fac_ws && m->fac_ws_bytes != bytes) m->release_fac_ws();
-    if (!m->fac_ws) {
-        if (hipMalloc(&m->fac_ws, bytes) != hipSuccess) {
-            m->fac_ws = nullptr;
-            set_error("device factorization workspace of " + std::to_string(bytes) + " bytes: allocation failed");
-            return MD_ERR_NOMEM;
-        }
-        m->fac_ws_bytes = bytes;
-    }
     void *ws = m->fac_ws;
     FacArgs A{};
     A.sn = m->d_fac; A.child = m->d_fchild; A.offrows = m->d_offrows; A.rel = m->d_rel;
@@ -1051,25 +1058,20 @@ int factor_device(md_mesh *m, CallSlot &slot, bool cleared) {
     double *base = static_cast<double *>(ws);
     A.P = base; A.S = A.P + nP; A.T = A.S + nS; A.U = A.T + nT; A.diag = A.U + nU;
     A.amax = fac_ws_words(m);
-    A.flag = reinterpret_cast<int *>(A.amax + 1);
+    A.flag = reinterpret_cast<int *>(A.amax + kFacWords - 1);
     A.pc = const_cast<void *>(m->dev.pc);
     A.pr = const_cast<void *>(m->dev.pr);
     A.solve64 = m->fp64() ? 1 : 0;
     A.stamp = &slot.head()->stamp[1];
     slot.queued = true;
-    hipError_t e = cleared ? hipSuccess : hipMemsetAsync(A.amax, 0, 2 * sizeof(unsigned long long), st);
-    if (e == hipSuccess) {
-        launch_fac_diag(st, A);
-        for (int h = 0; h < nh; ++h) {
-            const HeightLaunch &L = hl[h];
-            if (L.small > 0) launch_fac_small(st, A, f.hptr[h], L.small, L.sm);
-            launch_fac_height(st, A, f.hptr[h] + L.small, L.count, (L.mw + 63) / 64,
-                              fac_assembly(L.count, L.mm, L.mo, L.maps), L.tiles);
-        }
-        launch_publish(st, &slot.head()->stamp[2], A.flag, &slot.head()->flag);
-        e = hipGetLastError();
+    for (int h = 0; h < nh; ++h) {
+        const HeightLaunch &L = hl[h];
+        if (L.small > 0) launch_fac_small(st, A, f.hptr[h], L.small, L.sm);
+        launch_fac_height(st, A, f.hptr[h] + L.small, L.count, (L.mw + 63) / 64,
+                          fac_assembly(L.count, L.mm, L.mo, L.maps), L.tiles);
     }
-    if (e != hipSuccess) {
+    launch_publish(st, &slot.head()->stamp[2], A.flag, &slot.head()->flag);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) {
         slot.wait();
         m->release_fac_ws();
         set_error(std::string("device factorization: ") + hipGetErrorString(e));
@@ -1117,7 +1119,7 @@ int factor_upload(md_mesh *m) {
 struct Prep {
     const double *xyz = nullptr;
     bool full = false, need_analysis = false, need_factor = false, early = false;
-    bool cleared = false;        // the factorization's two words
+    bool weights_later = false;  // the cotan weights wait for the factorization's workspace
     Clock::time_point uploaded;  // when the upload was queued
 };
 
@@ -1142,8 +1144,10 @@ int prep_device_a(md_mesh *m, Prep &p, CallSlot &slot) {
     }
     const bool device = m->cfg.solver == MD_SOLVER_LDLT && m->cfg.factor_device;
     const bool factor = m->ncon > 0 && m->topo.nf > 0 && (p.full || p.need_analysis || !m->factored);
+    // the diagonal goes into the factorization's workspace: without one yet, the weights are left to
+    // prep_device_b (which runs mesh after mesh, so that workspaces that are not kept never add up)
     unsigned long long *words = factor && device ? fac_ws_words(m) : nullptr;
-    p.cleared = words && m->n > 0;
+    p.weights_later = factor && device && !words;
     hipError_t e = hipSuccess;
     // rest pose (when it changes) and the initial guess: the current mesh with the targets
     // pasted (arap.h:162-168, 277-281); in reference rest mode both come from the same upload
@@ -1153,12 +1157,13 @@ int prep_device_a(md_mesh *m, Prep &p, CallSlot &slot) {
         if (e == hipSuccess) e = upload_positions(m, p.xyz, nullptr, m->dev.pp, slot, words);
     }
     p.uploaded = Clock::now();
-    if (e == hipSuccess && (p.full || p.need_analysis)) {
-        e = compute_cotan(m);
-        if (e != hipSuccess) { set_error(std::string("cotan weights: ") + hipGetErrorString(e)); return MD_ERR_HIP; }
-    }
     m->initialized = true;
     m->iterated = false;
+    // (a factorization of weights that stand, after one that failed, computes them again for their diagonal)
+    if (e == hipSuccess && !p.weights_later && (p.full || p.need_analysis || words)) {
+        e = compute_cotan(m, words);
+        if (e != hipSuccess) { set_error(std::string("cotan weights: ") + hipGetErrorString(e)); return MD_ERR_HIP; }
+    }
     p.early = m->ncon == 0;  // arap.h:113-114
     p.need_factor = factor;
     if (e == hipSuccess && p.early) e = slot.wait();
@@ -1171,7 +1176,16 @@ int prep_device_a(md_mesh *m, Prep &p, CallSlot &slot) {
 int prep_device_b(md_mesh *m, Prep &p, CallSlot &slot) {
     if (!p.need_factor) return MD_OK;
     const bool pcg = m->cfg.solver == MD_SOLVER_PCG;
-    if (!pcg && m->cfg.factor_device) return factor_device(m, slot, p.cleared);
+    if (!pcg && m->cfg.factor_device) {
+        if (p.weights_later) {
+            if (int rc = fac_ws_ready(m)) return rc;
+            unsigned long long *words = fac_ws_words(m);
+            hipError_t e = hipMemsetAsync(words, 0, kFacWords * sizeof(*words), m->ctx->stream);
+            if (e == hipSuccess) e = compute_cotan(m, words);
+            if (e != hipSuccess) { set_error(std::string("cotan weights: ") + hipGetErrorString(e)); return MD_ERR_HIP; }
+        }
+        return factor_device(m, slot);
+    }
     if (int rc = pcg ? factor_pcg(m, slot) : factor_upload(m)) return rc;
     slot.queued = true;
     launch_publish(m->ctx->stream, &slot.head()->stamp[2], nullptr, nullptr);
