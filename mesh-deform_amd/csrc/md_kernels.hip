@@ -172,6 +172,67 @@ __global__ __launch_bounds__(kBlock) void k_cotan_slot(LaunchSet L, double *diag
     if (lane == 0) atomicMax(amax + slice % kFacMaxima * kFacMaxStride, top);
 }
 
+// Lane moves inside a row of 16 lanes (DPP control CTRL).
+template <int CTRL> __device__ __forceinline__ float dpp_move(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+template <int CTRL> __device__ __forceinline__ double dpp_move(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)u, CTRL, 0xF, 0xF, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), CTRL, 0xF, 0xF, true);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+// v + the value of the other row of each pair (Half: of the other half of the wavefront).
+template <bool Half> __device__ __forceinline__ void rows_swap(unsigned u, unsigned (&o)[2]) {
+    if constexpr (Half) {
+        const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        o[0] = a[0]; o[1] = a[1];
+    } else {
+        const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        o[0] = a[0]; o[1] = a[1];
+    }
+}
+template <bool Half> __device__ __forceinline__ float rows_sum(float v) {
+    unsigned a[2];
+    rows_swap<Half>(__builtin_bit_cast(unsigned, v), a);
+    return __builtin_bit_cast(float, a[0]) + __builtin_bit_cast(float, a[1]);
+}
+template <bool Half> __device__ __forceinline__ double rows_sum(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    unsigned lo[2], hi[2];
+    rows_swap<Half>((unsigned)u, lo);
+    rows_swap<Half>((unsigned)(u >> 32), hi);
+    return __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]) +
+           __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
+}
+// Sum over the wavefront, in every lane (quads, half rows, rows, row pairs, halves).
+template <typename T> __device__ __forceinline__ T wave_sum(T v) {
+    v += dpp_move<0xB1>(v);
+    v += dpp_move<0x4E>(v);
+    v += dpp_move<0x141>(v);
+    v += dpp_move<0x140>(v);
+    v = rows_sum<false>(v);
+    return rows_sum<true>(v);
+}
+// v of lane l (the same l in every lane).
+__device__ __forceinline__ double lane_value(double v, int l) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, l);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), l);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// One-rings longer than kRingSlots: where at most kFewLong lanes of a wavefront have one (a pole among
+// vertices of six neighbours), the wavefront takes their remaining slots together, a lane per slot, one
+// long ring after another: a round trip and nine sums (about 1.2 us) each, where every eight slots of
+// a ring are a round trip of the whole wavefront otherwise (the rotations of a UV sphere of 3,202 with poles
+// of 80 neighbours: 16 -> 8 us).
+constexpr int kRingSlots = 16, kFewLong = 4;
+// Lanes whose one-ring (wd > kRingSlots slots from s0; vertex iv) goes on past kRingSlots.
+__device__ __forceinline__ unsigned long long long_rings(const MD_G MeshDev &M, bool live, int iv, int s0) {
+    return __ballot(live && M.sell_col[(long long)(s0 + kRingSlots) * kSlice + iv % kSlice] != iv);
+}
+
 // ---- local step (arap.h:354-384) ----------------------------------------------------------
 
 // One Jacobi rotation of the symmetric 4x4 matrix a on the pair (P, Q); v accumulates the
@@ -413,16 +474,24 @@ __global__ __launch_bounds__(kBlock) void k_local(LaunchSet L) {
     int slice = (blockIdx.x - L.prefix[k]) * kSlicesPerBlock + (threadIdx.x >> 6);
     int lane = threadIdx.x & 63;
     if (slice >= M.nslices) return;
-    int iv = slice * kSlice + lane;
-    if (iv >= M.n) return;
+    const int iv = min(slice * kSlice + lane, M.n - 1);  // (the last slice's spare lanes help with long rings)
+    const bool live = slice * kSlice + lane < M.n;
     const T *A = aplanes<T>(M);
     int s0 = M.slice_ptr[slice], wd = M.slice_ptr[slice + 1] - s0;
-    d4 pi = M.pp[iv];
+    const d4 pi = M.pp[iv];
+    const V prev = reinterpret_cast<const V *>(M.quat)[iv];  // (early: its latency is hidden)
     T c[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    auto add = [&](T (&o)[9], T ax, T ay, T az, T ex, T ey, T ez) {
+        o[0] += ax * ex; o[1] += ax * ey; o[2] += ax * ez;
+        o[3] += ay * ex; o[4] += ay * ey; o[5] += ay * ez;
+        o[6] += az * ex; o[7] += az * ey; o[8] += az * ez;
+    };
     // 8 slots at a time: ids and edges first, then the neighbour gathers, then arithmetic
     // (slots past the slice width are clamped; they are padding with zero edges anyway)
     constexpr int kU = 8;
-    for (int q0 = 0; q0 < wd; q0 += kU) {
+    unsigned long long far = wd > kRingSlots ? long_rings(M, live, iv, s0) : 0;
+    if (__popcll(far) > kFewLong) far = 0;
+    for (int q0 = 0, end = far ? kRingSlots : wd; q0 < end; q0 += kU) {
         int jj[kU];
         T ex_[kU], ey_[kU], ez_[kU];
 #pragma unroll
@@ -438,16 +507,26 @@ __global__ __launch_bounds__(kBlock) void k_local(LaunchSet L) {
 #pragma unroll
         for (int u = 0; u < kU; ++u) pj[u] = M.pp[jj[u]];
 #pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            T ax = ex_[u], ay = ey_[u], az = ez_[u];
-            T ex = (T)(pi.x - pj[u].x), ey = (T)(pi.y - pj[u].y), ez = (T)(pi.z - pj[u].z);
-            c[0] += ax * ex; c[1] += ax * ey; c[2] += ax * ez;
-            c[3] += ay * ex; c[4] += ay * ey; c[5] += ay * ez;
-            c[6] += az * ex; c[7] += az * ey; c[8] += az * ez;
+        for (int u = 0; u < kU; ++u)
+            add(c, ex_[u], ey_[u], ez_[u], (T)(pi.x - pj[u].x), (T)(pi.y - pj[u].y), (T)(pi.z - pj[u].z));
+    }
+    for (; far; far &= far - 1) {
+        const int l = __ffsll(far) - 1;
+        const double px = lane_value(pi.x, l), py = lane_value(pi.y, l), pz = lane_value(pi.z, l);
+        T o[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+        for (int q = kRingSlots + lane; q < wd; q += 64) {
+            const long long g = (long long)(s0 + q) * kSlice + l;
+            const d4 pj = M.pp[M.sell_col[g]];
+            add(o, A[g], A[M.slots + g], A[2 * M.slots + g], (T)(px - pj.x), (T)(py - pj.y), (T)(pz - pj.z));
+        }
+#pragma unroll
+        for (int e = 0; e < 9; ++e) {
+            const T sum = wave_sum(o[e]);
+            if (lane == l) c[e] += sum;
         }
     }
+    if (!live) return;
     T qx, qy, qz, qw;
-    V prev = reinterpret_cast<const V *>(M.quat)[iv];
     best_rotation<T>(c, prev.x, prev.y, prev.z, prev.w, qx, qy, qz, qw);
     V out;
     out.x = qx; out.y = qy; out.z = qz; out.w = qw;
@@ -873,16 +952,6 @@ __device__ __forceinline__ int sub_find(const SubNode *N, int a, int b, int t) {
     return lo;
 }
 
-// v from the lane whose index is this lane's xor Q (Q = 1, 2: within a quad), by DPP.
-template <int Q>
-__device__ __forceinline__ double quad_xor(double v) {
-    constexpr int ctrl = Q == 1 ? 0xB1 : 0x4E;  // quad_perm [1,0,3,2] / [2,3,0,1]
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)u, ctrl, 0xF, 0xF, true);
-    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), ctrl, 0xF, 0xF, true);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
 // One subtree as the host lays it out: records [sub.x, sub.y), height table offset sub.z, sub.w
 // heights; rows [row.x, +row.y); forward positions [row.z, +row.w), backward off rows [ext.x, +ext.y).
 struct SubTree {
@@ -1036,14 +1105,8 @@ __global__ __launch_bounds__(BLOCK) void k_sub_fwd(LaunchSet L, SubLds D) {
 // 2,825 in FP64: 31 us (50), a batch's 7,413 in FP32: 59 us (73).
 template <typename T>
 __device__ __forceinline__ T quad_sum(T v) {
-    if constexpr (sizeof(T) == 8) {
-        v += quad_xor<1>(v);
-        v += quad_xor<2>(v);
-    } else {
-        v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));
-        v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, true));
-    }
-    return v;
+    v += dpp_move<0xB1>(v);
+    return v + dpp_move<0x4E>(v);
 }
 template <typename T, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_sub_bwd(LaunchSet L, SubLds D) {
@@ -1179,49 +1242,6 @@ __global__ __launch_bounds__(BLOCK) void k_sub_bwd(LaunchSet L, SubLds D) {
 template <typename T> __device__ __forceinline__ const T *wts(const MD_G MeshDev &M);
 template <> __device__ __forceinline__ const float *wts<float>(const MD_G MeshDev &M) { return M.w32; }
 template <> __device__ __forceinline__ const double *wts<double>(const MD_G MeshDev &M) { return M.w64; }
-
-// Lane moves inside a row of 16 lanes (DPP control CTRL).
-template <int CTRL> __device__ __forceinline__ float dpp_move(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
-}
-template <int CTRL> __device__ __forceinline__ double dpp_move(double v) {
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)u, CTRL, 0xF, 0xF, true);
-    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), CTRL, 0xF, 0xF, true);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-// v + the value of the other row of each pair (Half: of the other half of the wavefront).
-template <bool Half> __device__ __forceinline__ void rows_swap(unsigned u, unsigned (&o)[2]) {
-    if constexpr (Half) {
-        const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-        o[0] = a[0]; o[1] = a[1];
-    } else {
-        const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-        o[0] = a[0]; o[1] = a[1];
-    }
-}
-template <bool Half> __device__ __forceinline__ float rows_sum(float v) {
-    unsigned a[2];
-    rows_swap<Half>(__builtin_bit_cast(unsigned, v), a);
-    return __builtin_bit_cast(float, a[0]) + __builtin_bit_cast(float, a[1]);
-}
-template <bool Half> __device__ __forceinline__ double rows_sum(double v) {
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    unsigned lo[2], hi[2];
-    rows_swap<Half>((unsigned)u, lo);
-    rows_swap<Half>((unsigned)(u >> 32), hi);
-    return __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]) +
-           __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
-}
-// Sum over the wavefront, in every lane (quads, half rows, rows, row pairs, halves).
-template <typename T> __device__ __forceinline__ T wave_sum(T v) {
-    v += dpp_move<0xB1>(v);
-    v += dpp_move<0x4E>(v);
-    v += dpp_move<0x141>(v);
-    v += dpp_move<0x140>(v);
-    v = rows_sum<false>(v);
-    return rows_sum<true>(v);
-}
 
 // Six block sums, in every thread: a wavefront's by lane moves, the wavefronts' through LDS
 // (two LDS trees of eight barriers each took 4 of a CG step's 11 us). red is written once

@@ -31,3 +31,32 @@ def test_cotan_of_irregular_faces(segs, extra):
     np.testing.assert_allclose(w, w0, rtol=1e-12, atol=0)
     m.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("segs", [15, 16, 17, 24, 79, 80, 81, 150])
+@pytest.mark.parametrize("poles", [1, 4, 5, 6])
+def test_long_one_rings(segs, poles):
+    """Three spheres whose poles have `segs` neighbours, `poles` of the six held (held vertices share one
+    slice: at most four long rings in a slice are taken by the wavefront, more lane by lane)."""
+    if mdarap.device_count() == 0:
+        pytest.fail("no GPU visible: the HIP path cannot run")
+    one, tri1 = meshgen.uv_sphere(5, segs)
+    n = len(one)
+    xyz = np.concatenate([one + np.array([3.0 * k, 0.0, 0.0]) for k in range(3)])
+    tri = np.concatenate([tri1 + k * n for k in range(3)]).astype(np.int32)
+    pole = np.array([0, n - 1, n, 2 * n - 1, 2 * n, 3 * n - 1])[:poles]
+    side = np.concatenate([k * n + 1 + 2 * segs + np.arange(3) for k in range(3)])  # on each equator
+    held = np.sort(np.concatenate([pole, side])).astype(np.int32)
+    tgt = xyz[held] + np.where(np.isin(held, pole)[:, None], np.array([0.05, 0.0, 0.1]), 0.0)
+    ref = oracle.Arap(xyz, tri)
+    ref.set_constraints(held, tgt)
+    assert ref.deform(3)
+    ctx = mdarap.Context(0)
+    for prec, tol in ((mdarap.PREC_FP64, 1e-9), (mdarap.PREC_FP32_REFINE, 1e-5)):
+        print("case: segs=%d poles=%d precision=%d" % (segs, poles, prec), flush=True)
+        m = mdarap.Mesh(ctx, xyz, tri, mdarap.config(precision=prec))
+        m.set_constraints(held, tgt)
+        assert m.deform(3)
+        assert meshgen.relative_error(m.mesh, ref.mesh) < tol
+        m.close()
+    ctx.close()
