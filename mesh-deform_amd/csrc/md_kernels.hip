@@ -1098,11 +1098,12 @@ __global__ __launch_bounds__(BLOCK) void k_sub_fwd(LaunchSet L, SubLds D) {
 // owner's partials); per height
 //   off rows: -x of those inside, from LDS,
 //   columns:  x_s[q] = sum_p [Dinv_s; G_s][p, q] t[p], t = [z_s; off rows], four lanes per column
-//             (rows p = lane mod 4, joined by DPP: a front of up to 64 rows is one load of kSubAhead
+//             (rows p = lane mod 4, joined by DPP: a front of up to 4 kAhead rows is one load of kAhead
 //             entries per lane, made a height ahead).
 // A 10k icosphere's 91 subtrees in FP32: 9.5 us; one wavefront per subtree, one lane per column and
 // a round trip for the sources and one for the panel in every height took 19. The 164k icosphere's
-// 2,825 in FP64: 31 us (50), a batch's 7,413 in FP32: 59 us (73).
+// 2,825 in FP64: 31 us (50). A batch's 7,413 in FP32: 50 us (73), 59 with kSubAhead entries ahead and its
+// registers.
 template <typename T>
 __device__ __forceinline__ T quad_sum(T v) {
     v += dpp_move<0xB1>(v);
@@ -1158,14 +1159,16 @@ __global__ __launch_bounds__(BLOCK) void k_sub_bwd(LaunchSet L, SubLds D) {
     }
     __syncthreads();
     // column t of height h: its record and the first entries of the lane's rows
+    // (FP32 launches of many subtrees: fewer registers, seven wavefronts per SIMD instead of four)
+    constexpr int kAhead = BLOCK == kSubBlock || sizeof(T) == 8 ? kSubAhead : kSubAhead / 2;
     const int part = tid & 3;
-    T g[kSubAhead];
+    T g[kAhead];
     int item = 0;
     auto rows4 = [&](const SubNode &s, int q, int p0) {  // rows p0 + part, + 4, ...
         const int m = s.w + s.noff;
         const T *p = P + s.pr + q;
 #pragma unroll
-        for (int u = 0; u < kSubAhead; ++u) g[u] = p[(long long)min(p0 + part + 4 * u, m - 1) * s.w];
+        for (int u = 0; u < kAhead; ++u) g[u] = p[(long long)min(p0 + part + 4 * u, m - 1) * s.w];
     };
     auto load = [&](int a, int b, int t) {
         item = sub_find<&SubNode::pq>(N, a, b, t);
@@ -1197,10 +1200,10 @@ __global__ __launch_bounds__(BLOCK) void k_sub_bwd(LaunchSet L, SubLds D) {
             const V *zs = F + s.xs, *os = off + (s.ob - S.ext.x) - s.w;
             T ax = 0, ay = 0, az = 0;
             // row-major [Dinv_s; G_s]: entry (row p, column q) at p * w + q
-            for (int p0 = 0; p0 < m; p0 += 4 * kSubAhead) {
+            for (int p0 = 0; p0 < m; p0 += 4 * kAhead) {
                 if (p0 > 0) rows4(s, q, p0);
 #pragma unroll
-                for (int u0 = 0; u0 < kSubAhead; u0 += 4) {
+                for (int u0 = 0; u0 < kAhead; u0 += 4) {
                     if (p0 + 4 * u0 < m) {
 #pragma unroll
                         for (int u = u0; u < u0 + 4; ++u) {
