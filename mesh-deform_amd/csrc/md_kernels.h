@@ -209,14 +209,15 @@ inline FacAssembly fac_assembly(int count, int mm, int no, long long maps) {
 // and off rows each rounded up).
 void launch_fac_height(hipStream_t s, const FacArgs &A, int h0, int count, int nb, const FacAssembly &as, int tiles);
 // Fronts of m <= mm <= kFacSmallFront rows: every step of launch_fac_height for one front in one
-// workgroup (of one wavefront on heights of more than kSmallManyFronts fronts, else
-// of four), without the FP64 panel workspace.
+// workgroup, without the FP64 panel workspace: of one wavefront on heights of more than kSmallManyFronts
+// fronts of up to 48 rows (6,616: 50 us, with two 53; 1,380: 20 and 23), of two on heights of more than
+// kSmallManyWide with larger ones (1,137: 36 us, with one 49; 685: 25, with four 33), else of four.
 constexpr int kFacSmallFront = 64;
-constexpr int kSmallManyFronts = 1024;
+constexpr int kSmallManyFronts = 1024, kSmallManyWide = 512;
 void launch_fac_small(hipStream_t s, const FacArgs &A, int h0, int count, int mm);
 // Whether a height's `small` such fronts of `all` leave its general launches for the fused one: when
 // they are all of it, or at least 512 and the larger part (the 164k icosphere's second and third
-// heights: 116 and 114 us split, 140 and 152 together; a smaller share only adds a launch).
+// heights took 116 and 114 us split, 140 and 152 together; a smaller share only adds a launch).
 inline bool fac_split_small(int small, int all) { return small == all || (small >= 512 && 2 * small >= all); }
 // Internal-order vectors (positions, normals) to packed xyz in original order (internal: internal
 // id per original id); stamp: clock at the start (may be null).

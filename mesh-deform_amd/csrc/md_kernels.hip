@@ -2359,13 +2359,16 @@ __device__ __forceinline__ bool small_front(double *Fs, int w, double thr) {
 // front's row list staged in LDS for the searches) by all of its BLOCK threads, the sweeps by its
 // first wavefront in registers (small_front), and all of it out again: D^{-1} and G to the sweeps'
 // panels, U for the parent. BLOCK is 64 for many fronts (the leaves, which have no children) and 256
-// for few, where the additions of the children are the longer part. The FP64 panel workspace is not
-// used. 51 us for the 6,616 leaves of the 164k icosphere and 14 us for a single front of 52 columns; the
-// column-by-column Cholesky in LDS that stood here took 100 and 88 us (three barriers per column).
+// for few, where the additions of the children are the longer part; fronts of more than 48 rows, which
+// have children and whose LDS and registers hold four wavefronts' fronts per CU, take 128 where they
+// are many. Limited to two wavefronts per SIMD's registers (256), which 260 had halved. The FP64
+// panel workspace is not used. 50 us for the 6,616 leaves of the 164k icosphere, 70 for its 2,449 fronts of up to
+// 64 rows above them (92 with one wavefront each) and 14 us for a single front of 52 columns; the
+// column-by-column Cholesky in LDS that stood here took 100 us for the leaves and 88 for the single one.
 constexpr int kSmallSlotLanes = 4;  // lanes per pivot column for its original entries
 constexpr int kSmallAhead = 16;     // columns of a child's update matrix in flight
 template <int BLOCK, int NB>
-__global__ __launch_bounds__(BLOCK) void k_fac_small(FacArgs A, int h0) {
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void k_fac_small(FacArgs A, int h0) {
     const FacDev S = A.sn[h0 + blockIdx.x];
     const int tid = threadIdx.x, w = S.w, no = S.noff, m = S.m;
     if (A.stamp && h0 == 0 && blockIdx.x == 0 && tid == 0) *A.stamp = wall_clock64();
@@ -2497,13 +2500,18 @@ static void fac_small_of(hipStream_t s, const FacArgs &A, int h0, int count, int
     const dim3 grid(count), block(BLOCK);
     if (mm <= kIb) hipLaunchKernelGGL((k_fac_small<BLOCK, 1>), grid, block, 0, s, A, h0);
     else if (mm <= 2 * kIb) hipLaunchKernelGGL((k_fac_small<BLOCK, 2>), grid, block, 0, s, A, h0);
-    else if (mm <= 3 * kIb) hipLaunchKernelGGL((k_fac_small<BLOCK, 3>), grid, block, 0, s, A, h0);
-    else hipLaunchKernelGGL((k_fac_small<BLOCK, 4>), grid, block, 0, s, A, h0);
+    else hipLaunchKernelGGL((k_fac_small<BLOCK, 3>), grid, block, 0, s, A, h0);
 }
 void launch_fac_small(hipStream_t s, const FacArgs &A, int h0, int count, int mm) {
     if (count <= 0) return;
-    if (count > kSmallManyFronts) fac_small_of<64>(s, A, h0, count, mm);
-    else fac_small_of<256>(s, A, h0, count, mm);
+    if (mm > 3 * kIb) {
+        if (count > kSmallManyWide) hipLaunchKernelGGL((k_fac_small<128, 4>), dim3(count), dim3(128), 0, s, A, h0);
+        else hipLaunchKernelGGL((k_fac_small<256, 4>), dim3(count), dim3(256), 0, s, A, h0);
+    } else if (count > kSmallManyFronts) {
+        fac_small_of<64>(s, A, h0, count, mm);
+    } else {
+        fac_small_of<256>(s, A, h0, count, mm);
+    }
 }
 void launch_fac_height(hipStream_t s, const FacArgs &A, int h0, int count, int nb, const FacAssembly &as, int tiles) {
     if (count <= 0) return;
