@@ -78,9 +78,8 @@ typedef struct {
                           pair); 0 runs it on the host */
     int level_pairs;   /* MD_SOLVER_LDLT: 1 orders the free vertices so that every other sweep level
                           merges into its parents (about half the level launches, denser panels,
-                          the same fill) and the top levels, up to 400 columns (2000 where the
-                          rest pose is fixed), into one dense block; 0 keeps the plain
-                          nested-dissection order; default 1 */
+                          the same fill) and the top levels, up to 400 columns (700 where the rest
+                          pose is fixed), into one dense block; 0 keeps the plain nested-dissection order; default 1 */
 } md_config;
 
 typedef struct {

@@ -745,7 +745,7 @@ std::vector<int> pair_levels(const std::vector<int>& order, const std::vector<in
     // the top levels [cut, top] of at most top_columns columns together, or all of a small system. Below
     // the cut level 0 goes into the subtrees of the default budget and the others pair, so an even cut
     // leaves as many levels as the next one, for a wider top
-    const bool whole = m <= kWholeColumns;
+    const bool whole = m <= kTopColumns;
     int cut = top;
     {
         std::vector<int64_t> width(top + 1, 0);

@@ -21,15 +21,15 @@ constexpr int kMaxGroupWidth = 4096;
 // uses: the factor depends on the amalgamation and the pairing only, so a re-layout with any
 // budget keeps it (and the small budget pairs the low levels as well).
 constexpr int kPairBudget = 128;
-// Columns of the top sweep levels that level pairing merges into one supernode per root: each level
-// less saves two dependent launches per iteration (about 9 us) for a denser inverse. Where every deform
-// refactors (reference rest mode) a wider pivot block costs about 13 us per 64 columns and saves a height's
-// launches: 400 columns (UV spheres of 3,202, 10 iterations: 1110 -> 960 us; 680 columns no better). Where the
-// factor is kept, 2000 (drags of 10k icospheres, 10 iterations: 631 -> 520 us; 2600 gave 450 there but
-// slows 24 served meshes, bound by their bytes, from 3.76 to 4.07 ms). A whole system of at most
-// kWholeColumns becomes one supernode (a bar of 380 vertices, 20 iterations: 736 -> 500 us; a sphere of 642
-// with 5 iterations: 324 -> 337).
-constexpr int kTopColumns = 400, kTopColumnsKept = 2000, kWholeColumns = 400;
+// Columns of the top sweep levels that level pairing merges into one supernode per root, and of a whole
+// system that becomes one: each level less saves two dependent launches per iteration (about 9 us) for a
+// denser inverse. A wider pivot block costs the factorization about 13 us per 64 columns and saves a height's
+// launches (UV spheres of 3,202, a factorization and 10 iterations: 1110 -> 960 us, 680 columns no better; a
+// bar of 380 vertices whole, 20 iterations: 736 -> 500; a sphere of 642 whole, 5 iterations: 324 -> 337).
+// Where the factor is kept, 700 (10 iterations of 10k icospheres: 620 us with 400, 580 with 700). Wider still
+// would pay for one mesh (520 with 2000), but not in a mix, which is bound by its bytes (45 meshes, an
+// iteration: 0.630 ms with 400, 0.634 with 700, 0.71 with 2000).
+constexpr int kTopColumns = 400, kTopColumnsKept = 700;
 // Edge of the square panel tile one wavefront streams in the triangular sweeps.
 constexpr int kTile = 64;
 // Vertices per one-ring slice (one wavefront).
@@ -199,8 +199,8 @@ void symbolic(int n, const std::vector<int>& adj_ptr, const std::vector<int>& ad
 // order places a group's member supernodes right before their parent (after the members'
 // own subtrees, so the fill is unchanged) and group receives each position's group (-1:
 // none), so that symbolic() merges every group into one supernode: about half the levels,
-// for denser panels. The top levels of at most top_columns columns (everything, in a system of at
-// most kWholeColumns) are one group per root, their fill that of a dense block; the pairs lie below them.
+// for denser panels. The top levels of at most top_columns columns (everything, in a
+// system of at most kTopColumns) are one group per root, their fill that of a dense block; the pairs lie below them.
 std::vector<int> pair_levels(const std::vector<int>& order, const std::vector<int>& ptr, const std::vector<int>& adj,
                              int sub_budget, double amalg_ratio, int top_columns,
                              std::vector<int>& group);
