@@ -222,6 +222,14 @@ inline bool fac_split_small(int small, int all) { return small == all || (small 
 // Internal-order vectors (positions, normals) to packed xyz in original order (internal: internal
 // id per original id); stamp: clock at the start (may be null).
 void launch_pack_xyz(hipStream_t s, const d4 *v, const int *internal, int n, double *dst, unsigned long long *stamp);
+// The packed positions of `count` meshes, n vertices in blocks of kBlock threads from `block` each.
+struct PackEntry {
+    const MD_G d4 *x;
+    const MD_G int *internal;
+    MD_G double *dst;
+    int n, block;
+};
+void launch_pack_results(hipStream_t s, const PackEntry *e, int count, int blocks);
 // Packed xyz to internal order (p and/or pp; pp takes the targets tgt, internal order, for the
 // constrained ids [nf, n), and comes with identity rotations in quat).
 struct UnpackArgs {

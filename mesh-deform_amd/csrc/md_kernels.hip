@@ -1565,6 +1565,23 @@ __global__ __launch_bounds__(kBlock) void k_pack_xyz(const d4 *x, const int *int
     o[0] = p.x; o[1] = p.y; o[2] = p.z;
 }
 
+// The same for the results of several meshes, one launch (a launch per mesh is 8 us for the 10 a full
+// server finishes at a boundary, beside the next iteration's launches). The entries may lie in
+// pinned host memory; block b belongs to the last entry whose first block is not past it.
+__global__ __launch_bounds__(kBlock) void k_pack_results(const PackEntry *e, int count) {
+    int lo = 0, hi = count - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (e[mid].block <= (int)blockIdx.x) lo = mid; else hi = mid - 1;
+    }
+    const PackEntry E = e[lo];
+    const int v = ((int)blockIdx.x - E.block) * kBlock + threadIdx.x;
+    if (v >= E.n) return;
+    const d4 p = E.x[E.internal[v]];
+    MD_G double *o = E.dst + 3 * (size_t)v;
+    o[0] = p.x; o[1] = p.y; o[2] = p.z;
+}
+
 // Device workspace of the entry points that allocate nothing (md_mesh_normals_noalloc): one
 // array per GPU, set aside when the code object loads and held until the process ends. Host
 // code reaches it only through the address hipGetSymbolAddress returns on each device (the
@@ -2564,6 +2581,9 @@ void launch_publish(hipStream_t s, unsigned long long *stamp, const int *flag, i
     hipLaunchKernelGGL(k_publish, dim3(1), dim3(1), 0, s, stamp, flag, out);
 }
 
+void launch_pack_results(hipStream_t s, const PackEntry *e, int count, int blocks) {
+    if (count > 0 && blocks > 0) hipLaunchKernelGGL(k_pack_results, dim3(blocks), dim3(kBlock), 0, s, e, count);
+}
 void launch_scatter_entries(hipStream_t s, const TargetEntry *e, int k) {
     if (k > 0) hipLaunchKernelGGL(k_scatter_entries, dim3((k + kBlock - 1) / kBlock), dim3(kBlock), 0, s, e, k);
 }

@@ -262,6 +262,9 @@ struct md_server {
     size_t tgt_cap_host[2] = {0, 0};
     TargetEntry *tgt_dev = nullptr;
     size_t tgt_cap_dev = 0;
+    // results packed at a boundary: pinned entries by boundary parity, as the targets'
+    PackEntry *pack_host[2] = {nullptr, nullptr};
+    size_t pack_cap[2] = {0, 0};
     std::vector<double *> pinned_all;                     // guarded by mu
 
     double *take_pinned(ServedMesh *sm) {  // caller holds mu
@@ -342,6 +345,37 @@ void fail(Request &r, int status, const std::string &msg) {
         r.error = msg;
     }
     r.left = 0;
+}
+
+// Packs the positions of the requests that end at this boundary (mesh d_xyz, original order), behind the
+// boundary's launch.
+void pack_results(md_server *S, const std::vector<std::shared_ptr<Request>> &ending, hipStream_t st) {
+    size_t k = 0;
+    for (auto &r : ending) k += r->status == MD_OK;
+    if (k == 0) return;
+    hipError_t x = hipSuccess;
+    const int par = (int)(S->boundaries & 1);
+    if (S->pack_cap[par] < k) {
+        if (S->pack_host[par]) hipHostFree(S->pack_host[par]);
+        S->pack_host[par] = nullptr;
+        S->pack_cap[par] = 0;
+        x = hipHostMalloc((void **)&S->pack_host[par], sizeof(PackEntry) * 2 * k, hipHostMallocDefault);
+        if (x == hipSuccess) S->pack_cap[par] = 2 * k;
+    }
+    if (x == hipSuccess) {
+        int n = 0, blocks = 0;
+        for (auto &r : ending) {
+            if (r->status != MD_OK) continue;
+            md_mesh *m = r->sm->m;
+            S->pack_host[par][n++] = PackEntry{m->dev.pp, m->d_internal, m->d_xyz, m->n, blocks};
+            blocks += (m->n + kBlock - 1) / kBlock;
+        }
+        launch_pack_results(st, S->pack_host[par], n, blocks);
+        x = hipGetLastError();
+    }
+    if (x != hipSuccess)
+        for (auto &r : ending)
+            if (r->status == MD_OK) fail(*r, MD_ERR_HIP, std::string("packing the result: ") + hipGetErrorString(x));
 }
 
 // Admission at an iteration boundary (S->mu held), by plan_admission over the served meshes'
@@ -552,11 +586,10 @@ void server_loop(md_server *S) {
                 if (r->status == MD_OK && !(r->pinned = S->take_pinned(r->sm)))
                     fail(*r, MD_ERR_NOMEM, "pinned result buffer");
         }
-        // the positions are packed in original order straight into the pinned buffers (a burst to 24
-        // meshes of 5k to 60k vertices: 3.6 ms; with the scatter into the caller's order on the host 4.4) on the
-        // copy stream, after this boundary's
-        // launch (or, when nothing was launched, after everything queued so far), so the copies
+        // the positions are packed in original order on the device (each mesh's packed buffer, all in one
+        // launch behind the iteration's) and copied to the pinned buffers on the copy stream, so the copies
         // overlap the next launches; a mesh is not iterated again before its result is delivered
+        pack_results(S, ending, st);
         if (launched) hipEventRecord(S->ev[S->seq % 2], st);
         bool waited = false;
         for (auto &r : ending) {
@@ -568,8 +601,8 @@ void server_loop(md_server *S) {
                     waited = true;
                 }
                 md_mesh *m = r->sm->m;
-                launch_pack_xyz(S->copy_stream, m->dev.pp, m->d_internal, m->n, r->pinned, nullptr);
-                hipError_t x = hipGetLastError();
+                hipError_t x = hipMemcpyAsync(r->pinned, m->d_xyz, sizeof(double) * 3 * (size_t)m->n,
+                                              hipMemcpyDeviceToHost, S->copy_stream);
                 if (x != hipSuccess) fail(*r, MD_ERR_HIP, hipGetErrorString(x));
             }
             r->finish_seq = launched ? S->seq : 0;
@@ -816,6 +849,8 @@ extern "C" int md_server_destroy(md_server *S) {
     hipStreamSynchronize(S->copy_stream);
     for (double *p : S->pinned_all) hipHostFree(p);
     for (TargetEntry *p : S->tgt_host)
+        if (p) hipHostFree(p);
+    for (PackEntry *p : S->pack_host)
         if (p) hipHostFree(p);
     if (S->tgt_dev) hipFree(S->tgt_dev);
     // meshes evicted by the server stay on the host until their next use (md_mesh_* restores)
