@@ -2630,9 +2630,9 @@ static size_t sub_lds(const SubLds &D, int entries, int index_bytes, bool fp64) 
 }
 template <typename T, bool Fused>
 static void sub_fwd_of(hipStream_t s, LaunchSet L, int blocks, const SubLds &D, size_t lds) {
-    constexpr int kMany = Fused ? 64 : 128;
     if (D.block == kSubBlock) hipLaunchKernelGGL((k_sub_fwd<T, Fused, kSubBlock>), dim3(blocks), dim3(kSubBlock), lds, s, L, D);
-    else hipLaunchKernelGGL((k_sub_fwd<T, Fused, kMany>), dim3(blocks), dim3(kMany), lds, s, L, D);
+    else if (Fused || D.block == 64) hipLaunchKernelGGL((k_sub_fwd<T, Fused, 64>), dim3(blocks), dim3(64), lds, s, L, D);
+    else hipLaunchKernelGGL((k_sub_fwd<T, false, 128>), dim3(blocks), dim3(128), lds, s, L, D);
 }
 void launch_sub_fwd(hipStream_t s, LaunchSet L, int blocks, const SubLds &D, bool fused, bool fp64) {
     if (blocks <= 0) return;
@@ -2643,6 +2643,7 @@ void launch_sub_fwd(hipStream_t s, LaunchSet L, int blocks, const SubLds &D, boo
 template <typename T>
 static void sub_bwd_of(hipStream_t s, LaunchSet L, int blocks, const SubLds &D, size_t lds) {
     if (D.block == kSubBlock) hipLaunchKernelGGL((k_sub_bwd<T, kSubBlock>), dim3(blocks), dim3(kSubBlock), lds, s, L, D);
+    else if (D.block == 64) hipLaunchKernelGGL((k_sub_bwd<T, 64>), dim3(blocks), dim3(64), lds, s, L, D);
     else hipLaunchKernelGGL((k_sub_bwd<T, 128>), dim3(blocks), dim3(128), lds, s, L, D);
 }
 void launch_sub_bwd(hipStream_t s, LaunchSet L, int blocks, const SubLds &D, bool fp64) {

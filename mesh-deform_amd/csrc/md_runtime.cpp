@@ -98,7 +98,8 @@ hipError_t build_plan(Plan &plan, const std::vector<const MeshDev *> &meshes,
     plan.nlevels = 0;
     for (const Factor *f : factors) plan.nlevels = std::max(plan.nlevels, f->nlevels);
     int nl = plan.nlevels;
-    int ntables = 7 + 2 * nl;
+    constexpr int kLevelTable = 5 + 2 * kSubClasses;
+    int ntables = kLevelTable + 2 * nl;
     plan.h_prefix.assign((size_t)ntables * (na + 1), 0);
     plan.h_tbase.assign((size_t)ntables * (na + 1), 0);
     plan.off_fwd.assign(nl, 0);
@@ -118,26 +119,39 @@ hipError_t build_plan(Plan &plan, const std::vector<const MeshDev *> &meshes,
     table(2, plan.off_resid, plan.blk_resid,
           [&](int k) { return cdiv(meshes[k]->nslices_free, kSlicesPerBlock); });
     table(4, plan.off_apply, plan.blk_apply, [&](int k) { return cdiv(meshes[k]->nf, kBlock); });
-    table(5, plan.off_sub, plan.blk_sub, [&](int k) { return factors[k]->nsub; });
-    plan.sub = SubLds{};
-    for (const Factor *f : factors) {
-        plan.sub.fwd = std::max(plan.sub.fwd, f->sub_lds_fwd);
-        plan.sub.bwd = std::max(plan.sub.bwd, f->sub_lds_bwd);
-        plan.sub.off = std::max(plan.sub.off, f->sub_off);
-        plan.sub.nodes = std::max(plan.sub.nodes, f->sub_nodes);
-        plan.sub.heights = std::max(plan.sub.heights, f->sub_heights);
+    // bottom subtrees, by the LDS of their meshes' largest
+    auto lds_class = [&](int k) {
+        const int e = std::max(factors[k]->sub_lds_fwd, factors[k]->sub_lds_bwd);
+        int c = 0;
+        while (na > 1 && c < kSubClasses - 1 && e > kSubClassEntries[c]) ++c;
+        return c;
+    };
+    for (int c = 0; c < kSubClasses; ++c) {
+        Plan::Subtrees &u = plan.sub[c];
+        u = Plan::Subtrees{};
+        for (int k = 0; k < na; ++k) {
+            if (lds_class(k) != c) continue;
+            const Factor *f = factors[k];
+            u.lds.fwd = std::max(u.lds.fwd, f->sub_lds_fwd);
+            u.lds.bwd = std::max(u.lds.bwd, f->sub_lds_bwd);
+            u.lds.off = std::max(u.lds.off, f->sub_off);
+            u.lds.nodes = std::max(u.lds.nodes, f->sub_nodes);
+            u.lds.heights = std::max(u.lds.heights, f->sub_heights);
+        }
+        table(5 + 2 * c, u.off_fwd, u.blk_fwd, [&](int k) { return lds_class(k) == c ? factors[k]->nsub : 0; });
+        u.lds.block = u.blk_fwd <= kSubFew ? kSubBlock : na > 1 && c == 0 ? 64 : 128;
+        table(6 + 2 * c, u.off_bwd, u.blk_bwd, [&](int k) {
+            return lds_class(k) == c ? factors[k]->nsub + cdiv(meshes[k]->nlrows, u.lds.block) : 0;
+        });
     }
-    plan.sub.block = plan.blk_sub <= kSubFew ? kSubBlock : 0;
-    table(6, plan.off_subb, plan.blk_subb,
-          [&](int k) { return factors[k]->nsub + cdiv(meshes[k]->nlrows, sub_rows_bwd(plan.sub)); });
     table(3, plan.off_subf, plan.blk_subf,
-          [&](int k) { return factors[k]->nsub + cdiv(meshes[k]->nlrows, sub_rows_fwd(plan.sub)); });
+          [&](int k) { return factors[k]->nsub + cdiv(meshes[k]->nlrows, sub_rows_fused(plan.sub[0].lds)); });
     for (int l = 0; l < nl; ++l) {
-        table(7 + 2 * l, plan.off_fwd[l], plan.blk_fwd[l], [&](int k) {
+        table(kLevelTable + 2 * l, plan.off_fwd[l], plan.blk_fwd[l], [&](int k) {
             const Factor *f = factors[k];
             return l < f->nlevels ? f->ft_ptr[l + 1] - f->ft_ptr[l] : 0;
         });
-        table(8 + 2 * l, plan.off_bwd[l], plan.blk_bwd[l], [&](int k) {
+        table(kLevelTable + 1 + 2 * l, plan.off_bwd[l], plan.blk_bwd[l], [&](int k) {
             const Factor *f = factors[k];
             return l < f->nlevels ? f->bt_ptr[l + 1] - f->bt_ptr[l] : 0;
         });
@@ -224,20 +238,21 @@ void enqueue_iteration(const Plan &plan, hipStream_t stream, hipEvent_t *ev) {
         // one-mesh plans form the residual inside the subtree forward launch (subtree rows in
         // LDS, level rows by extra blocks): its phase is then empty and the forward phase
         // holds it; batches and server mixes keep k_residual (occupancy of the subtree sweep)
-        const bool fused = plan.nactive == 1 && plan.blk_sub <= kFusedResidualMaxSubtrees;
+        const bool fused = plan.nactive == 1 && plan.sub[0].blk_fwd <= kFusedResidualMaxSubtrees;
         if (!fused) launch_residual(stream, plan.set(plan.off_resid), plan.blk_resid, plan.fp64);
         if (ev && r == 0) hipEventRecord(ev[2], stream);
         if (fused)
-            launch_sub_fwd(stream, plan.set(plan.off_subf), plan.blk_subf, plan.sub, true, plan.fp64);
+            launch_sub_fwd(stream, plan.set(plan.off_subf), plan.blk_subf, plan.sub[0].lds, true, plan.fp64);
         else
-            launch_sub_fwd(stream, plan.set(plan.off_sub), plan.blk_sub, plan.sub, false, plan.fp64);
+            for (const Plan::Subtrees &u : plan.sub)
+                launch_sub_fwd(stream, plan.set(u.off_fwd), u.blk_fwd, u.lds, false, plan.fp64);
         for (int l = 0; l < plan.nlevels; ++l)
             launch_fwd(stream, plan.level_set(plan.off_fwd[l], true), plan.blk_fwd[l], l, plan.fp64);
         if (ev && r == 0) hipEventRecord(ev[3], stream);
         for (int l = plan.nlevels - 1; l >= 0; --l)
             launch_bwd(stream, plan.level_set(plan.off_bwd[l], false), plan.blk_bwd[l], l, plan.fp64);
         // subtrees, then p' += x (subtree rows inside their blocks, level rows in extra blocks)
-        launch_sub_bwd(stream, plan.set(plan.off_subb), plan.blk_subb, plan.sub, plan.fp64);
+        for (const Plan::Subtrees &u : plan.sub) launch_sub_bwd(stream, plan.set(u.off_bwd), u.blk_bwd, u.lds, plan.fp64);
         if (ev && r == 0) hipEventRecord(ev[4], stream);
     }
 }

@@ -50,12 +50,16 @@ private:
 struct Plan {
     int nactive = 0;
     int nlevels = 0;
-    int blk_face = 0, blk_slice = 0, blk_resid = 0, blk_apply = 0, blk_sub = 0;
-    int blk_subb = 0, off_subb = 0;    // k_sub_bwd: subtrees, then the p' update of level rows
+    int blk_face = 0, blk_slice = 0, blk_resid = 0, blk_apply = 0;
+    // bottom subtrees of the meshes of one LDS class (a one-mesh plan has only the first)
+    struct Subtrees {
+        SubLds lds{};                    // workgroup size, LDS of the largest
+        int blk_fwd = 0, off_fwd = 0;    // k_sub_fwd
+        int blk_bwd = 0, off_bwd = 0;    // k_sub_bwd: subtrees, then the p' update of level rows
+    } sub[kSubClasses];
     int blk_subf = 0, off_subf = 0;    // k_sub_fwd with the residual: subtrees, then the level rows
     std::vector<int> blk_fwd, blk_bwd;
-    int off_face = 0, off_slice = 0, off_resid = 0, off_apply = 0, off_sub = 0;
-    SubLds sub{};                      // bottom subtrees: workgroup size, LDS of the largest
+    int off_face = 0, off_slice = 0, off_resid = 0, off_apply = 0;
     std::vector<int> off_fwd, off_bwd;
     MeshDev *d_meshes = nullptr;       // views into d_tables: the mesh records,
     int *d_prefix = nullptr;           //   the prefix tables,
