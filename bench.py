@@ -8,7 +8,7 @@ Legs:
   plain   (the value): the 163,842-vertex noisy icosphere (7 subdivisions, sigma 0.01,
           seed 1234; 16,384 anchors at the bottom, 8,192 handles lifted 0.4), FP32 local step
           and FP32 block LDL^T with one FP64 residual refinement per iteration; W untimed and
-          K timed iterations replayed from hipGraphs; iterations/s.
+          K timed iterations, each launched directly; iterations/s.
   check   position error of that path (and of the FP64 path) against the FP64 CPU oracle
           after the same number of iterations from the same start (100, as many as fit the
           CPU time cap), the ARAP energy and iterations/s of each; the same for the Jacobi-PCG alternative
@@ -94,7 +94,7 @@ def plain_leg(ctx, pr, steps, warmup, tune=True, budget=None, fixed_ratio=None):
     m.iterate(steps)  # returns after the stream is synchronised
     ctx.synchronize()
     wall = time.perf_counter() - t0
-    # HIP events on the library's stream: graph replays, then one pass with events between
+    # HIP events on the library's stream: the same iterations, then one pass with events between
     # the phases (local, residual, forward sweeps, backward sweeps + update)
     ev_total_ms, phase_ms = m.time_iterations(0, steps)
     st = m.stats()
@@ -259,7 +259,7 @@ def served_leg(ctx, count, seconds, rate, iters, seed, sweep=(4000, 8000, 16000,
         m.autotune(iters=3)
     setup_s = time.perf_counter() - t0
     footprint = sum(m.stats()["device_bytes"] for m in meshes)
-    # the same meshes iterated one by one (each alone, its own graphs), `iters` iterations each
+    # the same meshes iterated one by one (each alone), `iters` iterations each
     for m in meshes:
         m.iterate(1)
     ctx.synchronize()
@@ -321,7 +321,7 @@ def batched_leg(ctx, count, iters, seed, tune=True, baseline=True):
 
     # plain: each mesh with its own tuned sweep layout and the library's default factor shape
     # (level pairs: fewer launches, the better choice for a mesh iterated alone), iterated alone
-    # (its own graphs), back to back
+    # back to back
     tune_plain_s, plain_s = 0.0, None
     if baseline:
         meshes = prepared(None)
@@ -331,7 +331,7 @@ def batched_leg(ctx, count, iters, seed, tune=True, baseline=True):
                 m.autotune(iters=3)
         tune_plain_s = time.perf_counter() - t0
         for m in meshes:
-            m.iterate(1)  # graph capture
+            m.iterate(1)  # warm-up
         ctx.synchronize()
         t0 = time.perf_counter()
         for m in meshes:
@@ -348,7 +348,7 @@ def batched_leg(ctx, count, iters, seed, tune=True, baseline=True):
     t0 = time.perf_counter()
     budget = b.autotune()[0] if tune else meshes[0].stats()["subtree_budget"]
     tune_batch_s = time.perf_counter() - t0
-    b.iterate(2)  # warm-up (graph capture)
+    b.iterate(2)  # warm-up
     ms = b.time_iterations(0, iters)
     b.close()
     total_iters = count * iters
@@ -490,13 +490,13 @@ def main():
     ap.add_argument("--batched-meshes", type=int, default=256)
     ap.add_argument("--batched-only", action="store_true", help="run only the batched leg (for profiling)")
     ap.add_argument("--no-plain-baseline", action="store_true",
-                    help="batched leg without the one-by-one baseline (profiling runs: one graph per mesh)")
+                    help="batched leg without the one-by-one baseline (profiling runs)")
     ap.add_argument("--subtree-budget", type=int, default=None,
                     help="fixed sweep layout of the plain leg and the traffic probe (no autotune)")
     ap.add_argument("--amalg-ratio", type=float, default=None,
                     help="fixed factor amalgamation of the plain leg and the traffic probe (no autotune)")
     ap.add_argument("--no-autotune", action="store_true",
-                    help="keep the default sweep layout (profiling runs: the tuner re-captures graphs)")
+                    help="keep the default sweep layout (profiling runs)")
     ap.add_argument("--traffic-probe", action="store_true",
                     help="only run the workload of the rocprofv3 --pmc traffic passes")
     ap.add_argument("--probe-iters", type=int, default=5)
@@ -561,7 +561,7 @@ def main():
                      "frac": round(achieved / PEAK_HBM_GBS, 4),
                      "traffic": None if traffic is None else int(traffic),
                      "kernel": "one ARAP iteration (k_local, k_sub_fwd with the residual, k_fwd per level, k_bwd "
-                               "per level, k_sub_bwd with the p' update), replayed from hipGraphs of 8 iterations; "
+                               "per level, k_sub_bwd with the p' update), launched directly; "
                                "HIP events on the library stream, time per iteration",
                      "algorithmic_bytes": cb["B_iter"], "ms_per_iteration": round(ev_step_ms, 5),
                      "canonical": cb,

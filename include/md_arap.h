@@ -62,9 +62,9 @@ typedef struct {
     int rest_mode;     /* md_rest_mode, default MD_REST_REFERENCE */
     int pcg_max_iters; /* MD_SOLVER_PCG: CG iterations per solve, default 200 */
     double pcg_tol;    /* MD_SOLVER_PCG: relative residual target, default 1e-7 */
-    int use_graph;     /* replay iterations from a captured hipGraph of 8 (PCG: of one), captured by
-                          the first call after a (re)layout that runs as many; the rest of a
-                          call's iterations is launched directly; default 1 */
+    int use_graph;     /* MD_SOLVER_PCG: replay iterations from a captured hipGraph of one, captured by
+                          the first call after a (re)layout; MD_SOLVER_LDLT launches every
+                          iteration directly; default 1 */
     int subtree_budget;/* MD_SOLVER_LDLT: LDS vector entries (at most 1024) of one bottom
                           subtree of the factor swept by one workgroup (fronts + columns of
                           its supernodes); 0 sweeps every supernode by level launches;

@@ -1,5 +1,5 @@
 // C ABI of the ARAP library: context, mesh (the AsRigidAsPossibleDeformation object of
-// inc/deform/arap.h), launch plans and graph replay. Batches and the server are in
+// inc/deform/arap.h), launch plans and their iterations. Batches and the server are in
 // md_serve.cpp.
 #include "md_runtime.h"
 
@@ -257,38 +257,36 @@ void enqueue_iteration(const Plan &plan, hipStream_t stream, hipEvent_t *ev) {
     }
 }
 
-// A graph of kGraphIterations iterations takes the bulk of a longer run. The rest is launched
-// directly: a launch costs the host under a microsecond here and the device 4.5 at least, while each
-// graph leaves about 8 us before the next one and its capture and instantiation take half a
-// millisecond (five iterations of a 642-vertex sphere: 190 us launched, 230 as one-iteration graphs).
-constexpr int kGraphIterations = 8;
-
-static hipError_t capture_iterations(Plan &plan, hipStream_t stream, int count, hipGraphExec_t *out) {
+// The direct solver's iterations are launched directly: 4 to 30 launches of 4 us and more each, which the
+// host queues at 1 to 3 us apiece, ahead of the device. Replayed from a graph of 8 iterations they run no
+// faster (an iteration, graph / direct: 642 vertices 27.2 / 27.2 us, 10k 48.5 / 49.3, 164k in FP32
+// 130.7 / 130.0, in FP64 195.3 / 194.2, a batch of 48 meshes 312 / 311), and the capture cost the call
+// that made it 0.13 to 1 ms. A PCG iteration is hundreds of short launches: it is captured, by the first
+// call, and replayed (900 CG steps of a 10k icosphere: 6.81 / 6.93 ms).
+static hipError_t capture_iteration(Plan &plan, hipStream_t stream) {
     hipGraph_t g = nullptr;
     MD_HIP_E(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-    for (int i = 0; i < count; ++i) enqueue_iteration(plan, stream, nullptr);
+    enqueue_iteration(plan, stream, nullptr);
     hipError_t e = hipStreamEndCapture(stream, &g);
     if (e != hipSuccess) return e;
-    e = hipGraphInstantiate(out, g, nullptr, nullptr, 0);
+    e = hipGraphInstantiate(&plan.graph, g, nullptr, nullptr, 0);
     hipGraphDestroy(g);
-    if (e != hipSuccess) *out = nullptr;
+    if (e != hipSuccess) plan.graph = nullptr;
     return e;
 }
 
 hipError_t prepare_iterations(Plan &plan, hipStream_t stream, int iters, bool use_graph) {
-    // a PCG iteration is already hundreds of launches: one-iteration graphs
-    const int count = plan.pcg ? 1 : kGraphIterations;
-    if (!use_graph || iters < count || plan.graph) return hipSuccess;
-    return capture_iterations(plan, stream, count, &plan.graph);
+    if (!use_graph || !plan.pcg || iters <= 0 || plan.graph) return hipSuccess;
+    return capture_iteration(plan, stream);
 }
 
 hipError_t run_iterations(Plan &plan, hipStream_t stream, int iters, bool use_graph) {
     if (iters <= 0) return hipSuccess;
     MD_HIP_E(prepare_iterations(plan, stream, iters, use_graph));
-    const int count = plan.pcg ? 1 : kGraphIterations;
-    if (use_graph)
-        for (; iters >= count; iters -= count) MD_HIP_E(hipGraphLaunch(plan.graph, stream));
-    for (; iters > 0; --iters) enqueue_iteration(plan, stream, nullptr);
+    for (; iters > 0; --iters) {
+        if (use_graph && plan.graph) MD_HIP_E(hipGraphLaunch(plan.graph, stream));
+        else enqueue_iteration(plan, stream, nullptr);
+    }
     return hipGetLastError();
 }
 

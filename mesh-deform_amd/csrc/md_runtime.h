@@ -77,7 +77,7 @@ struct Plan {
     int refine_steps = 1;
     bool pcg = false;
     int pcg_iters = 0;
-    hipGraphExec_t graph = nullptr;        // kGraphIterations iterations (PCG: one)
+    hipGraphExec_t graph = nullptr;        // one PCG iteration
     ~Plan();
     void drop_graph();
     LaunchSet set(int off) const {
@@ -103,8 +103,8 @@ hipError_t build_plan(Plan &plan, const std::vector<const MeshDev *> &meshes,
                       hipStream_t stream, bool sync = true, bool block_maps = false);
 // Enqueues one ARAP iteration (local step + refine_steps x (residual, sweeps)).
 void enqueue_iteration(const Plan &plan, hipStream_t stream, hipEvent_t *phase_events);
-// Runs `iters` iterations, the bulk of them from a captured graph when use_graph is set;
-// prepare_iterations captures what that many need, without running it.
+// Runs `iters` iterations (PCG: from a captured graph when use_graph is set; prepare_iterations captures
+// it without running it).
 hipError_t prepare_iterations(Plan &plan, hipStream_t stream, int iters, bool use_graph);
 hipError_t run_iterations(Plan &plan, hipStream_t stream, int iters, bool use_graph);
 

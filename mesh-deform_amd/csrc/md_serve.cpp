@@ -1,5 +1,5 @@
 // Batches (many prepared meshes iterated by the same launches, one launch per kernel per
-// level covering every mesh, replayed from one captured hipGraph) and the drag-request server.
+// level covering every mesh) and the drag-request server.
 #include <algorithm>
 #include <chrono>
 #include <condition_variable>
