@@ -245,6 +245,7 @@ struct md_mesh {
     // on every deform call (reference rest mode); others free it after each factorization
     void *fac_ws = nullptr;
     size_t fac_ws_bytes = 0;
+    hipEvent_t fac_ev = nullptr;   // after a deform call's factorization (kIterationsAhead)
     void release_fac_ws() {
         if (fac_ws) hipFree(fac_ws);
         fac_ws = nullptr;
@@ -272,5 +273,6 @@ struct md_mesh {
     ~md_mesh() {
         release_fac_ws();
         release_pin();
+        if (fac_ev) hipEventDestroy(fac_ev);
     }
 };

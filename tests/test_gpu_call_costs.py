@@ -1,8 +1,9 @@
 """Calls that must not pay for something else: the first long call of a mesh (no preparation of its
-iterations inside it)."""
+iterations inside it), and a call whose factorization fails (not all of its iterations)."""
 import statistics
 import time
 
+import numpy as np
 import pytest
 
 import meshgen
@@ -43,3 +44,37 @@ def test_first_long_call_costs_what_later_ones_do(ctx, warm):
         over.append(first - statistics.median(later))
         m.close()
     assert min(over) < 0.1, over
+
+
+@pytest.mark.parametrize("precision", [mdarap.PREC_FP64, mdarap.PREC_FP32_REFINE])
+@pytest.mark.parametrize("rest", [mdarap.REST_REFERENCE, mdarap.REST_FIXED])
+def test_failed_factorization_ends_a_long_call(ctx, precision, rest):
+    """A component without constraints fails the factorization: a call of 40,000 iterations (about a second
+    of them) returns False within 0.2 s, positions untouched, again on a second call; with the component
+    constrained the same mesh then gives what a fresh one does, bitwise."""
+    a, b = meshgen.sphere_problem(10, 16), meshgen.sphere_problem(8, 12)
+    xyz = np.concatenate([a.xyz, b.xyz + np.array([5.0, 0.0, 0.0])])
+    tri = np.concatenate([a.tri, b.tri + a.n]).astype(np.int32)
+    idx, tgt = a.constraints()
+    far = a.n + np.arange(3)
+
+    def mesh():
+        m = mdarap.Mesh(ctx, xyz, tri, mdarap.config(precision=precision, rest_mode=rest))
+        m.set_constraints(idx, tgt)
+        return m
+
+    m = mesh()
+    for k in range(2):
+        print("case: failed factorization, precision=%d rest=%d call %d" % (precision, rest, k), flush=True)
+        before = m.mesh.copy()
+        ms = _ms(lambda: m.deform(40000) and pytest.fail("a singular system was factored"))
+        assert ms < 200.0, ms
+        assert np.array_equal(m.mesh, before)
+    m.set_constraints(far, xyz[far])
+    ref = mesh()
+    ref.set_constraints(far, xyz[far])
+    for k in (0, 3, 8, 9, 20):
+        assert m.deform(k) and ref.deform(k)
+        assert np.all(np.isfinite(m.mesh)) and np.array_equal(m.mesh, ref.mesh)
+    m.close()
+    ref.close()
