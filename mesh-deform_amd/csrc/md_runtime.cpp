@@ -41,8 +41,10 @@ CallSlot::CallSlot(md_ctx *c) : ctx_(c) {
         }
     }
     void *h = nullptr;
-    if (!base_ && hipHostMalloc(&h, kHeadBytes + kStageBytes, hipHostMallocDefault) == hipSuccess)
-        base_ = static_cast<char *>(h);
+    if (!base_) {
+        if (hipHostMalloc(&h, kHeadBytes + kStageBytes, hipHostMallocDefault) == hipSuccess) base_ = static_cast<char *>(h);
+        else (void)hipGetLastError();
+    }
     if (base_) *head() = Head{};
 }
 CallSlot::~CallSlot() {
@@ -58,10 +60,13 @@ CallSlot::~CallSlot() {
     hipHostFree(base_);
 }
 
+// An error that a call reports is taken off the runtime's record: launches are judged by it
+// (hipGetLastError), also those of the calls that follow.
 #define MD_HIP(call)                                                                    \
     do {                                                                                \
         hipError_t e_ = (call);                                                         \
         if (e_ != hipSuccess) {                                                         \
+            (void)hipGetLastError();                                                    \
             md::set_error(std::string(#call) + ": " + hipGetErrorString(e_));           \
             return MD_ERR_HIP;                                                          \
         }                                                                               \
@@ -70,7 +75,10 @@ CallSlot::~CallSlot() {
 #define MD_HIP_E(call)                                                                  \
     do {                                                                                \
         hipError_t e_ = (call);                                                         \
-        if (e_ != hipSuccess) return e_;                                                \
+        if (e_ != hipSuccess) {                                                         \
+            (void)hipGetLastError();                                                    \
+            return e_;                                                                  \
+        }                                                                               \
     } while (0)
 
 Plan::~Plan() {
@@ -1018,6 +1026,7 @@ int fac_ws_ready(md_mesh *m) {
     if (m->fac_ws && m->fac_ws_bytes != bytes) m->release_fac_ws();
     if (m->fac_ws) return MD_OK;
     if (hipMalloc(&m->fac_ws, bytes) != hipSuccess) {
+        (void)hipGetLastError();
         m->fac_ws = nullptr;
         set_error("device factorization workspace of " + std::to_string(bytes) + " bytes: allocation failed");
         return MD_ERR_NOMEM;
@@ -2073,6 +2082,7 @@ extern "C" int md_copy_probe(md_ctx *ctx, size_t bytes, int repeats, double *gbp
     hipEvent_t e0 = nullptr, e1 = nullptr;
     hipError_t e = hipMalloc(&a, (size_t)n16 * 16);
     if (e == hipSuccess) e = hipMalloc(&b, (size_t)n16 * 16);
+    if (e != hipSuccess) (void)hipGetLastError();
     if (e == hipSuccess) e = hipMemsetAsync(a, 0, (size_t)n16 * 16, st);
     if (e == hipSuccess) launch_copy_probe(st, a, b, n16);  // warm-up
     if (e == hipSuccess) e = hipEventCreate(&e0);

@@ -29,7 +29,9 @@ public:
     hipError_t allocate() {
         release();
         if (size_ == 0) return hipSuccess;
-        return hipMalloc(&base_, size_);
+        const hipError_t e = hipMalloc(&base_, size_);
+        if (e != hipSuccess) (void)hipGetLastError();
+        return e;
     }
     void *at(size_t off) const { return static_cast<char *>(base_) + off; }
     char *base() const { return static_cast<char *>(base_); }

@@ -275,8 +275,10 @@ struct md_server {
             return p;
         }
         void *p = nullptr;
-        if (hipHostMalloc(&p, 3 * sizeof(double) * (size_t)std::max(1, sm->m->n), hipHostMallocDefault) != hipSuccess)
+        if (hipHostMalloc(&p, 3 * sizeof(double) * (size_t)std::max(1, sm->m->n), hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
             return nullptr;
+        }
         pinned_all.push_back((double *)p);
         return (double *)p;
     }
@@ -300,8 +302,10 @@ hipError_t apply_targets(md_server *S, const std::vector<std::shared_ptr<Request
         S->tgt_host[par] = nullptr;
         S->tgt_cap_host[par] = 0;
         const size_t cap = k + k / 2;
-        if (hipError_t e = hipHostMalloc((void **)&S->tgt_host[par], sizeof(TargetEntry) * cap, hipHostMallocDefault))
+        if (hipError_t e = hipHostMalloc((void **)&S->tgt_host[par], sizeof(TargetEntry) * cap, hipHostMallocDefault)) {
+            (void)hipGetLastError();
             return e;
+        }
         S->tgt_cap_host[par] = cap;
     }
     if (S->tgt_cap_dev < k) {
@@ -312,7 +316,10 @@ hipError_t apply_targets(md_server *S, const std::vector<std::shared_ptr<Request
         S->tgt_dev = nullptr;
         S->tgt_cap_dev = 0;
         const size_t cap = k + k / 2;
-        if (hipError_t e = hipMalloc((void **)&S->tgt_dev, sizeof(TargetEntry) * cap)) return e;
+        if (hipError_t e = hipMalloc((void **)&S->tgt_dev, sizeof(TargetEntry) * cap)) {
+            (void)hipGetLastError();
+            return e;
+        }
         S->tgt_cap_dev = cap;
     }
     TargetEntry *h = S->tgt_host[par];
@@ -361,6 +368,7 @@ void pack_results(md_server *S, const std::vector<std::shared_ptr<Request>> &end
         S->pack_cap[par] = 0;
         x = hipHostMalloc((void **)&S->pack_host[par], sizeof(PackEntry) * 2 * k, hipHostMallocDefault);
         if (x == hipSuccess) S->pack_cap[par] = 2 * k;
+        else (void)hipGetLastError();
     }
     if (x == hipSuccess) {
         int n = 0, blocks = 0;
@@ -688,6 +696,7 @@ extern "C" int md_server_add_mesh(md_server *S, md_mesh *m, int *mesh_id) {
     // md_server_wait / md_server_poll
     void *buf = nullptr;
     if (hipHostMalloc(&buf, 3 * sizeof(double) * (size_t)std::max(1, m->n), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
         set_error("md_server_add_mesh: pinned result buffer: allocation failed");
         return MD_ERR_NOMEM;
     }
