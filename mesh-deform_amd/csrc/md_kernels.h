@@ -247,7 +247,7 @@ struct UnpackArgs {
     unsigned long long *clear, *stamp;
 };
 void launch_unpack_xyz(hipStream_t s, const UnpackArgs &a, bool fp64);
-// Clock and *flag to pinned host memory.
+// Clock and *flag (may be null) to pinned host memory; nothing without a stamp.
 void launch_publish(hipStream_t s, unsigned long long *stamp, const int *flag, int *out);
 
 // Per-GPU device workspace of the non-allocating entry points (a static device array of

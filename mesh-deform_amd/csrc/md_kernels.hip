@@ -2578,7 +2578,7 @@ void launch_unpack_xyz(hipStream_t s, const UnpackArgs &a, bool fp64) {
     else hipLaunchKernelGGL(k_unpack_xyz<float>, dim3((a.n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, a);
 }
 void launch_publish(hipStream_t s, unsigned long long *stamp, const int *flag, int *out) {
-    hipLaunchKernelGGL(k_publish, dim3(1), dim3(1), 0, s, stamp, flag, out);
+    if (stamp) hipLaunchKernelGGL(k_publish, dim3(1), dim3(1), 0, s, stamp, flag, out);
 }
 
 void launch_pack_results(hipStream_t s, const PackEntry *e, int count, int blocks) {

@@ -48,8 +48,8 @@ CallSlot::CallSlot(md_ctx *c) : ctx_(c) {
     if (base_) *head() = Head{};
 }
 CallSlot::~CallSlot() {
-    if (!base_) return;
     if (queued) hipStreamSynchronize(ctx_->stream);
+    if (!base_) return;
     {
         std::lock_guard<std::mutex> g(ctx_->slot_mu);
         if (ctx_->slots.size() < kSlotsKept) {
@@ -833,12 +833,14 @@ hipError_t upload_positions(md_mesh *m, const double *xyz, d4 *p, d4 *pp, CallSl
     if (n == 0) return hipSuccess;
     if (slot.queued) MD_HIP_E(slot.wait());  // an earlier upload of the call may still read the block
     const size_t bytes = sizeof(double) * 3 * (size_t)n, tb = pp ? sizeof(double) * 3 * (size_t)(n - nf) : 0;
-    const bool staged = bytes + tb <= CallSlot::kStageBytes;
-    UnpackArgs a{m->d_xyz, m->d_internal, n, nf, m->d_tgt_xyz, p, pp, m->dev.quat, clear, &slot.head()->stamp[0]};
-    double *tgt = staged ? slot.data() + 3 * (size_t)n : slot.data();
-    if (tb > CallSlot::kStageBytes) {
+    const bool staged = bytes + tb <= slot.stage_bytes();
+    UnpackArgs a{m->d_xyz, m->d_internal, n, nf, m->d_tgt_xyz, p, pp, m->dev.quat, clear, slot.stamp(0)};
+    double *tgt = nullptr;
+    if (tb > slot.stage_bytes()) {
         m->tgt_stage.resize(3 * (size_t)(n - nf));
         tgt = m->tgt_stage.data();
+    } else if (tb) {
+        tgt = staged ? slot.data() + 3 * (size_t)n : slot.data();
     }
     slot.queued = true;
     if (staged) {
@@ -871,7 +873,7 @@ int download_packed(md_mesh *m, double *out, CallSlot &slot, const char *what, F
     };
     hipError_t e = hipSuccess;
     slot.queued = true;
-    if (bytes <= CallSlot::kStageBytes) {
+    if (slot.pinned() && bytes <= CallSlot::kStageBytes) {
         if (m->n > 0) fill(slot.data());
         e = hipGetLastError();
         if (e == hipSuccess) e = slot.wait();
@@ -914,14 +916,8 @@ int download_packed(md_mesh *m, double *out, CallSlot &slot, const char *what, F
 // Current positions to the caller's packed xyz (original order), packed on the device.
 template <class Arrived> int download_positions(md_mesh *m, double *xyz, CallSlot &slot, Arrived arrived) {
     return download_packed(m, xyz, slot, "position download", [&](double *dst) {
-        launch_pack_xyz(m->ctx->stream, m->dev.pp, m->d_internal, m->n, dst, &slot.head()->stamp[3]);
+        launch_pack_xyz(m->ctx->stream, m->dev.pp, m->d_internal, m->n, dst, slot.stamp(3));
     }, arrived);
-}
-
-int no_slot(const char *who) {
-    set_error(std::string(who) + ": pinned host block of " +
-              std::to_string(CallSlot::kHeadBytes + CallSlot::kStageBytes) + " bytes: allocation failed");
-    return MD_ERR_NOMEM;
 }
 
 // Cotan weights; with words (fac_ws_words), also the diagonal and its maximum for the factorization.
@@ -937,7 +933,7 @@ hipError_t compute_cotan(md_mesh *m, unsigned long long *words) {
 // With the PCG solver only the Jacobi diagonal is formed (queued on the device).
 int factor_pcg(md_mesh *m, CallSlot &slot) {
     const Plan &P = m->plan;
-    launch_publish(m->ctx->stream, &slot.head()->stamp[1], nullptr, nullptr);
+    launch_publish(m->ctx->stream, slot.stamp(1), nullptr, nullptr);
     launch_pcg_diag(m->ctx->stream, P.set(P.off_resid), P.blk_resid, m->fp64());
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) { set_error(std::string("PCG diagonal: ") + hipGetErrorString(e)); return MD_ERR_HIP; }
@@ -1084,7 +1080,7 @@ int factor_device(md_mesh *m, CallSlot &slot) {
     A.pc = const_cast<void *>(m->dev.pc);
     A.pr = const_cast<void *>(m->dev.pr);
     A.solve64 = m->fp64() ? 1 : 0;
-    A.stamp = &slot.head()->stamp[1];
+    A.stamp = slot.stamp(1);
     slot.queued = true;
     for (int h = 0; h < nh; ++h) {
         const HeightLaunch &L = hl[h];
@@ -1092,8 +1088,10 @@ int factor_device(md_mesh *m, CallSlot &slot) {
         launch_fac_height(st, A, f.hptr[h] + L.small, L.count, (L.mw + 63) / 64,
                           fac_assembly(L.count, L.mm, L.mo, L.maps), L.tiles);
     }
-    launch_publish(st, &slot.head()->stamp[2], A.flag, &slot.head()->flag);
-    if (hipError_t e = hipGetLastError(); e != hipSuccess) {
+    launch_publish(st, slot.stamp(2), A.flag, slot.flag());
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess && !slot.pinned()) e = hipMemcpyAsync(slot.flag(), A.flag, sizeof(int), hipMemcpyDeviceToHost, st);
+    if (e != hipSuccess) {
         slot.wait();
         m->release_fac_ws();
         set_error(std::string("device factorization: ") + hipGetErrorString(e));
@@ -1104,15 +1102,15 @@ int factor_device(md_mesh *m, CallSlot &slot) {
 
 // Result of a queued device factorization, after the stream has passed it. The workspace stays
 // with meshes that refactor on every deform call.
-int factor_finish(md_mesh *m, const CallSlot &slot) {
+int factor_finish(md_mesh *m, CallSlot &slot) {
     if (m->cfg.rest_mode != MD_REST_REFERENCE) m->release_fac_ws();
     m->factor_ms = slot.ms(1, 2);
-    if (slot.head()->flag == 1) {
+    if (*slot.flag() == 1) {
         set_error("factorization failed: a pivot block is not positive definite (a mesh component "
                   "without constraints?)");
         return MD_ERR_FACTOR;
     }
-    if (slot.head()->flag != 0) {
+    if (*slot.flag() != 0) {
         set_error("device factorization: inconsistent symbolic structure");
         return MD_ERR_INVALID;
     }
@@ -1210,12 +1208,12 @@ int prep_device_b(md_mesh *m, Prep &p, CallSlot &slot) {
     }
     if (int rc = pcg ? factor_pcg(m, slot) : factor_upload(m)) return rc;
     slot.queued = true;
-    launch_publish(m->ctx->stream, &slot.head()->stamp[2], nullptr, nullptr);
+    launch_publish(m->ctx->stream, slot.stamp(2), nullptr, nullptr);
     return MD_OK;
 }
 
 // After the stream has passed the queued work.
-int prep_finish(md_mesh *m, const Prep &p, const CallSlot &slot) {
+int prep_finish(md_mesh *m, const Prep &p, CallSlot &slot) {
     if (p.need_factor) {
         const bool device = m->cfg.solver == MD_SOLVER_LDLT && m->cfg.factor_device;
         const int rc = device ? factor_finish(m, slot) : MD_OK;
@@ -1265,7 +1263,6 @@ int setup_queue(md_mesh *m, const double *xyz, Prep &p, CallSlot &slot) {
 // The whole setup, waited for.
 int setup(md_mesh *m, const double *xyz, bool *early) {
     CallSlot slot(m->ctx);
-    if (!slot.ok()) return no_slot("setup");
     Prep p;
     int rc = setup_queue(m, xyz, p, slot);
     *early = p.early;
@@ -1664,7 +1661,6 @@ extern "C" int md_meshes_prepare(md_ctx *ctx, int count, md_mesh *const *meshes,
         }
     });
     CallSlot slot(ctx);  // one mesh at a time
-    if (!slot.ok()) return no_slot("md_meshes_prepare");
     for (int k = 0; k < nt; ++k) {
         int rc = prep_device_a(todo[k], preps[k], slot);
         prep_keep_rest(todo[k], preps[k]);
@@ -1711,7 +1707,6 @@ extern "C" int md_mesh_deform(md_mesh *m, int iterations, double *xyz, int *ok) 
     // everything is queued and waited for once: the setup, the iterations (arap.h:122-129) and the
     // packed positions; a factorization that failed leaves xyz untouched and the state that of the setup
     CallSlot slot(m->ctx);
-    if (!slot.ok()) return no_slot("md_mesh_deform");
     const bool dirty = m->dirty;
     Prep p;
     if (dirty) {
@@ -1738,7 +1733,7 @@ extern "C" int md_mesh_deform(md_mesh *m, int iterations, double *xyz, int *ok) 
         e = hipEventSynchronize(m->fac_ev);
         if (e != hipSuccess) { set_error(std::string("device factorization: ") + hipGetErrorString(e)); return MD_ERR_HIP; }
         // (a flag is reported by prep_finish below)
-        if (slot.head()->flag == 0 && (rc = iterate_queue(m, iterations - kIterationsAhead))) return rc;
+        if (*slot.flag() == 0 && (rc = iterate_queue(m, iterations - kIterationsAhead))) return rc;
     }
     double arrived_ms = 0.0;
     rc = download_positions(m, xyz, slot, [&]() -> int {  // write-back, arap.h:133-135
@@ -1786,7 +1781,6 @@ extern "C" int md_mesh_download(md_mesh *m, double *xyz) {
     hipSetDevice(m->ctx->device);
     if (int rc = ensure_resident(m, "md_mesh_download")) return rc;
     CallSlot slot(m->ctx);
-    if (!slot.ok()) return no_slot("md_mesh_download");
     return download_positions(m, xyz, slot, [] { return (int)MD_OK; });
 }
 
@@ -1873,7 +1867,6 @@ extern "C" int md_mesh_normals(md_mesh *m, double *nrm) {
     // face normals in the cotan step's per-face scratch (three doubles a face, rewritten whenever
     // weights are computed), vertex normals packed into the positions' device buffer: nothing is allocated
     CallSlot slot(m->ctx);
-    if (!slot.ok()) return no_slot("md_mesh_normals");
     const Plan &P = m->plan;
     return download_packed(m, nrm, slot, "md_mesh_normals", [&](double *dst) {
         launch_normals(m->ctx->stream, P.set(P.off_face), P.blk_face, P.set(P.off_slice), P.blk_slice, m->dev.fe_val,

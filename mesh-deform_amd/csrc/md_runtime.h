@@ -178,14 +178,17 @@ public:
     static constexpr size_t kStageBytes = size_t(5) << 18, kHeadBytes = 256;
     static constexpr size_t kSlotsKept = 4;
     explicit CallSlot(md_ctx *c);
-    ~CallSlot();  // waits for the stream if work of the call may still use the block
+    ~CallSlot();  // waits for the stream if work of the call may still use the block or the caller's buffers
     CallSlot(const CallSlot &) = delete;
     CallSlot &operator=(const CallSlot &) = delete;
-    bool ok() const { return base_ != nullptr; }
-    Head *head() const { return reinterpret_cast<Head *>(base_); }
+    // Without pinned memory for a block, the call copies through pageable memory and has no clocks.
+    bool pinned() const { return base_ != nullptr; }
+    size_t stage_bytes() const { return pinned() ? kStageBytes : 0; }
     double *data() const { return reinterpret_cast<double *>(base_ + kHeadBytes); }
+    int *flag() { return pinned() ? &head()->flag : &flag_; }
+    unsigned long long *stamp(int i) const { return pinned() ? &head()->stamp[i] : nullptr; }
     double ms(int from, int to) const {
-        return head()->stamp[to] > head()->stamp[from]
+        return pinned() && head()->stamp[to] > head()->stamp[from]
                    ? (double)(head()->stamp[to] - head()->stamp[from]) / ctx_->clock_khz : 0.0;
     }
     hipError_t wait() {
@@ -195,8 +198,10 @@ public:
     bool queued = false;
 
 private:
+    Head *head() const { return reinterpret_cast<Head *>(base_); }
     md_ctx *ctx_;
     char *base_ = nullptr;
+    int flag_ = 0;
 };
 }  // namespace md
 

@@ -360,17 +360,22 @@ void pack_results(md_server *S, const std::vector<std::shared_ptr<Request>> &end
     size_t k = 0;
     for (auto &r : ending) k += r->status == MD_OK;
     if (k == 0) return;
-    hipError_t x = hipSuccess;
     const int par = (int)(S->boundaries & 1);
     if (S->pack_cap[par] < k) {
         if (S->pack_host[par]) hipHostFree(S->pack_host[par]);
         S->pack_host[par] = nullptr;
         S->pack_cap[par] = 0;
-        x = hipHostMalloc((void **)&S->pack_host[par], sizeof(PackEntry) * 2 * k, hipHostMallocDefault);
-        if (x == hipSuccess) S->pack_cap[par] = 2 * k;
+        if (hipHostMalloc((void **)&S->pack_host[par], sizeof(PackEntry) * 2 * k, hipHostMallocDefault) == hipSuccess)
+            S->pack_cap[par] = 2 * k;
         else (void)hipGetLastError();
     }
-    if (x == hipSuccess) {
+    if (S->pack_cap[par] < k) {  // no pinned memory for the entries: a launch per result
+        for (auto &r : ending)
+            if (r->status == MD_OK) {
+                md_mesh *m = r->sm->m;
+                launch_pack_xyz(st, m->dev.pp, m->d_internal, m->n, m->d_xyz, nullptr);
+            }
+    } else {
         int n = 0, blocks = 0;
         for (auto &r : ending) {
             if (r->status != MD_OK) continue;
@@ -379,8 +384,8 @@ void pack_results(md_server *S, const std::vector<std::shared_ptr<Request>> &end
             blocks += (m->n + kBlock - 1) / kBlock;
         }
         launch_pack_results(st, S->pack_host[par], n, blocks);
-        x = hipGetLastError();
     }
+    const hipError_t x = hipGetLastError();
     if (x != hipSuccess)
         for (auto &r : ending)
             if (r->status == MD_OK) fail(*r, MD_ERR_HIP, std::string("packing the result: ") + hipGetErrorString(x));
