@@ -543,6 +543,21 @@ void sweep_levels(Factor& f, int sub_budget, std::vector<int>& sub_root, std::ve
 }
 }  // namespace
 
+void subtree_classes(const std::vector<SubSize>& meshes, std::vector<int>& cls) {
+    cls.assign(meshes.size(), 0);
+    long long all = 0;
+    for (const SubSize& m : meshes) all += m.nsub;
+    if (meshes.size() < 2 || all <= kSubFew) return;
+    int lowest = kSubClasses - 1;
+    for (size_t k = 0; k < meshes.size(); ++k) {
+        if (meshes[k].nsub == 0) continue;
+        while (cls[k] < kSubClasses - 1 && meshes[k].entries > kSubClassEntries[cls[k]]) ++cls[k];
+        lowest = std::min(lowest, cls[k]);
+    }
+    for (size_t k = 0; k < meshes.size(); ++k)
+        if (meshes[k].nsub == 0) cls[k] = lowest;
+}
+
 void device_layout(Factor& f, int sub_budget) {
     const int n = f.n, nn = f.ns;
     auto cdiv = [](int a, int b) { return (a + b - 1) / b; };

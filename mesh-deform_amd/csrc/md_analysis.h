@@ -205,6 +205,20 @@ std::vector<int> pair_levels(const std::vector<int>& order, const std::vector<in
                              int sub_budget, double amalg_ratio, int top_columns,
                              std::vector<int>& group);
 
+// LDS classes of the subtree launches of a plan of several meshes: entries up to kSubClassEntries[0] (about
+// budget 128), up to kSubClassEntries[1] (about 512), more. cls: a class per mesh. Every workgroup of a launch
+// gets the LDS of its largest subtree, which costs occupancy where the subtrees are more than run at once:
+// 45 meshes of 5k to 164k vertices with budgets tuned one by one (128 to 1024) take 0.77 ms per iteration in
+// one class, 0.69 in three. Up to kSubFew subtrees all run at once, and a further class is a further forward and
+// backward launch (8 meshes of 1k to 20k, 541 subtrees: 106 us an iteration in three classes, 70 in one), so
+// there is one; and a mesh without subtrees (level rows only) goes with the others.
+constexpr int kSubFew = 1024;
+constexpr int kSubClasses = 3, kSubClassEntries[kSubClasses - 1] = {192, 576};
+struct SubSize {
+    int nsub, entries;  // subtrees of a mesh, LDS vector entries of its largest
+};
+void subtree_classes(const std::vector<SubSize> &meshes, std::vector<int> &cls);
+
 // Device layout of a symbolic factor (partials, contribution lists, tiles, bottom subtrees)
 // for the given subtree budget; symbolic() calls it, and it may be called again to re-lay
 // the same structure out with another budget.

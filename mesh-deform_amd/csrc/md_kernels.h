@@ -154,18 +154,15 @@ void launch_bwd(hipStream_t s, LaunchSet L, int blocks, int level, bool fp64);
 // 12.5 / 11.1 us forward with the residual, 18.8 / 12.4 / 10.2 backward; 612 (FP32) 18.7 / 14.2 / 15.1 and
 // 20.8 / 14.8 / 12.2; 2,825 (FP64) 40 / 42 / 63 and 38 / 31 / 34; a batch's 7,413 (FP32, without the
 // residual) 38 / 34 / 47 and 57 / 59 / 80.
-// Launches over several meshes are split by the LDS of each mesh's largest subtree (kSubClassEntries,
-// about the budgets 128 and 512), since every workgroup of a launch gets the LDS of its largest: 45
-// meshes of 5k to 164k vertices with budgets tuned one by one (128 to 1024) 0.77 -> 0.69 ms per iteration.
-// The smallest class, whose subtrees are a supernode or two, takes 64 threads where they are many (the
+// Launches over several meshes are split by LDS class (subtree_classes), since every workgroup of a launch
+// gets the LDS of its largest subtree. The smallest class, whose subtrees are a supernode or two, takes 64 threads where they are many (the
 // same meshes all at 128: 0.75 -> 0.68 ms).
 // fused: the launch also forms the residual (one-mesh plans; blocks past the subtrees take
 // the level rows), else k_residual ran before it.
 struct SubLds {
     int block, nodes, heights, fwd, bwd, off;
 };
-constexpr int kSubBlock = 256, kSubFew = 1024;
-constexpr int kSubClasses = 3, kSubClassEntries[kSubClasses - 1] = {192, 576};
+constexpr int kSubBlock = 256;
 // Level rows per workgroup of the fused launch, past the subtrees (its threads).
 inline int sub_rows_fused(const SubLds &D) { return D.block == kSubBlock ? kSubBlock : 64; }
 void launch_sub_fwd(hipStream_t s, LaunchSet L, int blocks, const SubLds &D, bool fused, bool fp64);

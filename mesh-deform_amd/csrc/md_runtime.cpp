@@ -128,17 +128,15 @@ hipError_t build_plan(Plan &plan, const std::vector<const MeshDev *> &meshes,
           [&](int k) { return cdiv(meshes[k]->nslices_free, kSlicesPerBlock); });
     table(4, plan.off_apply, plan.blk_apply, [&](int k) { return cdiv(meshes[k]->nf, kBlock); });
     // bottom subtrees, by the LDS of their meshes' largest
-    auto lds_class = [&](int k) {
-        const int e = std::max(factors[k]->sub_lds_fwd, factors[k]->sub_lds_bwd);
-        int c = 0;
-        while (na > 1 && c < kSubClasses - 1 && e > kSubClassEntries[c]) ++c;
-        return c;
-    };
+    std::vector<SubSize> sizes;
+    for (const Factor *f : factors) sizes.push_back({f->nsub, std::max(f->sub_lds_fwd, f->sub_lds_bwd)});
+    std::vector<int> lds_class;
+    subtree_classes(sizes, lds_class);
     for (int c = 0; c < kSubClasses; ++c) {
         Plan::Subtrees &u = plan.sub[c];
         u = Plan::Subtrees{};
         for (int k = 0; k < na; ++k) {
-            if (lds_class(k) != c) continue;
+            if (lds_class[k] != c) continue;
             const Factor *f = factors[k];
             u.lds.fwd = std::max(u.lds.fwd, f->sub_lds_fwd);
             u.lds.bwd = std::max(u.lds.bwd, f->sub_lds_bwd);
@@ -146,10 +144,10 @@ hipError_t build_plan(Plan &plan, const std::vector<const MeshDev *> &meshes,
             u.lds.nodes = std::max(u.lds.nodes, f->sub_nodes);
             u.lds.heights = std::max(u.lds.heights, f->sub_heights);
         }
-        table(5 + 2 * c, u.off_fwd, u.blk_fwd, [&](int k) { return lds_class(k) == c ? factors[k]->nsub : 0; });
+        table(5 + 2 * c, u.off_fwd, u.blk_fwd, [&](int k) { return lds_class[k] == c ? factors[k]->nsub : 0; });
         u.lds.block = u.blk_fwd <= kSubFew ? kSubBlock : na > 1 && c == 0 ? 64 : 128;
         table(6 + 2 * c, u.off_bwd, u.blk_bwd, [&](int k) {
-            return lds_class(k) == c ? factors[k]->nsub + cdiv(meshes[k]->nlrows, u.lds.block) : 0;
+            return lds_class[k] == c ? factors[k]->nsub + cdiv(meshes[k]->nlrows, u.lds.block) : 0;
         });
     }
     table(3, plan.off_subf, plan.blk_subf,
