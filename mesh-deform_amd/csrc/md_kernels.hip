@@ -372,9 +372,20 @@ __host__ __device__ __forceinline__ void adj_column(const T (&a)[4][4], int col,
 // When that entry is small against |N|^3 the top eigenvalue is (nearly) repeated -- a rank-1
 // or reflection-ambiguous covariance -- the adjugate loses accuracy, and the warm-started
 // Jacobi sweeps decide instead. A zero covariance keeps the previous rotation.
+// The rotation does not depend on the covariance's scale, but the products on the way to it do, up to its
+// seventh power (FP32: past about 1e5 or below 1e-5 they leave the range): m is first scaled, exactly, by the
+// power of two that brings its largest entry into [0.5, 1).
 template <typename T>
-__host__ __device__ __forceinline__ bool best_rotation(const T (&m)[9], T px, T py, T pz, T pw, T &qx, T &qy, T &qz,
+__host__ __device__ __forceinline__ bool best_rotation(const T (&cov)[9], T px, T py, T pz, T pw, T &qx, T &qy, T &qz,
                                                        T &qw) {
+    T big = fabs(cov[0]);
+#pragma unroll
+    for (int i = 1; i < 9; ++i) big = fmax(big, fabs(cov[i]));
+    int e;
+    (void)frexp(big, &e);
+    T m[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) m[i] = ldexp(cov[i], -e);
     const T Sxx = m[0], Sxy = m[1], Sxz = m[2], Syx = m[3], Syy = m[4], Syz = m[5], Szx = m[6],
             Szy = m[7], Szz = m[8];
     const T f2 = Sxx * Sxx + Sxy * Sxy + Sxz * Sxz + Syx * Syx + Syy * Syy + Syz * Syz + Szx * Szx + Szy * Szy +
