@@ -90,7 +90,7 @@ struct Topology {
 // supernodes keep one partial of x_s (kr = 1); only the subtree root stores u_s (kc = 1,
 // the others kc = 0). Each supernode of a subtree has a 16-int record (SubNode layout:
 // c0, w, noff, forward front base, G offset, [Dinv; G] offset, contribution base, off-row
-// source base, u output or -1, x output, LDS column base of x, position / off-row / column
+// source base, u output or -1, x output, LDS column base of x, position (host emulation) / off-row / column
 // prefix within its height, 0, 0). Records of a subtree are contiguous and ordered by height; the
 // workgroup copies them to LDS and maps its items to supernodes by binary search over the
 // prefixes. LDS holds, forward, the fronts of the subtree's supernodes one after another in record

@@ -947,7 +947,7 @@ struct SubNode {
     int c0, w, noff, fb;     // columns, off rows, forward front base in LDS
     int pc, pr, cp, ob;      // G offset, [Dinv; G] offset, contribution entries, off-row sources
     int uo, xo, xs, pa;      // root: first update-slot entry (udst) or -1; x output, LDS column base
-                             //   of x, position prefix
+                             //   of x, position prefix (host emulation only)
     int pb, pq, pad0, pad1;  // off-row prefix, column prefix (within the height)
 };
 
@@ -1641,7 +1641,6 @@ __global__ __launch_bounds__(kBlock) void k_energy(LaunchSet L) {
     if (threadIdx.x == 0) M.energy_part[lb] = red[0];
 }
 
-// p'[iv[k]] = xyz[k] for k targets (internal ids), used to move handles without a re-setup.
 // The caller's packed xyz (original order, read in order: it may be pinned host memory) into
 // internal order: p[iv] (may be null), and pp[iv] (may be null) the same for free vertices, the constrained
 // ones (iv >= nf) taking their targets tgt[iv - nf] instead; with pp, identity rotations (arap.h:246-249).
@@ -1685,9 +1684,10 @@ __global__ __launch_bounds__(kBlock) void k_scatter_entries(const TargetEntry *e
 }
 
 // ---- numeric factorization (arap.h:337, SimplicialLDLT::compute) ------------------------
-// Multifrontal block LDL^T in FP64, one height of the supernodal tree at a time, one
-// workgroup per supernode. Every supernode's front lives in its own workspace blocks; the
-// children's update matrices are added in child order, so the factor is deterministic.
+// Multifrontal block LDL^T in FP64, one height of the supernodal tree at a time, each front by as many
+// workgroups as it has parts or tiles (small fronts by one). Every supernode's front lives in its own
+// workspace blocks; the children's update matrices are added in child order, so the factor is
+// deterministic.
 
 constexpr int kFacBlock = 256;
 
@@ -1723,7 +1723,7 @@ __device__ __forceinline__ FrontBuf front_buf(const FacArgs &A, const FacDev &S,
 // register and written once, so there is no zeroing, no read-modify-write and no barrier between
 // children. `per` workgroups per front, each `cols` columns (by rch ranges of rlen rows where one
 // child's inverse map would not fit); a wavefront takes four columns by 64 rows at a time, whose
-// children follow from one ballot, two children's entries (eight loads) in flight.
+// children follow from one ballot, three children's entries (kAsmAhead, twelve loads) in flight.
 // Bound by round trips (record, children, maps, entries): 7 us for a few fronts of 100 rows and 29 us a
 // height on average on the 164k icosphere, where scattering into the front in memory, child by child,
 // took 13 and 41.
@@ -2033,7 +2033,8 @@ static_assert(kFacBlock == 4 * 64, "four wavefronts");
 // callers outgrew the instruction cache, and its fetch was a third of a launch.
 // A chain of b pivots: per 16 of them 2,950 cycles of dependent FP64 arithmetic in the panel sweeps
 // (DPP and permlane broadcasts in place of LDS) and 1,900 for the exchange and the updates (one
-// v_mfma_f64_16x16x4 per 16 cycles and CU).
+// v_mfma_f64_16x16x4 per 16 cycles and CU): 19,400 for 64. As k_fac_inv0 runs it, its code not yet in the
+// instruction cache, 24,000 (10 us of the kernel's 15; loading the block takes 4, storing the inverse 0.7).
 __device__ __forceinline__ void invert64(const double *m, InvLds &work, int b, double thr, dv4 (&acc)[4], bool &bad) {
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
 #pragma unroll
@@ -2232,7 +2233,7 @@ __device__ __forceinline__ void block_put(bool below, const double (&v)[kTileVal
 // The last step of a front writes its panels: D^{-1} (minus the swept pivot block) and G. Tiles leave
 // through LDS, so one short loop stores every kind.
 // Bound by the chain of one tile per step: load, two products (1.7 us each at one MFMA per 16 cycles
-// and CU) and the inversion: 20 us a step of the 164k icosphere's top heights, whose other tiles
+// and CU) and the inversion (8 to 10): 20 us a step of the 164k icosphere's top heights, whose other tiles
 // run on CUs that the chain leaves idle. So the off rows and the update matrix are swept along: as
 // products after the sweeps (G = F D^{-1}, U -= G F^T, split over K) they took another 20 to 105 us a
 // height, waiting on their own chunks.
