@@ -320,8 +320,7 @@ def batched_leg(ctx, count, iters, seed, tune=True, baseline=True):
         return out
 
     # plain: each mesh with its own tuned sweep layout and the library's default factor shape
-    # (level pairs: fewer launches, the better choice for a mesh iterated alone), iterated alone
-    # back to back
+    # (level pairs: fewer launches, the better choice for a mesh iterated alone), back to back
     tune_plain_s, plain_s = 0.0, None
     if baseline:
         meshes = prepared(None)
