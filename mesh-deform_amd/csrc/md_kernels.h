@@ -155,8 +155,9 @@ void launch_bwd(hipStream_t s, LaunchSet L, int blocks, int level, bool fp64);
 // 20.8 / 14.8 / 12.2; 2,825 (FP64) 40 / 42 / 63 and 38 / 31 / 34; a batch's 7,413 (FP32, without the
 // residual) 38 / 34 / 47 and 57 / 59 / 80.
 // Launches over several meshes are split by LDS class (subtree_classes), since every workgroup of a launch
-// gets the LDS of its largest subtree. The smallest class, whose subtrees are a supernode or two, takes 64 threads where they are many (the
-// same meshes all at 128: 0.75 -> 0.68 ms).
+// gets the LDS of its largest subtree. The smallest class, whose subtrees are a supernode or two, takes 64
+// threads where they are many (45 meshes of 5k to 164k vertices all at budget 128: 0.75 -> 0.68 ms per
+// iteration).
 // fused: the launch also forms the residual (one-mesh plans; blocks past the subtrees take
 // the level rows), else k_residual ran before it.
 struct SubLds {
